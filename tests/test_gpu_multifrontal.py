@@ -76,6 +76,40 @@ def test_multifrontal_random_matrices(gpu):
     _check(n, A.indptr, A.indices, A.data, b)
 
 
+def _pattern(form):
+    """Small systems whose elimination trees are of every shape."""
+    rng = np.random.default_rng(11)
+    if form == "one":
+        return sp.csr_matrix([[2.0]])
+    if form == "diagonal":
+        return sp.diags(rng.uniform(1, 2, 200)).tocsr()
+    if form == "path":
+        return sp.diags([np.full(300, 4.0), np.full(299, 1.0), np.full(299, -1.0)], [0, 1, -1]).tocsr()
+    if form == "dense":
+        return sp.csr_matrix(rng.normal(size=(97, 97)) + 30 * np.eye(97))
+    if form == "star":
+        n = 700
+        A = sp.lil_matrix(np.diag(rng.uniform(4, 5, n)))
+        A[0, :] = rng.uniform(0.1, 1, n); A[:, 0] = rng.uniform(0.1, 1, n).reshape(-1, 1); A[0, 0] = 900.0
+        return A.tocsr()
+    if form == "two_parts":
+        L = sp.diags([np.full(40, 4.5), np.full(39, -1.0), np.full(39, -1.0)], [0, 1, -1])
+        G = sp.kron(L, sp.eye(40)) + sp.kron(sp.eye(40), L)
+        return sp.block_diag([G, G[:333, :333]]).tocsr()
+    n = 1500                                   # no locality: minimum degree is taken
+    r, c = rng.integers(0, n, 4 * n), rng.integers(0, n, 4 * n)
+    B = sp.coo_matrix((rng.normal(size=4 * n), (r, c)), shape=(n, n))
+    return (B + B.T + 25 * sp.eye(n)).tocsr()
+
+
+@pytest.mark.parametrize("form", ["one", "diagonal", "path", "dense", "star", "two_parts", "expander"])
+def test_multifrontal_pattern_forms(gpu, form):
+    A = _pattern(form)
+    A.sum_duplicates(); A.sort_indices()
+    b = np.random.default_rng(12).normal(size=A.shape[0])
+    _check(A.shape[0], A.indptr, A.indices, A.data, b)
+
+
 def test_multifrontal_singular_returns_status(gpu):
     rp = np.array([0, 2, 4, 6], np.int32)
     ci = np.array([0, 1, 0, 1, 1, 2], np.int32)

@@ -51,7 +51,7 @@ int xg_host_mf_plan(int n, const int* rowptr, const int* colind, const double* v
   xg::LuSymbolic s;
   xg::MfPlan p;
   try {
-    int st = xg::lu_analyse(n, rowptr, colind, values, s, false, true);
+    int st = xg::mf_analyse(n, rowptr, colind, values, s);
     if (st != XG_OK) return st;
     st = xg::mf_plan(s, rowptr, colind, p);
     if (st != XG_OK) return st;

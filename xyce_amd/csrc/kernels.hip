@@ -634,16 +634,20 @@ struct xg_lu {
 
   // symbolic analysis for the chosen (or automatically picked) method
   int analyse(const double* values, int want_method) {
+    const int n = (int)a_rowptr.size() - 1;
     LuSymbolic t;
-    int st = lu_analyse(s.n ? s.n : (int)a_rowptr.size() - 1, a_rowptr.data(), a_colind.data(), values, t, false, true);
-    if (st != XG_OK) return st;
-    const int n = t.n;
-    int m = want_method;
-    if (m == 0) m = (t.flops > 2e7 || n > 65535 || t.nlu > (1 << 24)) ? 2 : 1;
-    if (m == 1) {
-      st = lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true, false);
-      if (st != XG_OK) return st;
+    int m = want_method, st;
+    if (m == 0) {
+      m = 2;
+      if (n <= 65535) {
+        st = lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, false);
+        if (st != XG_OK) return st;
+        m = (t.flops > 2e7 || t.nlu > (1 << 24)) ? 2 : 1;
+      }
     }
+    st = m == 2 ? mf_analyse(n, a_rowptr.data(), a_colind.data(), values, t)
+                : lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
+    if (st != XG_OK) return st;
     s = std::move(t);
     method = m;
     return XG_OK;
@@ -686,7 +690,7 @@ struct xg_lu {
       const int rc = mfp->setup(s, a_rowptr.data(), a_colind.data(), (void*)stream, true);
       if (rc != XG_OK) return rc;
       // the plan holds what the kernels need; drop the host-side structure
-      std::vector<std::vector<int>>().swap(s.lcol);
+      for (auto* v : {&s.sfirst, &s.sparent, &s.srow_ptr, &s.srow, &s.rinv, &s.pinv}) std::vector<int>().swap(*v);
       have64 = false;
       return XG_OK;
     }

@@ -37,45 +37,30 @@ namespace xg {
 // ---------------------------------------------------------------------------
 int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p) {
   const int n = s.n;
-  if ((int)s.etree.size() != n || (int)s.lcol.size() != n) return XG_E_SETUP;
+  const int ns = (int)s.sfirst.size() - 1;
+  if (ns < 1 || (int)s.sparent.size() != ns || (int)s.srow_ptr.size() != ns + 1 || s.sfirst[ns] != n) return XG_E_SETUP;
   p = MfPlan();
   p.n = n;
-  const std::vector<int>& par = s.etree;
-  std::vector<int> nchild(n, 0);
-  for (int k = 0; k < n; ++k) if (par[k] >= 0) nchild[par[k]]++;
-  // fundamental supernodes: k joins k-1's supernode when k is k-1's parent,
-  // its only child, and the structures nest exactly
+  p.ns = ns;
+  p.sfirst = s.sfirst;
+  p.sparent = s.sparent;
   std::vector<int> snode(n);
-  p.sfirst.push_back(0);
-  for (int k = 0; k < n; ++k) {
-    const bool join = k > 0 && par[k - 1] == k && nchild[k] == 1 &&
-                      s.lcol[k - 1].size() == s.lcol[k].size() + 1;
-    if (!join && k > 0) p.sfirst.push_back(k);
-    snode[k] = (int)p.sfirst.size() - 1;
-  }
-  p.sfirst.push_back(n);
-  const int ns = p.ns = (int)p.sfirst.size() - 1;
-  // front index lists: pivots, then the last column's rows below
+  for (int t = 0; t < ns; ++t)
+    for (int k = p.sfirst[t]; k < p.sfirst[t + 1]; ++k) snode[k] = t;
+  // front index lists: pivots, then the rows below
   p.iptr.assign(ns + 1, 0);
   p.m.resize(ns);
   for (int t = 0; t < ns; ++t) {
-    const int last = p.sfirst[t + 1] - 1;
-    p.m[t] = (p.sfirst[t + 1] - p.sfirst[t]) + (int)s.lcol[last].size();
+    p.m[t] = (p.sfirst[t + 1] - p.sfirst[t]) + (s.srow_ptr[t + 1] - s.srow_ptr[t]);
     p.iptr[t + 1] = p.iptr[t] + p.m[t];
     p.max_m = std::max<long long>(p.max_m, p.m[t]);
+    if (p.sparent[t] >= 0 && p.sparent[t] <= t) return XG_E_SETUP;
   }
   p.idx.resize(p.iptr[ns]);
   for (int t = 0; t < ns; ++t) {
     int q = p.iptr[t];
     for (int c = p.sfirst[t]; c < p.sfirst[t + 1]; ++c) p.idx[q++] = c;
-    for (int r : s.lcol[p.sfirst[t + 1] - 1]) p.idx[q++] = r;
-  }
-  // parents, children, levels
-  p.sparent.assign(ns, -1);
-  for (int t = 0; t < ns; ++t) {
-    const int pk = par[p.sfirst[t + 1] - 1];
-    p.sparent[t] = pk >= 0 ? snode[pk] : -1;
-    if (p.sparent[t] >= 0 && p.sparent[t] <= t) return XG_E_SETUP;
+    for (int r = s.srow_ptr[t]; r < s.srow_ptr[t + 1]; ++r) p.idx[q++] = s.srow[r];
   }
   p.cptr.assign(ns + 1, 0);
   for (int t = 0; t < ns; ++t) if (p.sparent[t] >= 0) p.cptr[p.sparent[t] + 1]++;
@@ -87,7 +72,7 @@ int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p
   }
   std::vector<int> lvl(ns, 0);
   int maxl = 0;
-  for (int t = 0; t < ns; ++t) {       // children come before parents (postorder numbering)
+  for (int t = 0; t < ns; ++t) {       // children come before parents
     for (int c = p.cptr[t]; c < p.cptr[t + 1]; ++c) lvl[t] = std::max(lvl[t], lvl[p.clist[c]] + 1);
     maxl = std::max(maxl, lvl[t]);
   }

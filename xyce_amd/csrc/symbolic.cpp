@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <cmath>
 #include <deque>
+#include <future>
 #include <numeric>
 #include <stdexcept>
 
@@ -290,8 +291,11 @@ int etree_height(const Graph& g, const std::vector<int>& order) {
 // ordered recursively, then the separator.  Parts of at most `leaf` nodes get
 // approximate minimum degree.  Gives a shallow elimination tree (about
 // log2(n / leaf) separator levels) where minimum degree leaves long chains.
+//
+// widest (may be null): the largest separator, relative to the square root of
+// the part it divides.
 void nd_order(const Graph& g, std::vector<int> nodes, std::vector<int>& order, int leaf, std::vector<int>& tag,
-              int& stamp, std::vector<int>& lvl) {
+              int& stamp, std::vector<int>& lvl, double* widest = nullptr) {
   if ((int)nodes.size() <= leaf) { amd_order(g, nodes, order); return; }
   const int id = ++stamp;
   for (int v : nodes) tag[v] = id;
@@ -328,8 +332,8 @@ void nd_order(const Graph& g, std::vector<int> nodes, std::vector<int>& order, i
     std::vector<int> rest;
     for (int v : seq) tag[v] = -id;
     for (int v : nodes) if (tag[v] == id) rest.push_back(v);
-    nd_order(g, seq, order, leaf, tag, stamp, lvl);
-    nd_order(g, rest, order, leaf, tag, stamp, lvl);
+    nd_order(g, seq, order, leaf, tag, stamp, lvl, widest);
+    nd_order(g, rest, order, leaf, tag, stamp, lvl, widest);
     return;
   }
   const int nl = (int)lptr.size() - 1;
@@ -352,19 +356,15 @@ void nd_order(const Graph& g, std::vector<int> nodes, std::vector<int>& order, i
     for (int a : g[v]) if (tag[a] == id && lvl[a] == sep + 1) { beyond = true; break; }
     (beyond ? S : A).push_back(v);
   }
-  nd_order(g, std::move(A), order, leaf, tag, stamp, lvl);
-  nd_order(g, std::move(B), order, leaf, tag, stamp, lvl);
+  if (widest) *widest = std::max(*widest, (double)S.size() / std::sqrt((double)seq.size()));
+  nd_order(g, std::move(A), order, leaf, tag, stamp, lvl, widest);
+  nd_order(g, std::move(B), order, leaf, tag, stamp, lvl, widest);
   amd_order(g, S, order);
 }
 
-}  // namespace
-
-int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s, bool want_schedule,
-               bool keep_tree) {
-  s = LuSymbolic();
-  s.n = n; s.nnz_a = rowptr[n];
-  std::vector<int> match = max_transversal(n, rowptr, colind, values);  // A'(c,:) = A(match[c],:)
-  // A' pattern (row c of A' = row match[c] of A), symmetrised
+// A' = the rows of A permuted to the transversal's diagonal, symmetrised;
+// dense rows (beyond 10 sqrt(n)) apart, as AMD treats them
+Graph symmetric_graph(int n, const int* rowptr, const int* colind, const std::vector<int>& match) {
   Graph g(n);
   for (int c = 0; c < n; ++c) {
     const int r = match[c];
@@ -374,10 +374,257 @@ int lu_analyse(int n, const int* rowptr, const int* colind, const double* values
     }
   }
   for (auto& v : g) { std::sort(v.begin(), v.end()); v.erase(std::unique(v.begin(), v.end()), v.end()); }
-  // dense nodes last
+  return g;
+}
+
+void split_dense(const Graph& g, std::vector<int>& sparse_nodes, std::vector<int>& dense_nodes) {
+  const int n = (int)g.size();
   const int dense_thresh = std::max(16, (int)(10.0 * std::sqrt((double)n)));
-  std::vector<int> sparse_nodes, dense_nodes;
   for (int v = 0; v < n; ++v) ((int)g[v].size() > dense_thresh ? dense_nodes : sparse_nodes).push_back(v);
+}
+
+// ---- supernode tree of an elimination order (multifrontal analysis)
+struct SuperTree {
+  std::vector<int> order;            // elimination order (graph nodes), fronts contiguous
+  std::vector<int> sfirst, sparent, srow_ptr, srow;
+  double nnz = 0, flops = 0;         // of L+U and of the factorisation, padding included
+  double cost = 0;                   // modelled time of a refactor and a solve (us)
+};
+
+// Fronts whose merger with their parent stays within kMergeOrder rows, or
+// whose merger adds at most kMergeFill of explicit zeros to the merged pivot
+// columns, are merged (relaxed supernodes): a front costs a launch slot and a
+// tree level a chain of launches, which a few padded entries do not.
+constexpr int kMergeOrder = 32;
+constexpr double kMergeFill = 0.1;
+// cost model (us): a tree level's launches in refactor and solve, a 32-column
+// panel step, a GFLOP, a million front elements
+constexpr double kCostLevel = 40.0, kCostStep = 14.0, kCostGflop = 350.0, kCostMelem = 12.0;
+constexpr int kSmallFront = 64;      // orders up to this are factored by one wavefront
+
+SuperTree build_tree(const Graph& g, const std::vector<int>& order0) {
+  const int n = (int)order0.size();
+  SuperTree T;
+  std::vector<int> order(n), pos(n), parent(n, -1);
+  {
+    // elimination tree (Liu) of order0, then its postorder: the same fill,
+    // with the columns of a supernode next to each other
+    std::vector<int> par(n, -1), anc(n, -1), head(n, -1), next(n, -1), post;
+    for (int i = 0; i < n; ++i) pos[order0[i]] = i;
+    for (int i = 0; i < n; ++i)
+      for (int a : g[order0[i]]) {
+        int k = pos[a];
+        while (k != -1 && k < i) {
+          const int nx = anc[k];
+          anc[k] = i;
+          if (nx == -1) { par[k] = i; break; }
+          k = nx;
+        }
+      }
+    for (int i = n - 1; i >= 0; --i)
+      if (par[i] >= 0) { next[i] = head[par[i]]; head[par[i]] = i; }
+    post.reserve(n);
+    std::vector<int> stk;
+    for (int r = 0; r < n; ++r) {
+      if (par[r] >= 0) continue;
+      stk.push_back(r);
+      while (!stk.empty()) {
+        const int v = stk.back();
+        if (head[v] >= 0) { stk.push_back(head[v]); head[v] = next[head[v]]; }
+        else { post.push_back(v); stk.pop_back(); }
+      }
+    }
+    std::vector<int> where(n);
+    for (int i = 0; i < n; ++i) { where[post[i]] = i; order[i] = order0[post[i]]; }
+    for (int i = 0; i < n; ++i) if (par[i] >= 0) parent[where[i]] = where[par[i]];
+    for (int i = 0; i < n; ++i) pos[order[i]] = i;
+  }
+  // column structures (rows below the diagonal, unsorted) from A and the children's
+  std::vector<int> head(n, -1), next(n, -1), nchild(n, 0), mark(n, -1);
+  for (int i = n - 1; i >= 0; --i)
+    if (parent[i] >= 0) { next[i] = head[parent[i]]; head[parent[i]] = i; ++nchild[parent[i]]; }
+  std::vector<std::vector<int>> L(n);
+  for (int k = 0; k < n; ++k) {
+    mark[k] = k;
+    for (int a : g[order[k]]) {
+      const int i = pos[a];
+      if (i > k && mark[i] != k) { mark[i] = k; L[k].push_back(i); }
+    }
+    for (int c = head[k]; c >= 0; c = next[c])
+      for (int i : L[c])
+        if (mark[i] != k) { mark[i] = k; L[k].push_back(i); }
+  }
+  // fundamental supernodes: k joins k-1's when k is its parent, k-1 its only
+  // child, and the structures nest exactly
+  std::vector<int> first, snode(n);
+  for (int k = 0; k < n; ++k) {
+    const bool join = k > 0 && parent[k - 1] == k && nchild[k] == 1 && L[k - 1].size() == L[k].size() + 1;
+    if (!join) first.push_back(k);
+    snode[k] = (int)first.size() - 1;
+  }
+  first.push_back(n);
+  const int nf = (int)first.size() - 1;
+  // relaxed amalgamation, children before parents: each front merges the
+  // child that adds the fewest zeros while that is allowed
+  std::vector<int> np(nf), m(nf), par(nf, -1), into(nf);
+  std::vector<double> zeros(nf, 0.0);
+  std::vector<std::vector<int>> kids(nf);
+  for (int t = 0; t < nf; ++t) {
+    const int last = first[t + 1] - 1;
+    np[t] = first[t + 1] - first[t];
+    m[t] = np[t] + (int)L[last].size();
+    into[t] = t;
+    if (parent[last] >= 0) { par[t] = snode[parent[last]]; kids[par[t]].push_back(t); }
+  }
+  for (int t = 0; t < nf; ++t) {
+    std::vector<int>& cs = kids[t];
+    for (;;) {
+      int best = -1;
+      double bz = 0.0;
+      for (int i = 0; i < (int)cs.size(); ++i) {
+        const int c = cs[i];
+        const double z = (double)np[c] * (np[c] + m[t] - m[c]);
+        if (best < 0 || z < bz) { best = i; bz = z; }
+      }
+      if (best < 0) break;
+      const int c = cs[best];
+      const int mm = np[c] + m[t], pp = np[c] + np[t];
+      const double z = bz + zeros[c] + zeros[t];
+      if (mm > kMergeOrder && z > kMergeFill * (double)pp * mm) break;
+      cs[best] = cs.back();
+      cs.pop_back();
+      cs.insert(cs.end(), kids[c].begin(), kids[c].end());
+      std::vector<int>().swap(kids[c]);
+      into[c] = t;
+      np[t] = pp; m[t] = mm; zeros[t] = z;
+    }
+  }
+  // fronts in postorder of the merged tree, their pivots contiguous
+  std::vector<int> rep(nf), front(nf, -1);
+  for (int t = nf - 1; t >= 0; --t) rep[t] = into[t] == t ? t : rep[into[t]];
+  std::vector<std::vector<int>> members(nf);
+  for (int t = 0; t < nf; ++t) members[rep[t]].push_back(t);   // ascending: a child's columns before its parent's
+  T.order.reserve(n);
+  T.sfirst.push_back(0);
+  T.srow_ptr.push_back(0);
+  std::vector<int> newpos(n), stk, top, level;
+  for (int r = 0; r < nf; ++r) {
+    if (into[r] != r || par[r] >= 0) continue;
+    stk.push_back(r);
+    while (!stk.empty()) {
+      const int t = stk.back();
+      if (!kids[t].empty()) { stk.push_back(kids[t].back()); kids[t].pop_back(); continue; }
+      stk.pop_back();
+      front[t] = (int)top.size();
+      top.push_back(t);
+      for (int q : members[t])
+        for (int k = first[q]; k < first[q + 1]; ++k) { newpos[k] = (int)T.order.size(); T.order.push_back(order[k]); }
+      T.sfirst.push_back((int)T.order.size());
+    }
+  }
+  const int ns = (int)top.size();
+  T.sparent.assign(ns, -1);
+  level.assign(ns, 0);
+  int nl = 0;
+  for (int s = 0; s < ns; ++s) {
+    const int t = top[s];
+    if (par[t] >= 0) T.sparent[s] = front[rep[par[t]]];
+    const size_t b = T.srow.size();
+    for (int i : L[first[t + 1] - 1]) T.srow.push_back(newpos[i]);
+    std::sort(T.srow.begin() + b, T.srow.end());
+    T.srow_ptr.push_back((int)T.srow.size());
+    nl = std::max(nl, level[s] + 1);
+    if (T.sparent[s] >= 0) level[T.sparent[s]] = std::max(level[T.sparent[s]], level[s] + 1);
+  }
+  std::vector<int> maxp(nl, 0);
+  double elems = 0;
+  for (int s = 0; s < ns; ++s) {
+    const double p = T.sfirst[s + 1] - T.sfirst[s], mm = p + (T.srow_ptr[s + 1] - T.srow_ptr[s]);
+    if (mm > kSmallFront) maxp[level[s]] = std::max(maxp[level[s]], (int)p);
+    elems += mm * mm;
+    T.nnz += 2.0 * mm * p - p * p;
+    for (double k = 0; k < p; ++k) T.flops += 2.0 * (mm - k - 1) * (mm - k - 1) + (mm - k - 1);
+  }
+  T.cost = kCostLevel * nl + kCostGflop * T.flops * 1e-9 + kCostMelem * elems * 1e-6;
+  for (int l = 0; l < nl; ++l) T.cost += kCostStep * ((maxp[l] + 31) / 32);
+  return T;
+}
+
+}  // namespace
+
+// The order is the one whose tree the GPU is expected to factor and solve
+// soonest: nested dissection down to 64 or to 1024 nodes, or minimum degree.
+// On meshes and locally wired gate arrays dissection has the shallower tree
+// and also less fill on large meshes (512 x 512 nodes: 2.6 GFLOP and 19 levels
+// against 5.8 and 34), so minimum degree is tried only on small systems or when a
+// separator is wide for its part (no locality: an expander fills in less
+// under minimum degree).
+int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s) {
+  s = LuSymbolic();
+  s.n = n; s.nnz_a = rowptr[n];
+  const std::vector<int> match = max_transversal(n, rowptr, colind, values);
+  const Graph g = symmetric_graph(n, rowptr, colind, match);
+  std::vector<int> sparse_nodes, dense_nodes;
+  split_dense(g, sparse_nodes, dense_nodes);
+  // the candidates on host threads of their own
+  auto finish = [&](std::vector<int>& order) {
+    if (order.size() != sparse_nodes.size()) return SuperTree();
+    order.insert(order.end(), dense_nodes.begin(), dense_nodes.end());
+    return build_tree(g, order);
+  };
+  double widest = 0.0;
+  auto dissect = [&](int leaf, double* wide) {
+    std::vector<int> order, tag(n, 0), lvl(n, 0);
+    int stamp = 0;
+    order.reserve(n);
+    nd_order(g, sparse_nodes, order, leaf, tag, stamp, lvl, wide);
+    return finish(order);
+  };
+  auto min_degree = [&] {
+    std::vector<int> order;
+    order.reserve(n);
+    amd_order(g, sparse_nodes, order);
+    return finish(order);
+  };
+  const int m = (int)sparse_nodes.size();
+  SuperTree best;
+  auto consider = [&](SuperTree t) {
+    if (!t.order.empty() && (best.order.empty() || t.cost < best.cost)) best = std::move(t);
+  };
+  if (m > 64) {
+    std::future<SuperTree> coarse;
+    if (m > 1024) coarse = std::async(std::launch::async, dissect, 1024, (double*)nullptr);
+    consider(dissect(64, &widest));
+    if (coarse.valid()) consider(coarse.get());
+  }
+  if (best.order.empty() || m <= 8192 || widest > 3.0) consider(min_degree());
+  if (best.order.empty()) return XG_E_SETUP;
+  s.dense_tail = (int)dense_nodes.size();
+  s.perm_row.resize(n); s.perm_col.resize(n); s.rinv.resize(n); s.pinv.resize(n);
+  for (int i = 0; i < n; ++i) {
+    s.perm_col[i] = best.order[i];
+    s.perm_row[i] = match[best.order[i]];
+    s.pinv[best.order[i]] = i;
+    s.rinv[s.perm_row[i]] = i;
+  }
+  s.nlu = (int)std::min(best.nnz, 2147483647.0);
+  s.flops = best.flops;
+  s.sfirst = std::move(best.sfirst);
+  s.sparent = std::move(best.sparent);
+  s.srow_ptr = std::move(best.srow_ptr);
+  s.srow = std::move(best.srow);
+  return XG_OK;
+}
+
+
+int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s, bool want_schedule) {
+  s = LuSymbolic();
+  s.n = n; s.nnz_a = rowptr[n];
+  std::vector<int> match = max_transversal(n, rowptr, colind, values);  // A'(c,:) = A(match[c],:)
+  // A' pattern (row c of A' = row match[c] of A), symmetrised; dense nodes last
+  Graph g = symmetric_graph(n, rowptr, colind, match);
+  std::vector<int> sparse_nodes, dense_nodes;
+  split_dense(g, sparse_nodes, dense_nodes);
   std::vector<int> order;
   order.reserve(n);
   // small systems (the batched engine's classes): multiple minimum degree,
@@ -475,12 +722,6 @@ int lu_analyse(int n, const int* rowptr, const int* colind, const double* values
     double fl = 0;
     for (int k = 0; k < n; ++k) fl += 2.0 * (double)urow[k].size() * (double)urow[k].size() + (double)urow[k].size();
     s.flops = fl;
-  }
-  if (keep_tree) {
-    s.etree = parent;
-    s.lcol = urow;
-    s.rinv = rinv;
-    s.pinv = pinv;
   }
   if (!want_schedule) return XG_OK;
 

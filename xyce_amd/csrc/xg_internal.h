@@ -93,15 +93,14 @@ struct LuSymbolic {
   std::vector<int> bs_lvl_ptr, bs_rows;   // backward
   double flops = 0;
   int dense_tail = 0;
-  // elimination tree and column structure of L (rows below the diagonal,
-  // ascending) of B, kept when the multifrontal plan is wanted
-  std::vector<int> etree;
-  std::vector<std::vector<int>> lcol;
-  std::vector<int> rinv, pinv;   // A row -> B row, A col -> B col
+  std::vector<int> rinv, pinv;   // A row -> B row, A col -> B col (multifrontal analysis)
+  // supernode tree of the multifrontal analysis: front t eliminates the
+  // columns [sfirst[t], sfirst[t+1]) of B; its rows below them (ascending) are
+  // srow[srow_ptr[t] .. srow_ptr[t+1]); children come before parents
+  std::vector<int> sfirst, sparent, srow_ptr, srow;
 };
 
-// want_schedule: build the entry-level factor / solve schedules;
-// keep_tree: keep the elimination tree and the L column structure
+// want_schedule: build the entry-level factor / solve schedules
 // A square CSR pattern the symbolic analysis can read: rowptr[0] = 0,
 // non-decreasing, every column index in [0, n).
 inline bool valid_csr(int n, const int* rowptr, const int* colind) {
@@ -114,7 +113,11 @@ inline bool valid_csr(int n, const int* rowptr, const int* colind) {
 }
 
 int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s,
-               bool want_schedule = true, bool keep_tree = false);
+               bool want_schedule = true);
+
+// Analysis for the multifrontal method: permutations and the supernode tree
+// (s.nlu and s.flops are those of the tree's fronts)
+int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s);
 
 // Multifrontal plan of a symbolic analysis (multifrontal.hip)
 struct MfPlan {
