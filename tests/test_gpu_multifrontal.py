@@ -110,6 +110,43 @@ def test_multifrontal_pattern_forms(gpu, form):
     _check(A.shape[0], A.indptr, A.indices, A.data, b)
 
 
+def _coupled_blocks(sizes, sep, seed):
+    """Dense blocks coupled through a dense separator: fronts of order
+    size + sep with size pivots, then one of order sep."""
+    rng = np.random.default_rng(seed)
+    n = sum(sizes) + sep
+    M = np.zeros((n, n))
+    k = 0
+    for m in sizes:
+        M[k:k + m, k:k + m] = rng.normal(size=(m, m))
+        M[k:k + m, n - sep:] = rng.normal(size=(m, sep))
+        M[n - sep:, k:k + m] = rng.normal(size=(sep, m))
+        k += m
+    M[n - sep:, n - sep:] = rng.normal(size=(sep, sep))
+    return sp.csr_matrix(M + 3.0 * np.sqrt(n) * np.eye(n))
+
+
+@pytest.mark.parametrize("sizes,sep", [((65,), 1), ((64, 64), 1), ((33, 31, 32), 33), ((96, 97), 32), ((95, 34), 64),
+                                       ((128, 1), 65), ((66, 160), 97), ((300,), 129)])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_multifrontal_front_edges(gpu, sizes, sep, fp32):
+    """Front orders and pivot counts around the panel width (32) and the tile
+    sizes (64, 96) of the blocked factorisation."""
+    A = _coupled_blocks(sizes, sep, 17)
+    A.sort_indices()
+    n = A.shape[0]
+    b = np.random.default_rng(18).normal(size=n)
+    if not fp32:
+        _check(n, A.indptr, A.indices, A.data, b)
+        return
+    s = X.DirectSolver(n, A.indptr, A.indices, method=2)
+    s.set_precision(1, ir_tol=1e-12, ir_max=10)
+    st, x = s.doSolve(A.data, b)
+    ps = s.precision_stats()
+    assert st == 0 and ps["fp64_fallbacks"] == 0 and ps["fp32_pivot_failures"] == 0
+    assert np.max(np.abs(A @ x - b)) <= 1e-12 * np.max(np.abs(b))
+
+
 def test_multifrontal_singular_returns_status(gpu):
     rp = np.array([0, 2, 4, 6], np.int32)
     ci = np.array([0, 1, 0, 1, 1, 2], np.int32)

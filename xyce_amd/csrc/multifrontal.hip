@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 #include <stdexcept>
+#include <type_traits>
 #include <vector>
 
 #include "xg_internal.h"
@@ -154,8 +155,17 @@ struct MfDev {
 
 constexpr int kMfTiny = 64;     // fronts up to this order: one wavefront, the front in LDS
 constexpr int kMfPanel = 32;    // panel width of the blocked factorisation (64 spills the register panel)
-constexpr int kMfRowsPerLoad = 64 / kMfPanel;   // L21 rows a 64-lane load covers
 constexpr int kMfSolveBlock = 1024;
+
+// f(0), f(1), ... f(N - 1) with the index a constant in each
+template <int N, int K = 0, class F>
+__device__ __forceinline__ void mf_for(const F& f) {
+  if constexpr (K < N) {
+    f(std::integral_constant<int, K>{});
+    mf_for<N, K + 1>(f);
+  }
+}
+#define MF_INLINE __attribute__((always_inline))
 
 template <class T>
 __global__ void k_mf_fill(T* F, long long total) {
@@ -352,140 +362,34 @@ __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list,
   if (hard && t == 0) atomicOr(bad + 1, 1);
 }
 
-// larger fronts, blocked by panels of kMfPanel columns; all fronts of a level
-// in one launch per panel index (entries {front, block, dbuf slot, 0}).
-// (1) every workgroup (one wavefront) factors the pw x pw diagonal block in
-// registers (lane t owns row t, the pivot row broadcast across lanes), then
-// solves a 64-row block of L21 (x U11 = row) or a 64-column block of U12
-// (L11 x = column).  Block 0 also stores the block's factors in its dbuf
-// slot; the update launch copies them into the front (the front's other
-// workgroups may still be reading the unfactored block).
-template <class T>
-__global__ void __launch_bounds__(64) k_mf_panel(MfDev d, const int4* ent, int p0, T* F, T* dbuf, int* bad) {
-  __shared__ T D[kMfPanel][kMfPanel + 1];
-  __shared__ T Rd[kMfPanel];
-  __shared__ T Tl[64][kMfPanel + 1];
-  const int4 e = ent[blockIdx.x];
-  const int s = e.x, blk = e.y, slot = e.z;
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const int pw = min(kMfPanel, np - p0);
-  const int base = p0 + pw, rest = ms - base, nrb = (rest + 63) / 64;
-  T* Fs = F + d.fo[s];
-  const int t = threadIdx.x;
-  T r[kMfPanel];
-#pragma unroll
-  for (int q = 0; q < kMfPanel; ++q)
-    r[q] = (t < pw && q < pw) ? Fs[(long long)(p0 + t) * ms + p0 + q] : (T)0;
-  // (loops keep constant trip counts so that the register arrays stay
-  // register-resident after full unrolling)
-  bool fail = false, stop = false;
-#pragma unroll
-  for (int k = 0; k < kMfPanel; ++k) {
-    if (k < pw && !stop) {
-      const T piv = mf_bcast(r[k], k);
-      if (mf_bad_pivot(piv)) {
-        fail = true;
-        stop = true;
-      } else {
-        const bool upd = t > k && t < pw;
-        const T l = upd ? r[k] / piv : (T)0;
-        if (upd) {
-          r[k] = l;
-          if (!(fabs((double)l) <= 1.0e3)) fail = true;
-        }
-#pragma unroll
-        for (int q = 0; q < kMfPanel; ++q) {
-          if (q > k) {
-            const T u = mf_bcast(r[q], k);
-            if (upd) r[q] -= l * u;
-          }
-        }
-      }
-    }
-  }
-  if (t < kMfPanel) {
-#pragma unroll
-    for (int q = 0; q < kMfPanel; ++q) D[t][q] = r[q];
-    // pivot reciprocals, all at once: the row solves below multiply
-    Rd[t] = t < pw ? (T)1 / D[t][t] : (T)0;
-  }
-  __syncthreads();
-  if (blk == 0) {
-    T* db = dbuf + (long long)slot * kMfPanel * kMfPanel;
-    for (int i = 0; i < pw; ++i)
-      if (t < pw) db[i * kMfPanel + t] = D[i][t];
-  }
-  if (rest > 0 && blk < nrb) {
-    // L21 rows [r0, r0 + 64), staged through LDS for coalesced access
-    const int r0 = base + blk * 64;
-    {
-      // all loads issued before the LDS stores (one wait, not one per row)
-      T v[kMfPanel];
-#pragma unroll
-      for (int it = 0; it < kMfPanel; ++it) {
-        const int rr = t / kMfPanel + kMfRowsPerLoad * it, q = t % kMfPanel;
-        v[it] = (r0 + rr < ms && q < pw) ? Fs[(long long)(r0 + rr) * ms + p0 + q] : (T)0;
-      }
-#pragma unroll
-      for (int it = 0; it < kMfPanel; ++it) Tl[t / kMfPanel + kMfRowsPerLoad * it][t % kMfPanel] = v[it];
-    }
-    __syncthreads();
-    T a[kMfPanel];
-#pragma unroll
-    for (int q = 0; q < kMfPanel; ++q) a[q] = Tl[t][q];
-    const bool valid = r0 + t < ms;
-#pragma unroll
-    for (int k = 0; k < kMfPanel; ++k) {
-      if (k < pw) {
-        a[k] = a[k] * Rd[k];
-        if (valid && !(fabs((double)a[k]) <= 1.0e3)) fail = true;
-#pragma unroll
-        for (int q = 0; q < kMfPanel; ++q)
-          if (q > k) a[q] -= a[k] * D[k][q];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kMfPanel; ++q) Tl[t][q] = a[q];
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < kMfPanel; ++it) {
-      const int rr = t / kMfPanel + kMfRowsPerLoad * it, q = t % kMfPanel;
-      if (r0 + rr < ms && q < pw) Fs[(long long)(r0 + rr) * ms + p0 + q] = Tl[rr][q];
-    }
-  } else if (rest > 0) {
-    // U12 columns [c0, c0 + 64): lane t owns column c0 + t
-    const int c = base + (blk - nrb) * 64 + t;
-    const bool valid = c < ms;
-    T b[kMfPanel];
-#pragma unroll
-    for (int q = 0; q < kMfPanel; ++q) b[q] = (valid && q < pw) ? Fs[(long long)(p0 + q) * ms + c] : (T)0;
-#pragma unroll
-    for (int k = 0; k < kMfPanel; ++k) {
-      if (k < pw) {
-#pragma unroll
-        for (int q = 0; q < kMfPanel; ++q)
-          if (q > k) b[q] -= D[q][k] * b[k];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kMfPanel; ++q)
-      if (valid && q < pw) Fs[(long long)(p0 + q) * ms + c] = b[q];
-  }
-  if (__any(fail) && t == 0) atomicMin(bad, d.sfirst[s] + p0 + 1);
-  if (__any(stop) && t == 0) atomicOr(bad + 1, 1);
-}
-
-// (2) trailing update F[i][j] -= sum_q L[i][q] U[q][j], i, j >= p0 + pw, one
-// 64x64 tile per workgroup (entries {front, tile row, tile column, dbuf
-// slot}; tile row -1: the front has nothing below the panel), the panel's L
-// rows and U columns staged in LDS.  Tile (0, 0) or the -1 entry copies the
-// panel's diagonal-block factors from dbuf into the front.
-// Trailing update of the larger fronts on the matrix cores: the 64x64 tile
-// of a workgroup as 4 wavefronts x 2 x 2 blocks of 16 x 16, rank-4 products
-// per v_mfma_{f64,f32}_16x16x4 (A: lane l holds row l % 16, column l / 16 of
-// the 16 x 4 block; B: row l / 16, column l % 16 of the 4 x 16 block;
-// accumulator register r of lane l: column l % 16, row l / 16 + 4 r for FP64
-// and 4 (l / 16) + r for FP32).
+// Larger fronts: blocked by panels of kMfPanel columns, one launch per panel
+// index over all fronts of a level.  Launch j (p0 = 32 j) does two things at
+// once: the rank-32 update by panel j - 1 and the factorisation of panel j.
+//   panel entries {front, i, -1, slot}: blocks 2 i and 2 i + 1 of the front's
+//     64-row blocks of L21 and 64-column blocks of U12.  Wavefronts 1 and 2
+//     apply panel j - 1's update to a block each (matrix cores) while wavefront
+//     0 updates and factors the 32 x 32 diagonal block in registers (lane t
+//     owns row t, the pivot row broadcast with readlane); wavefronts 1 and 2
+//     then solve their blocks by substitution.  Every workgroup of a front
+//     factors the diagonal block for itself, so no workgroup waits for
+//     another; the first stores the factors in the front's dbuf slot (the
+//     others may still be reading the unfactored block), and launch j + 1
+//     copies them into the front.
+//   update entries {front, tile row, tile column, slot}: a 96 x 64 tile of the
+//     rest, -= L U of panel j - 1.
+//   copy entries {front, 0, -2, slot}: only the copy of panel j - 1's diagonal.
+// The launch after the last panel holds the update entries of the Schur
+// complement.  The chain of panels is what bounds a tree's top: one launch per
+// panel instead of a panel and an update launch, and no operand passes through
+// LDS on its way to the matrix cores, so that a step is one round of loads, the
+// diagonal's 32 dependent pivots and a substitution (16.8 us where the two
+// launches took 31.6, on the 865-order root of a 512 x 512 grid; 10.7 to 20 us
+// with FP32 factors and up to 720 workgroups).
+//
+// v_mfma_{f64,f32}_16x16x4: lane l holds A's row l % 16, column l / 16 of the
+// 16 x 4 block, B's row l / 16, column l % 16 of the 4 x 16 block; accumulator
+// register r of lane l: column l % 16, row l / 16 + 4 r for FP64 and
+// 4 (l / 16) + r for FP32.
 typedef double mf_d4 __attribute__((ext_vector_type(4)));
 typedef float mf_f4 __attribute__((ext_vector_type(4)));
 template <class T> struct MfAcc;
@@ -504,74 +408,316 @@ template <> struct MfAcc<float> {
   }
 };
 
+// acc = F[i0.., j0..] - F[i0.., q0..q0+kw) F[q0..q0+kw, j0..) on NA x NB blocks
+// of 16 x 16 by one wavefront (i0 < i1, j0 < j1).  Rows from i1 and columns from
+// j1 on repeat the last one (the caller drops them), so that no load is conditional; addresses
+// are a uniform base and a 32-bit offset.  Every load is issued before the
+// first product.
 template <class T>
-__global__ void __launch_bounds__(256) k_mf_update(MfDev d, const int4* ent, int p0, T* F, const T* dbuf) {
-  constexpr int TB = 64, KB = kMfPanel;
-  __shared__ T Ls[TB][KB + 1];
-  __shared__ T Us[KB][TB + 1];
-  const int4 e = ent[blockIdx.x];
-  const int s = e.x;
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const int pw = min(kMfPanel, np - p0);
-  const int base = p0 + pw;
-  T* Fs = F + d.fo[s];
-  if (e.y <= 0 && e.z <= 0) {
-    const T* db = dbuf + (long long)e.w * kMfPanel * kMfPanel;
-    for (int q = threadIdx.x; q < pw * kMfPanel; q += blockDim.x) {
-      const int i = q / kMfPanel, j = q % kMfPanel;
-      if (j < pw) Fs[(long long)(p0 + i) * ms + p0 + j] = db[q];
+__device__ __forceinline__ T mf_at(const T* base, unsigned byte_off) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + byte_off);
+}
+
+template <class T, int NA, int NB>
+__device__ __forceinline__ void mf_update_blocks(const T* Fs, long long ld, int i0, int i1, int j0, int j1, int q0,
+                                                 int kw, int lane, typename MfAcc<T>::V (&acc)[NA][NB]) {
+  const int lr = lane & 15, lk = lane >> 4;
+  const unsigned row = (unsigned)ld * sizeof(T);
+  unsigned cj[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) cj[b] = (unsigned)(min(j0 + 16 * b + lr, j1 - 1) - j0) * sizeof(T);
+  const T* C = Fs + i0 * ld + j0;
+#pragma unroll
+  for (int a = 0; a < NA; ++a)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const unsigned o = (unsigned)(min(i0 + 16 * a + MfAcc<T>::row(lk, r), i1 - 1) - i0) * row;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[a][b][r] = mf_at(C, o + cj[b]);
+    }
+  if (kw <= 0) return;
+  T l[NA][kMfPanel / 4], u[NB][kMfPanel / 4];
+  const T* Lb = Fs + i0 * ld + q0;
+  const T* Ub = Fs + q0 * ld + j0;
+#pragma unroll
+  for (int a = 0; a < NA; ++a) {
+    const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row;
+#pragma unroll
+    for (int k = 0; k < kMfPanel / 4; ++k) l[a][k] = mf_at(Lb, o + (unsigned)min(4 * k + lk, kw - 1) * (unsigned)sizeof(T));
+  }
+#pragma unroll
+  for (int k = 0; k < kMfPanel / 4; ++k) {
+    const unsigned o = (unsigned)min(4 * k + lk, kw - 1) * row;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) u[b][k] = mf_at(Ub, o + cj[b]);
+  }
+#pragma unroll
+  for (int k = 0; k < kMfPanel / 4; ++k) {
+    const bool in = 4 * k + lk < kw;
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+      const T lv = in ? -l[a][k] : (T)0;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) acc[a][b] = MfAcc<T>::mma(lv, u[b][k], acc[a][b]);
     }
   }
-  if (e.y < 0) return;
-  const int i0 = base + e.y * TB, j0 = base + e.z * TB;
-  {
-    // the L21 rows and U12 columns of the tile (zero beyond the front and the
-    // panel), all loads issued before the LDS stores
-    T lv[TB * KB / 256], uv[TB * KB / 256];
+}
+
+// reciprocal of a pivot in four stages that run between the products of a row
+// update: the hardware estimate of the mantissa's reciprocal, two Newton steps
+// (one for FP32), the exponent (apart, so that no step over- or underflows)
+template <class T> struct MfRecip;
+template <> struct MfRecip<double> {
+  double p, m, x;
+  __device__ __forceinline__ void stage(int i) {
+    if (i == 0) { m = __builtin_amdgcn_frexp_mant(p); x = __builtin_amdgcn_rcp(m); }
+    if (i == 1 || i == 2) x = fma(fma(-m, x, 1.0), x, x);
+    if (i == 3) x = __builtin_amdgcn_ldexp(x, -__builtin_amdgcn_frexp_exp(p));
+  }
+};
+template <> struct MfRecip<float> {
+  float p, m, x;
+  __device__ __forceinline__ void stage(int i) {
+    if (i == 0) { m = __builtin_amdgcn_frexp_mantf(p); x = __builtin_amdgcn_rcpf(m); }
+    if (i == 2) x = fmaf(fmaf(-m, x, 1.0f), x, x);
+    if (i == 3) x = __builtin_amdgcn_ldexpf(x, -__builtin_amdgcn_frexp_expf(p));
+  }
+};
+
+// row[q] -= l * (row k's element q) for q in [q0, N), the lanes' rows in
+// registers: eight broadcasts before the products that use them (a broadcast
+// is usable two cycles after it issues), the next pivot's reciprocal in between
+template <int N, class T>
+__device__ __forceinline__ void mf_row_update(T (&v)[N], T l, int k, int q0, MfRecip<T>& rec) {
 #pragma unroll
-    for (int it = 0; it < TB * KB / 256; ++it) {
-      const int x = threadIdx.x + it * 256;
-      const int r = x / KB, q = x % KB;
-      const int gi = i0 + r;
-      lv[it] = (gi < ms && q < pw) ? Fs[(long long)gi * ms + p0 + q] : (T)0;
-      const int qq = x / TB, c = x % TB;
-      const int gj = j0 + c;
-      uv[it] = (gj < ms && qq < pw) ? Fs[(long long)(p0 + qq) * ms + gj] : (T)0;
+  for (int c = 0; c < N; c += 8) {
+    T u[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (c + q >= q0 && c + q < N) u[q] = mf_bcast(v[c + q < N ? c + q : 0], k);
+    if (c + 7 >= q0) __builtin_amdgcn_sched_barrier(0);
+    if (c >= N - 32) rec.stage((c - (N - 32)) / 8);
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (c + q >= q0 && c + q < N) v[c + q < N ? c + q : 0] -= l * u[q];
+  }
+}
+
+// right-looking LU of the rows in registers (lane t: row t), pivots [0, NP) of
+// N columns; lanes from `rows` on count for nothing.  first: lowest column with
+// a bad pivot or a multiplier beyond KLU's threshold; rd: lane k's reciprocal
+// of pivot k.  Constant trip counts keep the rows in registers.
+template <int N, int NP, class T>
+__device__ __forceinline__ void mf_factor_rows(T (&v)[N], int lane, int rows, int np, int& first, bool& hard, T& rd) {
+  MfRecip<T> rec;
+  T piv = mf_bcast(v[0], 0);
+  rec.p = piv;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) rec.stage(i);
+  mf_for<NP>([&](auto kc) MF_INLINE {
+    constexpr int k = kc, k1 = k + 1 < N ? k + 1 : k;
+    if (k >= np) return;
+    const T rp = rec.x;
+    if (!(fabs((double)piv) > 0.0) || !isfinite((double)piv)) { first = min(first, k); hard = true; }
+    if (lane == k) rd = rp;
+    const bool upd = lane > k && lane < rows;
+    const T l = upd ? v[k] * rp : (T)0;
+    if (upd) v[k] = l;
+    if (!(fabs((double)l) <= 1.0e3)) first = min(first, k);
+    if constexpr (k1 > k) v[k1] -= l * mf_bcast(v[k1], k);
+    piv = mf_bcast(v[k1], k1);
+    rec.p = piv;
+    mf_row_update<N>(v, l, k, k + 2, rec);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+}
+
+// LDS written by a wavefront's lanes is visible to its other lanes
+__device__ __forceinline__ void mf_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+constexpr int kMfStep = 192;              // threads of a step workgroup: three wavefronts
+constexpr int kMfTileRows = 96;           // rows of an update tile: 32 per wavefront
+constexpr int kMfDs = kMfPanel + 2;       // row stride of the diagonal factors in LDS (16-byte pairs)
+constexpr int kMfTile = 64 * (kMfPanel + 1) > kMfPanel * 65 ? 64 * (kMfPanel + 1) : kMfPanel * 65;
+
+template <class T>
+__global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2))) k_mf_step(MfDev d, const int4* ent, int p0, T* F, T* dbuf, int half,
+                                                     int* bad) {
+  constexpr int PW = kMfPanel;
+  __shared__ __attribute__((aligned(16))) T Du[PW * kMfDs];   // U11 by rows
+  __shared__ __attribute__((aligned(16))) T Dl[PW * kMfDs];   // L11 by columns; the updated block before it is factored
+  __shared__ T Rd[PW];
+  __shared__ T Ts[2][kMfTile];
+  const int4 e = ent[blockIdx.x];
+  const int s = e.x, slot = e.w;
+  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
+  const int base = min(np, p0 + PW), q0 = p0 - PW, kw = q0 >= 0 ? min(PW, np - q0) : 0;
+  T* Fs = F + d.fo[s];
+  const long long ld = ms;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
+  typedef typename MfAcc<T>::V V;
+  if (kw > 0 && e.y == 0 && e.z <= 0) {
+    // the front's first entry: panel j - 1's diagonal factors into the front
+    const T* db = dbuf + ((long long)slot * 2 + (half ^ 1)) * PW * PW;
+    for (int x = t; x < PW * PW; x += kMfStep) {
+      const int i = x / PW, j = x % PW;
+      if (i < kw && j < kw) Fs[(q0 + i) * ld + q0 + j] = db[x];
     }
+  }
+  if (e.z == -2) return;
+  if (e.z >= 0) {
+    const int i0 = base + e.y * kMfTileRows + 32 * wave, j0 = base + e.z * 64;
+    if (i0 >= ms) return;      // these rows of the tile lie beyond the front
+    V acc[2][4];
+    mf_update_blocks<T, 2, 4>(Fs, ld, i0, ms, j0, ms, q0, kw, lane, acc);
 #pragma unroll
-    for (int it = 0; it < TB * KB / 256; ++it) {
-      const int x = threadIdx.x + it * 256;
-      Ls[x / KB][x % KB] = lv[it];
-      Us[x / TB][x % TB] = uv[it];
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int gi = i0 + 16 * a + MfAcc<T>::row(lk, r), gj = j0 + 16 * b + lr;
+          if (gi < ms && gj < ms) Fs[gi * ld + gj] = acc[a][b][r];
+        }
+    return;
+  }
+  // ---- the diagonal (wavefront 0) and two blocks (wavefronts 1, 2) of panel j
+  const int pw = base - p0, rest = ms - base, nrb = (rest + 63) / 64;
+  const int blk = 2 * e.y + wave - 1;
+  const bool has = wave > 0 && blk < 2 * nrb, lower = blk < nrb;
+  T* Tl = Ts[wave > 1];
+  const int o0 = base + (lower ? blk : blk - nrb) * 64;     // first row or column of the block
+  if (wave == 0) {
+    V acc[2][2];
+    mf_update_blocks<T, 2, 2>(Fs, ld, p0, base, p0, base, q0, kw, lane, acc);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 16 * a + MfAcc<T>::row(lk, r), j = 16 * b + lr;
+          // beyond the panel's width: the identity
+          Dl[i * kMfDs + j] = (i < pw && j < pw) ? acc[a][b][r] : (i == j ? (T)1 : (T)0);
+        }
+  } else if (has && lower) {
+    V acc[4][2];
+    mf_update_blocks<T, 4, 2>(Fs, ld, o0, ms, p0, base, q0, kw, lane, acc);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          Tl[(16 * a + MfAcc<T>::row(lk, r)) * (PW + 1) + 16 * b + lr] = acc[a][b][r];
+  } else if (has) {
+    V acc[2][4];
+    mf_update_blocks<T, 2, 4>(Fs, ld, p0, base, o0, ms, q0, kw, lane, acc);
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Tl[(16 * a + MfAcc<T>::row(lk, r)) * 65 + 16 * b + lr] = acc[a][b][r];
+  }
+  mf_wave_fence();          // each wavefront reads back its own tile: no wait for the others
+  int failed = PW;          // first column whose pivot or multiplier fails
+  bool hard = false;
+  T v[PW];
+  if (wave == 0) {
+    const int row = lane & 31;
+#pragma unroll
+    for (int q = 0; q < PW; ++q) v[q] = Dl[row * kMfDs + q];
+    T rd = (T)1;
+    mf_factor_rows<PW, PW>(v, lane, PW, PW, failed, hard, rd);
+    if (lane < PW) Rd[lane] = rd;
+  } else if (has && lower) {
+#pragma unroll
+    for (int q = 0; q < PW; ++q) v[q] = Tl[lane * (PW + 1) + q];
+  } else if (has) {
+#pragma unroll
+    for (int q = 0; q < PW; ++q) v[q] = Tl[q * 65 + lane];
+  }
+  __syncthreads();
+  if (wave == 0 && lane < PW) {
+#pragma unroll
+    for (int q = 0; q < PW; ++q) {
+      Du[lane * kMfDs + q] = v[q];
+      Dl[q * kMfDs + lane] = v[q];
+    }
+    if (e.y == 0) {
+      T* db = dbuf + ((long long)slot * 2 + half) * PW * PW + lane * PW;
+#pragma unroll
+      for (int q = 0; q < PW; ++q) db[q] = v[q];
     }
   }
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int wr = (wave >> 1) * 32, wc = (wave & 1) * 32, lr = lane & 15, lk = lane >> 4;
-  typedef typename MfAcc<T>::V V;
-  V acc[2][2];
+  if (has) {
+    if (lower) {
+      const bool valid = o0 + lane < ms;
+      // row k + 1 of U11 is read while row k is applied (z, zero, is tied to
+      // v[k] so that at most two rows are held in registers)
+      int z = 0;
+      T u[PW], un[PW];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+      for (int q = 0; q < PW; ++q) u[q] = Du[q];
+      T r = Rd[0];
+      mf_for<PW>([&](auto kc) MF_INLINE {
+        constexpr int k = kc, k1 = k + 1 < PW ? k + 1 : k;
+        asm volatile("" : "+v"(z) : "v"(v[k]));
+        const T rn = Rd[k1 + z];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = V{};
+        for (int q = k + 2; q < PW; ++q) un[q] = Du[z + k1 * kMfDs + q];
+        v[k] *= r;
+        if (valid && !(fabs((double)v[k]) <= 1.0e3)) failed = min(failed, k);
 #pragma unroll
-  for (int k = 0; k < KB; k += 4) {
-    const T a0 = Ls[wr + lr][k + lk], a1 = Ls[wr + 16 + lr][k + lk];
-    const T b0 = Us[k + lk][wc + lr], b1 = Us[k + lk][wc + 16 + lr];
-    acc[0][0] = MfAcc<T>::mma(a0, b0, acc[0][0]);
-    acc[0][1] = MfAcc<T>::mma(a0, b1, acc[0][1]);
-    acc[1][0] = MfAcc<T>::mma(a1, b0, acc[1][0]);
-    acc[1][1] = MfAcc<T>::mma(a1, b1, acc[1][1]);
+        for (int q = k + 1; q < PW; ++q) v[q] -= v[k] * u[q];
+#pragma unroll
+        for (int q = k + 2; q < PW; ++q) u[q] = un[q];
+        r = rn;
+        __builtin_amdgcn_sched_barrier(0);
+      });
+#pragma unroll
+      for (int q = 0; q < PW; ++q) Tl[lane * (PW + 1) + q] = v[q];
+    } else {
+      const int c = o0 + lane;
+      int z = 0;
+      T u[PW], un[PW];
+#pragma unroll
+      for (int q = 0; q < PW; ++q) u[q] = Dl[q];
+      mf_for<PW>([&](auto kc) MF_INLINE {
+        constexpr int k = kc, k1 = k + 1 < PW ? k + 1 : k;
+        asm volatile("" : "+v"(z) : "v"(v[k]));
+#pragma unroll
+        for (int q = k + 2; q < PW; ++q) un[q] = Dl[z + k1 * kMfDs + q];
+#pragma unroll
+        for (int q = k + 1; q < PW; ++q) v[q] -= u[q] * v[k];
+#pragma unroll
+        for (int q = k + 2; q < PW; ++q) u[q] = un[q];
+        __builtin_amdgcn_sched_barrier(0);
+      });
+#pragma unroll
+      for (int q = 0; q < PW; ++q)
+        if (c < ms && q < pw) Fs[(p0 + q) * ld + c] = v[q];
+    }
   }
+  __syncthreads();
+  // the L21 blocks, row by row
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gi = i0 + wr + 16 * a + MfAcc<T>::row(lk, r), gj = j0 + wc + 16 * b + lr;
-        if (gi < ms && gj < ms) Fs[(long long)gi * ms + gj] -= acc[a][b][r];
-      }
+  for (int w = 0; w < 2; ++w) {
+    const int b = 2 * e.y + w, r0 = base + b * 64;
+    if (b >= nrb) break;
+    for (int x = t; x < 64 * PW; x += kMfStep) {
+      const int i = x / PW, q = x % PW;
+      if (r0 + i < ms && q < pw) Fs[(r0 + i) * ld + p0 + q] = Ts[w][i * (PW + 1) + q];
+    }
+  }
+  if (failed < pw) atomicMin(bad, d.sfirst[s] + p0 + failed + 1);
+  if (__any(hard) && lane == 0) atomicOr(bad + 1, 1);
 }
 
 // sums over c in [c0, c1) of F[r + k][c] v[c] for the rows r .. r + nr - 1
@@ -879,14 +1025,13 @@ struct MfLu::Impl {
   DevVec<int> tiny_list, big_list;
   DevVec<int4> aent;              // assembly entries of the larger fronts {front, first row, alo offset, 0}
   DevVec<int> alo;                // per entry and child: first child row at or after the entry's first row
-  DevVec<int4> pent, uent;        // panel and update launch entries
-  DevVec<double> dbuf;            // diagonal-block factors, one 32x32 slot per front of a panel launch
+  DevVec<int4> sent;              // entries of the panel steps
+  DevVec<double> dbuf;            // diagonal-block factors, two 32 x 32 slots per larger front of a level
   std::vector<int> tiny_off, tiny_maxm, big_off;
   int big_maxm = 0;
   std::vector<int> aoff;          // per level: offset into aent
-  // blocked launches: per level, per panel index j
-  struct PanelLaunch { int p0, poff, pcnt, uoff, ucnt; };
-  std::vector<std::vector<PanelLaunch>> pl_of_level;
+  struct Step { int p0, off, cnt; };
+  std::vector<std::vector<Step>> steps;   // per level: its panel steps
   MfDev dev() const {
     MfDev d;
     d.sfirst = sfirst.p; d.m = m.p; d.fo = fo.p; d.iptr = iptr.p; d.idx = idx.p; d.cptr = cptr.p;
@@ -927,12 +1072,12 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   // fronts of the level in each panel launch)
   const int nl = (int)P.lvl_ptr.size() - 1;
   std::vector<int> tl, bl;
-  std::vector<int4> pe, ue;
+  std::vector<int4> se;
   int max_slots = 1;
   I.tiny_off.assign(nl + 1, 0);
   I.big_off.assign(nl + 1, 0);
   I.tiny_maxm.assign(nl, 0);
-  I.pl_of_level.assign(nl, {});
+  I.steps.assign(nl, {});
   I.big_maxm = 0;
   for (int l = 0; l < nl; ++l) {
     I.tiny_off[l] = (int)tl.size();
@@ -949,39 +1094,38 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
         maxp = std::max(maxp, (P.sfirst[t + 1] - P.sfirst[t] + kMfPanel - 1) / kMfPanel);
       }
     }
-    for (int j = 0; j < maxp; ++j) {
-      Impl::PanelLaunch L{j * kMfPanel, (int)pe.size(), 0, (int)ue.size(), 0};
-      int slot = 0;
-      for (int b = I.big_off[l]; b < (int)bl.size(); ++b) {
-        const int t = bl[b];
-        const int np = P.sfirst[t + 1] - P.sfirst[t];
-        if (np <= L.p0) continue;
-        const int pw = std::min(kMfPanel, np - L.p0);
-        const int rest = P.m[t] - L.p0 - pw;
-        const int nrb = (rest + 63) / 64;
-        if (rest > 0) {
-          for (int blk = 0; blk < 2 * nrb; ++blk) pe.push_back(make_int4(t, blk, slot, 0));
-          for (int ti = 0; ti < nrb; ++ti)
-            for (int tj = 0; tj < nrb; ++tj) ue.push_back(make_int4(t, ti, tj, slot));
-        } else {
-          pe.push_back(make_int4(t, 0, slot, 0));
-          ue.push_back(make_int4(t, -1, -1, slot));
+    const int nb = (int)bl.size() - I.big_off[l];
+    max_slots = std::max(max_slots, nb);
+    for (int j = 0; nb > 0 && j <= maxp; ++j) {
+      Impl::Step S{j * kMfPanel, (int)se.size(), 0};
+      // the panels first (they are the longer chain), then the update tiles
+      for (int pass = 0; pass < 2; ++pass)
+        for (int slot = 0; slot < nb; ++slot) {
+          const int t = bl[I.big_off[l] + slot];
+          const int np = P.sfirst[t + 1] - P.sfirst[t];
+          if (S.p0 >= np + kMfPanel) continue;                 // finished at an earlier step
+          const int rest = P.m[t] - std::min(np, S.p0 + kMfPanel);
+          const int nrb = (rest + 63) / 64;
+          if (pass == 0) {
+            if (S.p0 < np)
+              for (int i = 0; i < std::max(1, nrb); ++i) se.push_back(make_int4(t, i, -1, slot));
+            else if (rest == 0) se.push_back(make_int4(t, 0, -2, slot));
+          } else if (j > 0) {
+            // after the last panel tile (0, 0) copies the diagonal
+            for (int ti = 0; ti * kMfTileRows < rest; ++ti)
+              for (int tj = 0; tj < nrb; ++tj) se.push_back(make_int4(t, ti, tj, slot));
+          }
         }
-        ++slot;
-      }
-      L.pcnt = (int)pe.size() - L.poff;
-      L.ucnt = (int)ue.size() - L.uoff;
-      max_slots = std::max(max_slots, slot);
-      I.pl_of_level[l].push_back(L);
+      S.cnt = (int)se.size() - S.off;
+      I.steps[l].push_back(S);
     }
   }
   I.tiny_off[nl] = (int)tl.size();
   I.big_off[nl] = (int)bl.size();
   MFCHK(I.tiny_list.up(tl, st));
   MFCHK(I.big_list.up(bl, st));
-  MFCHK(I.pent.up(pe, st));
-  MFCHK(I.uent.up(ue, st));
-  MFCHK(I.dbuf.alloc((size_t)max_slots * kMfPanel * kMfPanel));
+  MFCHK(I.sent.up(se, st));
+  MFCHK(I.dbuf.alloc((size_t)max_slots * 2 * kMfPanel * kMfPanel));
   // assembly of the larger fronts: 32 parent rows per workgroup (the tiny
   // fronts assemble their children inside their factor kernel)
   std::vector<int4> ae;
@@ -1042,12 +1186,9 @@ static int mf_factor_enqueue(MfLu::Impl& I, const double* vals_dev, int nnz, T* 
       hipLaunchKernelGGL(k_mf_factor_tiny<T>, dim3(nt), dim3(64), (size_t)mm * (mm + 1) * sizeof(T), st, d,
                          I.tiny_list.p + I.tiny_off[l], F, I.bad.p);
     }
-    for (const auto& L : I.pl_of_level[l]) {
-      hipLaunchKernelGGL(k_mf_panel<T>, dim3(L.pcnt), dim3(64), 0, st, d, I.pent.p + L.poff, L.p0, F, dbuf,
-                         I.bad.p);
-      hipLaunchKernelGGL(k_mf_update<T>, dim3(L.ucnt), dim3(256), 0, st, d, I.uent.p + L.uoff, L.p0, F,
-                         (const T*)dbuf);
-    }
+    for (const auto& S : I.steps[l])
+      hipLaunchKernelGGL(k_mf_step<T>, dim3(S.cnt), dim3(kMfStep), 0, st, d, I.sent.p + S.off, S.p0, F, dbuf,
+                         (S.p0 / kMfPanel) & 1, I.bad.p);
   }
   MFCHK(hipGetLastError());
   return XG_OK;
