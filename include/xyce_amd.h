@@ -159,11 +159,10 @@ int xg_combine_dev(xg_circuit* c, const double* q0, const double* q2, double* rh
  * ordering, N_LAS_AmesosSolver.C:335).  values may be NULL; if given they
  * steer the transversal toward large entries. */
 int xg_lu_symbolic(int n, const int* rowptr, const int* colind, const double* values, xg_lu** out);
-/* The same with the factorisation method chosen: 0 automatic (multifrontal
- * when the level-scheduled program would exceed 2e7 flops, 65535 unknowns or
- * 2^24 factor entries), 1 level-scheduled entry LU (small systems), 2
- * multifrontal (supernodal fronts, level by level over the elimination
- * tree; for power grids and gate arrays). */
+/* The same with the factorisation method chosen: 0 automatic (level-scheduled
+ * up to 128 unknowns, multifrontal above), 1 level-scheduled entry LU (small
+ * systems), 2 multifrontal (supernodal fronts, level by level over the
+ * elimination tree). */
 int xg_lu_symbolic_ex(int n, const int* rowptr, const int* colind, const double* values, int method, xg_lu** out);
 int xg_lu_destroy(xg_lu* lu);
 /* Numeric refactor with the symbolic pivot order (KLU NumericFactorization,
@@ -179,9 +178,10 @@ int xg_lu_destroy(xg_lu* lu);
 int xg_lu_numeric(xg_lu* lu, const double* vals);
 /* Solve A x = b with the last factors (:396); NaN -> XG_E_NAN, x zeroed.
  * transpose != 0 solves A^T x = b (doSolve(reuse_factors, transpose),
- * N_LAS_Solver.h:95-107; Amesos SetUseTranspose): level-scheduled method
- * with FP64 factors only (XG_E_ARG otherwise; Xyce's transient path does not
- * use it). */
+ * N_LAS_Solver.h:95-107; Amesos SetUseTranspose): FP64 factors of the
+ * level-scheduled method, which a handle with an automatic method makes when
+ * first asked, up to 65535 unknowns and 2e7 flops (XG_E_ARG otherwise; Xyce's
+ * transient path does not use it). */
 int xg_lu_solve(xg_lu* lu, const double* b, double* x, int transpose);
 /* xg_lu_numeric / xg_lu_solve on device arrays (HIP device memory); same
  * semantics; each call returns when its outputs are complete. */

@@ -160,6 +160,37 @@ def test_malformed_pattern_is_rejected(case):
     X.host_lu_analyse(3, np.array([0, 2, 4, 6], np.int32), np.array([0, 1, 0, 1, 1, 2], np.int32))
 
 
+@pytest.mark.parametrize("name", ["rings", "grids", "gates", "star", "clique", "path", "diagonal"])
+def test_multifrontal_plan_covers_every_column(name):
+    """The plan of systems around the dissection's leaf size (64) and of extreme
+    shapes: built, every front square and within the system, at least the
+    factor entries a dense diagonal needs."""
+    def csr(M):
+        rp = np.concatenate([[0], np.cumsum(M.sum(1))]).astype(np.int32)
+        return M.shape[0], rp, np.nonzero(M)[1].astype(np.int32)
+    if name == "star":
+        pats = []
+        for n in (2, 65, 200):
+            M = np.eye(n, dtype=int); M[0] = 1; M[:, 0] = 1
+            pats.append(csr(M))
+    elif name == "clique":
+        pats = [csr(np.ones((n, n), int)) for n in (1, 64, 65, 90)]
+    elif name == "path":
+        pats = [csr(np.eye(n, dtype=int) + np.eye(n, k=1, dtype=int) + np.eye(n, k=-1, dtype=int)) for n in (64, 65, 66, 300, 2000)]
+    elif name == "diagonal":
+        pats = [(n, np.arange(n + 1, dtype=np.int32), np.arange(n, dtype=np.int32)) for n in (1, 64, 65, 200_000)]
+    else:
+        cs = {"rings": [C.ring(s) for s in range(3, 140, 2)],
+              "grids": [C.power_grid(a, b, pad_pitch=4, n_sinks=4) for a, b in ((1, 70), (2, 33), (8, 8), (9, 8), (33, 40))],
+              "gates": [C.gate_dag(k, seed=k) for k in (20, 40, 45, 300, 1100)]}[name]
+        hp = [X.host_pattern(c) for c in cs]
+        pats = [(h["n"], h["rowptr"], h["colind"]) for h in hp]
+    for n, rp, ci in pats:
+        p = X.host_mf_plan(n, rp, ci)
+        assert 1 <= p["supernodes"] <= n and 1 <= p["levels"] <= p["supernodes"] and 1 <= p["max_front"] <= n
+        assert n <= p["nnz_lu"] <= p["front_elements"] and p["front_elements"] <= p["supernodes"] * p["max_front"] ** 2
+
+
 @pytest.mark.parametrize("name", ["ring", "grid", "gates"])
 def test_patterns_are_one_strongly_connected_block(name):
     import scipy.sparse as sp

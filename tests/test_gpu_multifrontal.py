@@ -202,3 +202,26 @@ def test_power_grid_512_full_size(gpu):
     assert s.numeric(J) == 0
     st, x2 = s.solve(rhs)
     assert np.array_equal(x, x2)
+
+
+@pytest.mark.parametrize("name,method", [("ring125", 1), ("ring127", 2), ("gates200", 2)])
+def test_automatic_method_solves_both_ways(gpu, name, method):
+    """Either side of the automatic method's line: A x = b, A^T x = b (whatever
+    the method), again after a refactor, and the no-allocation solve."""
+    import ctypes
+    import torch
+    c = C.gate_dag(200, seed=4) if name == "gates200" else C.ring(int(name[4:]), seed=2, mc_seed=2)
+    n, rp, ci, J, b = _jacobian(c, 5)
+    s = X.DirectSolver(n, rp, ci)
+    assert s.info()["method"] == method
+    for vals in (J, J * (1.0 + 0.1 * np.random.default_rng(3).uniform(size=J.size))):
+        A = sp.csr_matrix((vals, ci, rp), shape=(n, n)).toarray()
+        st, x = s.doSolve(vals, b)
+        assert st == 0 and np.linalg.norm(A @ x - b) <= 1e-12 * np.linalg.norm(b)
+        st, xt = s.doSolve(vals, b, reuse_factors=True, transpose=True)
+        assert st == 0 and np.linalg.norm(A.T @ xt - b) <= 1e-12 * np.linalg.norm(b)
+        bd, xd = torch.from_numpy(b).cuda(), torch.zeros(n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        P = lambda t: ctypes.c_void_p(t.data_ptr())
+        assert X.lib().xg_lu_solve_noalloc(s.h, P(bd), P(xd)) == 0
+        assert np.array_equal(xd.cpu().numpy(), x)

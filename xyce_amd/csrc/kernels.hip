@@ -632,22 +632,44 @@ struct xg_lu {
   // with the handle; null if the lookup failed)
   double* scratch_work = nullptr;
 
-  // symbolic analysis for the chosen (or automatically picked) method
+  // a handle whose method was picked here (asked 0) also solves A^T x = b where
+  // the level-scheduled method can hold the system: from factors of its own,
+  // made when a transpose solve first needs them
+  int asked = 0;
+  xg_lu* tlu = nullptr;
+  bool tlu_current = false;
+
+  ~xg_lu() { if (tlu) (void)xg_lu_destroy(tlu); }
+
+  bool level_fits(const double* values) const {
+    const int n = (int)a_rowptr.size() - 1;
+    if (n > 65535) return false;
+    LuSymbolic t;
+    return lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, false) == XG_OK && t.flops <= 2e7 &&
+           t.nlu <= (1 << 24);
+  }
+
+  // symbolic analysis for the chosen (or automatically picked) method.  The
+  // line: up to 128 unknowns one workgroup walks the levels of the entry program
+  // about as fast as the multifrontal launches follow each other, and its first
+  // pass needs no graph (ring of 103 unknowns: refactor and solve 196 us against
+  // 188, first pass 226 against 285); above, its levels grow with the system and
+  // the supernode tree's do not (gate array of 298: 758 us against 242, of 1481:
+  // 6990 against 562).
+  static constexpr int kLevelMaxN = 128;
   int analyse(const double* values, int want_method) {
     const int n = (int)a_rowptr.size() - 1;
     LuSymbolic t;
-    int m = want_method, st;
-    if (m == 0) {
-      m = 2;
-      if (n <= 65535) {
-        st = lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, false);
-        if (st != XG_OK) return st;
-        m = (t.flops > 2e7 || t.nlu > (1 << 24)) ? 2 : 1;
-      }
-    }
-    st = m == 2 ? mf_analyse(n, a_rowptr.data(), a_colind.data(), values, t)
-                : lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
+    int m = want_method ? want_method : n <= kLevelMaxN ? 1 : 2;
+    int st = m == 2 ? mf_analyse(n, a_rowptr.data(), a_colind.data(), values, t)
+                    : lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
     if (st != XG_OK) return st;
+    // what the level-scheduled method can hold keeps its no-allocation solve
+    if (want_method == 0 && m == 2 && 4 * (size_t)n + t.srow.size() + 256 > kScratchDoubles && level_fits(values)) {
+      m = 1;
+      st = lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
+      if (st != XG_OK) return st;
+    }
     s = std::move(t);
     method = m;
     return XG_OK;
@@ -1380,6 +1402,7 @@ int xg_lu_symbolic_ex(int n, const int* rowptr, const int* colind, const double*
   lu->a_rowptr.assign(rowptr, rowptr + n + 1);
   lu->a_colind.assign(colind, colind + rowptr[n]);
   lu->s.n = n;
+  lu->asked = method;
   try {
     int st = lu->analyse(values, method);
     if (st != XG_OK) return st;
@@ -1428,6 +1451,7 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
   HIPCHK(hipMemcpyAsync(lu->avals.p, vals, sizeof(double) * lu->s.nnz_a, in, s));
   lu->have64 = false;
   lu->soft64 = false;
+  lu->tlu_current = false;
   int bad = 0, hard = 0, st;
   if (lu->mode == 1) {
     st = lu->factor_any(true, &bad, &hard);
@@ -1469,10 +1493,33 @@ int xg_lu_numeric(xg_lu* lu, const double* vals) { return lu_numeric_impl(lu, va
 
 int xg_lu_numeric_dev(xg_lu* lu, const double* vals) { return lu_numeric_impl(lu, vals, true); }
 
+static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, bool dev);
+
+// A^T x = b on a handle that took the multifrontal method by itself: the
+// level-scheduled factors of the current values
+static int lu_solve_transpose_auto(xg_lu* lu, const double* b, double* x, bool dev) {
+  if (!lu->tlu) {
+    try {
+      if (!lu->level_fits(nullptr)) return XG_E_ARG;
+    } catch (...) {
+      return XG_E_SETUP;
+    }
+    const int st = xg_lu_symbolic_ex(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 1, &lu->tlu);
+    if (st != XG_OK) return st;
+  }
+  if (!lu->tlu_current) {
+    const int st = lu_numeric_impl(lu->tlu, lu->avals.p, true);
+    if (st != XG_OK) return st < 0 ? st : XG_E_ARG;
+    lu->tlu_current = true;
+  }
+  return lu_solve_impl(lu->tlu, b, x, 1, dev);
+}
+
 static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, bool dev) {
   if (!lu || !b || !x) return XG_E_ARG;
   // transpose solves: the level-scheduled method with plain FP64 factors
-  if (transpose && (lu->method != 1 || lu->mode == 1 || !lu->have64 || lu->soft64)) return XG_E_ARG;
+  if (transpose && (lu->mode == 1 || !lu->have64 || lu->soft64)) return XG_E_ARG;
+  if (transpose && lu->method != 1) return lu->asked == 0 ? lu_solve_transpose_auto(lu, b, x, dev) : XG_E_ARG;
   hipStream_t s = lu->stream;
   const int n = lu->s.n;
   HIPCHK(hipMemcpyAsync(lu->b.p, b, sizeof(double) * n, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));

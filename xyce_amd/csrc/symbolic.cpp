@@ -328,19 +328,27 @@ void nd_order(const Graph& g, std::vector<int> nodes, std::vector<int>& order, i
   }
   bfs(root, seq, lptr);
   if (seq.size() < nodes.size()) {
-    // disconnected: the component and the rest are independent
-    std::vector<int> rest;
-    for (int v : seq) tag[v] = -id;
-    for (int v : nodes) if (tag[v] == id) rest.push_back(v);
-    nd_order(g, seq, order, leaf, tag, stamp, lvl, widest);
-    nd_order(g, rest, order, leaf, tag, stamp, lvl, widest);
+    std::vector<std::vector<int>> parts;
+    size_t at = 0;
+    // disconnected: the components are independent; the small ones together
+    std::vector<int> small;
+    for (;;) {
+      if ((int)seq.size() <= leaf) small.insert(small.end(), seq.begin(), seq.end());
+      else parts.push_back(seq);
+      for (int v : seq) tag[v] = -id;
+      while (at < nodes.size() && tag[nodes[at]] != id) ++at;
+      if (at == nodes.size()) break;
+      bfs(nodes[at], seq, lptr);
+    }
+    amd_order(g, small, order);
+    for (auto& p : parts) nd_order(g, std::move(p), order, leaf, tag, stamp, lvl, widest);
     return;
   }
   const int nl = (int)lptr.size() - 1;
   if (nl < 3) { amd_order(g, nodes, order); return; }
   const int half = (int)seq.size() / 2;
   int mid = 1;
-  while (mid < nl - 1 && lptr[mid + 1] <= half) ++mid;
+  while (mid < nl - 2 && lptr[mid + 1] <= half) ++mid;   // a level beyond the separator remains
   // smallest level within a window around the middle that keeps both sides
   // at least a third of the nodes
   int sep = mid;
@@ -356,6 +364,7 @@ void nd_order(const Graph& g, std::vector<int> nodes, std::vector<int>& order, i
     for (int a : g[v]) if (tag[a] == id && lvl[a] == sep + 1) { beyond = true; break; }
     (beyond ? S : A).push_back(v);
   }
+  if (B.empty() || S.empty()) { amd_order(g, nodes, order); return; }
   if (widest) *widest = std::max(*widest, (double)S.size() / std::sqrt((double)seq.size()));
   nd_order(g, std::move(A), order, leaf, tag, stamp, lvl, widest);
   nd_order(g, std::move(B), order, leaf, tag, stamp, lvl, widest);
