@@ -9,7 +9,7 @@
 //
 //   assemble  F_s = A entries of s's columns + extend-add of the children's
 //             Schur complements (the j-th children of a level in launch j,
-//             rows split over workgroups: a fixed order, no atomics)
+//             rows split over workgroups: a fixed order)
 //   factor    dense LU of the pivot block, L21, U12 and the Schur complement
 //             F22 -= L21 U12; small fronts one workgroup each, large fronts
 //             blocked by 32-column panels (diagonal block in LDS, row-parallel
@@ -120,10 +120,10 @@ int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p
     const double np = p.sfirst[t + 1] - p.sfirst[t], mm = p.m[t];
     for (double k = 0; k < np; ++k) p.flops += 2.0 * (mm - k - 1) * (mm - k - 1) + (mm - k - 1);
   }
-  // A entries -> front elements: entry (i,j) of B goes to the front whose
-  // pivots hold min(i,j)
-  p.amap.resize(s.nnz_a);
-  std::vector<int> pos_in(0);
+  // A entries by front row: entry (i,j) of B goes to the front whose pivots
+  // hold min(i,j)
+  std::vector<int> arow_of(s.nnz_a), acol_of(s.nnz_a);
+  p.arow.assign((size_t)p.vo[ns] + 1, 0);
   for (int r = 0; r < n; ++r) {
     const int i = s.rinv[r];
     for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) {
@@ -139,7 +139,20 @@ int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p
       };
       const int li = local(i), lj = local(j);
       if (li < 0 || lj < 0) return XG_E_SETUP;
-      p.amap[k] = p.fo[t] + (long long)li * p.m[t] + lj;
+      arow_of[k] = p.vo[t] + li;
+      acol_of[k] = lj;
+      ++p.arow[arow_of[k] + 1];
+    }
+  }
+  for (size_t q = 1; q < p.arow.size(); ++q) p.arow[q] += p.arow[q - 1];
+  p.acol.resize(s.nnz_a);
+  p.aslot.resize(s.nnz_a);
+  {
+    std::vector<int> f(p.arow.begin(), p.arow.end() - 1);
+    for (int k = 0; k < s.nnz_a; ++k) {
+      const int q = f[arow_of[k]]++;
+      p.acol[q] = acol_of[k];
+      p.aslot[q] = k;
     }
   }
   return XG_OK;
@@ -148,9 +161,24 @@ int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
+// what a kernel needs to know of a front and of a child, each in one load
+struct MfFront {
+  long long fo;                 // its elements (row-major, order m)
+  int m, np;                    // order, pivots
+  int first, idx;               // first column, index list
+  int c0, c1;                   // children
+  int vo, pad;                  // its rows' slots in the front vectors and in arow
+};
+struct MfChild {
+  long long src;                // the Schur complement's first element
+  int ld, nu;                   // its row stride and order
+  int em, vsrc;                 // parent positions of its rows; their slots in the front vectors
+};
 struct MfDev {
   const int* sfirst; const int* m; const long long* fo; const int* iptr; const int* idx;
   const int* cptr; const int* clist; const int* eptr; const int* emap; const int* vo;
+  const MfFront* front; const MfChild* child;
+  const int* arow; const int* acol; const int* aslot;
 };
 
 constexpr int kMfTiny = 64;     // fronts up to this order: one wavefront, the front in LDS
@@ -166,18 +194,6 @@ __device__ __forceinline__ void mf_for(const F& f) {
   }
 }
 #define MF_INLINE __attribute__((always_inline))
-
-template <class T>
-__global__ void k_mf_fill(T* F, long long total) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < total) F[i] = (T)0;
-}
-
-template <class T>
-__global__ void k_mf_scatter(int nnz, const double* vals, const long long* amap, T* F) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < nnz) F[amap[k]] += (T)vals[k];
-}
 
 // value of v in lane `src` (wave-uniform) of the wavefront
 __device__ __forceinline__ double mf_bcast(double v, int src) {
@@ -195,171 +211,6 @@ __device__ __forceinline__ T mf_wave_sum(T v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
-}
-
-// assembly of the children's Schur complements into a larger front: one
-// workgroup per kMfAsmRows rows of the parent (entries {front, first row,
-// offset into `alo`}); the children are added one after another in their
-// fixed order, so every parent element receives the same sums in the same
-// order on every refactor (no atomics).  A child's rows map to increasing
-// parent rows; alo holds, per entry and child, the first child row that lands
-// at or after the entry's first row.  The four wavefronts take the child rows
-// in turn (wave w: rows a0 + w, a0 + w + 4, ...), lanes over 256-column
-// chunks; a chunk's parent column positions are loaded once, and each wave
-// loads four rows' child and parent values before it stores any, so a row
-// costs two memory round trips shared with the wave's other rows.
-constexpr int kMfAsmRows = 16;
-
-template <class T>
-__global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, const int* alo, T* F) {
-  const int4 e = ent[blockIdx.x];
-  const int s = e.x, ms = d.m[s];
-  const int r1 = min(ms, e.y + kMfAsmRows);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  T* Fs = F + d.fo[s];
-  for (int c = d.cptr[s]; c < d.cptr[s + 1]; ++c) {
-    const int ch = d.clist[c];
-    const int mc = d.m[ch], npc = d.sfirst[ch + 1] - d.sfirst[ch], nu = mc - npc;
-    const int* em = d.emap + d.eptr[ch];
-    const T* Fc = F + d.fo[ch];
-    const int a0 = alo[e.z + (c - d.cptr[s])] + wave;
-    for (int c0 = 0; c0 < nu; c0 += 256) {
-      const int b0 = c0 + lane;
-      int eb[4];
-      bool ok[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int b = b0 + 64 * q;
-        ok[q] = b < nu;
-        eb[q] = ok[q] ? em[b] : 0;
-      }
-      for (int a = a0; a < nu; a += 16) {
-        // rows a, a + 4, a + 8, a + 12 of this wave (those that land in the range)
-        int pr[4];
-        bool in[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const int ak = a + 4 * k;
-          pr[k] = ak < nu ? em[ak] : r1;
-          in[k] = pr[k] < r1;
-        }
-        if (!in[0]) break;
-        T cv[4][4], pv[4][4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const T* crow = Fc + (long long)(npc + a + 4 * k) * mc + npc;
-          const T* prow = Fs + (long long)(in[k] ? pr[k] : 0) * ms;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            cv[k][q] = (in[k] && ok[q]) ? crow[b0 + 64 * q] : (T)0;
-            pv[k][q] = (in[k] && ok[q]) ? prow[eb[q]] : (T)0;
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          T* prow = Fs + (long long)(in[k] ? pr[k] : 0) * ms;
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            if (in[k] && ok[q]) prow[eb[q]] = pv[k][q] + cv[k][q];
-        }
-        if (!in[3]) break;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-template <class T>
-__device__ __forceinline__ bool mf_bad_pivot(T d) {
-  const double v = (double)d;
-  return !(fabs(v) > 0.0) || !isfinite(v);
-}
-
-// fronts of order <= 64: one wavefront per front, the front staged in LDS
-// (row stride m + 1) and its children's updates added there, then
-// right-looking over its pivots with lane i owning row i
-template <class T>
-__global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list, T* F, int* bad) {
-  extern __shared__ unsigned char mf_sm[];
-  T* A = reinterpret_cast<T*>(mf_sm);
-  const int s = list[blockIdx.x];
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const int ld = ms + 1;
-  T* Fs = F + d.fo[s];
-  const int t = threadIdx.x;
-  for (int i0 = 0; i0 < ms; i0 += 16) {
-    T v[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) v[q] = (t < ms && i0 + q < ms) ? Fs[(long long)(i0 + q) * ms + t] : (T)0;
-#pragma unroll
-    for (int q = 0; q < 16; ++q)
-      if (t < ms && i0 + q < ms) A[(i0 + q) * ld + t] = v[q];
-  }
-  __syncthreads();
-  // the children's Schur complements, one child after another (a child's
-  // update has at most ms rows and columns: lane t adds column t)
-  for (int c = d.cptr[s]; c < d.cptr[s + 1]; ++c) {
-    const int ch = d.clist[c];
-    const int mc = d.m[ch], npc = d.sfirst[ch + 1] - d.sfirst[ch], nu = mc - npc;
-    const int* em = d.emap + d.eptr[ch];
-    const T* Fc = F + d.fo[ch];
-    const int eb = t < nu ? em[t] : 0;     // lane t: parent position of the child's row/column t
-    const T* cb = Fc + (long long)npc * mc + npc + t;
-    int a = 0;
-    for (; a + 16 <= nu; a += 16) {
-      T v[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) v[q] = t < nu ? cb[(long long)(a + q) * mc] : (T)0;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) {
-        const int pr = __builtin_amdgcn_readlane(eb, a + q);
-        if (t < nu) A[pr * ld + eb] += v[q];
-      }
-    }
-    for (; a + 4 <= nu; a += 4) {
-      T v[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = t < nu ? cb[(long long)(a + q) * mc] : (T)0;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int pr = __builtin_amdgcn_readlane(eb, a + q);
-        if (t < nu) A[pr * ld + eb] += v[q];
-      }
-    }
-    for (; a < nu; ++a) {
-      const int pr = __builtin_amdgcn_readlane(eb, a);
-      if (t < nu) A[pr * ld + eb] += cb[(long long)a * mc];
-    }
-    __syncthreads();
-  }
-  bool fail = false, hard = false;
-  for (int k = 0; k < np; ++k) {
-    const T piv = A[k * ld + k];
-    if (mf_bad_pivot(piv)) { fail = true; hard = true; break; }
-    if (t > k && t < ms) {
-      T* ri = A + t * ld;
-      const T* rk = A + k * ld;
-      const T l = ri[k] / piv;
-      ri[k] = l;
-      if (!(fabs((double)l) <= 1.0e3)) fail = true;
-      int j = k + 1;
-      for (; j + 8 <= ms; j += 8) {
-        T u[8], a[8];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) u[q] = rk[j + q];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) a[q] = ri[j + q];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) ri[j + q] = a[q] - l * u[q];
-      }
-      for (; j < ms; ++j) ri[j] -= l * rk[j];
-    }
-    __syncthreads();
-  }
-  for (int i = 0; i < ms; ++i)
-    if (t < ms) Fs[(long long)i * ms + t] = A[i * ld + t];
-  if (__any(fail) && t == 0) atomicMin(bad, d.sfirst[s] + 1);
-  if (hard && t == 0) atomicOr(bad + 1, 1);
 }
 
 // Larger fronts: blocked by panels of kMfPanel columns, one launch per panel
@@ -537,6 +388,148 @@ __device__ __forceinline__ void mf_wave_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Assembly of a larger front: A's entries plus the children's Schur
+// complements, one child after another in their fixed order, so that every
+// element receives the same sums in the same order on every refactor.  One
+// workgroup per range of rows and columns (entries {front, first row, rows,
+// offset into alo}, {first column, columns, 0, 0}; at most kMfAsm elements, held
+// in LDS until they are complete, so a front is written once and never cleared
+// or read back).  Wavefront w owns the rows with index % 4 = w: no wavefront
+// waits for another.  alo holds, per entry and child, the child's rows [x, y)
+// that land in the range; a child's rows map to increasing parent rows.  Per
+// child and 256 columns a wavefront issues the loads of up to four rows at
+// once (512 x 512 grid, all levels: 263 us with A's entries in, where clearing the
+// fronts, scattering A and adding the children in memory took 400).
+constexpr int kMfAsmRows = 16;
+constexpr int kMfAsm = 4096;
+
+template <class T>
+__global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, const int2* alo, const double* vals,
+                                                     T* F) {
+  __shared__ T R[kMfAsm];
+  const int4 e = ent[2 * blockIdx.x], ec = ent[2 * blockIdx.x + 1];
+  const MfFront f = d.front[e.x];
+  const int r0 = e.y, rows = e.z, j0 = ec.x, w = ec.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int i = wave; i < rows; i += 4) {
+    for (int j = lane; j < w; j += 64) R[i * w + j] = (T)0;
+    mf_wave_fence();
+    const int* ar = d.arow + f.vo + r0 + i;
+    for (int q = ar[0] + lane; q < ar[1]; q += 64) {
+      const int j = d.acol[q] - j0;
+      // (an entry listed twice in a row adds up)
+      if (j >= 0 && j < w) atomicAdd(&R[i * w + j], (T)vals[d.aslot[q]]);
+    }
+  }
+  mf_wave_fence();
+  const int2* lo = alo + e.w;
+  for (int c = f.c0; c < f.c1; ++c) {
+    const MfChild ch = d.child[c];
+    const int2 ab = lo[c - f.c0];
+    if (ab.x >= ab.y) continue;
+    const int* em = d.emap + ch.em;
+    // slot k: the child's row that lands on this wavefront's row 4 k + wave
+    const int er = ab.x + lane < ab.y ? em[ab.x + lane] - r0 : -1;
+    int a[kMfAsmRows / 4];
+#pragma unroll
+    for (int k = 0; k < kMfAsmRows / 4; ++k) {
+      const unsigned long long hit = __ballot(er == 4 * k + wave);
+      a[k] = hit ? ab.x + (int)__builtin_ctzll(hit) : -1;
+    }
+    const T* Fc = F + ch.src;
+    for (int c0 = lane; c0 - lane < ch.nu; c0 += 256) {
+      int eb[4];
+      T cv[kMfAsmRows / 4][4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int b = c0 + 64 * q;
+        const int j = b < ch.nu ? em[b] - j0 : -1;
+        eb[q] = j < w ? j : -1;
+      }
+#pragma unroll
+      for (int k = 0; k < kMfAsmRows / 4; ++k) {
+        if (a[k] < 0) continue;
+        const T* crow = Fc + (long long)a[k] * ch.ld;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int b = c0 + 64 * q;
+          cv[k][q] = b < ch.nu ? crow[b] : (T)0;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < kMfAsmRows / 4; ++k) {
+        if (a[k] < 0) continue;
+        T* prow = R + (4 * k + wave) * w;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if (eb[q] >= 0) prow[eb[q]] += cv[k][q];
+      }
+    }
+    mf_wave_fence();
+  }
+  T* Fs = F + f.fo + (long long)r0 * f.m + j0;
+  for (int i = wave; i < rows; i += 4)
+    for (int j = lane; j < w; j += 64) Fs[(long long)i * f.m + j] = R[i * w + j];
+}
+
+// Fronts of order at most N (32 or 64): one wavefront per front.  A's entries
+// and the children's updates are added in LDS (row stride N + 1), one child
+// after another; then lane t holds row t in registers and the pivot rows are
+// broadcast from there: a pivot costs its reciprocal and the row updates, no
+// LDS traffic (512 x 512 grid, all levels: 300 us, 656 with the elimination in LDS).
+template <class T, int N>
+__global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list, const double* vals, T* F, int* bad) {
+  constexpr int ld = N + 1;
+  __shared__ T A[N * ld];
+  const MfFront f = d.front[list[blockIdx.x]];
+  const int ms = f.m, np = f.np, t = threadIdx.x;
+  if (t < ms) {
+    T* row = A + t * ld;
+    for (int j = 0; j < ms; ++j) row[j] = (T)0;
+    const int q1 = d.arow[f.vo + t + 1];
+    for (int q = d.arow[f.vo + t]; q < q1; ++q) row[d.acol[q]] += (T)vals[d.aslot[q]];
+  }
+  mf_wave_fence();
+  // a child's update has at most ms rows and columns: lane t adds column t
+  for (int c = f.c0; c < f.c1; ++c) {
+    const MfChild ch = d.child[c];
+    const int nu = ch.nu;
+    const int eb = t < nu ? d.emap[ch.em + t] : 0;   // parent position of the child's row/column t
+    const T* cb = F + ch.src + t;
+    for (int a = 0; a < nu; a += 16) {
+      T v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = (t < nu && a + q < nu) ? cb[(long long)(a + q) * ch.ld] : (T)0;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) {
+        if (a + q >= nu) break;
+        const int pr = __builtin_amdgcn_readlane(eb, a + q);
+        if (t < nu) A[pr * ld + eb] += v[q];
+      }
+    }
+    mf_wave_fence();
+  }
+  T v[N];
+  const T* own = A + (t < N ? t : 0) * ld;
+#pragma unroll
+  for (int q = 0; q < N; ++q) v[q] = (t < ms && q < ms) ? own[q] : (T)0;
+  int first = N;
+  bool hard = false;
+  T rd = (T)0;
+  mf_factor_rows<N, N>(v, t, ms, np, first, hard, rd);
+  if (t < ms) {
+    T* row = A + t * ld;
+#pragma unroll
+    for (int q = 0; q < N; ++q) row[q] = v[q];
+  }
+  mf_wave_fence();
+  T* Fs = F + f.fo;
+  for (int i = 0; i < ms; ++i)
+    if (t < ms) Fs[(long long)i * ms + t] = A[i * ld + t];
+  if (first < np) atomicMin(bad, f.first + first + 1);
+  if (__any(hard) && t == 0) atomicOr(bad + 1, 1);
 }
 
 constexpr int kMfStep = 192;              // threads of a step workgroup: three wavefronts
@@ -1018,16 +1011,18 @@ struct MfLu::Impl {
     for (auto& g : graphs)
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
   }
-  DevVec<int> sfirst, m, iptr, idx, cptr, clist, eptr, emap, vo, prow, pcol, bad;
-  DevVec<long long> fo, amap;
+  DevVec<int> sfirst, m, iptr, idx, cptr, clist, eptr, emap, vo, prow, pcol, bad, arow, acol, aslot;
+  DevVec<long long> fo;
+  DevVec<MfFront> front;
+  DevVec<MfChild> child;
   DevVec<double> F64, V64, y64, b64;
   DevVec<float> F32, V32, y32;
   DevVec<int> tiny_list, big_list;
-  DevVec<int4> aent;              // assembly entries of the larger fronts {front, first row, alo offset, 0}
-  DevVec<int> alo;                // per entry and child: first child row at or after the entry's first row
+  DevVec<int4> aent;              // assembly entries of the larger fronts, two each
+  DevVec<int2> alo;               // per entry and child: the child's rows in the entry's range
   DevVec<int4> sent;              // entries of the panel steps
   DevVec<double> dbuf;            // diagonal-block factors, two 32 x 32 slots per larger front of a level
-  std::vector<int> tiny_off, tiny_maxm, big_off;
+  std::vector<int> tiny_off, tiny_half, big_off;   // fronts up to order 32 at [tiny_off, tiny_half), up to 64 from there
   int big_maxm = 0;
   std::vector<int> aoff;          // per level: offset into aent
   struct Step { int p0, off, cnt; };
@@ -1036,6 +1031,7 @@ struct MfLu::Impl {
     MfDev d;
     d.sfirst = sfirst.p; d.m = m.p; d.fo = fo.p; d.iptr = iptr.p; d.idx = idx.p; d.cptr = cptr.p;
     d.clist = clist.p; d.eptr = eptr.p; d.emap = emap.p; d.vo = vo.p;
+    d.front = front.p; d.child = child.p; d.arow = arow.p; d.acol = acol.p; d.aslot = aslot.p;
     return d;
   }
 };
@@ -1051,7 +1047,7 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   const MfPlan& P = I.P;
   // every index a kernel reads is checked here
   for (int v : P.idx) if (v < 0 || v >= P.n) return XG_E_SETUP;
-  for (long long a : P.amap) if (a < 0 || a >= P.fo[P.ns]) return XG_E_SETUP;
+  for (int k : P.aslot) if (k < 0 || k >= s.nnz_a) return XG_E_SETUP;
   for (int c : P.clist) if (c < 0 || c >= P.ns) return XG_E_SETUP;
   for (int t = 0; t < P.ns; ++t) {
     if (P.m[t] < P.sfirst[t + 1] - P.sfirst[t] || P.sfirst[t + 1] <= P.sfirst[t]) return XG_E_SETUP;
@@ -1060,10 +1056,25 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
       if (e > P.eptr[t] && P.emap[e] <= P.emap[e - 1]) return XG_E_SETUP;   // assembly bisects the map
     }
   }
+  std::vector<MfFront> fr(P.ns);
+  std::vector<MfChild> chv(P.clist.size());
+  for (int t = 0; t < P.ns; ++t) {
+    const int np = P.sfirst[t + 1] - P.sfirst[t];
+    fr[t] = MfFront{P.fo[t], P.m[t], np, P.sfirst[t], P.iptr[t], P.cptr[t], P.cptr[t + 1], P.vo[t], 0};
+    for (int i = 0; i < P.m[t]; ++i)
+      for (int q = P.arow[P.vo[t] + i]; q < P.arow[P.vo[t] + i + 1]; ++q)
+        if (P.acol[q] < 0 || P.acol[q] >= P.m[t]) return XG_E_SETUP;
+  }
+  for (size_t c = 0; c < P.clist.size(); ++c) {
+    const int t = P.clist[c], np = P.sfirst[t + 1] - P.sfirst[t];
+    chv[c] = MfChild{P.fo[t] + (long long)np * P.m[t] + np, P.m[t], P.m[t] - np, P.eptr[t], P.vo[t] + np};
+  }
   hipStream_t st = I.st;
+  MFCHK(I.front.up(fr, st)); MFCHK(I.child.up(chv, st));
+  MFCHK(I.arow.up(P.arow, st)); MFCHK(I.acol.up(P.acol, st)); MFCHK(I.aslot.up(P.aslot, st));
   MFCHK(I.sfirst.up(P.sfirst, st)); MFCHK(I.m.up(P.m, st)); MFCHK(I.iptr.up(P.iptr, st)); MFCHK(I.idx.up(P.idx, st));
   MFCHK(I.cptr.up(P.cptr, st)); MFCHK(I.clist.up(P.clist, st)); MFCHK(I.eptr.up(P.eptr, st));
-  MFCHK(I.emap.up(P.emap, st)); MFCHK(I.vo.up(P.vo, st)); MFCHK(I.fo.up(P.fo, st)); MFCHK(I.amap.up(P.amap, st));
+  MFCHK(I.emap.up(P.emap, st)); MFCHK(I.vo.up(P.vo, st)); MFCHK(I.fo.up(P.fo, st));
   MFCHK(I.prow.up(s.perm_row, st)); MFCHK(I.pcol.up(s.perm_col, st));
   MFCHK(I.bad.alloc(2));
   MFCHK(I.F64.alloc(P.fo[P.ns])); MFCHK(I.V64.alloc(P.vo[P.ns])); MFCHK(I.y64.alloc(P.n)); MFCHK(I.b64.alloc(P.n));
@@ -1076,24 +1087,26 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   int max_slots = 1;
   I.tiny_off.assign(nl + 1, 0);
   I.big_off.assign(nl + 1, 0);
-  I.tiny_maxm.assign(nl, 0);
+  I.tiny_half.assign(nl, 0);
   I.steps.assign(nl, {});
   I.big_maxm = 0;
   for (int l = 0; l < nl; ++l) {
     I.tiny_off[l] = (int)tl.size();
     I.big_off[l] = (int)bl.size();
     int maxp = 0;
+    std::vector<int> mid;
     for (int q = P.lvl_ptr[l]; q < P.lvl_ptr[l + 1]; ++q) {
       const int t = P.lvl_s[q];
       if (P.m[t] <= kMfTiny) {
-        tl.push_back(t);
-        I.tiny_maxm[l] = std::max(I.tiny_maxm[l], P.m[t]);
+        (P.m[t] <= kMfTiny / 2 ? tl : mid).push_back(t);
       } else {
         bl.push_back(t);
         I.big_maxm = std::max(I.big_maxm, P.m[t]);
         maxp = std::max(maxp, (P.sfirst[t + 1] - P.sfirst[t] + kMfPanel - 1) / kMfPanel);
       }
     }
+    I.tiny_half[l] = (int)tl.size();
+    tl.insert(tl.end(), mid.begin(), mid.end());
     const int nb = (int)bl.size() - I.big_off[l];
     max_slots = std::max(max_slots, nb);
     for (int j = 0; nb > 0 && j <= maxp; ++j) {
@@ -1126,28 +1139,32 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   MFCHK(I.big_list.up(bl, st));
   MFCHK(I.sent.up(se, st));
   MFCHK(I.dbuf.alloc((size_t)max_slots * 2 * kMfPanel * kMfPanel));
-  // assembly of the larger fronts: 32 parent rows per workgroup (the tiny
-  // fronts assemble their children inside their factor kernel)
+  // assembly of the larger fronts, ranges of rows and columns (the tiny fronts
+  // assemble themselves inside their factor kernel)
   std::vector<int4> ae;
-  std::vector<int> lo;
+  std::vector<int2> lo;
   I.aoff.assign(nl + 1, 0);
   for (int l = 0; l < nl; ++l) {
-    I.aoff[l] = (int)ae.size();
+    I.aoff[l] = (int)ae.size() / 2;
     for (int b = I.big_off[l]; b < I.big_off[l + 1]; ++b) {
-      const int t = bl[b];
-      if (P.cptr[t + 1] == P.cptr[t]) continue;
-      for (int r0 = 0; r0 < P.m[t]; r0 += kMfAsmRows) {
-        ae.push_back(make_int4(t, r0, (int)lo.size(), 0));
+      const int t = bl[b], m = P.m[t];
+      const int w = std::min(m, kMfAsm / 4), rows = std::min(kMfAsmRows, kMfAsm / w);
+      for (int r0 = 0; r0 < m; r0 += rows) {
+        const int off = (int)lo.size();
         for (int c = P.cptr[t]; c < P.cptr[t + 1]; ++c) {
           const int ch = P.clist[c];
           const int* eb = P.emap.data() + P.eptr[ch];
           const int* ee = P.emap.data() + P.eptr[ch + 1];
-          lo.push_back((int)(std::lower_bound(eb, ee, r0) - eb));
+          lo.push_back(make_int2((int)(std::lower_bound(eb, ee, r0) - eb), (int)(std::lower_bound(eb, ee, r0 + rows) - eb)));
+        }
+        for (int j0 = 0; j0 < m; j0 += w) {
+          ae.push_back(make_int4(t, r0, std::min(rows, m - r0), off));
+          ae.push_back(make_int4(j0, std::min(w, m - j0), 0, 0));
         }
       }
     }
   }
-  I.aoff[nl] = (int)ae.size();
+  I.aoff[nl] = (int)ae.size() / 2;
   MFCHK(I.aent.up(ae, st));
   MFCHK(I.alo.up(lo, st));
   MFCHK(hipStreamSynchronize(st));
@@ -1170,22 +1187,21 @@ template <class T>
 static int mf_factor_enqueue(MfLu::Impl& I, const double* vals_dev, int nnz, T* F) {
   const MfPlan& P = I.P;
   hipStream_t st = I.st;
-  const long long tot = P.fo[P.ns];
-  hipLaunchKernelGGL(k_mf_fill<T>, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, F, tot);
-  hipLaunchKernelGGL(k_mf_scatter<T>, dim3((nnz + 255) / 256), dim3(256), 0, st, nnz, vals_dev, I.amap.p, F);
   hipLaunchKernelGGL(k_mf_flag_init<T>, dim3(1), dim3(1), 0, st, I.bad.p);
   const MfDev d = I.dev();
   T* dbuf = reinterpret_cast<T*>(I.dbuf.p);
   const int nl = (int)P.lvl_ptr.size() - 1;
   for (int l = 0; l < nl; ++l) {
     const int na = I.aoff[l + 1] - I.aoff[l];
-    if (na) hipLaunchKernelGGL(k_mf_assemble<T>, dim3(na), dim3(256), 0, st, d, I.aent.p + I.aoff[l], I.alo.p, F);
-    const int nt = I.tiny_off[l + 1] - I.tiny_off[l];
-    if (nt) {
-      const int mm = I.tiny_maxm[l];
-      hipLaunchKernelGGL(k_mf_factor_tiny<T>, dim3(nt), dim3(64), (size_t)mm * (mm + 1) * sizeof(T), st, d,
-                         I.tiny_list.p + I.tiny_off[l], F, I.bad.p);
-    }
+    if (na)
+      hipLaunchKernelGGL(k_mf_assemble<T>, dim3(na), dim3(256), 0, st, d, I.aent.p + 2 * I.aoff[l], I.alo.p, vals_dev, F);
+    const int n32 = I.tiny_half[l] - I.tiny_off[l], n64 = I.tiny_off[l + 1] - I.tiny_half[l];
+    if (n32)
+      hipLaunchKernelGGL((k_mf_factor_tiny<T, kMfTiny / 2>), dim3(n32), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l],
+                         vals_dev, F, I.bad.p);
+    if (n64)
+      hipLaunchKernelGGL((k_mf_factor_tiny<T, kMfTiny>), dim3(n64), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_half[l],
+                         vals_dev, F, I.bad.p);
     for (const auto& S : I.steps[l])
       hipLaunchKernelGGL(k_mf_step<T>, dim3(S.cnt), dim3(kMfStep), 0, st, d, I.sent.p + S.off, S.p0, F, dbuf,
                          (S.p0 / kMfPanel) & 1, I.bad.p);

@@ -127,7 +127,9 @@ struct MfPlan {
   std::vector<int> m;              // front order (pivots + rows below)
   std::vector<long long> fo;       // front element offsets (row-major fronts), fo[ns] = total
   std::vector<int> iptr, idx;      // front index lists (B indices), pivots first
-  std::vector<long long> amap;     // A slot -> front element
+  // A's entries by front row: row i of front t holds those at
+  // [arow[vo[t] + i], arow[vo[t] + i + 1]): front column and A slot
+  std::vector<int> arow, acol, aslot;
   std::vector<int> cptr, clist;    // children of each supernode
   std::vector<int> eptr, emap;     // per supernode: parent-local index of each row below its pivots
   std::vector<int> lvl_ptr, lvl_s; // supernodes by level, leaves first
