@@ -175,15 +175,14 @@ struct MfChild {
   int em, vsrc;                 // parent positions of its rows; their slots in the front vectors
 };
 struct MfDev {
-  const int* sfirst; const int* m; const long long* fo; const int* iptr; const int* idx;
-  const int* cptr; const int* clist; const int* eptr; const int* emap; const int* vo;
-  const MfFront* front; const MfChild* child;
+  const int* sfirst; const int* m; const long long* fo;
+  const MfFront* front; const MfChild* child; const int* emap;
+  const int* bidx; const int* xidx;      // of the fronts' rows: index into b, into x
   const int* arow; const int* acol; const int* aslot;
 };
 
 constexpr int kMfTiny = 64;     // fronts up to this order: one wavefront, the front in LDS
 constexpr int kMfPanel = 32;    // panel width of the blocked factorisation (64 spills the register panel)
-constexpr int kMfSolveBlock = 1024;
 
 // f(0), f(1), ... f(N - 1) with the index a constant in each
 template <int N, int K = 0, class F>
@@ -233,9 +232,9 @@ __device__ __forceinline__ T mf_wave_sum(T v) {
 // complement.  The chain of panels is what bounds a tree's top: one launch per
 // panel instead of a panel and an update launch, and no operand passes through
 // LDS on its way to the matrix cores, so that a step is one round of loads, the
-// diagonal's 32 dependent pivots and a substitution (16.8 us where the two
-// launches took 31.6, on the 865-order root of a 512 x 512 grid; 10.7 to 20 us
-// with FP32 factors and up to 720 workgroups).
+// diagonal's 32 dependent pivots and a substitution (12.5 us where the two
+// launches took 31.6, on the 865-order root of a 512 x 512 grid: loads and update
+// 3.8 us, pivots 4.5, substitution and stores 3.3; mean over all its steps 14.2).
 //
 // v_mfma_{f64,f32}_16x16x4: lane l holds A's row l % 16, column l / 16 of the
 // 16 x 4 block, B's row l / 16, column l % 16 of the 4 x 16 block; accumulator
@@ -287,31 +286,46 @@ __device__ __forceinline__ void mf_update_blocks(const T* Fs, long long ld, int 
       for (int b = 0; b < NB; ++b) acc[a][b][r] = mf_at(C, o + cj[b]);
     }
   if (kw <= 0) return;
+  // step k of the product takes the columns 8 lk + k of L (a lane's eight lie
+  // next to each other in memory) and the same rows of U
   T l[NA][kMfPanel / 4], u[NB][kMfPanel / 4];
   const T* Lb = Fs + i0 * ld + q0;
   const T* Ub = Fs + q0 * ld + j0;
+  if (kw == kMfPanel) {
+    typedef T Pair __attribute__((ext_vector_type(2), aligned(sizeof(T))));
 #pragma unroll
-  for (int a = 0; a < NA; ++a) {
-    const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row;
+    for (int a = 0; a < NA; ++a) {
+      const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row + 8 * lk * (unsigned)sizeof(T);
 #pragma unroll
-    for (int k = 0; k < kMfPanel / 4; ++k) l[a][k] = mf_at(Lb, o + (unsigned)min(4 * k + lk, kw - 1) * (unsigned)sizeof(T));
+      for (int k = 0; k < kMfPanel / 4; k += 2) {
+        const Pair p = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(Lb) + o + k * sizeof(T));
+        l[a][k] = -p.x;
+        l[a][k + 1] = -p.y;
+      }
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+      const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row;
+#pragma unroll
+      for (int k = 0; k < kMfPanel / 4; ++k) {
+        const T v = mf_at(Lb, o + (unsigned)min(8 * lk + k, kw - 1) * (unsigned)sizeof(T));
+        l[a][k] = 8 * lk + k < kw ? -v : (T)0;
+      }
+    }
   }
 #pragma unroll
   for (int k = 0; k < kMfPanel / 4; ++k) {
-    const unsigned o = (unsigned)min(4 * k + lk, kw - 1) * row;
+    const unsigned o = (unsigned)min(8 * lk + k, kw - 1) * row;
 #pragma unroll
     for (int b = 0; b < NB; ++b) u[b][k] = mf_at(Ub, o + cj[b]);
   }
 #pragma unroll
-  for (int k = 0; k < kMfPanel / 4; ++k) {
-    const bool in = 4 * k + lk < kw;
+  for (int k = 0; k < kMfPanel / 4; ++k)
 #pragma unroll
-    for (int a = 0; a < NA; ++a) {
-      const T lv = in ? -l[a][k] : (T)0;
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc[a][b] = MfAcc<T>::mma(lv, u[b][k], acc[a][b]);
-    }
-  }
+      for (int b = 0; b < NB; ++b) acc[a][b] = MfAcc<T>::mma(l[a][k], u[b][k], acc[a][b]);
 }
 
 // reciprocal of a pivot in four stages that run between the products of a row
@@ -354,33 +368,60 @@ __device__ __forceinline__ void mf_row_update(T (&v)[N], T l, int k, int q0, MfR
   }
 }
 
-// right-looking LU of the rows in registers (lane t: row t), pivots [0, NP) of
-// N columns; lanes from `rows` on count for nothing.  first: lowest column with
-// a bad pivot or a multiplier beyond KLU's threshold; rd: lane k's reciprocal
-// of pivot k.  Constant trip counts keep the rows in registers.
-template <int N, int NP, class T>
-__device__ __forceinline__ void mf_factor_rows(T (&v)[N], int lane, int rows, int np, int& first, bool& hard, T& rd) {
+// right-looking LU of the rows in registers (lane t: row t), the first np <= N
+// pivots; rd: lane k's reciprocal of pivot k.  Constant trip counts keep the
+// rows in registers.
+template <int N, class T>
+__device__ __forceinline__ void mf_factor_rows(T (&v)[N], int lane, int np, T& rd) {
   MfRecip<T> rec;
-  T piv = mf_bcast(v[0], 0);
-  rec.p = piv;
+  rec.p = mf_bcast(v[0], 0);
 #pragma unroll
   for (int i = 0; i < 4; ++i) rec.stage(i);
-  mf_for<NP>([&](auto kc) MF_INLINE {
+  mf_for<N>([&](auto kc) MF_INLINE {
     constexpr int k = kc, k1 = k + 1 < N ? k + 1 : k;
     if (k >= np) return;
     const T rp = rec.x;
-    if (!(fabs((double)piv) > 0.0) || !isfinite((double)piv)) { first = min(first, k); hard = true; }
-    if (lane == k) rd = rp;
-    const bool upd = lane > k && lane < rows;
-    const T l = upd ? v[k] * rp : (T)0;
-    if (upd) v[k] = l;
-    if (!(fabs((double)l) <= 1.0e3)) first = min(first, k);
+    rd = lane == k ? rp : rd;
+    const T l = lane > k ? v[k] * rp : (T)0;
+    v[k] = lane > k ? l : v[k];
     if constexpr (k1 > k) v[k1] -= l * mf_bcast(v[k1], k);
-    piv = mf_bcast(v[k1], k1);
-    rec.p = piv;
+    rec.p = mf_bcast(v[k1], k1);
     mf_row_update<N>(v, l, k, k + 2, rec);
     __builtin_amdgcn_sched_barrier(0);
   });
+}
+
+__device__ __forceinline__ unsigned mf_abs_high(double v) {
+  return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32) & 0x7fffffffu;
+}
+__device__ __forceinline__ unsigned mf_abs_high(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+
+// the lowest of the first np columns of factored rows (lane t: row t, t < rows;
+// also in memory, at(k)) with a bad pivot or a multiplier beyond KLU's
+// threshold, or N.  The high words of absolute values order like the values, NaN
+// last: one maximum over the multipliers and the pivot's word tell whether
+// anything has to be looked at.
+template <int N, class T, class At>
+__device__ __forceinline__ int mf_check_rows(const T (&v)[N], int lane, int rows, int np, const At& at, bool& hard) {
+  unsigned top = 0, piv = mf_abs_high((T)1);
+  // (the comparisons are made here: kept from the factorisation they would spill)
+  asm volatile("" : "+v"(lane), "+v"(np));
+  const int lim = min(lane, np), own = lane < np ? lane : -1;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const unsigned h = mf_abs_high(v[k]);
+    top = max(top, lim > k ? h : 0);
+    piv = own == k ? h : piv;
+  }
+  const bool look = lane < rows && (top >= mf_abs_high((T)1.0e3) || piv == 0 || piv >= mf_abs_high((T)INFINITY));
+  int first = N;
+  if (__any(look) && lane < rows)
+    for (int k = min(min(np, N) - 1, lane); k >= 0; --k) {
+      const double a = fabs((double)at(k));
+      const bool p = lane == k;
+      if (p ? !(a > 0.0) || !isfinite(a) : !(a <= 1.0e3)) { first = k; hard |= p; }
+    }
+  return first;
 }
 
 // LDS written by a wavefront's lanes is visible to its other lanes
@@ -515,16 +556,16 @@ __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list,
   const T* own = A + (t < N ? t : 0) * ld;
 #pragma unroll
   for (int q = 0; q < N; ++q) v[q] = (t < ms && q < ms) ? own[q] : (T)0;
-  int first = N;
   bool hard = false;
   T rd = (T)0;
-  mf_factor_rows<N, N>(v, t, ms, np, first, hard, rd);
+  mf_factor_rows<N>(v, t, np, rd);
   if (t < ms) {
     T* row = A + t * ld;
 #pragma unroll
     for (int q = 0; q < N; ++q) row[q] = v[q];
   }
   mf_wave_fence();
+  const int first = mf_check_rows<N>(v, t, ms, np, [&](int k) MF_INLINE { return A[t * ld + k]; }, hard);
   T* Fs = F + f.fo;
   for (int i = 0; i < ms; ++i)
     if (t < ms) Fs[(long long)i * ms + t] = A[i * ld + t];
@@ -543,7 +584,6 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
   constexpr int PW = kMfPanel;
   __shared__ __attribute__((aligned(16))) T Du[PW * kMfDs];   // U11 by rows
   __shared__ __attribute__((aligned(16))) T Dl[PW * kMfDs];   // L11 by columns; the updated block before it is factored
-  __shared__ T Rd[PW];
   __shared__ T Ts[2][kMfTile];
   const int4 e = ent[blockIdx.x];
   const int s = e.x, slot = e.w;
@@ -585,6 +625,7 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
   T* Tl = Ts[wave > 1];
   const int o0 = base + (lower ? blk : blk - nrb) * 64;     // first row or column of the block
   if (wave == 0) {
+    __builtin_amdgcn_s_setprio(3);       // the others wait for this wavefront: its loads first
     V acc[2][2];
     mf_update_blocks<T, 2, 2>(Fs, ld, p0, base, p0, base, q0, kw, lane, acc);
 #pragma unroll
@@ -626,8 +667,8 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
     for (int q = 0; q < PW; ++q) v[q] = Dl[row * kMfDs + q];
     T rd = (T)1;
-    mf_factor_rows<PW, PW>(v, lane, PW, PW, failed, hard, rd);
-    if (lane < PW) Rd[lane] = rd;
+    mf_factor_rows<PW>(v, lane, PW, rd);
+    if (lane < PW) Du[lane * kMfDs + PW] = rd;      // the pivots' reciprocals behind the rows
   } else if (has && lower) {
 #pragma unroll
     for (int q = 0; q < PW; ++q) v[q] = Tl[lane * (PW + 1) + q];
@@ -642,51 +683,72 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
       Du[lane * kMfDs + q] = v[q];
       Dl[q * kMfDs + lane] = v[q];
     }
-    if (e.y == 0) {
-      T* db = dbuf + ((long long)slot * 2 + half) * PW * PW + lane * PW;
-#pragma unroll
-      for (int q = 0; q < PW; ++q) db[q] = v[q];
-    }
   }
   __syncthreads();
+  if (wave == 0)
+    failed = mf_check_rows<PW>(v, lane, PW, PW, [&](int k) MF_INLINE { return Du[lane * kMfDs + k]; }, hard);
+  if (wave == 0 && e.y == 0 && lane < PW) {
+    T* db = dbuf + ((long long)slot * 2 + half) * PW * PW + lane * PW;
+#pragma unroll
+    for (int q = 0; q < PW; ++q) db[q] = v[q];
+  }
   if (has) {
+    // the factors' rows come two values at a time from LDS; row k + 1 is read
+    // while row k is applied (its address is tied to v[k], so that no more than
+    // two rows are held in registers)
+    typedef T Pair __attribute__((ext_vector_type(2)));
+    typedef const __attribute__((address_space(3))) T* Lds;
+    typedef const __attribute__((address_space(3))) Pair* LdsPair;
+    Lds pd = (Lds)(lower ? Du : Dl);
+    T u[PW], un[PW];
+    auto fetch = [&](auto kc, T (&to)[PW]) MF_INLINE {
+      constexpr int k = kc;
+#pragma unroll
+      for (int q = (k + 1) & ~1; q < PW; q += 2) {
+        const Pair p = *(LdsPair)(pd + k * kMfDs + q);
+        to[q] = p.x;
+        to[q + 1] = p.y;
+      }
+    };
+    fetch(std::integral_constant<int, 0>{}, u);
     if (lower) {
       const bool valid = o0 + lane < ms;
-      // row k + 1 of U11 is read while row k is applied (z, zero, is tied to
-      // v[k] so that at most two rows are held in registers)
-      int z = 0;
-      T u[PW], un[PW];
-#pragma unroll
-      for (int q = 0; q < PW; ++q) u[q] = Du[q];
-      T r = Rd[0];
+      T r = pd[PW], rn = r;
       mf_for<PW>([&](auto kc) MF_INLINE {
-        constexpr int k = kc, k1 = k + 1 < PW ? k + 1 : k;
-        asm volatile("" : "+v"(z) : "v"(v[k]));
-        const T rn = Rd[k1 + z];
-#pragma unroll
-        for (int q = k + 2; q < PW; ++q) un[q] = Du[z + k1 * kMfDs + q];
+        constexpr int k = kc;
+        asm volatile("" : "+v"(pd) : "v"(v[k]));
+        if constexpr (k + 1 < PW) {
+          fetch(std::integral_constant<int, k + 1>{}, un);
+          rn = pd[(k + 1) * kMfDs + PW];
+        }
         v[k] *= r;
+        r = rn;
         if (valid && !(fabs((double)v[k]) <= 1.0e3)) failed = min(failed, k);
 #pragma unroll
         for (int q = k + 1; q < PW; ++q) v[q] -= v[k] * u[q];
 #pragma unroll
         for (int q = k + 2; q < PW; ++q) u[q] = un[q];
-        r = rn;
         __builtin_amdgcn_sched_barrier(0);
       });
+      // the lane's row of L21: 32 values next to each other
+      if (valid) {
+        T* to = Fs + (o0 + lane) * ld + p0;
+        if (pw == PW) {
+          typedef T Pair8 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
 #pragma unroll
-      for (int q = 0; q < PW; ++q) Tl[lane * (PW + 1) + q] = v[q];
+          for (int q = 0; q < PW; q += 2) *reinterpret_cast<Pair8*>(to + q) = Pair8{v[q], v[q + 1]};
+        } else {
+#pragma unroll
+          for (int q = 0; q < PW; ++q)
+            if (q < pw) to[q] = v[q];
+        }
+      }
     } else {
       const int c = o0 + lane;
-      int z = 0;
-      T u[PW], un[PW];
-#pragma unroll
-      for (int q = 0; q < PW; ++q) u[q] = Dl[q];
       mf_for<PW>([&](auto kc) MF_INLINE {
-        constexpr int k = kc, k1 = k + 1 < PW ? k + 1 : k;
-        asm volatile("" : "+v"(z) : "v"(v[k]));
-#pragma unroll
-        for (int q = k + 2; q < PW; ++q) un[q] = Dl[z + k1 * kMfDs + q];
+        constexpr int k = kc;
+        asm volatile("" : "+v"(pd) : "v"(v[k]));
+        if constexpr (k + 1 < PW) fetch(std::integral_constant<int, k + 1>{}, un);
 #pragma unroll
         for (int q = k + 1; q < PW; ++q) v[q] -= u[q] * v[k];
 #pragma unroll
@@ -698,276 +760,336 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
         if (c < ms && q < pw) Fs[(p0 + q) * ld + c] = v[q];
     }
   }
-  __syncthreads();
-  // the L21 blocks, row by row
-#pragma unroll
-  for (int w = 0; w < 2; ++w) {
-    const int b = 2 * e.y + w, r0 = base + b * 64;
-    if (b >= nrb) break;
-    for (int x = t; x < 64 * PW; x += kMfStep) {
-      const int i = x / PW, q = x % PW;
-      if (r0 + i < ms && q < pw) Fs[(r0 + i) * ld + p0 + q] = Ts[w][i * (PW + 1) + q];
-    }
-  }
   if (failed < pw) atomicMin(bad, d.sfirst[s] + p0 + failed + 1);
   if (__any(hard) && lane == 0) atomicOr(bad + 1, 1);
 }
 
-// sums over c in [c0, c1) of F[r + k][c] v[c] for the rows r .. r + nr - 1
-// (nr <= 4, wave-uniform) of a row-major front, by one wavefront: every lane
-// keeps eight loads in flight (four rows, two column blocks), so the four rows
-// share their memory round trips; row k's sum is returned in out[k] in every
-// lane
-template <class T>
-__device__ __forceinline__ void mf_rows_dot4(const T* Fs, long long ms, int r, int nr, const T* v, int c0, int c1,
-                                             int lane, T out[4]) {
-  const T* row[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) row[k] = Fs + (long long)(r + (k < nr ? k : 0)) * ms;
-  T a[4], b[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) { a[k] = (T)0; b[k] = (T)0; }
-  int c = c0 + lane;
-  for (; c + 64 < c1; c += 128) {
-    const T v0 = v[c], v1 = v[c + 64];
-    T f0[4], f1[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { f0[k] = row[k][c]; f1[k] = row[k][c + 64]; }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { a[k] += f0[k] * v0; b[k] += f1[k] * v1; }
-  }
-  if (c < c1) {
-    const T v0 = v[c];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) a[k] += row[k][c] * v0;
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) out[k] = mf_wave_sum(a[k] + b[k]);
-}
-
 // ---- solves.  V holds, per front, the vector of its index list: y on the
-// pivot rows, the update for the parent below them.
+// pivot rows, the update for the parent below them.  The right-hand side is
+// read, and the solution written, in A's numbering.
 
-// sum the children's updates into the front's vector Vl (LDS)
-template <class T>
-__device__ __forceinline__ void mf_gather_children(const MfDev& d, int s, const T* V, T* Vl) {
-  for (int c = d.cptr[s]; c < d.cptr[s + 1]; ++c) {
-    const int ch = d.clist[c];
-    const int npc = d.sfirst[ch + 1] - d.sfirst[ch], nu = d.m[ch] - npc;
-    const T* Vc = V + d.vo[ch];
-    const int* em = d.emap + d.eptr[ch];
-    for (int a = threadIdx.x; a < nu; a += blockDim.x) Vl[em[a]] += Vc[npc + a];
-    __syncthreads();
+// partial sums of this lane (to be added over the wavefront) of F[r + k][c] x(c)
+// over c in [c0, c1), for the NR rows from r on (rows from nr on repeat the
+// last): 4 NR loads in flight, so the rows share their memory round trips
+template <int NR, class T, class X>
+__device__ __forceinline__ void mf_rows_part(const T* Fs, long long ld, int r, int nr, int c0, int c1, int lane,
+                                             const X& x, T (&acc)[NR]) {
+  const T* row[NR];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) { row[k] = Fs + (long long)(r + min(k, nr - 1)) * ld; acc[k] = (T)0; }
+  for (int c = c0; c < c1; c += 256) {
+    T xv[4], f[NR][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int j = c + 64 * q + lane, jj = min(j, c1 - 1);
+#pragma unroll
+      for (int k = 0; k < NR; ++k) f[k][q] = row[k][jj];
+      xv[q] = j < c1 ? x(jj) : (T)0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int k = 0; k < NR; ++k)
+        if (c + 64 * q < c1) acc[k] += f[k][q] * xv[q];
   }
 }
 
-// forward, fronts of order <= 64: one wavefront, lane i owns row i
+// forward, fronts of order <= 64: one wavefront, lane i owns row i; sixteen
+// columns of the rows are loaded before the pivots that use them
 template <class T>
-__global__ void __launch_bounds__(64) k_mf_fwd_tiny(MfDev d, const int* list, const T* F, T* V, const double* b,
-                                                    T* yg) {
+__global__ void __launch_bounds__(64) k_mf_fwd_tiny(MfDev d, const int* list, const T* F, T* V, const double* b) {
   __shared__ T Vl[kMfTiny];
-  const int s = list[blockIdx.x];
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const T* Fs = F + d.fo[s];
-  const int* ix = d.idx + d.iptr[s];
-  const int t = threadIdx.x;
-  Vl[t] = t < np ? (T)b[ix[t]] : (T)0;
-  __syncthreads();
-  mf_gather_children(d, s, V, Vl);
-  T v = Vl[t];
-  for (int k = 0; k < np; ++k) {
-    const T yk = mf_bcast(v, k);
-    if (t > k && t < ms) v -= Fs[(long long)t * ms + k] * yk;
+  const MfFront f = d.front[list[blockIdx.x]];
+  const int ms = f.m, np = f.np, t = threadIdx.x;
+  Vl[t] = t < np ? (T)b[d.bidx[f.idx + t]] : (T)0;
+  mf_wave_fence();
+  // the next child's values are loaded while this one's are added
+  MfChild ch{};
+  int e = -1;
+  T v = (T)0;
+  auto fetch = [&](int c) MF_INLINE {
+    e = -1;
+    if (c >= f.c1) return;
+    ch = d.child[c];
+    if (t < ch.nu) { e = d.emap[ch.em + t]; v = V[ch.vsrc + t]; }
+  };
+  fetch(f.c0);
+  for (int c = f.c0; c < f.c1; ++c) {
+    const int ec = e;
+    const T vc = v;
+    fetch(c + 1);
+    if (ec >= 0) Vl[ec] += vc;
+    mf_wave_fence();
   }
-  if (t < ms) V[d.vo[s] + t] = v;
-  if (t < np) yg[ix[t]] = v;
-}
-
-// forward, larger fronts: one workgroup per front, the vector in LDS; the
-// unit-lower L11 by 64-row blocks (rows updated by a row-wise product with the
-// solved part, then the block's triangle solved by one wavefront from LDS),
-// then the rows below the pivots updated by L21 y
-template <class T>
-__global__ void __launch_bounds__(kMfSolveBlock) k_mf_fwd_big(MfDev d, const int* list, const T* F, T* V,
-                                                             const double* b, T* yg, int ldsv) {
-  extern __shared__ unsigned char mf_sm[];
-  T* Bl = reinterpret_cast<T*>(mf_sm);          // 64 x 65 block
-  const int s = list[blockIdx.x];
-  T* Vl = ldsv ? Bl + 64 * 65 : V + d.vo[s];    // the front's vector (ms)
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const T* Fs = F + d.fo[s];
-  const int* ix = d.idx + d.iptr[s];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
-  for (int i = t; i < ms; i += blockDim.x) Vl[i] = i < np ? (T)b[ix[i]] : (T)0;
-  __syncthreads();
-  mf_gather_children(d, s, V, Vl);
-  for (int b0 = 0; b0 < np; b0 += 64) {
-    const int bw = min(64, np - b0);
-    if (b0 > 0) {
-      for (int rr = 4 * wave; rr < bw; rr += 4 * nw) {
-        const int nr = min(4, bw - rr);
-        T acc[4];
-        mf_rows_dot4(Fs, ms, b0 + rr, nr, Vl, 0, b0, lane, acc);
-        if (lane == 0)
+  v = Vl[t];
+  const T* row = F + f.fo + (long long)min(t, ms - 1) * ms;
+  for (int k0 = 0; k0 < np; k0 += 16) {
+    T l[16];
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (k < nr) Vl[b0 + rr + k] -= acc[k];
-      }
-    }
-    {
-      T v[64 * 64 / kMfSolveBlock];
+    for (int q = 0; q < 16; ++q) l[q] = row[min(k0 + q, np - 1)];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int it = 0; it < 64 * 64 / kMfSolveBlock; ++it) {
-        const int x = t + it * kMfSolveBlock, i = x >> 6, j = x & 63;
-        v[it] = (i < bw && j < i) ? Fs[(long long)(b0 + i) * ms + b0 + j] : (T)0;
-      }
-#pragma unroll
-      for (int it = 0; it < 64 * 64 / kMfSolveBlock; ++it) {
-        const int x = t + it * kMfSolveBlock;
-        Bl[(x >> 6) * 65 + (x & 63)] = v[it];
-      }
+    for (int q = 0; q < 16; ++q) {
+      const T yk = mf_bcast(v, k0 + q);
+      const T w = v - l[q] * yk;
+      v = (k0 + q < np && t > k0 + q) ? w : v;
     }
-    __syncthreads();
-    if (wave == 0) {
-      T v = lane < bw ? Vl[b0 + lane] : (T)0;
-      for (int k = 0; k < bw; ++k) {
-        const T yk = mf_bcast(v, k);
-        if (lane > k && lane < bw) v -= Bl[lane * 65 + k] * yk;
-      }
-      if (lane < bw) Vl[b0 + lane] = v;
-    }
-    __syncthreads();
   }
-  for (int rr = np + 4 * wave; rr < ms; rr += 4 * nw) {
-    const int nr = min(4, ms - rr);
-    T acc[4];
-    mf_rows_dot4(Fs, ms, rr, nr, Vl, 0, np, lane, acc);
-    if (lane == 0)
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (k < nr) Vl[rr + k] -= acc[k];
-  }
-  __syncthreads();
-  if (ldsv)
-    for (int i = t; i < ms; i += blockDim.x) V[d.vo[s] + i] = Vl[i];
-  for (int i = t; i < np; i += blockDim.x) yg[ix[i]] = Vl[i];
+  if (t < ms) V[f.vo + t] = v;
 }
 
 // backward, fronts of order <= 64 (roots first): x = U11^-1 (y - U12 x_below)
 template <class T>
-__global__ void __launch_bounds__(64) k_mf_bwd_tiny(MfDev d, const int* list, const T* F, T* x) {
-  __shared__ T Xl[kMfTiny];
-  const int s = list[blockIdx.x];
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const T* Fs = F + d.fo[s];
-  const int* ix = d.idx + d.iptr[s];
-  const int t = threadIdx.x;
-  if (t < ms) Xl[t] = x[ix[t]];           // y on the pivot rows, solved x below
-  __syncthreads();
-  T v = Xl[t];
+__global__ void __launch_bounds__(64) k_mf_bwd_tiny(MfDev d, const int* list, const T* F, const T* V, double* x,
+                                                    int* nan_flag) {
+  const MfFront f = d.front[list[blockIdx.x]];
+  const int ms = f.m, np = f.np, t = threadIdx.x;
+  const int g = t < ms ? d.xidx[f.idx + t] : 0;
+  // lane t: y of pivot t, or the solved x of row t below the pivots
+  T v = t < np ? V[f.vo + t] : t < ms ? (T)x[g] : (T)0;
+  const T* row = F + f.fo + (long long)min(t, np - 1) * ms;
+  // each lane's pivot reciprocal first (in parallel): the sweep multiplies
+  const T rd = (T)1 / row[min(t, np - 1)];
+  for (int k1 = ms; k1 > 0; k1 -= 16) {
+    T u[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) u[q] = row[max(k1 - 1 - q, 0)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int k = k1 - 1 - q;
+      if (k < 0) break;
+      T xk = mf_bcast(v, k);
+      if (k < np) {
+        xk *= mf_bcast(rd, k);
+        if (t == k) v = xk;
+      }
+      if (t < k && t < np) v -= u[q] * xk;
+    }
+  }
   if (t < np) {
-    const T* row = Fs + (long long)t * ms;
-    int u = np;
-    for (; u + 4 <= ms; u += 4) {
-      const T f0 = row[u], f1 = row[u + 1], f2 = row[u + 2], f3 = row[u + 3];
-      v -= f0 * Xl[u];
-      v -= f1 * Xl[u + 1];
-      v -= f2 * Xl[u + 2];
-      v -= f3 * Xl[u + 3];
-    }
-    for (; u < ms; ++u) v -= row[u] * Xl[u];
+    x[g] = (double)v;
+    if (!isfinite((double)v)) atomicOr(nan_flag, 1);
   }
-  // each lane's pivot reciprocal first (in parallel), so that the serial
-  // sweep multiplies instead of dividing
-  const T rd = t < np ? (T)1 / Fs[(long long)t * ms + t] : (T)0;
-  for (int k = np - 1; k >= 0; --k) {
-    const T xk = mf_bcast(v, k) * mf_bcast(rd, k);
-    if (t == k) v = xk;
-    else if (t < k) v -= Fs[(long long)t * ms + k] * xk;
-  }
-  if (t < np) x[ix[t]] = v;
 }
 
-// backward, larger fronts: rows minus U12 x_below (row-wise products), then
-// U11 by 64-row blocks from the bottom
+// Larger fronts: one workgroup per front solves the pivot block (L11 or U11) by
+// 64-row blocks with the vector in LDS.  While wavefront 0 solves a block's
+// triangle (64 dependent steps), wavefronts 1 to 13 form the products of the
+// next block's rows (five each) with everything solved before this block, load
+// those rows' part inside it, and the next triangle; so between two triangles
+// stands one 64 x 64 product from registers.  The rows outside the pivot block
+// (L21 y, U12 x_below) are split over the GPU by the _rows kernels where they
+// have more than kMfSplit elements, which one workgroup would need longer for
+// than a launch takes (5 us).  512 x 512 grid, all levels, forward and
+// backward: 1.08 ms, 1.38 ms before the overlap and the split.
+constexpr int kMfSolve = 1024;
+constexpr int kMfSplit = 49152;
+constexpr int kMfTri = 64 * 65;
+constexpr int kMfNext = 5;                     // rows of the next block per wavefront
+
 template <class T>
-__global__ void __launch_bounds__(kMfSolveBlock) k_mf_bwd_big(MfDev d, const int* list, const T* F, T* V, T* x,
-                                                             int ldsv) {
+__device__ __forceinline__ void mf_load_tri(const T* Fs, long long ld, int b0, int bw, int t, int nt, T* tri) {
+  T v[5];
+#pragma unroll
+  for (int it = 0; it < 5; ++it) {
+    const int x = t + it * nt, i = min(x >> 6, bw - 1), j = min(x & 63, bw - 1);
+    v[it] = Fs[(b0 + i) * ld + b0 + j];
+  }
+#pragma unroll
+  for (int it = 0; it < 5; ++it) {
+    const int x = t + it * nt;
+    if (x < 4096) tri[(x >> 6) * 65 + (x & 63)] = v[it];
+  }
+}
+
+template <class T>
+__global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* list, const T* F, T* V, const double* b,
+                                                        int ldsv) {
   extern __shared__ unsigned char mf_sm[];
-  T* Bl = reinterpret_cast<T*>(mf_sm);          // 64 x 65 block
-  const int s = list[blockIdx.x];
-  T* Xl = ldsv ? Bl + 64 * 65 : V + d.vo[s];    // scratch (ms); V is not read by the backward solve
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
-  const T* Fs = F + d.fo[s];
-  const int* ix = d.idx + d.iptr[s];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = blockDim.x >> 6;
-  for (int i = t; i < ms; i += blockDim.x) Xl[i] = x[ix[i]];
+  T* tri = reinterpret_cast<T*>(mf_sm);
+  const int2 en = list[blockIdx.x];             // front, rows below the pivots left to k_mf_fwd_rows
+  const MfFront f = d.front[en.x];
+  T* x = ldsv ? tri + 2 * kMfTri : V + f.vo;    // the front's vector
+  const int ms = f.m, np = f.np;
+  const long long ld = ms;
+  const T* Fs = F + f.fo;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  mf_load_tri(Fs, ld, 0, min(64, np), t, kMfSolve, tri);
+  for (int i = t; i < ms; i += kMfSolve) x[i] = i < np ? (T)b[d.bidx[f.idx + i]] : (T)0;
   __syncthreads();
-  for (int rr = 4 * wave; rr < np; rr += 4 * nw) {
-    const int nr = min(4, np - rr);
-    T acc[4];
-    mf_rows_dot4(Fs, ms, rr, nr, Xl, np, ms, lane, acc);
-    if (lane == 0)
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (k < nr) Xl[rr + k] -= acc[k];
-  }
-  __syncthreads();
-  for (int b1 = np; b1 > 0; b1 -= 64) {
-    const int b0 = max(0, b1 - 64), bw = b1 - b0;
-    if (b1 < np) {
-      for (int rr = 4 * wave; rr < bw; rr += 4 * nw) {
-        const int nr = min(4, bw - rr);
-        T acc[4];
-        mf_rows_dot4(Fs, ms, b0 + rr, nr, Xl, b1, np, lane, acc);
-        if (lane == 0)
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (k < nr) Xl[b0 + rr + k] -= acc[k];
-      }
-    }
-    {
-      T v[64 * 64 / kMfSolveBlock];
-#pragma unroll
-      for (int it = 0; it < 64 * 64 / kMfSolveBlock; ++it) {
-        const int x = t + it * kMfSolveBlock, i = x >> 6, j = x & 63;
-        v[it] = (i < bw && j >= i && j < bw) ? Fs[(long long)(b0 + i) * ms + b0 + j] : (T)0;
-      }
-#pragma unroll
-      for (int it = 0; it < 64 * 64 / kMfSolveBlock; ++it) {
-        const int x = t + it * kMfSolveBlock;
-        Bl[(x >> 6) * 65 + (x & 63)] = v[it];
-      }
-    }
+  for (int c = f.c0; c < f.c1; ++c) {
+    const MfChild ch = d.child[c];
+    for (int a = t; a < ch.nu; a += kMfSolve) x[d.emap[ch.em + a]] += V[ch.vsrc + a];
     __syncthreads();
+  }
+  if (en.y && ldsv)
+    for (int i = np + t; i < ms; i += kMfSolve) V[f.vo + i] = x[i];
+  const int nb = (np + 63) / 64;
+  for (int k = 0; k < nb; ++k) {
+    const int b0 = 64 * k, r = b0 + 64 + kMfNext * (wave - 1);
+    const bool mine = wave > 0 && kMfNext * (wave - 1) < 64 && r < np;
+    const int nr = min(kMfNext, min(np, b0 + 128) - r);
+    T acc[kMfNext], pre[kMfNext];
     if (wave == 0) {
-      T v = lane < bw ? Xl[b0 + lane] : (T)0;
-      const T rd = lane < bw ? (T)1 / Bl[lane * 65 + lane] : (T)0;
-      for (int k = bw - 1; k >= 0; --k) {
-        const T xk = mf_bcast(v, k) * mf_bcast(rd, k);
-        if (lane == k) v = xk;
-        else if (lane < k) v -= Bl[lane * 65 + k] * xk;
+      const int bw = min(64, np - b0);
+      const T* tr = tri + (k & 1) * kMfTri + lane * 65;
+      T v = lane < bw ? x[b0 + lane] : (T)0;
+#pragma unroll 16
+      for (int j = 0; j < bw; ++j) {
+        const T yj = mf_bcast(v, j);
+        const T l = tr[j];
+        if (lane > j) v -= l * yj;
       }
-      if (lane < bw) Xl[b0 + lane] = v;
+      if (lane < bw) x[b0 + lane] = v;
+    } else {
+      if (mine) {
+#pragma unroll
+        for (int i = 0; i < kMfNext; ++i) pre[i] = Fs[(r + min(i, nr - 1)) * ld + b0 + lane];
+        mf_rows_part<kMfNext>(Fs, ld, r, nr, 0, b0, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
+      }
+      if (k + 1 < nb)
+        mf_load_tri(Fs, ld, b0 + 64, min(64, np - b0 - 64), t - 64, kMfSolve - 64, tri + ((k + 1) & 1) * kMfTri);
+    }
+    __syncthreads();
+    if (mine) {
+      const T y = x[b0 + lane];
+#pragma unroll
+      for (int i = 0; i < kMfNext; ++i) acc[i] = mf_wave_sum(acc[i] + pre[i] * y);
+      if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < kMfNext; ++i)
+          if (i < nr) x[r + i] -= acc[i];
     }
     __syncthreads();
   }
-  for (int i = t; i < np; i += blockDim.x) x[ix[i]] = Xl[i];
+  if (!en.y)
+    for (int r = np + 4 * wave; r < ms; r += 4 * (kMfSolve / 64)) {
+      const int nr = min(4, ms - r);
+      T acc[4];
+      mf_rows_part<4>(Fs, ld, r, nr, 0, np, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        acc[k] = mf_wave_sum(acc[k]);
+        if (lane == 0 && k < nr) x[r + k] -= acc[k];
+      }
+    }
+  if (!ldsv) return;
+  __syncthreads();
+  for (int i = t; i < (en.y ? np : ms); i += kMfSolve) V[f.vo + i] = x[i];
+}
+
+// rows below the pivots of a split front, 16 per workgroup (entries {front, row})
+template <class T>
+__global__ void __launch_bounds__(256) k_mf_fwd_rows(MfDev d, const int2* ent, const T* F, T* V) {
+  const int2 en = ent[blockIdx.x];
+  const MfFront f = d.front[en.x];
+  const int lane = threadIdx.x & 63, r = en.y + 4 * (threadIdx.x >> 6), nr = min(4, f.m - r);
+  if (nr <= 0) return;
+  T* v = V + f.vo;
+  T acc[4];
+  mf_rows_part<4>(F + f.fo, f.m, r, nr, 0, f.np, lane, [&](int j) MF_INLINE { return v[j]; }, acc);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    acc[k] = mf_wave_sum(acc[k]);
+    if (lane == 0 && k < nr) v[r + k] -= acc[k];
+  }
+}
+
+// pivot rows of a split front minus U12 x_below, 16 per workgroup
+template <class T>
+__global__ void __launch_bounds__(256) k_mf_bwd_rows(MfDev d, const int2* ent, const T* F, T* V, const double* x) {
+  const int2 en = ent[blockIdx.x];
+  const MfFront f = d.front[en.x];
+  const int lane = threadIdx.x & 63, r = en.y + 4 * (threadIdx.x >> 6), nr = min(4, f.np - r);
+  if (nr <= 0) return;
+  const int* ix = d.xidx + f.idx;
+  T acc[4];
+  mf_rows_part<4>(F + f.fo, f.m, r, nr, f.np, f.m, lane, [&](int j) MF_INLINE { return (T)x[ix[j]]; }, acc);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    acc[k] = mf_wave_sum(acc[k]);
+    if (lane == 0 && k < nr) V[f.vo + r + k] -= acc[k];
+  }
 }
 
 template <class T>
-__global__ void k_mf_perm_in(int n, const int* prow, const double* b, double* bp) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) bp[i] = b[prow[i]];
-}
-template <class T>
-__global__ void k_mf_perm_out(int n, const int* pcol, const T* xp, double* x, int* nan_flag) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n) {
-    const double v = (double)xp[j];
-    x[pcol[j]] = v;
-    if (!isfinite(v)) atomicOr(nan_flag, 1);
+__global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* list, const T* F, T* V, double* xg,
+                                                        int ldsv, int* nan_flag) {
+  extern __shared__ unsigned char mf_sm[];
+  T* tri = reinterpret_cast<T*>(mf_sm);
+  const int2 en = list[blockIdx.x];             // front, U12 x_below already subtracted by k_mf_bwd_rows
+  const MfFront f = d.front[en.x];
+  T* x = ldsv ? tri + 2 * kMfTri : V + f.vo;
+  const int ms = f.m, np = f.np;
+  const long long ld = ms;
+  const T* Fs = F + f.fo;
+  const int* ix = d.xidx + f.idx;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int nb = (np + 63) / 64;
+  mf_load_tri(Fs, ld, 64 * (nb - 1), np - 64 * (nb - 1), t, kMfSolve, tri + ((nb - 1) & 1) * kMfTri);
+  for (int i = t; i < (en.y ? np : ms); i += kMfSolve)
+    if (i >= np) x[i] = (T)xg[ix[i]];
+    else if (ldsv) x[i] = V[f.vo + i];
+  __syncthreads();
+  if (!en.y && ms > np) {
+    for (int r = 4 * wave; r < np; r += 4 * (kMfSolve / 64)) {
+      const int nr = min(4, np - r);
+      T acc[4];
+      mf_rows_part<4>(Fs, ld, r, nr, np, ms, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        acc[k] = mf_wave_sum(acc[k]);
+        if (lane == 0 && k < nr) x[r + k] -= acc[k];
+      }
+    }
+    __syncthreads();
   }
+  for (int k = nb - 1; k >= 0; --k) {
+    const int b0 = 64 * k, bw = min(64, np - b0);
+    const int i0 = kMfNext * (wave - 1), r = b0 - 64 + i0;
+    const bool mine = wave > 0 && i0 < 64 && k > 0;
+    const int nr = min(kMfNext, 64 - i0);
+    T acc[kMfNext], pre[kMfNext];
+    if (wave == 0) {
+      const T* tr = tri + (k & 1) * kMfTri + lane * 65;
+      T v = lane < bw ? x[b0 + lane] : (T)0;
+      const T rd = lane < bw ? (T)1 / tr[lane] : (T)0;
+#pragma unroll 16
+      for (int j = bw - 1; j >= 0; --j) {
+        const T xj = mf_bcast(v, j) * mf_bcast(rd, j);
+        const T u = tr[j];
+        if (lane == j) v = xj;
+        if (lane < j) v -= u * xj;
+      }
+      if (lane < bw) x[b0 + lane] = v;
+    } else {
+      if (mine) {
+#pragma unroll
+        for (int i = 0; i < kMfNext; ++i) pre[i] = Fs[(r + min(i, nr - 1)) * ld + b0 + min(lane, bw - 1)];
+        mf_rows_part<kMfNext>(Fs, ld, r, nr, b0 + bw, np, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
+      }
+      if (k > 0) mf_load_tri(Fs, ld, b0 - 64, 64, t - 64, kMfSolve - 64, tri + ((k - 1) & 1) * kMfTri);
+    }
+    __syncthreads();
+    if (mine) {
+      const T y = lane < bw ? x[b0 + lane] : (T)0;
+#pragma unroll
+      for (int i = 0; i < kMfNext; ++i) acc[i] = mf_wave_sum(acc[i] + pre[i] * y);
+      if (lane == 0)
+#pragma unroll
+        for (int i = 0; i < kMfNext; ++i)
+          if (i < nr) x[r + i] -= acc[i];
+    }
+    __syncthreads();
+  }
+  bool bad = false;
+  for (int i = t; i < np; i += kMfSolve) {
+    const double v = (double)x[i];
+    xg[ix[i]] = v;
+    bad |= !isfinite(v);
+  }
+  if (bad) atomicOr(nan_flag, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -1011,26 +1133,28 @@ struct MfLu::Impl {
     for (auto& g : graphs)
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
   }
-  DevVec<int> sfirst, m, iptr, idx, cptr, clist, eptr, emap, vo, prow, pcol, bad, arow, acol, aslot;
+  DevVec<int> sfirst, m, emap, bidx, xidx, bad, arow, acol, aslot;
   DevVec<long long> fo;
   DevVec<MfFront> front;
   DevVec<MfChild> child;
-  DevVec<double> F64, V64, y64, b64;
-  DevVec<float> F32, V32, y32;
-  DevVec<int> tiny_list, big_list;
+  DevVec<double> F64, V64;
+  DevVec<float> F32, V32;
+  DevVec<int> tiny_list;
+  DevVec<int2> big_list;          // larger fronts {front, 1: rows outside the pivot block split over the GPU}
+  DevVec<int2> frow, brow;        // entries of those rows {front, first row}
   DevVec<int4> aent;              // assembly entries of the larger fronts, two each
   DevVec<int2> alo;               // per entry and child: the child's rows in the entry's range
   DevVec<int4> sent;              // entries of the panel steps
   DevVec<double> dbuf;            // diagonal-block factors, two 32 x 32 slots per larger front of a level
   std::vector<int> tiny_off, tiny_half, big_off;   // fronts up to order 32 at [tiny_off, tiny_half), up to 64 from there
   int big_maxm = 0;
+  std::vector<int> frow_off, brow_off;   // per level
   std::vector<int> aoff;          // per level: offset into aent
   struct Step { int p0, off, cnt; };
   std::vector<std::vector<Step>> steps;   // per level: its panel steps
   MfDev dev() const {
     MfDev d;
-    d.sfirst = sfirst.p; d.m = m.p; d.fo = fo.p; d.iptr = iptr.p; d.idx = idx.p; d.cptr = cptr.p;
-    d.clist = clist.p; d.eptr = eptr.p; d.emap = emap.p; d.vo = vo.p;
+    d.sfirst = sfirst.p; d.m = m.p; d.fo = fo.p; d.emap = emap.p; d.bidx = bidx.p; d.xidx = xidx.p;
     d.front = front.p; d.child = child.p; d.arow = arow.p; d.acol = acol.p; d.aslot = aslot.p;
     return d;
   }
@@ -1072,17 +1196,20 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   hipStream_t st = I.st;
   MFCHK(I.front.up(fr, st)); MFCHK(I.child.up(chv, st));
   MFCHK(I.arow.up(P.arow, st)); MFCHK(I.acol.up(P.acol, st)); MFCHK(I.aslot.up(P.aslot, st));
-  MFCHK(I.sfirst.up(P.sfirst, st)); MFCHK(I.m.up(P.m, st)); MFCHK(I.iptr.up(P.iptr, st)); MFCHK(I.idx.up(P.idx, st));
-  MFCHK(I.cptr.up(P.cptr, st)); MFCHK(I.clist.up(P.clist, st)); MFCHK(I.eptr.up(P.eptr, st));
-  MFCHK(I.emap.up(P.emap, st)); MFCHK(I.vo.up(P.vo, st)); MFCHK(I.fo.up(P.fo, st));
-  MFCHK(I.prow.up(s.perm_row, st)); MFCHK(I.pcol.up(s.perm_col, st));
+  MFCHK(I.sfirst.up(P.sfirst, st)); MFCHK(I.m.up(P.m, st)); MFCHK(I.emap.up(P.emap, st)); MFCHK(I.fo.up(P.fo, st));
+  std::vector<int> bi(P.idx.size()), xi(P.idx.size());
+  for (size_t q = 0; q < P.idx.size(); ++q) { bi[q] = s.perm_row[P.idx[q]]; xi[q] = s.perm_col[P.idx[q]]; }
+  MFCHK(I.bidx.up(bi, st)); MFCHK(I.xidx.up(xi, st));
   MFCHK(I.bad.alloc(2));
-  MFCHK(I.F64.alloc(P.fo[P.ns])); MFCHK(I.V64.alloc(P.vo[P.ns])); MFCHK(I.y64.alloc(P.n)); MFCHK(I.b64.alloc(P.n));
-  if (want_fp32) { MFCHK(I.F32.alloc(P.fo[P.ns])); MFCHK(I.V32.alloc(P.vo[P.ns])); MFCHK(I.y32.alloc(P.n)); }
+  MFCHK(I.F64.alloc(P.fo[P.ns])); MFCHK(I.V64.alloc(P.vo[P.ns]));
+  if (want_fp32) { MFCHK(I.F32.alloc(P.fo[P.ns])); MFCHK(I.V32.alloc(P.vo[P.ns])); }
   // per level: tiny fronts (one launch), larger fronts (blocked panels, all
   // fronts of the level in each panel launch)
   const int nl = (int)P.lvl_ptr.size() - 1;
   std::vector<int> tl, bl;
+  std::vector<int2> bl2, fre, bre;
+  I.frow_off.assign(nl + 1, 0);
+  I.brow_off.assign(nl + 1, 0);
   std::vector<int4> se;
   int max_slots = 1;
   I.tiny_off.assign(nl + 1, 0);
@@ -1107,6 +1234,15 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
     }
     I.tiny_half[l] = (int)tl.size();
     tl.insert(tl.end(), mid.begin(), mid.end());
+    I.frow_off[l] = (int)fre.size();
+    I.brow_off[l] = (int)bre.size();
+    for (int q = I.big_off[l]; q < (int)bl.size(); ++q) {
+      const int t = bl[q], m = P.m[t], np = P.sfirst[t + 1] - P.sfirst[t];
+      const bool split = (long long)np * (m - np) > kMfSplit;
+      bl2.push_back(make_int2(t, split));
+      for (int r = np; split && r < m; r += 16) fre.push_back(make_int2(t, r));
+      for (int r = 0; split && r < np; r += 16) bre.push_back(make_int2(t, r));
+    }
     const int nb = (int)bl.size() - I.big_off[l];
     max_slots = std::max(max_slots, nb);
     for (int j = 0; nb > 0 && j <= maxp; ++j) {
@@ -1136,7 +1272,11 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   I.tiny_off[nl] = (int)tl.size();
   I.big_off[nl] = (int)bl.size();
   MFCHK(I.tiny_list.up(tl, st));
-  MFCHK(I.big_list.up(bl, st));
+  I.frow_off[nl] = (int)fre.size();
+  I.brow_off[nl] = (int)bre.size();
+  MFCHK(I.big_list.up(bl2, st));
+  MFCHK(I.frow.up(fre, st));
+  MFCHK(I.brow.up(bre, st));
   MFCHK(I.sent.up(se, st));
   MFCHK(I.dbuf.alloc((size_t)max_slots * 2 * kMfPanel * kMfPanel));
   // assembly of the larger fronts, ranges of rows and columns (the tiny fronts
@@ -1249,46 +1389,46 @@ static int mf_factor_t(MfLu::Impl& I, const double* vals_dev, int nnz, T* F, int
 }
 
 template <class T>
-static int mf_solve_enqueue(MfLu::Impl& I, const T* F, T* V, T* y, double* bp, const double* b_dev, double* x_dev,
-                            int* nan_flag) {
+static int mf_solve_enqueue(MfLu::Impl& I, const T* F, T* V, const double* b_dev, double* x_dev, int* nan_flag) {
   const MfPlan& P = I.P;
   hipStream_t st = I.st;
   const MfDev d = I.dev();
-  const int n = P.n;
-  // the larger fronts keep their vector in LDS when it fits in 64 KB with the
-  // 64x65 block, else in their slice of V
-  const size_t blk_bytes = 64 * 65 * sizeof(T);
-  const bool ldsv = blk_bytes + (size_t)I.big_maxm * sizeof(T) <= 65536;
-  const size_t big_lds = blk_bytes + (ldsv ? (size_t)I.big_maxm * sizeof(T) : 0);
-  hipLaunchKernelGGL(k_mf_perm_in<T>, dim3((n + 255) / 256), dim3(256), 0, st, n, I.prow.p, b_dev, bp);
+  // the larger fronts keep their vector in LDS when it fits beside the two
+  // triangles, else in their slice of V
+  const size_t tri = 2 * kMfTri * sizeof(T);
+  const bool ldsv = tri + (size_t)I.big_maxm * sizeof(T) <= 150 * 1024;
+  const size_t lds = tri + (ldsv ? (size_t)I.big_maxm * sizeof(T) : 0);
   const int nl = (int)P.lvl_ptr.size() - 1;
   for (int l = 0; l < nl; ++l) {
     const int nt = I.tiny_off[l + 1] - I.tiny_off[l], nb = I.big_off[l + 1] - I.big_off[l];
-    if (nt)
-      hipLaunchKernelGGL(k_mf_fwd_tiny<T>, dim3(nt), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l], F, V,
-                         bp, y);
+    const int nr = I.frow_off[l + 1] - I.frow_off[l];
+    if (nt) hipLaunchKernelGGL(k_mf_fwd_tiny<T>, dim3(nt), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l], F, V, b_dev);
     if (nb)
-      hipLaunchKernelGGL(k_mf_fwd_big<T>, dim3(nb), dim3(kMfSolveBlock), big_lds, st, d, I.big_list.p + I.big_off[l],
-                         F, V, bp, y, (int)ldsv);
+      hipLaunchKernelGGL(k_mf_fwd_big<T>, dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F, V, b_dev,
+                         (int)ldsv);
+    if (nr) hipLaunchKernelGGL(k_mf_fwd_rows<T>, dim3(nr), dim3(256), 0, st, d, I.frow.p + I.frow_off[l], F, V);
   }
   for (int l = nl - 1; l >= 0; --l) {
     const int nt = I.tiny_off[l + 1] - I.tiny_off[l], nb = I.big_off[l + 1] - I.big_off[l];
+    const int nr = I.brow_off[l + 1] - I.brow_off[l];
+    if (nr)
+      hipLaunchKernelGGL(k_mf_bwd_rows<T>, dim3(nr), dim3(256), 0, st, d, I.brow.p + I.brow_off[l], F, V,
+                         (const double*)x_dev);
     if (nb)
-      hipLaunchKernelGGL(k_mf_bwd_big<T>, dim3(nb), dim3(kMfSolveBlock), big_lds, st, d, I.big_list.p + I.big_off[l],
-                         F, V, y, (int)ldsv);
+      hipLaunchKernelGGL(k_mf_bwd_big<T>, dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F, V, x_dev,
+                         (int)ldsv, nan_flag);
     if (nt)
-      hipLaunchKernelGGL(k_mf_bwd_tiny<T>, dim3(nt), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l], F, y);
+      hipLaunchKernelGGL(k_mf_bwd_tiny<T>, dim3(nt), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l], F, (const T*)V,
+                         x_dev, nan_flag);
   }
-  hipLaunchKernelGGL(k_mf_perm_out<T>, dim3((n + 255) / 256), dim3(256), 0, st, n, I.pcol.p, y, x_dev, nan_flag);
   MFCHK(hipGetLastError());
   return XG_OK;
 }
 
 template <class T>
-static int mf_solve_t(MfLu::Impl& I, const T* F, T* V, T* y, double* bp, const double* b_dev, double* x_dev,
-                      int* nan_flag) {
-  const void* key[8] = {(const void*)2, F, V, y, bp, b_dev, x_dev, nan_flag};
-  return mf_replay(I, key, 8, [&] { return mf_solve_enqueue<T>(I, F, V, y, bp, b_dev, x_dev, nan_flag); });
+static int mf_solve_t(MfLu::Impl& I, const T* F, T* V, const double* b_dev, double* x_dev, int* nan_flag) {
+  const void* key[8] = {(const void*)2, F, V, b_dev, x_dev, nan_flag, nullptr, nullptr};
+  return mf_replay(I, key, 8, [&] { return mf_solve_enqueue<T>(I, F, V, b_dev, x_dev, nan_flag); });
 }
 
 int MfLu::factor(const double* vals_dev, int nnz, bool fp32, int* bad, int* hard) {
@@ -1304,9 +1444,9 @@ int MfLu::solve(const double* b_dev, double* x_dev, bool fp32, int* nan_flag) {
   Impl& I = *impl_;
   if (fp32) {
     if (!I.F32.p) return XG_E_ARG;
-    return mf_solve_t<float>(I, I.F32.p, I.V32.p, I.y32.p, I.b64.p, b_dev, x_dev, nan_flag);
+    return mf_solve_t<float>(I, I.F32.p, I.V32.p, b_dev, x_dev, nan_flag);
   }
-  return mf_solve_t<double>(I, I.F64.p, I.V64.p, I.y64.p, I.b64.p, b_dev, x_dev, nan_flag);
+  return mf_solve_t<double>(I, I.F64.p, I.V64.p, b_dev, x_dev, nan_flag);
 }
 
 static size_t round32(size_t v) { return (v + 31) & ~(size_t)31; }
@@ -1322,7 +1462,13 @@ int MfLu::solve_ext(const double* b_dev, double* x_dev, int* nan_flag, double* w
   double* V = work;
   double* y = V + round32((size_t)P.vo[P.ns]);
   double* bp = y + round32((size_t)P.n);
-  return mf_solve_t<double>(I, I.F64.p, V, y, bp, b_dev, x_dev, nan_flag);
+  // through the work area, so that the captured graph does not hold the
+  // caller's addresses
+  MFCHK(hipMemcpyAsync(bp, b_dev, sizeof(double) * P.n, hipMemcpyDeviceToDevice, I.st));
+  const int rc = mf_solve_t<double>(I, I.F64.p, V, bp, y, nan_flag);
+  if (rc != XG_OK) return rc;
+  MFCHK(hipMemcpyAsync(x_dev, y, sizeof(double) * P.n, hipMemcpyDeviceToDevice, I.st));
+  return XG_OK;
 }
 
 }  // namespace xg
