@@ -208,3 +208,52 @@ def test_gate_array_full_load_host_and_device_arrays(gpu):
     for a, b in zip(dmm, hm):
         assert np.array_equal(a.cpu().numpy(), b)
     assert min(td) < min(th)
+
+
+@pytest.mark.parametrize("stages", [5, 1501])
+def test_host_and_device_loads_agree_on_both_sides_of_the_staging(gpu, stages):
+    """Small host-array loads go through the pinned staging, larger ones through
+    copies: both give the device-array calls' bits, added to what the arrays
+    hold, and leave entries of other devices alone."""
+    import torch
+    c = C.ring(stages, seed=stages, mc_seed=stages)
+    d = X.DeviceMgr(c)
+    L = X.lib()
+    rng = np.random.default_rng(stages)
+    x = rng.uniform(0.0, 1.8, d.n)
+    d.set_solver_state(order=2, h=1e-12, time=0.2e-9)
+    sta, sto, _ = d.updateState(x + 0.01, np.zeros(d.nsta), np.zeros(d.nsto))
+    sn, on, lim = d.updateState(x, sta, sto)
+    into = {k: rng.normal(size=d.n) for k in ("F", "Q", "B", "dFdxdVp", "dQdxdVp")}
+    base = {k: v.copy() for k, v in into.items()}
+    d.loadDAEVectors(into)
+    dF, dQ = d.loadDAEMatrices()
+    q0, q2 = rng.normal(size=d.n) * 1e-15, rng.normal(size=d.n) * 1e-5
+    rhs, J = d.combine(q0, q2)
+    rhs0, _ = d.combine(q0)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    xs, sas, sos, snd, ond = g(x), g(sta), g(sto), torch.zeros(d.nsta, dtype=torch.float64, device="cuda"), g(sto)
+    flag = ctypes.c_int(-1)
+    torch.cuda.synchronize()
+    assert L.xg_update_state_dev(d.h, P(xs), P(sas), P(sos), P(snd), P(ond), ctypes.byref(flag)) == 0
+    assert flag.value == lim
+    np.testing.assert_array_equal(snd.cpu().numpy(), sn)
+    np.testing.assert_array_equal(ond.cpu().numpy(), on)
+    dv = {k: g(base[k]) for k in base}
+    dm = [torch.zeros(d.nnz, dtype=torch.float64, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    assert L.xg_load_vectors_dev(d.h, *[P(dv[k]) for k in ("F", "Q", "B", "dFdxdVp", "dQdxdVp")]) == 0
+    assert L.xg_load_matrices_dev(d.h, P(dm[0]), P(dm[1])) == 0
+    for k in into:
+        np.testing.assert_array_equal(dv[k].cpu().numpy(), into[k])
+    np.testing.assert_array_equal(dm[0].cpu().numpy(), dF)
+    np.testing.assert_array_equal(dm[1].cpu().numpy(), dQ)
+    q0d, q2d, r = g(q0), g(q2), torch.zeros(d.n, dtype=torch.float64, device="cuda")
+    j = torch.zeros(d.nnz, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    assert L.xg_combine_dev(d.h, P(q0d), P(q2d), P(r), P(j)) == 0
+    np.testing.assert_array_equal(r.cpu().numpy(), rhs)
+    np.testing.assert_array_equal(j.cpu().numpy(), J)
+    assert L.xg_combine_dev(d.h, P(q0d), None, P(r), None) == 0
+    np.testing.assert_array_equal(r.cpu().numpy(), rhs0)

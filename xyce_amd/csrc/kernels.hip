@@ -57,31 +57,61 @@ struct EvalArgs {
   const double* x;
   const double* sto_cur; const double* sto_nxt_in; const double* sta_cur;
   double* sto_out; double* sta_out;
+  const int* sta0; const int* sto0;      // Xyce's layout: each device's first entry
   double* rec;
   int* limited;
   MosFlags fl;
 };
 
+// XY: store and state in the caller's vectors, a device's entries next to each
+// other (read and written in pairs; the devices of a wavefront follow each other
+// there too, so the lines are used whole), else in the planes of the resident
+// engine.  Bound by memory: 300k MOSFETs 51 us
+// on the caller's vectors, where the planes' conversions (72 us) and the evaluation
+// on them (78 us) took 150.
+template <bool XY>
 __global__ void __launch_bounds__(256) k_mos1_eval(EvalArgs a) {
+  typedef double Pair __attribute__((ext_vector_type(2), aligned(8)));
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.n_mos) return;
   const int N = a.n_mos;
   const double* k = a.cls + (size_t)a.mcls[i] * KSTRIDE;
   double volt[6], sc[6], sn[6], ac[8];
+  const int s0 = XY ? a.sto0[i] : 0, t0 = XY ? a.sta0[i] : 0;
+  if (XY) {
+#pragma unroll
+    for (int j = 0; j < 6; j += 2) {
+      const Pair c = *reinterpret_cast<const Pair*>(a.sto_cur + s0 + j);
+      const Pair n = *reinterpret_cast<const Pair*>(a.sto_nxt_in + s0 + j);
+      sc[j] = c.x; sc[j + 1] = c.y; sn[j] = n.x; sn[j + 1] = n.y;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      const Pair c = *reinterpret_cast<const Pair*>(a.sta_cur + t0 + j);
+      ac[j] = c.x; ac[j + 1] = c.y;
+    }
+  } else {
+    for (int j = 0; j < 6; ++j) { sc[j] = a.sto_cur[(size_t)j * N + i]; sn[j] = a.sto_nxt_in[(size_t)j * N + i]; }
+    for (int j = 0; j < 8; ++j) ac[j] = a.sta_cur[(size_t)j * N + i];
+  }
   for (int j = 0; j < 6; ++j) volt[j] = a.x[a.lid[6 * i + j]];
-  for (int j = 0; j < 6; ++j) { sc[j] = a.sto_cur[(size_t)j * N + i]; sn[j] = a.sto_nxt_in[(size_t)j * N + i]; }
-  for (int j = 0; j < 8; ++j) ac[j] = a.sta_cur[(size_t)j * N + i];
   const unsigned long long m = a.mask[i];
   double* rec = a.rec;
   auto emit = [&](int plane, double v) { if (m >> plane & 1ull) rec[(size_t)plane * N + i] = v; };
   // the store and state inputs are all in registers before the first output
   // is written (the outputs may be the input arrays)
   auto keep = [&](int j, double v) {
-    if (j < 6) a.sto_out[(size_t)j * N + i] = v;
-    else a.sta_out[(size_t)(j - 6) * N + i] = v;
+    if (j < 6) a.sto_out[XY ? (size_t)(s0 + j) : (size_t)j * N + i] = v;
+    else a.sta_out[XY ? (size_t)(t0 + j - 6) : (size_t)(j - 6) * N + i] = v;
   };
   const int lim = mos1_eval(k, a.tvbi[i], a.beta[i], a.tvto[i], volt, sc, sn, ac, a.fl, keep, emit);
-  if (lim) atomicOr(a.limited, 1);
+  if (lim) *a.limited = 1;       // (every writer writes the same value)
+}
+
+// x into the circuit's vector (entry n: ground)
+__global__ void k_take_x(int n, const double* x, double* to) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= n) to[i] = i < n ? x[i] : 0.0;
 }
 
 struct SrcArgs {
@@ -114,31 +144,96 @@ __device__ __forceinline__ double wg_sum_fixed(double v, double* sh) {
   return t;
 }
 
+// The caller's arrays that a load's result goes to (each may be null): added to
+// what they hold, or stored (staging that the host adds from)
+template <int N>
+struct OutArgs {
+  double* p[N];
+  int add;
+  __device__ __forceinline__ void put(int i, int r, double v) const {
+    if (p[i]) p[i][r] = add ? p[i][r] + v : v;
+  }
+};
+
+// Long rows and slots (beyond kGatherLong terms) are summed in two passes:
+// chunks of at most kGatherChunk terms, one workgroup each, into partial sums
+// (fixed-order workgroup reduction), then one wavefront per long entry adds its
+// chunks' partials.  Chunk c covers terms [cb[c], ce[c]); kind 0 = record terms,
+// 1 = linear CSR entries (vectors only).
+constexpr int kGatherChunk = 2048;
+
 // Per row: F/Q/dFdxdVp/dQdxdVp from the record terms (device order), then the
 // linear part's row sums (FilteredMatrix::axpy, N_LAS_FilteredMatrix.C:511-536),
 // then B from the sources (DeviceMgr::loadBVectorsforSources).  Long rows are
-// left to k_gather_vectors_long.
-__global__ void k_gather_vectors(int n, int n_mos, const int* __restrict__ vg_ptr, const int* __restrict__ vg_ent,
-                                 const double* __restrict__ rec, const int* __restrict__ rowptr,
-                                 const int* __restrict__ colind, const double* __restrict__ linF,
-                                 const double* __restrict__ linQ, const double* __restrict__ x, SrcArgs s,
-                                 double* F, double* Q, double* B, double* FL, double* QL) {
+// left to the workgroups from row_blocks on, one per chunk (ck, cb, ce), and
+// k_gather_vectors_fin.
+__global__ void __launch_bounds__(256) k_gather_vectors(
+    int n, int n_mos, const int* __restrict__ vg_ptr, const int* __restrict__ vg_ent, const double* __restrict__ rec,
+    const int* __restrict__ rowptr, const int* __restrict__ colind, const double* __restrict__ linF,
+    const double* __restrict__ linQ, const double* __restrict__ x, SrcArgs s, double* F, double* Q, double* B,
+    double* FL, double* QL, OutArgs<5> out, int row_blocks, const int* __restrict__ ck, const int* __restrict__ cb,
+    const int* __restrict__ ce, double* part) {
+  if ((int)blockIdx.x >= row_blocks) {
+    __shared__ double sh[16];
+    const int c = blockIdx.x - row_blocks;
+    double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+    if (ck[c] == 0) {
+#pragma unroll 4
+      for (int e = cb[c] + (int)threadIdx.x; e < ce[c]; e += 256) {
+        const int ent = vg_ent[e];
+        const int dev = ent >> 6, plane = ent & 63;
+        const double v = rec[(size_t)plane * n_mos + dev];
+        const int vid = d_rec_vec_id(plane);
+        if (vid == 0) a0 += v; else if (vid == 1) a1 += v; else if (vid == 2) a2 += v; else a3 += v;
+      }
+    } else {
+      for (int k = cb[c] + (int)threadIdx.x; k < ce[c]; k += blockDim.x) {
+        const double xv = x[colind[k]];
+        if (linF[k] != 0.0) a0 += linF[k] * xv;
+        if (linQ[k] != 0.0) a1 += linQ[k] * xv;
+      }
+    }
+    a0 = wg_sum_fixed(a0, sh); a1 = wg_sum_fixed(a1, sh); a2 = wg_sum_fixed(a2, sh); a3 = wg_sum_fixed(a3, sh);
+    if (threadIdx.x == 0) {
+      part[4 * c] = a0; part[4 * c + 1] = a1; part[4 * c + 2] = a2; part[4 * c + 3] = a3;
+    }
+    return;
+  }
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
   if (vg_ptr[r + 1] - vg_ptr[r] + rowptr[r + 1] - rowptr[r] > kGatherLong) return;
   double f = 0.0, q = 0.0, fl = 0.0, ql = 0.0;
-  for (int e = vg_ptr[r]; e < vg_ptr[r + 1]; ++e) {
-    const int ent = vg_ent[e];
-    const int dev = ent >> 6, plane = ent & 63;
-    const double v = rec[(size_t)plane * n_mos + dev];
-    const int vid = d_rec_vec_id(plane);
-    if (vid == 0) f += v; else if (vid == 1) q += v; else if (vid == 2) fl += v; else ql += v;
+  // (eight terms and four CSR entries at a time: a row waits for memory that often)
+  const int e1 = vg_ptr[r + 1];
+  for (int e = vg_ptr[r]; e < e1; e += 8) {
+    int ent[8];
+    double v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ent[j] = vg_ent[min(e + j, e1 - 1)];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = rec[(size_t)(ent[j] & 63) * n_mos + (ent[j] >> 6)];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (e + j >= e1) break;
+      const int vid = d_rec_vec_id(ent[j] & 63);
+      if (vid == 0) f += v[j]; else if (vid == 1) q += v[j]; else if (vid == 2) fl += v[j]; else ql += v[j];
+    }
   }
   double sf = 0.0, sq = 0.0;
-  for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) {
-    const double xv = x[colind[k]];
-    if (linF[k] != 0.0) sf += linF[k] * xv;
-    if (linQ[k] != 0.0) sq += linQ[k] * xv;
+  const int k1 = rowptr[r + 1];
+  for (int k = rowptr[r]; k < k1; k += 4) {
+    double xv[4], lf[4], lq[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int kk = min(k + j, k1 - 1);
+      xv[j] = x[colind[kk]]; lf[j] = linF[kk]; lq[j] = linQ[kk];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (k + j >= k1) break;
+      if (lf[j] != 0.0) sf += lf[j] * xv[j];
+      if (lq[j] != 0.0) sq += lq[j] * xv[j];
+    }
   }
   f += sf; q += sq;
   double b = 0.0;
@@ -148,41 +243,7 @@ __global__ void k_gather_vectors(int n, int n_mos, const int* __restrict__ vg_pt
     if (ent & 1) b -= v; else b += v;
   }
   F[r] = f; Q[r] = q; B[r] = b; FL[r] = fl; QL[r] = ql;
-}
-
-// Long rows and slots are summed in two passes: chunks of at most
-// kGatherChunk terms, one workgroup each, into partial sums (fixed-order
-// workgroup reduction), then one thread per long entry adds its chunks'
-// partials in chunk order.  Chunk c covers terms [cb[c], ce[c]) of entry
-// ci[c]; kind 0 = record terms, 1 = linear CSR entries (vectors only).
-constexpr int kGatherChunk = 2048;
-
-__global__ void __launch_bounds__(256) k_gather_vectors_part(
-    int n_mos, const int* __restrict__ ck, const int* __restrict__ cb, const int* __restrict__ ce,
-    const int* __restrict__ vg_ent, const double* __restrict__ rec, const int* __restrict__ colind,
-    const double* __restrict__ linF, const double* __restrict__ linQ, const double* __restrict__ x, double* part) {
-  __shared__ double sh[16];
-  const int c = blockIdx.x;
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
-  if (ck[c] == 0) {
-    for (int e = cb[c] + (int)threadIdx.x; e < ce[c]; e += blockDim.x) {
-      const int ent = vg_ent[e];
-      const int dev = ent >> 6, plane = ent & 63;
-      const double v = rec[(size_t)plane * n_mos + dev];
-      const int vid = d_rec_vec_id(plane);
-      if (vid == 0) a0 += v; else if (vid == 1) a1 += v; else if (vid == 2) a2 += v; else a3 += v;
-    }
-  } else {
-    for (int k = cb[c] + (int)threadIdx.x; k < ce[c]; k += blockDim.x) {
-      const double xv = x[colind[k]];
-      if (linF[k] != 0.0) a0 += linF[k] * xv;
-      if (linQ[k] != 0.0) a1 += linQ[k] * xv;
-    }
-  }
-  a0 = wg_sum_fixed(a0, sh); a1 = wg_sum_fixed(a1, sh); a2 = wg_sum_fixed(a2, sh); a3 = wg_sum_fixed(a3, sh);
-  if (threadIdx.x == 0) {
-    part[4 * c] = a0; part[4 * c + 1] = a1; part[4 * c + 2] = a2; part[4 * c + 3] = a3;
-  }
+  out.put(0, r, f); out.put(1, r, q); out.put(2, r, b); out.put(3, r, fl); out.put(4, r, ql);
 }
 
 // one wavefront per long row: record-term chunks [rc[3l], rc[3l+1]), CSR
@@ -195,7 +256,8 @@ __device__ __forceinline__ double wave_sum_fixed(double v) {
 
 __global__ void __launch_bounds__(64) k_gather_vectors_fin(const int* __restrict__ rows, const int* __restrict__ rc,
                                                           const double* __restrict__ part, SrcArgs s, double* F,
-                                                          double* Q, double* B, double* FL, double* QL) {
+                                                          double* Q, double* B, double* FL, double* QL,
+                                                          OutArgs<5> out) {
   const int l = blockIdx.x, lane = threadIdx.x;
   const int r = rows[l];
   double f = 0.0, q = 0.0, fl = 0.0, ql = 0.0, sf = 0.0, sq = 0.0;
@@ -214,64 +276,65 @@ __global__ void __launch_bounds__(64) k_gather_vectors_fin(const int* __restrict
     if (ent & 1) b -= v; else b += v;
   }
   F[r] = f; Q[r] = q; B[r] = b; FL[r] = fl; QL[r] = ql;
+  out.put(0, r, f); out.put(1, r, q); out.put(2, r, b); out.put(3, r, fl); out.put(4, r, ql);
 }
-
-#pragma clang fp contract(off)
-__device__ __forceinline__ double jac_combine_k(double a, double dq, double b, double df) { return a * dq + b * df; }
-#pragma clang fp contract(fast)
 
 // Per CSR slot: dFdx, dQdx from the record terms, + the linear matrices
-// (FilteredMatrix::addToMatrix), optionally J = a*dQdx + b*dFdx
-// (EpetraMatrix::linearCombo N_LAS_EpetraMatrix.C:629) scattered to LU storage.
-__global__ void k_gather_matrices(int nnz, int n_mos, const int* __restrict__ mg_ptr, const int* __restrict__ mg_ent,
-                                  const double* __restrict__ rec, const double* __restrict__ linF,
-                                  const double* __restrict__ linQ, double* dFdx, double* dQdx, double a, double b,
-                                  double* J, double* lu, const int* __restrict__ a2lu) {
+// (FilteredMatrix::addToMatrix).  Long slots are left to the workgroups from
+// slot_blocks on, one per chunk, and k_gather_matrices_fin.
+__global__ void __launch_bounds__(256) k_gather_matrices(int nnz, int n_mos, const int* __restrict__ mg_ptr,
+                                                         const int* __restrict__ mg_ent, const double* __restrict__ rec,
+                                                         const double* __restrict__ linF, const double* __restrict__ linQ,
+                                                         double* dFdx, double* dQdx, OutArgs<2> out, int slot_blocks,
+                                                         const int* __restrict__ cb, const int* __restrict__ ce,
+                                                         double* part) {
+  if ((int)blockIdx.x >= slot_blocks) {
+    __shared__ double sh[16];
+    const int c = blockIdx.x - slot_blocks;
+    double df = 0.0, dq = 0.0;
+#pragma unroll 4
+    for (int e = cb[c] + (int)threadIdx.x; e < ce[c]; e += 256) {
+      const int ent = mg_ent[e];
+      const int dev = ent >> 6, plane = ent & 63;
+      const double v = rec[(size_t)plane * n_mos + dev];
+      if (plane < R_JQ0) df += v; else dq += v;
+    }
+    df = wg_sum_fixed(df, sh);
+    dq = wg_sum_fixed(dq, sh);
+    if (threadIdx.x == 0) { part[2 * c] = df; part[2 * c + 1] = dq; }
+    return;
+  }
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nnz) return;
-  if (mg_ptr[s + 1] - mg_ptr[s] > kGatherLong) return;   // k_gather_matrices_long
+  if (mg_ptr[s + 1] - mg_ptr[s] > kGatherLong) return;
   double df = 0.0, dq = 0.0;
-  for (int e = mg_ptr[s]; e < mg_ptr[s + 1]; ++e) {
-    const int ent = mg_ent[e];
-    const int dev = ent >> 6, plane = ent & 63;
-    const double v = rec[(size_t)plane * n_mos + dev];
-    if (plane < R_JQ0) df += v; else dq += v;
+  const double lf = linF[s], lq = linQ[s];
+  const int e1 = mg_ptr[s + 1];
+  for (int e = mg_ptr[s]; e < e1; e += 4) {
+    int ent[4];
+    double v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) ent[j] = mg_ent[min(e + j, e1 - 1)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = rec[(size_t)(ent[j] & 63) * n_mos + (ent[j] >> 6)];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (e + j >= e1) break;
+      if ((ent[j] & 63) < R_JQ0) df += v[j]; else dq += v[j];
+    }
   }
-  if (linF[s] != 0.0) df += linF[s];
-  if (linQ[s] != 0.0) dq += linQ[s];
-  if (dFdx) { dFdx[s] = df; dQdx[s] = dq; }
-  if (J || lu) {
-    const double j = jac_combine_k(a, dq, b, df);
-    if (J) J[s] = j;
-    if (lu) lu[a2lu[s]] = j;
-  }
+  if (lf != 0.0) df += lf;
+  if (lq != 0.0) dq += lq;
+  dFdx[s] = df; dQdx[s] = dq;
+  out.put(0, s, df); out.put(1, s, dq);
 }
 
-// Long CSR slots: chunk partial sums of dFdx and dQdx terms ...
-__global__ void __launch_bounds__(256) k_gather_matrices_part(int n_mos, const int* __restrict__ cb,
-                                                              const int* __restrict__ ce, const int* __restrict__ mg_ent,
-                                                              const double* __restrict__ rec, double* part) {
-  __shared__ double sh[16];
-  const int c = blockIdx.x;
-  double df = 0.0, dq = 0.0;
-  for (int e = cb[c] + (int)threadIdx.x; e < ce[c]; e += blockDim.x) {
-    const int ent = mg_ent[e];
-    const int dev = ent >> 6, plane = ent & 63;
-    const double v = rec[(size_t)plane * n_mos + dev];
-    if (plane < R_JQ0) df += v; else dq += v;
-  }
-  df = wg_sum_fixed(df, sh);
-  dq = wg_sum_fixed(dq, sh);
-  if (threadIdx.x == 0) { part[2 * c] = df; part[2 * c + 1] = dq; }
-}
-
-// ... then one wavefront per long slot over its chunks [sc[l], sc[l + 1])
+// one wavefront per long slot over its chunks [sc[l], sc[l + 1])
 __global__ void __launch_bounds__(64) k_gather_matrices_fin(const int* __restrict__ slots, const int* __restrict__ sc,
                                                            const double* __restrict__ part,
                                                            const double* __restrict__ linF,
                                                            const double* __restrict__ linQ, double* dFdx, double* dQdx,
-                                                           double a, double b, double* J, double* lu,
-                                                           const int* __restrict__ a2lu) {
+                                                           OutArgs<2> out) {
   const int l = blockIdx.x, lane = threadIdx.x;
   const int s = slots[l];
   double df = 0.0, dq = 0.0;
@@ -281,20 +344,26 @@ __global__ void __launch_bounds__(64) k_gather_matrices_fin(const int* __restric
   if (lane != 0) return;
   if (linF[s] != 0.0) df += linF[s];
   if (linQ[s] != 0.0) dq += linQ[s];
-  if (dFdx) { dFdx[s] = df; dQdx[s] = dq; }
-  if (J || lu) {
-    const double j = jac_combine_k(a, dq, b, df);
-    if (J) J[s] = j;
-    if (lu) lu[a2lu[s]] = j;
-  }
+  dFdx[s] = df; dQdx[s] = dq;
+  out.put(0, s, df); out.put(1, s, dq);
 }
 
 // OneStep::obtainResidual (N_TIA_OneStep.C:219-289) / NoTimeIntegration (DC).
 #pragma clang fp contract(off)
-__global__ void k_combine_rhs(int n, int dcop, int order, double h, const double* F, const double* Q, const double* B,
-                              const double* FL, const double* QL, const double* q0, const double* q2, double* rhs) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// the residual (threads [0, n)) and the Jacobian (OneStep::obtainJacobian; from
+// thread n rounded up to 256 on); rhs, J and q2 may be null
+__global__ void __launch_bounds__(256) k_combine(int n, int nnz, int dcop, int order, double h, const double* F,
+                                                 const double* Q, const double* B, const double* FL, const double* QL,
+                                                 const double* q0, const double* q2, double* rhs, double a, double b,
+                                                 const double* dFdx, const double* dQdx, double* J) {
+  const int row_blocks = (n + 255) / 256;
+  if ((int)blockIdx.x >= row_blocks) {
+    const int s = (blockIdx.x - row_blocks) * 256 + threadIdx.x;
+    if (s < nnz && J) J[s] = a * dQdx[s] + b * dFdx[s];
+    return;
+  }
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n || !rhs) return;
   double r;
   if (dcop) {
     r = 1.0 * F[i] + -1.0 * B[i];
@@ -304,7 +373,7 @@ __global__ void k_combine_rhs(int n, int dcop, int order, double h, const double
     r = 1.0 * Q[i] + -1.0 * q0[i];
     if (order == 2) {
       r = (1.0 / h) * r + 0.5 * F[i] + -0.5 * B[i];
-      r = r + 0.5 * q2[i];
+      r = r + 0.5 * (q2 ? q2[i] : 0.0);
     } else {
       r = (1.0 / h) * r + 1.0 * F[i] + -1.0 * B[i];
     }
@@ -314,12 +383,6 @@ __global__ void k_combine_rhs(int n, int dcop, int order, double h, const double
     r = r + (order == 2 ? 0.5 : 1.0) * FL[i];
   }
   rhs[i] = r;
-}
-
-__global__ void k_combine_jac(int nnz, double a, double b, const double* dFdx, const double* dQdx, double* J) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nnz) return;
-  J[s] = a * dQdx[s] + b * dFdx[s];
 }
 #pragma clang fp contract(fast)
 
@@ -549,18 +612,6 @@ __global__ void k_axpy_f64(int n, const double* d, double* x) {
 __global__ void k_axpy_neg_f64(int n, const double* d, double* x) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] -= d[i];
-}
-
-// state permutation between the Xyce layout and the SoA planes
-__global__ void k_sta_to_soa(int n_mos, int nslots, const int* off0, const double* xy, double* soa) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_mos) return;
-  for (int j = 0; j < nslots; ++j) soa[(size_t)j * n_mos + i] = xy[off0[i] + j];
-}
-__global__ void k_soa_to_sta(int n_mos, int nslots, const int* off0, const double* soa, double* xy) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_mos) return;
-  for (int j = 0; j < nslots; ++j) xy[off0[i] + j] = soa[(size_t)j * n_mos + i];
 }
 
 inline unsigned nblk(size_t n, unsigned b = 256) { return (unsigned)((n + b - 1) / b); }
@@ -954,18 +1005,26 @@ struct xg_circuit {
   DBuf<int> mcls, lid, sta0, sto0;
   DBuf<unsigned long long> mask;
   DBuf<double> sto_cur, sto_nxt, sta_cur, sta_nxt, rec;
-  DBuf<double> x, F, Q, B, FL, QL, rhs, q0, q2, dFdx, dQdx, J, linF, linQ;
+  DBuf<double> x, F, Q, B, FL, QL, rhs, q0, q2, dFdx, dQdx, J, linF, linQ;   // rhs .. J: host-array calls
   DBuf<int> rowptr, colind, vg_ptr, vg_ent, mg_ptr, mg_ent, bg_ptr, bg_ent, src_wave, wave_type, wave_off, limited;
   // long rows / slots: chunk lists (kind, begin, end), per-entry chunk ranges, partial sums
   DBuf<int> long_rows, long_slots, vck, vcb, vce, vrc, mcb, mce, msc;
   DBuf<double> vpart, mpart;
   int n_long_rows = 0, n_long_slots = 0, n_vchunks = 0, n_mchunks = 0;
-  DBuf<double> wave_data, xy_sta, xy_sto;
+  DBuf<double> wave_data, xy_sta, xy_sto, xy_sta_next, xy_sto_next;   // host-array calls: the caller's vectors
+  int* hlimited = nullptr;      // pinned: the limiter flag of xg_update_state
   xg_solver_state ss{};
   // pinned host staging for the loads into host arrays (allocated on first use)
   double* hstage = nullptr;
   size_t hstage_n = 0;
-  ~xg_circuit() { if (hstage) (void)hipHostFree(hstage); }
+  ~xg_circuit() {
+    if (hstage) (void)hipHostFree(hstage);
+    if (hlimited) (void)hipHostFree(hlimited);
+  }
+  // vectors up to this many doubles in all go through the staging: the kernels
+  // read and write it directly, which costs them a few microseconds where every
+  // copy costs about ten (ring of 101 stages, one load: 268 -> 106 us)
+  static constexpr size_t kStageDirect = 32768;
   hipError_t stage(size_t cnt) {
     if (cnt <= hstage_n) return hipSuccess;
     if (hstage) { (void)hipHostFree(hstage); hstage = nullptr; hstage_n = 0; }
@@ -1052,14 +1111,15 @@ static int circuit_upload(xg_circuit* c) {
   HIPCHK(c->wave_type.upload(h.wave_type, s)); HIPCHK(c->wave_off.upload(h.wave_off, s));
   HIPCHK(c->wave_data.upload(h.wave_data, s));
   HIPCHK(c->limited.alloc(1));
-  HIPCHK(c->xy_sta.alloc(std::max(1, h.nsta))); HIPCHK(c->xy_sto.alloc(std::max(1, h.nsto)));
+  HIPCHK(hipHostMalloc((void**)&c->hlimited, sizeof(int), hipHostMallocDefault));
   k_fill<<<nblk(n + 1), 256, 0, s>>>(c->x.p, n + 1, 0.0);
   HIPCHK(hipStreamSynchronize(s));
   return XG_OK;
 }
 
-static void gather_vectors(xg_circuit* c);
-static void gather_matrices(xg_circuit* c);
+static void gather_vectors(xg_circuit* c, const OutArgs<5>& out);
+static void gather_matrices(xg_circuit* c, const OutArgs<2>& out);
+static void combine(xg_circuit* c, const double* q0, const double* q2, double* rhs, double* J);
 
 static SrcArgs src_args(xg_circuit* c) {
   SrcArgs a;
@@ -1094,23 +1154,16 @@ int circuit_load(xg_circuit* c) {
     a.limited = c->limited.p;
     a.fl.dcop = c->ss.dcop; a.fl.tran = c->ss.tran; a.fl.init_jct = c->ss.init_jct; a.fl.newton_iter = c->ss.newton_iter;
     a.fl.tranop = c->ss.tranop;
-    k_mos1_eval<<<nblk(N), 256, 0, s>>>(a);
+    k_mos1_eval<false><<<nblk(N), 256, 0, s>>>(a);
   }
-  gather_vectors(c);
-  gather_matrices(c);
+  gather_vectors(c, OutArgs<5>{});
+  gather_matrices(c, OutArgs<2>{});
   HIPCHK(hipGetLastError());
   return XG_OK;
 }
 
 int circuit_combine(xg_circuit* c, const double* q0, const double* q2, double* rhs, double* J) {
-  HostCircuit& h = c->hc;
-  hipStream_t s = c->stream;
-  const int n = h.n;
-  k_combine_rhs<<<nblk(n), 256, 0, s>>>(n, c->ss.dcop, c->ss.order, c->ss.h, c->F.p, c->Q.p, c->B.p, c->FL.p,
-                                        c->QL.p, c->ss.dcop ? c->F.p : q0, c->ss.dcop ? c->F.p : q2, rhs);
-  double a, b;
-  if (c->ss.dcop) { a = 1.0e-20; b = 1.0; } else { a = 1.0 / c->ss.h; b = c->ss.order == 2 ? 0.5 : 1.0; }
-  k_combine_jac<<<nblk(h.nnz), 256, 0, s>>>(h.nnz, a, b, c->dFdx.p, c->dQdx.p, J);
+  combine(c, q0, q2, rhs, J);
   HIPCHK(hipGetLastError());
   return XG_OK;
 }
@@ -1202,59 +1255,63 @@ static int update_state_impl(xg_circuit* c, const double* x, const double* sta_c
   HostCircuit& h = c->hc;
   hipStream_t s = c->stream;
   const int N = h.n_mos;
+  const size_t n = h.n, nsta = N > 0 ? h.nsta : 0, nsto = N > 0 ? h.nsto : 0;
   if (N > 0 && (!sta_cur || !sto_cur || !sta_next || !sto_next)) return XG_E_ARG;
-  const hipMemcpyKind in = dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-  HIPCHK(hipMemcpyAsync(c->x.p, x, sizeof(double) * h.n, in, s));
-  k_fill<<<1, 1, 0, s>>>(c->x.p + h.n, 1, 0.0);
-  if (N > 0) {
-    const double* sc = sta_cur;
-    const double* oc = sto_cur;
-    const double* on = sto_next;
-    if (!dev) {
-      HIPCHK(hipMemcpyAsync(c->xy_sta.p, sta_cur, sizeof(double) * h.nsta, hipMemcpyHostToDevice, s));
-      sc = c->xy_sta.p;
+  EvalArgs a{};
+  const double* xs = x;
+  a.sta_cur = sta_cur; a.sto_cur = sto_cur; a.sto_nxt_in = sto_next; a.sta_out = sta_next; a.sto_out = sto_next;
+  const bool direct = !dev && n + 2 * (nsta + nsto) <= xg_circuit::kStageDirect;
+  if (direct) {
+    HIPCHK(c->stage(n + 2 * (nsta + nsto)));
+    double* p = c->hstage;
+    auto put = [&](const double* from, size_t cnt) {
+      if (cnt) std::memcpy(p, from, cnt * sizeof(double));
+      double* at = p;
+      p += cnt;
+      return at;
+    };
+    xs = put(x, n);
+    a.sta_cur = put(sta_cur, nsta); a.sto_cur = put(sto_cur, nsto);
+    a.sta_out = put(sta_next, nsta);
+    a.sto_nxt_in = a.sto_out = put(sto_next, nsto);
+  } else if (!dev) {
+    if (N > 0 && !c->xy_sto_next.p) {
+      HIPCHK(c->xy_sta.alloc(nsta)); HIPCHK(c->xy_sto.alloc(nsto));
+      HIPCHK(c->xy_sta_next.alloc(nsta)); HIPCHK(c->xy_sto_next.alloc(nsto));
     }
-    k_sta_to_soa<<<nblk(N), 256, 0, s>>>(N, 8, c->sta0.p, sc, c->sta_cur.p);
-    if (!dev) {
-      HIPCHK(hipMemcpyAsync(c->xy_sto.p, sto_cur, sizeof(double) * h.nsto, hipMemcpyHostToDevice, s));
-      oc = c->xy_sto.p;
+    HIPCHK(hipMemcpyAsync(c->x.p, x, sizeof(double) * n, hipMemcpyHostToDevice, s));
+    if (N > 0) {
+      HIPCHK(hipMemcpyAsync(c->xy_sta.p, sta_cur, sizeof(double) * nsta, hipMemcpyHostToDevice, s));
+      HIPCHK(hipMemcpyAsync(c->xy_sto.p, sto_cur, sizeof(double) * nsto, hipMemcpyHostToDevice, s));
+      HIPCHK(hipMemcpyAsync(c->xy_sta_next.p, sta_next, sizeof(double) * nsta, hipMemcpyHostToDevice, s));
+      HIPCHK(hipMemcpyAsync(c->xy_sto_next.p, sto_next, sizeof(double) * nsto, hipMemcpyHostToDevice, s));
     }
-    k_sta_to_soa<<<nblk(N), 256, 0, s>>>(N, 6, c->sto0.p, oc, c->sto_cur.p);
-    if (!dev) {
-      HIPCHK(hipMemcpyAsync(c->xy_sto.p, sto_next, sizeof(double) * h.nsto, hipMemcpyHostToDevice, s));
-      on = c->xy_sto.p;
-    }
-    k_sta_to_soa<<<nblk(N), 256, 0, s>>>(N, 6, c->sto0.p, on, c->sto_nxt.p);
+    a.sta_cur = c->xy_sta.p; a.sto_cur = c->xy_sto.p; a.sta_out = c->xy_sta_next.p;
+    a.sto_nxt_in = a.sto_out = c->xy_sto_next.p;
   }
-  k_fill<<<1, 1, 0, s>>>(c->limited.p, 1, 0);
+  if (dev || direct) k_take_x<<<nblk(n + 1), 256, 0, s>>>((int)n, xs, c->x.p);
+  *c->hlimited = 0;
   if (N > 0) {
-    EvalArgs a;
     a.n_mos = N; a.cls = c->cls.p; a.mcls = c->mcls.p; a.tvbi = c->tvbi.p; a.beta = c->beta.p; a.tvto = c->tvto.p;
-    a.lid = c->lid.p; a.mask = c->mask.p; a.x = c->x.p; a.sto_cur = c->sto_cur.p; a.sto_nxt_in = c->sto_nxt.p;
-    a.sta_cur = c->sta_cur.p; a.sto_out = c->sto_nxt.p; a.sta_out = c->sta_nxt.p; a.rec = c->rec.p;
-    a.limited = c->limited.p;
+    a.lid = c->lid.p; a.mask = c->mask.p; a.x = c->x.p; a.sta0 = c->sta0.p; a.sto0 = c->sto0.p; a.rec = c->rec.p;
+    a.limited = c->hlimited;
     a.fl.dcop = c->ss.dcop; a.fl.tran = c->ss.tran; a.fl.init_jct = c->ss.init_jct; a.fl.newton_iter = c->ss.newton_iter;
     a.fl.tranop = c->ss.tranop;
-    k_mos1_eval<<<nblk(N), 256, 0, s>>>(a);
+    // (a device's thread reads its entries before it writes any: the next
+    // vectors may be the current ones)
+    k_mos1_eval<true><<<nblk(N), 256, 0, s>>>(a);
     HIPCHK(hipGetLastError());
-    // in-place read of sto_nxt_in vs write of sto_out: each thread reads its
-    // own inputs before writing its own outputs, so aliasing is safe.
-    if (dev) {
-      k_soa_to_sta<<<nblk(N), 256, 0, s>>>(N, 8, c->sta0.p, c->sta_nxt.p, sta_next);
-      k_soa_to_sta<<<nblk(N), 256, 0, s>>>(N, 6, c->sto0.p, c->sto_nxt.p, sto_next);
-    } else {
-      // the caller's other entries come back unchanged
-      HIPCHK(hipMemcpyAsync(c->xy_sta.p, sta_next, sizeof(double) * h.nsta, hipMemcpyHostToDevice, s));
-      k_soa_to_sta<<<nblk(N), 256, 0, s>>>(N, 8, c->sta0.p, c->sta_nxt.p, c->xy_sta.p);
-      HIPCHK(hipMemcpyAsync(sta_next, c->xy_sta.p, sizeof(double) * h.nsta, hipMemcpyDeviceToHost, s));
-      k_soa_to_sta<<<nblk(N), 256, 0, s>>>(N, 6, c->sto0.p, c->sto_nxt.p, c->xy_sto.p);
-      HIPCHK(hipMemcpyAsync(sto_next, c->xy_sto.p, sizeof(double) * h.nsto, hipMemcpyDeviceToHost, s));
+    if (!dev && !direct) {
+      HIPCHK(hipMemcpyAsync(sta_next, c->xy_sta_next.p, sizeof(double) * nsta, hipMemcpyDeviceToHost, s));
+      HIPCHK(hipMemcpyAsync(sto_next, c->xy_sto_next.p, sizeof(double) * nsto, hipMemcpyDeviceToHost, s));
     }
   }
-  int lim = 0;
-  HIPCHK(hipMemcpyAsync(&lim, c->limited.p, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  if (limited) *limited = lim;
+  if (direct && N > 0) {
+    std::memcpy(sta_next, a.sta_out, nsta * sizeof(double));
+    std::memcpy(sto_next, a.sto_out, nsto * sizeof(double));
+  }
+  if (limited) *limited = *c->hlimited;
   return XG_OK;
 }
 
@@ -1268,79 +1325,79 @@ int xg_update_state_dev(xg_circuit* c, const double* x, const double* sta_cur, c
   return update_state_impl(c, x, sta_cur, sto_cur, sta_next, sto_next, limited, true);
 }
 
-// Adds k device arrays of m entries each (this handle's contributions) into
-// the caller's arrays: device arrays by a kernel on the handle's stream, host
-// arrays through the pinned staging buffer.  Each output entry becomes
-// caller's value + contribution, one rounding, as a master's "+=" into a
-// vector the loader has zeroed or other devices have filled.
-static int accumulate_out(xg_circuit* c, int k, const double* const* src, double* const* dst, size_t m, bool dev) {
-  hipStream_t s = c->stream;
-  if (dev) {
-    for (int i = 0; i < k; ++i)
-      if (dst[i] && m) k_axpy_f64<<<nblk(m), 256, 0, s>>>((int)m, src[i], dst[i]);
-    HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(s));
-    return XG_OK;
-  }
-  int used = 0;
-  for (int i = 0; i < k; ++i) used += dst[i] != nullptr;
-  if (used == 0 || m == 0) { HIPCHK(hipStreamSynchronize(s)); return XG_OK; }
-  HIPCHK(c->stage((size_t)used * m));
-  for (int i = 0, j = 0; i < k; ++i)
-    if (dst[i]) HIPCHK(hipMemcpyAsync(c->hstage + (size_t)(j++) * m, src[i], sizeof(double) * m, hipMemcpyDeviceToHost, s));
-  HIPCHK(hipStreamSynchronize(s));
-  for (int i = 0, j = 0; i < k; ++i) {
-    if (!dst[i]) continue;
-    const double* st = c->hstage + (size_t)(j++) * m;
-    double* d = dst[i];
-    for (size_t e = 0; e < m; ++e) d[e] += st[e];
-  }
-  return XG_OK;
-}
-
-static void gather_vectors(xg_circuit* c) {
+static void gather_vectors(xg_circuit* c, const OutArgs<5>& out) {
   HostCircuit& h = c->hc;
   hipStream_t s = c->stream;
-  const int n = h.n;
-  k_gather_vectors<<<nblk(n), 256, 0, s>>>(n, h.n_mos, c->vg_ptr.p, c->vg_ent.p, c->rec.p, c->rowptr.p, c->colind.p,
-                                           c->linF.p, c->linQ.p, c->x.p, src_args(c), c->F.p, c->Q.p, c->B.p, c->FL.p, c->QL.p);
-  if (c->n_long_rows) {
-    k_gather_vectors_part<<<c->n_vchunks, 256, 0, s>>>(h.n_mos, c->vck.p, c->vcb.p, c->vce.p, c->vg_ent.p, c->rec.p,
-                                                       c->colind.p, c->linF.p, c->linQ.p, c->x.p, c->vpart.p);
+  const int n = h.n, rb = (int)nblk(n);
+  k_gather_vectors<<<rb + c->n_vchunks, 256, 0, s>>>(n, h.n_mos, c->vg_ptr.p, c->vg_ent.p, c->rec.p, c->rowptr.p,
+                                                     c->colind.p, c->linF.p, c->linQ.p, c->x.p, src_args(c), c->F.p,
+                                                     c->Q.p, c->B.p, c->FL.p, c->QL.p, out, rb, c->vck.p, c->vcb.p,
+                                                     c->vce.p, c->vpart.p);
+  if (c->n_long_rows)
     k_gather_vectors_fin<<<c->n_long_rows, 64, 0, s>>>(c->long_rows.p, c->vrc.p, c->vpart.p, src_args(c), c->F.p,
-                                                       c->Q.p, c->B.p, c->FL.p, c->QL.p);
-  }
+                                                       c->Q.p, c->B.p, c->FL.p, c->QL.p, out);
 }
 
-static void gather_matrices(xg_circuit* c) {
+static void gather_matrices(xg_circuit* c, const OutArgs<2>& out) {
   HostCircuit& h = c->hc;
   hipStream_t s = c->stream;
-  k_gather_matrices<<<nblk(h.nnz), 256, 0, s>>>(h.nnz, h.n_mos, c->mg_ptr.p, c->mg_ent.p, c->rec.p, c->linF.p,
-                                               c->linQ.p, c->dFdx.p, c->dQdx.p, 0.0, 0.0, nullptr, nullptr, nullptr);
-  if (c->n_long_slots) {
-    k_gather_matrices_part<<<c->n_mchunks, 256, 0, s>>>(h.n_mos, c->mcb.p, c->mce.p, c->mg_ent.p, c->rec.p, c->mpart.p);
+  const int sb = (int)nblk(h.nnz);
+  k_gather_matrices<<<sb + c->n_mchunks, 256, 0, s>>>(h.nnz, h.n_mos, c->mg_ptr.p, c->mg_ent.p, c->rec.p, c->linF.p,
+                                                     c->linQ.p, c->dFdx.p, c->dQdx.p, out, sb, c->mcb.p, c->mce.p,
+                                                     c->mpart.p);
+  if (c->n_long_slots)
     k_gather_matrices_fin<<<c->n_long_slots, 64, 0, s>>>(c->long_slots.p, c->msc.p, c->mpart.p, c->linF.p, c->linQ.p,
-                                                         c->dFdx.p, c->dQdx.p, 0.0, 0.0, nullptr, nullptr, nullptr);
+                                                         c->dFdx.p, c->dQdx.p, out);
+}
+
+// A load into K arrays of m entries of the caller's: each output entry becomes
+// caller's value + contribution, one rounding, as a master's "+=" into a vector
+// the loader has zeroed or other devices have filled.  Device arrays are added
+// to by the gather itself; host arrays through the pinned staging, which a small
+// load's gather writes directly.
+extern "C++" template <int K, class Gather>
+int load_into(xg_circuit* c, double* const (&dst)[K], const double* const (&src)[K], size_t m, bool dev,
+                     Gather gather) {
+  hipStream_t s = c->stream;
+  OutArgs<K> out{};
+  size_t used = 0;
+  for (int i = 0; i < K; ++i) used += dst[i] != nullptr;
+  const bool direct = !dev && used * m <= xg_circuit::kStageDirect;
+  if (!dev && used * m) HIPCHK(c->stage(used * m));
+  if (dev || direct) {
+    out.add = dev;
+    for (int i = 0, j = 0; i < K; ++i)
+      if (dst[i]) out.p[i] = dev ? dst[i] : c->hstage + (size_t)(j++) * m;
   }
+  gather(c, out);
+  HIPCHK(hipGetLastError());
+  if (!dev && !direct)
+    for (int i = 0, j = 0; i < K; ++i)
+      if (dst[i]) HIPCHK(hipMemcpyAsync(c->hstage + (size_t)(j++) * m, src[i], sizeof(double) * m, hipMemcpyDeviceToHost, s));
+  HIPCHK(hipStreamSynchronize(s));
+  if (!dev)
+    for (int i = 0, j = 0; i < K; ++i) {
+      if (!dst[i]) continue;
+      const double* st = c->hstage + (size_t)(j++) * m;
+      double* d = dst[i];
+      for (size_t e = 0; e < m; ++e) d[e] += st[e];
+    }
+  return XG_OK;
 }
 
 static int load_vectors_impl(xg_circuit* c, double* F, double* Q, double* B, double* dFdxdVp, double* dQdxdVp,
                              bool dev) {
   if (!c) return XG_E_ARG;
-  gather_vectors(c);
-  HIPCHK(hipGetLastError());
-  const double* src[5] = {c->F.p, c->Q.p, c->B.p, c->FL.p, c->QL.p};
-  double* dst[5] = {F, Q, B, dFdxdVp, dQdxdVp};
-  return accumulate_out(c, 5, src, dst, (size_t)c->hc.n, dev);
+  const double* const src[5] = {c->F.p, c->Q.p, c->B.p, c->FL.p, c->QL.p};
+  double* const dst[5] = {F, Q, B, dFdxdVp, dQdxdVp};
+  return load_into(c, dst, src, (size_t)c->hc.n, dev, gather_vectors);
 }
 
 static int load_matrices_impl(xg_circuit* c, double* dFdx_vals, double* dQdx_vals, bool dev) {
   if (!c) return XG_E_ARG;
-  gather_matrices(c);
-  HIPCHK(hipGetLastError());
-  const double* src[2] = {c->dFdx.p, c->dQdx.p};
-  double* dst[2] = {dFdx_vals, dQdx_vals};
-  return accumulate_out(c, 2, src, dst, (size_t)c->hc.nnz, dev);
+  const double* const src[2] = {c->dFdx.p, c->dQdx.p};
+  double* const dst[2] = {dFdx_vals, dQdx_vals};
+  return load_into(c, dst, src, (size_t)c->hc.nnz, dev, gather_matrices);
 }
 
 int xg_load_vectors(xg_circuit* c, double* F, double* Q, double* B, double* dFdxdVp, double* dQdxdVp) {
@@ -1359,27 +1416,46 @@ int xg_load_matrices_dev(xg_circuit* c, double* dFdx_vals, double* dQdx_vals) {
   return load_matrices_impl(c, dFdx_vals, dQdx_vals, true);
 }
 
+static void combine(xg_circuit* c, const double* q0, const double* q2, double* rhs, double* J) {
+  const HostCircuit& h = c->hc;
+  double a, b;
+  if (c->ss.dcop) { a = 1.0e-20; b = 1.0; } else { a = 1.0 / c->ss.h; b = c->ss.order == 2 ? 0.5 : 1.0; }
+  k_combine<<<nblk(h.n) + nblk(h.nnz), 256, 0, c->stream>>>(h.n, h.nnz, c->ss.dcop, c->ss.order, c->ss.h, c->F.p, c->Q.p,
+                                                            c->B.p, c->FL.p, c->QL.p, q0, q2, rhs, a, b, c->dFdx.p,
+                                                            c->dQdx.p, J);
+}
+
 static int combine_impl(xg_circuit* c, const double* q0, const double* q2, double* rhs, double* jac_vals, bool dev) {
   if (!c) return XG_E_ARG;
   HostCircuit& h = c->hc;
   hipStream_t s = c->stream;
-  const int n = h.n;
-  const hipMemcpyKind in = dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-  const hipMemcpyKind out = dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-  if (!c->ss.dcop) {
-    if (!q0) return XG_E_ARG;
-    HIPCHK(hipMemcpyAsync(c->q0.p, q0, sizeof(double) * n, in, s));
-    if (q2) HIPCHK(hipMemcpyAsync(c->q2.p, q2, sizeof(double) * n, in, s));
-    else k_fill<<<nblk(n), 256, 0, s>>>(c->q2.p, n, 0.0);
+  const size_t n = h.n, nnz = h.nnz;
+  if (c->ss.dcop) q0 = q2 = nullptr;
+  else if (!q0) return XG_E_ARG;
+  if (dev) {
+    combine(c, q0, q2, rhs, jac_vals);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s));
+    return XG_OK;
   }
-  k_combine_rhs<<<nblk(n), 256, 0, s>>>(n, c->ss.dcop, c->ss.order, c->ss.h, c->F.p, c->Q.p, c->B.p, c->FL.p, c->QL.p,
-                                        c->q0.p, c->q2.p, c->rhs.p);
-  double a, b;
-  if (c->ss.dcop) { a = 1.0e-20; b = 1.0; } else { a = 1.0 / c->ss.h; b = c->ss.order == 2 ? 0.5 : 1.0; }
-  k_combine_jac<<<nblk(h.nnz), 256, 0, s>>>(h.nnz, a, b, c->dFdx.p, c->dQdx.p, c->J.p);
+  if (3 * n + nnz <= xg_circuit::kStageDirect) {
+    HIPCHK(c->stage(3 * n + nnz));
+    double* p = c->hstage;
+    if (q0) std::memcpy(p, q0, n * sizeof(double));
+    if (q2) std::memcpy(p + n, q2, n * sizeof(double));
+    combine(c, q0 ? p : nullptr, q2 ? p + n : nullptr, rhs ? p + 2 * n : nullptr, jac_vals ? p + 3 * n : nullptr);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(s));
+    if (rhs) std::memcpy(rhs, p + 2 * n, n * sizeof(double));
+    if (jac_vals) std::memcpy(jac_vals, p + 3 * n, nnz * sizeof(double));
+    return XG_OK;
+  }
+  if (q0) HIPCHK(hipMemcpyAsync(c->q0.p, q0, sizeof(double) * n, hipMemcpyHostToDevice, s));
+  if (q2) HIPCHK(hipMemcpyAsync(c->q2.p, q2, sizeof(double) * n, hipMemcpyHostToDevice, s));
+  combine(c, q0 ? c->q0.p : nullptr, q2 ? c->q2.p : nullptr, c->rhs.p, c->J.p);
   HIPCHK(hipGetLastError());
-  if (rhs) HIPCHK(hipMemcpyAsync(rhs, c->rhs.p, sizeof(double) * n, out, s));
-  if (jac_vals) HIPCHK(hipMemcpyAsync(jac_vals, c->J.p, sizeof(double) * h.nnz, out, s));
+  if (rhs) HIPCHK(hipMemcpyAsync(rhs, c->rhs.p, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+  if (jac_vals) HIPCHK(hipMemcpyAsync(jac_vals, c->J.p, sizeof(double) * nnz, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   return XG_OK;
 }
