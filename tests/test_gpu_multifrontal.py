@@ -225,3 +225,53 @@ def test_automatic_method_solves_both_ways(gpu, name, method):
         P = lambda t: ctypes.c_void_p(t.data_ptr())
         assert X.lib().xg_lu_solve_noalloc(s.h, P(bd), P(xd)) == 0
         assert np.array_equal(xd.cpu().numpy(), x)
+
+
+def _level_case(name):
+    rng = np.random.default_rng(8)
+    if name == "one":
+        A = sp.csr_matrix(np.array([[2.5]]))
+    elif name.startswith("arrow"):          # a last row and column of n - 1 entries
+        n = int(name[5:])
+        A = sp.lil_matrix((n, n))
+        A[n - 1, :] = rng.uniform(-1, 1, n)
+        A[:, n - 1] = rng.uniform(-1, 1, n)[:, None]
+        A.setdiag(2.0 + n * rng.uniform(size=n))
+    else:
+        m = int(name[4:])
+        A = sp.kronsum(sp.diags([-1, 2.1, -1.1], [-1, 0, 1], shape=(m, m)),
+                       sp.diags([-1, 2.2, -0.9], [-1, 0, 1], shape=(m, m)))
+    A = sp.csr_matrix(A)
+    A.sort_indices()
+    return A
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("name", ["one", "arrow24", "arrow27", "arrow130", "arrow700", "grid8", "grid12", "grid13", "grid15"])
+def test_level_factors_in_lds_and_beyond(gpu, name, fp32):
+    """Level-scheduled systems whose factors and program fit LDS and the next
+    larger ones, with targets and rows of up to 700 terms: both directions,
+    after a refactor, a zero pivot and a value that is not finite.  Row sums are
+    dominated, so a backward-stable solve's residual is n eps."""
+    A = _level_case(name)
+    n = A.shape[0]
+    b = np.random.default_rng(9).normal(size=n)
+    s = X.DirectSolver(n, A.indptr, A.indices, method=1)
+    if fp32:
+        s.set_precision(1)
+    for k in (1.0, -3.0):
+        B = sp.csr_matrix((A.data * k, A.indices, A.indptr), shape=A.shape)
+        assert s.numeric(B.data) == 0
+        st, x = s.solve(b)
+        assert st == 0 and np.max(np.abs(B @ x - b)) <= 1e-12 * np.max(np.abs(b))
+        if not fp32:
+            st, xt = s.solve(b, transpose=True)
+            assert st == 0 and np.max(np.abs(B.T @ xt - b)) <= 1e-12 * np.max(np.abs(b))
+    assert s.numeric(A.data * 0.0) > 0
+    assert s.numeric(A.data) == 0
+    bad = b.copy()
+    bad[n // 2] = np.nan
+    st, x = s.solve(bad)
+    assert st != 0 and not x.any()
+    st, x = s.solve(b)
+    assert st == 0 and np.max(np.abs(A @ x - b)) <= 1e-12 * np.max(np.abs(b))

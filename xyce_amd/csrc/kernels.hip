@@ -436,15 +436,19 @@ __global__ void k_lu_factor_level(int t0, int t1, const int* __restrict__ tgt, c
 
 // pivot check: non-finite or zero pivot, or a multiplier beyond KLU's
 // threshold (|l_ij| > 1/0.001: KLU would have re-pivoted) -> bad = row + 1
+__global__ void k_flag_init(int* bad) {
+  bad[0] = 0x7fffffff;
+  bad[1] = 0;
+}
 template <class T>
-__global__ void k_lu_pivots(int n, const int* lu_rowptr, const int* diag, const T* lu, int* bad) {
+__global__ void k_lu_pivots(int n, const int* lu_rowptr, const int* diag, const T* lu, int* bad, int* fail) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double d = (double)lu[diag[i]];
   const bool hard = !(fabs(d) > 0.0) || !isfinite(d);
   bool b = hard;
   for (int p = lu_rowptr[i]; p < diag[i] && !b; ++p) b = !(fabs((double)lu[p]) <= 1.0e3);
-  if (b) atomicMin(bad, i + 1);
+  if (b) { atomicMin(bad, i + 1); *fail = 1; }
   if (hard) atomicOr(bad + 1, 1);   // a zero or non-finite pivot (else only the threshold)
 }
 
@@ -485,7 +489,174 @@ __global__ void __launch_bounds__(1024) k_lu_solve_1wg(int n, const int* __restr
     if (!isfinite(v)) bad = 1;
     x[pcol[j]] = v;
   }
-  if (bad) atomicOr(nan_flag, 1);
+  if (bad) *nan_flag = 1;
+}
+
+// The same factorisation and solves for systems whose factors and program fit
+// LDS: one launch each that stages both, walks the levels there and, for the
+// factorisation, tests the pivots.  From memory a level costs three dependent
+// loads (target, operands' positions, operands); from LDS its barrier and the
+// longest target, and targets and rows of more than kLuLong operations (a supply
+// row's) are summed by a wavefront.  Host arrays go through pinned staging that
+// the kernels read and write.  Ring of 103 unknowns, refactor and solve on host
+// arrays: 197 us with the kernels above, which larger systems keep, 72 here, of
+// which 46 are the two calls' launches and waits (7 unknowns).
+constexpr int kLuSmall = 512;             // threads
+constexpr int kLuLong = 24;
+constexpr size_t kLuSmallLds = 65024;     // (beside 16 bytes of static LDS)
+
+struct LuSmall {
+  int n, nlu, nnz_a;
+  const unsigned* prog;                   // packed program (LuProgram::pack)
+  int words_f, words_s;                   // its factor and its solve part
+  int nlev, nops, nfl, nbl;
+};
+
+template <class T>
+__device__ __forceinline__ T lu_wave_sum(T v) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// factor program: level bounds [nlev + 1], first operation of each target
+// [nlu + 1], targets [nlu] (position, position of the divisor or 0xffff),
+// operations [nops] (position of l, of u), diagonal positions and row starts [n]
+template <class T>
+__global__ void __launch_bounds__(kLuSmall) k_lu_small_factor(LuSmall P, const double* vals, double* keep,
+                                                             const int* a2lu, T* lu, int* verdict) {
+  extern __shared__ unsigned char lu_sm[];
+  T* A = reinterpret_cast<T*>(lu_sm);
+  unsigned* W = reinterpret_cast<unsigned*>(A + P.nlu + (P.nlu & 1));
+  __shared__ int first, any_hard;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = kLuSmall / 64;
+  if (t == 0) { first = 0x7fffffff; any_hard = 0; }
+  for (int i = t; i < P.nlu; i += kLuSmall) A[i] = (T)0;
+  for (int i = t; i < P.words_f; i += kLuSmall) W[i] = P.prog[i];
+  __syncthreads();
+  for (int i = t; i < P.nnz_a; i += kLuSmall) {
+    const double v = vals[i];
+    A[a2lu[i]] = (T)v;
+    if (keep) keep[i] = v;                // (values from the pinned staging)
+  }
+  const unsigned* lvl = W;
+  const unsigned* op0 = lvl + P.nlev + 1;
+  const unsigned* tgt = op0 + P.nlu + 1;
+  const unsigned* ops = tgt + P.nlu;
+  const unsigned* rows = ops + P.nops;
+  __syncthreads();
+  for (int l = 0; l < P.nlev; ++l) {
+    const int t0 = lvl[l], t1 = lvl[l + 1];
+    for (int i = t0 + t; i < t1; i += kLuSmall) {
+      const int o0 = op0[i], o1 = op0[i + 1];
+      if (o1 - o0 > kLuLong) continue;
+      const unsigned w = tgt[i];
+      T v = A[w & 0xffff];
+      for (int o = o0; o < o1; ++o) {
+        const unsigned q = ops[o];
+        v -= A[q & 0xffff] * A[q >> 16];
+      }
+      if ((w >> 16) != 0xffffu) v /= A[w >> 16];
+      A[w & 0xffff] = v;
+    }
+    // (a level's long targets: few, found by every wavefront)
+    for (int i0 = t0; i0 < t1; i0 += 64) {
+      const int i = i0 + lane;
+      unsigned long long m = __ballot(i < t1 && (int)(op0[i + 1] - op0[i]) > kLuLong);
+      for (int k = 0; m; ++k, m &= m - 1) {
+        if (k % nw != wave) continue;
+        const int j = i0 + (int)__builtin_ctzll(m);
+        T s = (T)0;
+        for (int o = (int)op0[j] + lane; o < (int)op0[j + 1]; o += 64) {
+          const unsigned q = ops[o];
+          s += A[q & 0xffff] * A[q >> 16];
+        }
+        s = lu_wave_sum(s);
+        if (lane == 0) {
+          const unsigned w = tgt[j];
+          T v = A[w & 0xffff] - s;
+          if ((w >> 16) != 0xffffu) v /= A[w >> 16];
+          A[w & 0xffff] = v;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = t; i < P.n; i += kLuSmall) {
+    const int dg = rows[i] & 0xffff, r0 = rows[i] >> 16;
+    const double d = (double)A[dg];
+    const bool hard = !(fabs(d) > 0.0) || !isfinite(d);
+    bool b = hard;
+    for (int p = r0; p < dg && !b; ++p) b = !(fabs((double)A[p]) <= 1.0e3);
+    if (b) atomicMin(&first, i + 1);
+    if (hard) any_hard = 1;
+  }
+  for (int i = t; i < P.nlu; i += kLuSmall) lu[i] = A[i];
+  __syncthreads();
+  if (t == 0) { verdict[0] = first == 0x7fffffff ? 0 : first; verdict[1] = any_hard; }
+}
+
+// solve program: forward level bounds [nfl + 1], backward [nbl + 1], their rows
+// [n + n] (row, then its positions: start | diagonal << 16), end of the last row
+// and column indices in halves
+template <class T>
+__global__ void __launch_bounds__(kLuSmall) k_lu_small_solve(LuSmall P, const T* lu, const int* prow, const int* pcol,
+                                                            const double* b, double* x, int* nan_flag) {
+  extern __shared__ unsigned char lu_sm[];
+  T* A = reinterpret_cast<T*>(lu_sm);
+  T* y = A + P.nlu;
+  unsigned* W = reinterpret_cast<unsigned*>(y + P.n + ((P.nlu + P.n) & 1));
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nw = kLuSmall / 64;
+  for (int i = t; i < P.nlu; i += kLuSmall) A[i] = lu[i];
+  for (int i = t; i < P.words_s; i += kLuSmall) W[i] = P.prog[P.words_f + i];
+  for (int i = t; i < P.n; i += kLuSmall) y[i] = (T)b[prow[i]];
+  const unsigned* fl = W;
+  const unsigned* bl = fl + P.nfl + 1;
+  const unsigned* frow = bl + P.nbl + 1;
+  const unsigned* brow = frow + P.n;
+  const unsigned* pos = brow + P.n;               // [n + 1]: start | diagonal << 16
+  const unsigned short* col = reinterpret_cast<const unsigned short*>(pos + P.n + 1);
+  __syncthreads();
+  for (int pass = 0; pass < 2; ++pass) {
+    const unsigned* lv = pass ? bl : fl;
+    const unsigned* row = pass ? brow : frow;
+    const int nl = pass ? P.nbl : P.nfl;
+    for (int l = 0; l < nl; ++l) {
+      const int t0 = lv[l], t1 = lv[l + 1];
+      for (int k = t0 + t; k < t1; k += kLuSmall) {
+        const int i = row[k], dg = pos[i] >> 16;
+        const int p0 = pass ? dg + 1 : pos[i] & 0xffff, p1 = pass ? pos[i + 1] & 0xffff : dg;
+        if (p1 - p0 > kLuLong) continue;
+        T v = y[i];
+        for (int p = p0; p < p1; ++p) v -= A[p] * y[col[p]];
+        y[i] = pass ? v / A[dg] : v;
+      }
+      for (int k0 = t0; k0 < t1; k0 += 64) {
+        const int k = k0 + lane, i = k < t1 ? (int)row[k] : 0, dg = pos[i] >> 16;
+        const int p0 = pass ? dg + 1 : pos[i] & 0xffff, p1 = pass ? pos[i + 1] & 0xffff : dg;
+        unsigned long long m = __ballot(k < t1 && p1 - p0 > kLuLong);
+        for (int q = 0; m; ++q, m &= m - 1) {
+          if (q % nw != wave) continue;
+          const int src = (int)__builtin_ctzll(m);
+          const int ii = __shfl(i, src), a0 = __shfl(p0, src), a1 = __shfl(p1, src), d = __shfl(dg, src);
+          T s = (T)0;
+          for (int p = a0 + lane; p < a1; p += 64) s += A[p] * y[col[p]];
+          s = lu_wave_sum(s);
+          if (lane == 0) {
+            const T v = y[ii] - s;
+            y[ii] = pass ? v / A[d] : v;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  bool bad = false;
+  for (int j = t; j < P.n; j += kLuSmall) {
+    const double v = (double)y[j];
+    bad |= !isfinite(v);
+    x[pcol[j]] = v;
+  }
+  if (bad) *nan_flag = 1;
 }
 
 // transpose solves B^T z = c = U^T L^T z: U^T by the backward levels in reverse
@@ -543,7 +714,7 @@ __global__ void k_permute_out(int n, const int* pcol, const T* y, double* x, int
   if (j < n) {
     const double v = (double)y[j];
     x[pcol[j]] = v;
-    if (!isfinite(v)) atomicOr(nan_flag, 1);
+    if (!isfinite(v)) *nan_flag = 1;
   }
 }
 
@@ -609,6 +780,10 @@ __global__ void k_axpy_f64(int n, const double* d, double* x) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] += d[i];
 }
+__global__ void k_copy_f64(size_t n, const double* a, double* b) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) b[i] = a[i];
+}
 __global__ void k_axpy_neg_f64(int n, const double* d, double* x) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] -= d[i];
@@ -667,6 +842,18 @@ struct xg_lu {
   DBuf<unsigned long long> red;
   std::vector<int> h_flvl, h_fs, h_bs;
   bool one_wg = true;
+  bool small = false;           // factors and program fit LDS (k_lu_small_*)
+  LuSmall sm{};
+  DBuf<unsigned> prog;
+  size_t lds_f[2] = {0, 0}, lds_s[2] = {0, 0};   // dynamic LDS, FP64 and FP32
+  // pinned: first failing pivot + 1 and whether one was zero or not finite (small
+  // systems), a non-finite solution, a failed pivot (other level systems)
+  int* hflag = nullptr;
+  int* nan_flag() const { return hflag + 2; }
+  // pinned staging of small host arrays, read and written by the kernels
+  double* hstage = nullptr;
+  bool staged = false;          // the next factorisation reads its values there and keeps them
+  static constexpr size_t kStage = 32768;
   std::vector<int> a_rowptr, a_colind;
   // precision: 0 = FP64 factors; 1 = FP32 factors + FP64 iterative refinement
   int mode = 0;
@@ -690,7 +877,11 @@ struct xg_lu {
   xg_lu* tlu = nullptr;
   bool tlu_current = false;
 
-  ~xg_lu() { if (tlu) (void)xg_lu_destroy(tlu); }
+  ~xg_lu() {
+    if (tlu) (void)xg_lu_destroy(tlu);
+    if (hflag) (void)hipHostFree(hflag);
+    if (hstage) (void)hipHostFree(hstage);
+  }
 
   bool level_fits(const double* values) const {
     const int n = (int)a_rowptr.size() - 1;
@@ -701,12 +892,12 @@ struct xg_lu {
   }
 
   // symbolic analysis for the chosen (or automatically picked) method.  The
-  // line: up to 128 unknowns one workgroup walks the levels of the entry program
-  // about as fast as the multifrontal launches follow each other, and its first
-  // pass needs no graph (ring of 103 unknowns: refactor and solve 196 us against
-  // 188, first pass 226 against 285); above, its levels grow with the system and
-  // the supernode tree's do not (gate array of 298: 758 us against 242, of 1481:
-  // 6990 against 562).
+  // line: up to 128 unknowns the levels are walked in LDS, one launch each for
+  // factors and solve (ring of 103 unknowns: refactor and solve 72 us against 117
+  // with the multifrontal launches, of 33: 57 against 91; a grid of 104, with
+  // three times the levels: 155 against 109); above, the levels grow with the
+  // system, the supernode tree's do not, and soon LDS is full (12 x 12 grid: 206
+  // us against 117, 16 x 16: 742 against 161, gate array of 298: 734 against 159).
   static constexpr int kLevelMaxN = 128;
   int analyse(const double* values, int want_method) {
     const int n = (int)a_rowptr.size() - 1;
@@ -750,6 +941,16 @@ struct xg_lu {
 
   int upload() {
     hipStream_t st = stream;
+    if (!hflag) HIPCHK(hipHostMalloc((void**)&hflag, 4 * sizeof(int), hipHostMallocDefault));
+    if (!hstage && (size_t)s.nnz_a <= kStage && 2 * (size_t)s.n <= kStage)
+      HIPCHK(hipHostMalloc((void**)&hstage, std::max((size_t)s.nnz_a, 2 * (size_t)s.n) * sizeof(double),
+                           hipHostMallocDefault));
+    // (a re-pivot keeps the buffers of values and vectors: their sizes are the pattern's)
+    if (!avals.p) {
+      HIPCHK(avals.alloc(s.nnz_a)); HIPCHK(b.alloc(s.n)); HIPCHK(x.alloc(s.n)); HIPCHK(r.alloc(s.n)); HIPCHK(d.alloc(s.n));
+      HIPCHK(flag.alloc(2)); HIPCHK(red.alloc(2));
+      k_flag_init<<<1, 1, 0, st>>>(flag.p);
+    }
     {
       const int rc = setup_long_rows();
       if (rc != XG_OK) return rc;
@@ -757,8 +958,6 @@ struct xg_lu {
     if (method == 2) {
       HIPCHK(prow.upload(s.perm_row, st)); HIPCHK(pcol.upload(s.perm_col, st));
       HIPCHK(arp.upload(a_rowptr, st)); HIPCHK(aci.upload(a_colind, st));
-      HIPCHK(flag.alloc(2)); HIPCHK(red.alloc(2));
-      HIPCHK(avals.alloc(s.nnz_a)); HIPCHK(b.alloc(s.n)); HIPCHK(x.alloc(s.n)); HIPCHK(r.alloc(s.n)); HIPCHK(d.alloc(s.n));
       mfp = std::make_unique<MfLu>();
       const int rc = mfp->setup(s, a_rowptr.data(), a_colind.data(), (void*)stream, true);
       if (rc != XG_OK) return rc;
@@ -776,19 +975,71 @@ struct xg_lu {
     HIPCHK(bs_ptr.upload(s.bs_lvl_ptr, st)); HIPCHK(bs_rows.upload(s.bs_rows, st));
     HIPCHK(prow.upload(s.perm_row, st)); HIPCHK(pcol.upload(s.perm_col, st));
     HIPCHK(arp.upload(a_rowptr, st)); HIPCHK(aci.upload(a_colind, st));
-    HIPCHK(flag.alloc(2)); HIPCHK(red.alloc(2));
-    HIPCHK(lu.alloc(s.nlu)); HIPCHK(avals.alloc(s.nnz_a)); HIPCHK(y.alloc(s.n)); HIPCHK(b.alloc(s.n));
-    HIPCHK(x.alloc(s.n)); HIPCHK(r.alloc(s.n)); HIPCHK(d.alloc(s.n));
+    HIPCHK(lu.alloc(s.nlu)); HIPCHK(y.alloc(s.n));
     if (mode == 1) { HIPCHK(lu32.alloc(s.nlu)); HIPCHK(y32.alloc(s.n)); }
     h_flvl = s.f_lvl_ptr; h_fs = s.fs_lvl_ptr; h_bs = s.bs_lvl_ptr;
     have_t = false;   // a new pattern: the transpose column lists are rebuilt when next needed
     const int nlev = (int)s.f_lvl_ptr.size() - 1;
     one_wg = s.nlu <= (1 << 20) && nlev <= 4096 && s.n <= (1 << 16);
+    {
+      const int rc = pack_small();
+      if (rc != XG_OK) return rc;
+    }
     have64 = false;
     return XG_OK;
   }
 
+  // the program of the LDS-resident kernels, where it and the factors fit
+  int pack_small() {
+    small = false;
+    const size_t nops = s.f_ops.size() / 2, nlev = s.f_lvl_ptr.size() - 1;
+    if (s.nlu >= 0xffff || s.n >= 0xffff) return XG_OK;
+    std::vector<unsigned> w;
+    w.insert(w.end(), s.f_lvl_ptr.begin(), s.f_lvl_ptr.end());
+    w.insert(w.end(), s.f_op_ptr.begin(), s.f_op_ptr.end());
+    for (int t = 0; t < s.nlu; ++t)
+      w.push_back((unsigned)s.f_tgt[t] | (s.f_div[t] >= 0 ? (unsigned)s.f_div[t] << 16 : 0xffff0000u));
+    for (size_t o = 0; o < nops; ++o) w.push_back((unsigned)s.f_ops[2 * o] | (unsigned)s.f_ops[2 * o + 1] << 16);
+    for (int i = 0; i < s.n; ++i) w.push_back((unsigned)s.lu_diag[i] | (unsigned)s.lu_rowptr[i] << 16);
+    sm.words_f = (int)w.size();
+    w.insert(w.end(), s.fs_lvl_ptr.begin(), s.fs_lvl_ptr.end());
+    w.insert(w.end(), s.bs_lvl_ptr.begin(), s.bs_lvl_ptr.end());
+    w.insert(w.end(), s.fs_rows.begin(), s.fs_rows.end());
+    w.insert(w.end(), s.bs_rows.begin(), s.bs_rows.end());
+    for (int i = 0; i < s.n; ++i) w.push_back((unsigned)s.lu_rowptr[i] | (unsigned)s.lu_diag[i] << 16);
+    w.push_back((unsigned)s.nlu);
+    for (int p = 0; p < s.nlu; p += 2)
+      w.push_back((unsigned)s.lu_colind[p] | (p + 1 < s.nlu ? (unsigned)s.lu_colind[p + 1] << 16 : 0u));
+    sm.words_s = (int)w.size() - sm.words_f;
+    for (int k = 0; k < 2; ++k) {
+      const size_t e = k ? 4 : 8;
+      lds_f[k] = (s.nlu + 1) * e + 4 * (size_t)sm.words_f;
+      lds_s[k] = (s.nlu + s.n + 1) * e + 4 * (size_t)sm.words_s;
+    }
+    if (lds_f[0] > kLuSmallLds || lds_s[0] > kLuSmallLds) return XG_OK;
+    sm.n = s.n; sm.nlu = s.nlu; sm.nnz_a = s.nnz_a;
+    sm.nlev = (int)nlev; sm.nops = (int)nops;
+    sm.nfl = (int)s.fs_lvl_ptr.size() - 1; sm.nbl = (int)s.bs_lvl_ptr.size() - 1;
+    HIPCHK(prog.upload(w, stream));
+    HIPCHK(hipStreamSynchronize(stream));
+    sm.prog = prog.p;
+    small = true;
+    return XG_OK;
+  }
+
   // numeric factorisation of the values in `avals`, into FP64 or FP32 storage
+  template <class T>
+  int factor_small(T* f, int* bad_out, int* hard_out) {
+    const bool st = staged;
+    staged = false;
+    k_lu_small_factor<T><<<1, kLuSmall, lds_f[sizeof(T) == 4], stream>>>(sm, st ? hstage : avals.p, st ? avals.p : nullptr,
+                                                                         a2lu.p, f, hflag);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(stream));
+    *bad_out = hflag[0];
+    *hard_out = hflag[1];
+    return XG_OK;
+  }
   template <class T>
   int factor_device(T* f) {
     const int nlev = (int)h_flvl.size() - 1;
@@ -807,11 +1058,14 @@ struct xg_lu {
   }
   template <class T>
   int check_pivots(const T* f, int* bad_out, int* hard_out) {
-    int init[2] = {0x7fffffff, 0};
-    HIPCHK(hipMemcpyAsync(flag.p, init, sizeof(init), hipMemcpyHostToDevice, stream));
-    k_lu_pivots<T><<<nblk(s.n), 256, 0, stream>>>(s.n, lu_rowptr.p, lu_diag.p, f, flag.p);
+    hflag[3] = 0;
+    k_lu_pivots<T><<<nblk(s.n), 256, 0, stream>>>(s.n, lu_rowptr.p, lu_diag.p, f, flag.p, hflag + 3);
+    HIPCHK(hipStreamSynchronize(stream));
+    *bad_out = *hard_out = 0;
+    if (!hflag[3]) return XG_OK;
     int res[2];
     HIPCHK(hipMemcpyAsync(res, flag.p, sizeof(res), hipMemcpyDeviceToHost, stream));
+    k_flag_init<<<1, 1, 0, stream>>>(flag.p);
     HIPCHK(hipStreamSynchronize(stream));
     *bad_out = res[0] == 0x7fffffff ? 0 : res[0];
     *hard_out = res[1];
@@ -868,7 +1122,9 @@ struct xg_lu {
   template <class T>
   int solve_device(const T* f, T* yy, const double* db, double* dx, int* nan_flag) {
     const int n = s.n;
-    if (one_wg) {
+    if (small) {
+      k_lu_small_solve<T><<<1, kLuSmall, lds_s[sizeof(T) == 4], stream>>>(sm, f, prow.p, pcol.p, db, dx, nan_flag);
+    } else if (one_wg) {
       k_lu_solve_1wg<T><<<1, 1024, 0, stream>>>(n, lu_rowptr.p, lu_colind.p, lu_diag.p, f, (int)h_fs.size() - 1,
                                                 fs_ptr.p, fs_rows.p, (int)h_bs.size() - 1, bs_ptr.p, bs_rows.p,
                                                 prow.p, pcol.p, db, yy, dx, nan_flag);
@@ -889,29 +1145,28 @@ struct xg_lu {
   // *hard = 1 if a pivot was zero or not finite)
   int factor_any(bool fp32, int* bad, int* hard) {
     if (method == 2) return mfp->factor(avals.p, s.nnz_a, fp32, bad, hard);
+    if (small) return fp32 ? factor_small<float>(lu32.p, bad, hard) : factor_small<double>(lu.p, bad, hard);
     const int st = fp32 ? factor_device<float>(lu32.p) : factor_device<double>(lu.p);
     if (st != XG_OK) return st;
     return fp32 ? check_pivots<float>(lu32.p, bad, hard) : check_pivots<double>(lu.p, bad, hard);
   }
   int solve_any(bool fp32, const double* db, double* dx) {
-    if (method == 2) return mfp->solve(db, dx, fp32, flag.p + 1);
-    return fp32 ? solve_device<float>(lu32.p, y32.p, db, dx, flag.p + 1)
-                : solve_device<double>(lu.p, y.p, db, dx, flag.p + 1);
+    if (method == 2) return mfp->solve(db, dx, fp32, nan_flag());
+    return fp32 ? solve_device<float>(lu32.p, y32.p, db, dx, nan_flag()) : solve_device<double>(lu.p, y.p, db, dx, nan_flag());
   }
   // FP64-factor solve whose work vectors and flag are the caller's device
   // memory `work` (work_doubles() doubles, 256-byte aligned) instead of the
-  // handle's buffers; *nan_flag is the first word of the work area
+  // handle's buffers
   size_t work_doubles() const {
     const size_t flag_d = 32;                       // one int, padded to 256 bytes
     if (method == 2) return flag_d + mfp->solve_work_doubles();
     return flag_d + (((size_t)s.n + 31) & ~(size_t)31);
   }
   int solve_with_work(const double* db, double* dx, double* work) {
-    int* nan_flag = reinterpret_cast<int*>(work);
     double* w = work + 32;
-    k_fill<<<1, 1, 0, stream>>>(nan_flag, 1, 0);
-    if (method == 2) return mfp->solve_ext(db, dx, nan_flag, w);
-    return solve_device<double>(lu.p, w, db, dx, nan_flag);
+    *nan_flag() = 0;
+    if (method == 2) return mfp->solve_ext(db, dx, nan_flag(), w);
+    return solve_device<double>(lu.p, w, db, dx, nan_flag());
   }
   // FP64 factors whose multipliers exceeded KLU's threshold: solve, then
   // refine x += A^-1 r against A in FP64 while the residual decreases, up to
@@ -971,7 +1226,7 @@ struct xg_lu {
       if (rel <= ir_tol) break;
       if (it >= ir_max || !(rel < prev)) {
         // refinement does not converge with the FP32 factors: FP64 factors
-        HIPCHK(hipMemsetAsync(flag.p + 1, 0, sizeof(int), stream));
+        *nan_flag() = 0;             // (residual() has waited for the stream)
         if (!have64) {
           int bad64 = 0, hard64 = 0;
           st = factor_any(false, &bad64, &hard64);
@@ -1469,7 +1724,8 @@ int xg_combine_dev(xg_circuit* c, const double* q0, const double* q2, double* rh
 }
 
 // ---------------- LU ----------------
-int xg_lu_symbolic_ex(int n, const int* rowptr, const int* colind, const double* values, int method, xg_lu** out) {
+static int lu_create(int n, const int* rowptr, const int* colind, const double* values, int method, hipStream_t stream,
+                     xg_lu** out) {
   if (n <= 0 || !rowptr || !colind || !out || method < 0 || method > 2) return XG_E_ARG;
   if (!xg::valid_csr(n, rowptr, colind)) return XG_E_ARG;
   int ndev = 0;
@@ -1485,14 +1741,21 @@ int xg_lu_symbolic_ex(int n, const int* rowptr, const int* colind, const double*
   } catch (...) {
     return XG_E_SETUP;
   }
-  if (hipStreamCreate(&lu->stream) != hipSuccess) return XG_E_HIP;
-  lu->own_stream = true;
+  lu->stream = stream;
+  if (!stream) {
+    if (hipStreamCreate(&lu->stream) != hipSuccess) return XG_E_HIP;
+    lu->own_stream = true;
+  }
   int st = lu->upload();
   if (st != XG_OK) return st;
   // the no-allocation solve's work area on this device (looked up once per device)
   if (scratch_address(&lu->scratch_work) != XG_OK) lu->scratch_work = nullptr;
   *out = lu.release();
   return XG_OK;
+}
+
+int xg_lu_symbolic_ex(int n, const int* rowptr, const int* colind, const double* values, int method, xg_lu** out) {
+  return lu_create(n, rowptr, colind, values, method, nullptr, out);
 }
 
 int xg_lu_symbolic(int n, const int* rowptr, const int* colind, const double* values, xg_lu** out) {
@@ -1523,8 +1786,15 @@ static int lu_factor64(xg_lu* lu, bool fp32_failed, int* bad, int* hard) {
 static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
   if (!lu || !vals) return XG_E_ARG;
   hipStream_t s = lu->stream;
-  const hipMemcpyKind in = dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-  HIPCHK(hipMemcpyAsync(lu->avals.p, vals, sizeof(double) * lu->s.nnz_a, in, s));
+  const size_t nnz = lu->s.nnz_a;
+  if (!dev && lu->hstage) {
+    // small host arrays: the copy kernel reads the staging (a copy of its own costs more than it)
+    std::memcpy(lu->hstage, vals, nnz * sizeof(double));
+    if (lu->small) lu->staged = true;
+    else k_copy_f64<<<nblk(nnz), 256, 0, s>>>(nnz, lu->hstage, lu->avals.p);
+  } else if (vals != lu->avals.p) {
+    HIPCHK(hipMemcpyAsync(lu->avals.p, vals, sizeof(double) * nnz, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
+  }
   lu->have64 = false;
   lu->soft64 = false;
   lu->tlu_current = false;
@@ -1597,30 +1867,47 @@ static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, b
   if (transpose && (lu->mode == 1 || !lu->have64 || lu->soft64)) return XG_E_ARG;
   if (transpose && lu->method != 1) return lu->asked == 0 ? lu_solve_transpose_auto(lu, b, x, dev) : XG_E_ARG;
   hipStream_t s = lu->stream;
-  const int n = lu->s.n;
-  HIPCHK(hipMemcpyAsync(lu->b.p, b, sizeof(double) * n, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
-  k_fill<<<1, 1, 0, s>>>(lu->flag.p + 1, 1, 0);
+  const size_t n = lu->s.n;
+  const bool direct = !dev && lu->hstage;
+  // (one small kernel: it reads and writes the staging itself)
+  const bool inplace = direct && lu->small && lu->have64 && !lu->soft64 && !transpose;
+  if (direct) {
+    std::memcpy(lu->hstage, b, n * sizeof(double));
+    if (!inplace) k_copy_f64<<<nblk(n), 256, 0, s>>>(n, lu->hstage, lu->b.p);
+  } else if (b != lu->b.p) {
+    HIPCHK(hipMemcpyAsync(lu->b.p, b, sizeof(double) * n, dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
+  }
+  *lu->nan_flag() = 0;
   int st;
-  if (transpose) st = lu->solve_transpose(lu->b.p, lu->x.p, lu->flag.p + 1);
+  if (transpose) st = lu->solve_transpose(lu->b.p, lu->x.p, lu->nan_flag());
   else if (lu->mode == 1 && !lu->have64) st = lu->solve_refined(lu->b.p, lu->x.p);
   else if (lu->soft64) st = lu->solve_refined64(lu->b.p, lu->x.p);
-  else st = lu->solve_any(false, lu->b.p, lu->x.p);
+  else st = lu->solve_any(false, inplace ? lu->hstage : lu->b.p, inplace ? lu->hstage + n : lu->x.p);
   if (st != XG_OK) return st;
-  int nanf = 0;
-  HIPCHK(hipMemcpyAsync(&nanf, lu->flag.p + 1, sizeof(int), hipMemcpyDeviceToHost, s));
-  if (dev) {
-    HIPCHK(hipStreamSynchronize(s));
-    // the solve kernels flag every non-finite result
-    if (nanf) { k_fill<<<nblk(n), 256, 0, s>>>(x, (size_t)n, 0.0); HIPCHK(hipStreamSynchronize(s)); return XG_E_NAN; }
-    HIPCHK(hipMemcpyAsync(x, lu->x.p, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-    HIPCHK(hipStreamSynchronize(s));
-    return XG_OK;
-  }
-  HIPCHK(hipMemcpyAsync(x, lu->x.p, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+  // the result goes out before the wait; a non-finite one, which every solve
+  // kernel flags, is replaced by zeros after it
+  if (direct && !inplace) k_copy_f64<<<nblk(n), 256, 0, s>>>(n, lu->x.p, lu->hstage + n);
+  else if (!direct && x != lu->x.p)
+    HIPCHK(hipMemcpyAsync(x, lu->x.p, sizeof(double) * n, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  bool bad = nanf != 0;
-  for (int i = 0; i < n && !bad; ++i) bad = !std::isfinite(x[i]);
-  if (bad) { std::fill(x, x + n, 0.0); return XG_E_NAN; }
+  if (*lu->nan_flag()) {
+    if (dev) {
+      k_fill<<<nblk(n), 256, 0, s>>>(x, n, 0.0);
+      HIPCHK(hipStreamSynchronize(s));
+    } else {
+      std::fill(x, x + n, 0.0);
+    }
+    return XG_E_NAN;
+  }
+  if (direct) std::memcpy(x, lu->hstage + n, n * sizeof(double));
+  if (!dev && (transpose || !lu->have64 || lu->soft64)) {
+    // (refined and transposed ones are summed up outside the checked kernels)
+    for (size_t i = 0; i < n; ++i) {
+      if (std::isfinite(x[i])) continue;
+      std::fill(x, x + n, 0.0);
+      return XG_E_NAN;
+    }
+  }
   return XG_OK;
 }
 
@@ -1643,10 +1930,8 @@ int xg_lu_solve_noalloc(xg_lu* lu, const double* b, double* x) {
   hipStream_t s = lu->stream;
   int st = lu->solve_with_work(b, x, lu->scratch_work);
   if (st != XG_OK) return st;
-  int nanf = 0;
-  HIPCHK(hipMemcpyAsync(&nanf, lu->scratch_work, sizeof(int), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
-  if (nanf) {
+  if (*lu->nan_flag()) {
     k_fill<<<nblk(lu->s.n), 256, 0, s>>>(x, (size_t)lu->s.n, 0.0);
     HIPCHK(hipStreamSynchronize(s));
     return XG_E_NAN;
@@ -1693,3 +1978,43 @@ int xg_lu_info(const xg_lu* lu, double* info) {
 }
 
 }  // extern "C"
+
+namespace xg {
+
+int lu_create_on(int n, const int* rowptr, const int* colind, int method, void* stream, xg_lu** out) {
+  return lu_create(n, rowptr, colind, nullptr, method, (hipStream_t)stream, out);
+}
+
+LuDev lu_dev(xg_lu* lu) { return LuDev{lu->avals.p, lu->b.p, lu->x.p}; }
+
+// With plain FP64 multifrontal factors the solve is enqueued behind the
+// factorisation and both are judged after one wait; factors that turn out to
+// need new pivots or refinement go the ordinary way, as every other handle does.
+int lu_step(xg_lu* lu, int* numeric) {
+  *numeric = 0;
+  if (lu->method == 2 && lu->mode == 0 && !lu->repivot_futile) {
+    lu->have64 = lu->soft64 = lu->tlu_current = false;
+    *lu->nan_flag() = 0;
+    int st = lu->mfp->factor_begin(lu->avals.p, lu->s.nnz_a, false);
+    if (st != XG_OK) return st;
+    st = lu->mfp->solve(lu->b.p, lu->x.p, false, lu->nan_flag());
+    if (st != XG_OK) return st;
+    HIPCHK(hipStreamSynchronize(lu->stream));
+    int bad = 0, hard = 0;
+    st = lu->mfp->factor_end(&bad, &hard);
+    if (st != XG_OK) return st;
+    if (!bad) {
+      lu->have64 = true;
+      if (!*lu->nan_flag()) return XG_OK;
+      k_fill<<<nblk(lu->s.n), 256, 0, lu->stream>>>(lu->x.p, (size_t)lu->s.n, 0.0);
+      HIPCHK(hipGetLastError());
+      return XG_E_NAN;
+    }
+  }
+  const int st = lu_numeric_impl(lu, lu->avals.p, true);
+  if (st < 0) return st;
+  *numeric = st;
+  return st > 0 ? XG_OK : lu_solve_impl(lu, lu->b.p, lu->x.p, 0, true);
+}
+
+}  // namespace xg

@@ -521,7 +521,7 @@ __global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, c
 // broadcast from there: a pivot costs its reciprocal and the row updates, no
 // LDS traffic (512 x 512 grid, all levels: 300 us, 656 with the elimination in LDS).
 template <class T, int N>
-__global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list, const double* vals, T* F, int* bad) {
+__global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list, const double* vals, T* F, int* bad, int* fail) {
   constexpr int ld = N + 1;
   __shared__ T A[N * ld];
   const MfFront f = d.front[list[blockIdx.x]];
@@ -569,7 +569,7 @@ __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list,
   T* Fs = F + f.fo;
   for (int i = 0; i < ms; ++i)
     if (t < ms) Fs[(long long)i * ms + t] = A[i * ld + t];
-  if (first < np) atomicMin(bad, f.first + first + 1);
+  if (first < np) { atomicMin(bad, f.first + first + 1); *fail = 1; }
   if (__any(hard) && t == 0) atomicOr(bad + 1, 1);
 }
 
@@ -580,7 +580,7 @@ constexpr int kMfTile = 64 * (kMfPanel + 1) > kMfPanel * 65 ? 64 * (kMfPanel + 1
 
 template <class T>
 __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2))) k_mf_step(MfDev d, const int4* ent, int p0, T* F, T* dbuf, int half,
-                                                     int* bad) {
+                                                     int* bad, int* fail) {
   constexpr int PW = kMfPanel;
   __shared__ __attribute__((aligned(16))) T Du[PW * kMfDs];   // U11 by rows
   __shared__ __attribute__((aligned(16))) T Dl[PW * kMfDs];   // L11 by columns; the updated block before it is factored
@@ -760,7 +760,7 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
         if (c < ms && q < pw) Fs[(p0 + q) * ld + c] = v[q];
     }
   }
-  if (failed < pw) atomicMin(bad, d.sfirst[s] + p0 + failed + 1);
+  if (failed < pw) { atomicMin(bad, d.sfirst[s] + p0 + failed + 1); *fail = 1; }
   if (__any(hard) && lane == 0) atomicOr(bad + 1, 1);
 }
 
@@ -869,7 +869,7 @@ __global__ void __launch_bounds__(64) k_mf_bwd_tiny(MfDev d, const int* list, co
   }
   if (t < np) {
     x[g] = (double)v;
-    if (!isfinite((double)v)) atomicOr(nan_flag, 1);
+    if (!isfinite((double)v)) *nan_flag = 1;
   }
 }
 
@@ -1089,7 +1089,12 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* li
     xg[ix[i]] = v;
     bad |= !isfinite(v);
   }
-  if (bad) atomicOr(nan_flag, 1);
+  if (bad) *nan_flag = 1;
+}
+
+__global__ void k_mf_flag_init(int* bad) {
+  bad[0] = 0x7fffffff;
+  bad[1] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1129,7 +1134,9 @@ struct MfLu::Impl {
   MfPlan P;
   hipStream_t st = nullptr;
   std::vector<MfGraph> graphs;
+  int* fail = nullptr;            // pinned: raised by a factorisation whose pivots fail
   ~Impl() {
+    if (fail) (void)hipHostFree(fail);
     for (auto& g : graphs)
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
   }
@@ -1201,6 +1208,8 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   for (size_t q = 0; q < P.idx.size(); ++q) { bi[q] = s.perm_row[P.idx[q]]; xi[q] = s.perm_col[P.idx[q]]; }
   MFCHK(I.bidx.up(bi, st)); MFCHK(I.xidx.up(xi, st));
   MFCHK(I.bad.alloc(2));
+  if (!I.fail) MFCHK(hipHostMalloc((void**)&I.fail, sizeof(int), hipHostMallocDefault));
+  hipLaunchKernelGGL(k_mf_flag_init, dim3(1), dim3(1), 0, st, I.bad.p);
   MFCHK(I.F64.alloc(P.fo[P.ns])); MFCHK(I.V64.alloc(P.vo[P.ns]));
   if (want_fp32) { MFCHK(I.F32.alloc(P.fo[P.ns])); MFCHK(I.V32.alloc(P.vo[P.ns])); }
   // per level: tiny fronts (one launch), larger fronts (blocked panels, all
@@ -1316,18 +1325,11 @@ long long MfLu::front_elements() const { return impl_->P.fo.empty() ? 0 : impl_-
 int MfLu::levels() const { return (int)impl_->P.lvl_ptr.size() - 1; }
 int MfLu::supernodes() const { return impl_->P.ns; }
 
-template <class T>
-__global__ void k_mf_flag_init(int* bad) {
-  bad[0] = 0x7fffffff;
-  bad[1] = 0;
-}
-
 // the launches of one refactor (no host work: the sequence is captured)
 template <class T>
 static int mf_factor_enqueue(MfLu::Impl& I, const double* vals_dev, int nnz, T* F) {
   const MfPlan& P = I.P;
   hipStream_t st = I.st;
-  hipLaunchKernelGGL(k_mf_flag_init<T>, dim3(1), dim3(1), 0, st, I.bad.p);
   const MfDev d = I.dev();
   T* dbuf = reinterpret_cast<T*>(I.dbuf.p);
   const int nl = (int)P.lvl_ptr.size() - 1;
@@ -1338,13 +1340,13 @@ static int mf_factor_enqueue(MfLu::Impl& I, const double* vals_dev, int nnz, T* 
     const int n32 = I.tiny_half[l] - I.tiny_off[l], n64 = I.tiny_off[l + 1] - I.tiny_half[l];
     if (n32)
       hipLaunchKernelGGL((k_mf_factor_tiny<T, kMfTiny / 2>), dim3(n32), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l],
-                         vals_dev, F, I.bad.p);
+                         vals_dev, F, I.bad.p, I.fail);
     if (n64)
       hipLaunchKernelGGL((k_mf_factor_tiny<T, kMfTiny>), dim3(n64), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_half[l],
-                         vals_dev, F, I.bad.p);
+                         vals_dev, F, I.bad.p, I.fail);
     for (const auto& S : I.steps[l])
       hipLaunchKernelGGL(k_mf_step<T>, dim3(S.cnt), dim3(kMfStep), 0, st, d, I.sent.p + S.off, S.p0, F, dbuf,
-                         (S.p0 / kMfPanel) & 1, I.bad.p);
+                         (S.p0 / kMfPanel) & 1, I.bad.p, I.fail);
   }
   MFCHK(hipGetLastError());
   return XG_OK;
@@ -1376,16 +1378,10 @@ static int mf_replay(MfLu::Impl& I, const void* const* key, int nkey, Enqueue en
 }
 
 template <class T>
-static int mf_factor_t(MfLu::Impl& I, const double* vals_dev, int nnz, T* F, int* bad_out, int* hard_out) {
+static int mf_factor_t(MfLu::Impl& I, const double* vals_dev, int nnz, T* F) {
   const void* key[8] = {(const void*)1, vals_dev, F, (const void*)(long long)nnz, nullptr, nullptr, nullptr, nullptr};
-  int rc = mf_replay(I, key, 8, [&] { return mf_factor_enqueue<T>(I, vals_dev, nnz, F); });
-  if (rc != XG_OK) return rc;
-  int res[2];
-  MFCHK(hipMemcpyAsync(res, I.bad.p, sizeof(res), hipMemcpyDeviceToHost, I.st));
-  MFCHK(hipStreamSynchronize(I.st));
-  *bad_out = res[0] == 0x7fffffff ? 0 : res[0];
-  *hard_out = res[1];
-  return XG_OK;
+  *I.fail = 0;
+  return mf_replay(I, key, 8, [&] { return mf_factor_enqueue<T>(I, vals_dev, nnz, F); });
 }
 
 template <class T>
@@ -1431,13 +1427,35 @@ static int mf_solve_t(MfLu::Impl& I, const T* F, T* V, const double* b_dev, doub
   return mf_replay(I, key, 8, [&] { return mf_solve_enqueue<T>(I, F, V, b_dev, x_dev, nan_flag); });
 }
 
-int MfLu::factor(const double* vals_dev, int nnz, bool fp32, int* bad, int* hard) {
+int MfLu::factor_begin(const double* vals_dev, int nnz, bool fp32) {
   Impl& I = *impl_;
   if (fp32) {
     if (!I.F32.p) return XG_E_ARG;
-    return mf_factor_t<float>(I, vals_dev, nnz, I.F32.p, bad, hard);
+    return mf_factor_t<float>(I, vals_dev, nnz, I.F32.p);
   }
-  return mf_factor_t<double>(I, vals_dev, nnz, I.F64.p, bad, hard);
+  return mf_factor_t<double>(I, vals_dev, nnz, I.F64.p);
+}
+
+// The kernels raise the pinned flag and leave the details on the device, where
+// they are looked at (and cleared) only then.
+int MfLu::factor_end(int* bad, int* hard) {
+  Impl& I = *impl_;
+  *bad = *hard = 0;
+  if (!*I.fail) return XG_OK;
+  int res[2];
+  MFCHK(hipMemcpyAsync(res, I.bad.p, sizeof(res), hipMemcpyDeviceToHost, I.st));
+  hipLaunchKernelGGL(k_mf_flag_init, dim3(1), dim3(1), 0, I.st, I.bad.p);
+  MFCHK(hipStreamSynchronize(I.st));
+  *bad = res[0] == 0x7fffffff ? 0 : res[0];
+  *hard = res[1];
+  return XG_OK;
+}
+
+int MfLu::factor(const double* vals_dev, int nnz, bool fp32, int* bad, int* hard) {
+  const int rc = factor_begin(vals_dev, nnz, fp32);
+  if (rc != XG_OK) return rc;
+  MFCHK(hipStreamSynchronize(impl_->st));
+  return factor_end(bad, hard);
 }
 
 int MfLu::solve(const double* b_dev, double* x_dev, bool fp32, int* nan_flag) {

@@ -140,7 +140,8 @@ struct MfPlan {
 int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p);
 
 // Multifrontal factorisation on the GPU (multifrontal.hip); the stream is a
-// hipStream_t, vectors are device pointers in A's numbering.
+// hipStream_t, vectors are device pointers in A's numbering; nan_flag is pinned
+// host or device memory that a non-finite solution sets to 1.
 class MfLu {
  public:
   struct Impl;
@@ -153,6 +154,9 @@ class MfLu {
   // was zero or not finite (else every failure is a multiplier beyond KLU's
   // threshold)
   int factor(const double* vals_dev, int nnz, bool fp32, int* bad, int* hard);
+  // the same in two parts: enqueued, and its verdict once the stream has been waited for
+  int factor_begin(const double* vals_dev, int nnz, bool fp32);
+  int factor_end(int* bad, int* hard);
   int solve(const double* b_dev, double* x_dev, bool fp32, int* nan_flag);
   // FP64 solve whose front vectors, work vector and permuted right-hand side
   // are the caller's device memory `work` (solve_work_doubles() doubles,
@@ -191,6 +195,16 @@ int circuit_combine(xg_circuit* c, const double* q0, const double* q2, double* r
 // MOSFET state / store history: 0 zero both, 1 current <- next (a step or
 // operating point accepted), 2 next <- current (a step rejected)
 int circuit_history(xg_circuit* c, int op);
+
+// ---- the drop-in LU on a caller's stream (a hipStream_t), for the
+// single-circuit engine (kernels.hip): the values and the right-hand side are
+// written into its own buffers, the solution is left there
+int lu_create_on(int n, const int* rowptr, const int* colind, int method, void* stream, xg_lu** out);
+struct LuDev { double *vals, *b, *x; };
+LuDev lu_dev(xg_lu* lu);          // (the handle keeps them, also over a re-pivot)
+// factors the values and solves; waits for the stream.  *numeric > 0: singular
+// (nothing solved).  Returns XG_OK, XG_E_NAN (x zeroed) or an error.
+int lu_step(xg_lu* lu, int* numeric);
 
 // learned-predictor network (mlp.hip): forward on a caller stream (a
 // hipStream_t), and its dimensions
