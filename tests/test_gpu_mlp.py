@@ -67,6 +67,14 @@ def test_forward_and_gradients_match_oracle(gpu, in_dim, width, hidden, out_dim,
             off += n
 
 
+@pytest.mark.parametrize("width,hidden,rows", [(64, 9, 64), (128, 7, 192), (192, 1, 320), (64, 8, 1088)])
+def test_grouped_weight_gradients(gpu, width, hidden, rows):
+    """Weight and bias gradients over two groups of layers, one to 17 steps of the
+    sum over rows, 64- and 128-row tiles' remainders: as the oracle's, whose
+    bf16 roundings of the activations they share (2e-2, as for the small nets)."""
+    test_forward_and_gradients_match_oracle(gpu, 128, width, hidden, 64, rows)
+
+
 def test_adam_step_matches_oracle(gpu):
     in_dim, width, hidden, out_dim, rows = 128, 128, 1, 64, 64
     net = X.MLP(in_dim, width, hidden, out_dim, max_rows=rows, seed=3)

@@ -65,7 +65,19 @@ struct GemmArgs {
   const float* Zin;                   // EPI_GELU_BWD: pre-activation of this layer
 };
 
-constexpr int BN = 64, BK = 64, LDS_K = BK + 8;
+constexpr int BN = 64, BK = 64;
+
+// Place of (row, k) in a staged tile: rows of 64 halves without padding, the
+// eight 16-byte groups of a row exchanged by the row's bits so that no LDS access
+// of the product meets a bank twice as often as it must: 16 consecutive rows at
+// one group (operand reads) fall on 16 different quads of banks, and so do the
+// rows 8 apart that a transposed operand's pairs are stored to (with rows padded
+// to 72 halves those eight fell on one bank: weight gradients of 2048 rows 40 us,
+// 23 now).
+__device__ __forceinline__ int lds_at(int row, int k) {
+  const int f = ((row >> 3) ^ (((row >> 1) & 3) << 1)) & 7;
+  return row * BK + (((k >> 3) ^ f) << 3) + (k & 7);
+}
 
 // A tile of T rows (of A or B as the product reads them) by BK of k, from
 // memory to registers and from there to LDS.  Straight operands are rows of
@@ -92,17 +104,17 @@ struct Stage {
     if (!TR) {
 #pragma unroll
       for (int i = 0; i < N; ++i)
-        *reinterpret_cast<u32x4*>(&lds[((t >> 3) + 32 * i) * LDS_K + (t & 7) * 8]) = v[i];
+        *reinterpret_cast<u32x4*>(&lds[lds_at((t >> 3) + 32 * i, (t & 7) * 8)]) = v[i];
     } else {
 #pragma unroll
       for (int i = 0; i < N; i += 2) {
         const u32x4 a = v[i], b = v[i + 1];
-        unsigned short* to = lds + ((t & 7) * 8 + 32 * i) * LDS_K + (t >> 3) * 2;
+        const int r = (t & 7) * 8 + 32 * i, k = (t >> 3) * 2;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           // rows 2 j and 2 j + 1: (k, k + 1) side by side
-          *reinterpret_cast<unsigned*>(to + (2 * j) * LDS_K) = __builtin_amdgcn_perm(b[j], a[j], 0x05040100u);
-          *reinterpret_cast<unsigned*>(to + (2 * j + 1) * LDS_K) = __builtin_amdgcn_perm(b[j], a[j], 0x07060302u);
+          *reinterpret_cast<unsigned*>(&lds[lds_at(r + 2 * j, k)]) = __builtin_amdgcn_perm(b[j], a[j], 0x05040100u);
+          *reinterpret_cast<unsigned*>(&lds[lds_at(r + 2 * j + 1, k)]) = __builtin_amdgcn_perm(b[j], a[j], 0x07060302u);
         }
       }
     }
@@ -113,24 +125,26 @@ struct Stage {
 // BM / 64 blocks of v_mfma_f32_32x32x16_bf16 (A: lane l holds row l%32, k =
 // 8*(l/32)..+7; B likewise by column; D register r of lane l is row 8*(r/4) +
 // 4*(l/32) + r%4, column l%32).  At these sizes a tile's chain of k steps bounds
-// the product (8 to 32 steps of 64, one or two tiles per CU), so four steps are
-// in flight from memory in registers while LDS holds two, with one barrier per
-// step; and the tiles that share rows of A sit on one XCD (consecutive
-// workgroups go to the eight XCDs in turn), so that A crosses to one L2 only.
-// Forward of 4096 rows (1600 -> 3 x 512 -> 256) 53.0 us, 78.5 with one 64 x 64 x 32
-// step at a time; weight gradient 512 x 1600 over 2048 rows 22 us, 53.  Every element accumulates k in ascending order of
-// 16 whatever the tile, so the tile size does not change a result.
-constexpr int kAhead = 4;
+// the product (8 to 32 steps of 64, one or two tiles per CU), so two steps are in
+// flight from memory in registers while LDS holds two, with one barrier per step
+// (four in flight take the registers of more tiles per CU: forward of 8192 rows
+// 72 us against 75, training on 8192 rows 294 us a step against 328); and the tiles
+// that share rows of A sit on one XCD (consecutive workgroups go to the eight
+// XCDs in turn), so that A crosses to one L2 only.  Forward of 4096 rows (1600 ->
+// 3 x 512 -> 256) 50.2 us, 78.5 with one 64 x 64 x 32 step at a time.  Every
+// element accumulates k in ascending order of 16 whatever the tile, so the tile
+// size does not change a result.
+constexpr int kAhead = 2;
+constexpr long long kWideTiles = 512;   // (the dispatch of 128-row tiles)
 
 template <bool TA, bool TB, int EPI, int BM>
-__global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) unsigned short As[2][BM * LDS_K];
-  __shared__ __attribute__((aligned(16))) unsigned short Bs[2][BN * LDS_K];
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int id, unsigned short (*As)[BM * BK],
+                                          unsigned short (*Bs)[BN * BK]) {
   constexpr int MI = BM / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   // workgroup id -> tile: ids id, id + 8, ... (one XCD) walk the columns of a row of tiles
-  const int nt = g.N / BN, mt = g.M / BM, id = blockIdx.x;
+  const int nt = g.N / BN, mt = g.M / BM;
   const int full = mt / 8 * 8 * nt;               // ids of whole groups of eight tile rows
   int tm, tn;
   if (id < full) {
@@ -145,61 +159,87 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
   f32x16 acc[MI] = {};
   Stage<TA, BM> sa[kAhead];
   Stage<TB, BN> sb[kAhead];
+  // Loads are never skipped (past the end they repeat the last step's): a
+  // branch around one makes the compiler wait for all that are in flight.
+  const int klast = g.K - BK;
 #pragma unroll
-  for (int d = 0; d < kAhead; ++d)
-    if (d * BK < g.K) {
-      sa[d].load(g.A, g.lda, m0, d * BK, tid);
-      sb[d].load(g.B, g.ldb, n0, d * BK, tid);
+  for (int d = 0; d < kAhead; ++d) {
+    sa[d].load(g.A, g.lda, m0, min(d * BK, klast), tid);
+    sb[d].load(g.B, g.ldb, n0, min(d * BK, klast), tid);
+  }
+  auto multiply = [&](const unsigned short* at, const unsigned short* bt) {
+#pragma unroll
+    for (int kk = 0; kk < BK; kk += 16) {
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(&bt[lds_at(wn * 32 + (lane & 31), kk + 8 * (lane >> 5))]);
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        const bf16x8 a =
+            *reinterpret_cast<const bf16x8*>(&at[lds_at((wm * MI + i) * 32 + (lane & 31), kk + 8 * (lane >> 5))]);
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i], 0, 0, 0);
+      }
     }
-  for (int k0 = 0; k0 < g.K; k0 += kAhead * BK) {
+  };
+  int k0 = 0;
+  for (; k0 + kAhead * BK < g.K; k0 += kAhead * BK) {
 #pragma unroll
     for (int d = 0; d < kAhead; ++d) {
-      const int k = k0 + d * BK;
-      if (k >= g.K) break;
-      unsigned short *at = As[d & 1], *bt = Bs[d & 1];
-      sa[d].store(at, tid);
-      sb[d].store(bt, tid);
-      if (k + kAhead * BK < g.K) {
-        sa[d].load(g.A, g.lda, m0, k + kAhead * BK, tid);
-        sb[d].load(g.B, g.ldb, n0, k + kAhead * BK, tid);
-      }
+      sa[d].store(As[d & 1], tid);
+      sb[d].store(Bs[d & 1], tid);
+      const int k = min(k0 + (d + kAhead) * BK, klast);
+      sa[d].load(g.A, g.lda, m0, k, tid);
+      sb[d].load(g.B, g.ldb, n0, k, tid);
       __syncthreads();
-      // ---- matrix cores
-#pragma unroll
-      for (int kk = 0; kk < BK; kk += 16) {
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(&bt[(wn * 32 + (lane & 31)) * LDS_K + kk + 8 * (lane >> 5)]);
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-          const bf16x8 a =
-              *reinterpret_cast<const bf16x8*>(&at[((wm * MI + i) * 32 + (lane & 31)) * LDS_K + kk + 8 * (lane >> 5)]);
-          acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[i], 0, 0, 0);
-        }
-      }
+      multiply(As[d & 1], Bs[d & 1]);
+      // (else the later steps' operands are waited for and packed here too)
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // ---- epilogue
+  // the epilogue's operands, beside the last steps
   const int col = n0 + wn * 32 + (lane & 31);
+  const int row0 = m0 + wm * MI * 32 + 4 * (lane >> 5);
+  float bias = 0.0f, zin[MI * 16];
+  if (EPI == EPI_BIAS_F32 || EPI == EPI_BIAS_GELU || EPI == EPI_BIAS_GELU_H) bias = g.bias[col];
+  if (EPI == EPI_GELU_BWD)
+#pragma unroll
+    for (int r = 0; r < MI * 16; ++r)
+      zin[r] = g.Zin[(size_t)(row0 + (r >> 4) * 32 + 8 * ((r & 15) >> 2) + (r & 3)) * g.ldc + col];
+#pragma unroll
+  for (int d = 0; d < kAhead; ++d) {
+    if (k0 + d * BK >= g.K) break;
+    sa[d].store(As[d & 1], tid);
+    sb[d].store(Bs[d & 1], tid);
+    __syncthreads();
+    multiply(As[d & 1], Bs[d & 1]);
+  }
+  // ---- epilogue
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int row = m0 + (wm * MI + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+      const int row = row0 + i * 32 + 8 * (r >> 2) + (r & 3);
       const size_t o = (size_t)row * g.ldc + col;
       const float v = acc[i][r];
       if (EPI == EPI_F32) {
         g.C[o] = v;
       } else if (EPI == EPI_BIAS_F32) {
-        g.C[o] = v + g.bias[col];
+        g.C[o] = v + bias;
       } else if (EPI == EPI_BIAS_GELU) {
-        const float z = v + g.bias[col];
+        const float z = v + bias;
         g.C[o] = z;
         g.H[o] = f2bf(gelu(z));
       } else if (EPI == EPI_BIAS_GELU_H) {
-        g.H[o] = f2bf(gelu(v + g.bias[col]));
+        g.H[o] = f2bf(gelu(v + bias));
       } else {
-        g.H[o] = f2bf(v * gelu_d(g.Zin[o]));
+        g.H[o] = f2bf(v * gelu_d(zin[i * 16 + r]));
       }
     }
+}
+
+template <bool TA, bool TB, int EPI, int BM>
+__global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) unsigned short As[2][BM * BK];
+  __shared__ __attribute__((aligned(16))) unsigned short Bs[2][BN * BK];
+  gemm_tile<TA, TB, EPI, BM>(g, blockIdx.x, As, Bs);
 }
 
 // loss = sum_rows sum_j mask (y - t)^2 / count, dY = 2 mask (y - t) / count
@@ -222,26 +262,14 @@ __global__ void k_mse(int n, int count, const float* y, const float* t, const fl
   }
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
-__global__ void k_sum(int n, const double* p, double* out) {
-  __shared__ double red[256];
-  double s = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) s += p[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = red[0];
-}
 
 // bias gradients: column sums of a bf16 [rows][N] matrix, two passes (chunks of
-// 256 rows, then over chunks; the second for all layers in one launch).  The
-// chunk pass is bound by its loads' latency: eight rows in flight
-// (2048 x 512: 4.4 us, 9.9 one row at a time).
-__global__ void k_colsum_part(int rows, int N, const unsigned short* d, float* part) {
-  const int col = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int r0 = blockIdx.y * 256 + (threadIdx.x >> 6) * 64;
+// 256 rows, then over chunks).  The chunk pass is bound by its loads' latency:
+// eight rows in flight.
+__device__ __forceinline__ void colsum_part(int rows, int N, const unsigned short* d, float* part, int bx, int by,
+                                            float* red) {
+  const int col = bx * 64 + (threadIdx.x & 63);
+  const int r0 = by * 256 + (threadIdx.x >> 6) * 64;
   float s = 0.0f;
   // (rows are a multiple of 64: a wavefront's 64 rows all exist or none does)
   if (r0 < rows)
@@ -252,17 +280,64 @@ __global__ void k_colsum_part(int rows, int N, const unsigned short* d, float* p
 #pragma unroll
       for (int q = 0; q < 8; ++q) s += bf2f(v[q]);
     }
-  __shared__ float red[256];
   red[threadIdx.x] = s;
   __syncthreads();
   if (threadIdx.x < 64) {
     const float t = red[threadIdx.x] + red[threadIdx.x + 64] + red[threadIdx.x + 128] + red[threadIdx.x + 192];
-    part[(size_t)blockIdx.y * N + col] = t;
+    part[(size_t)by * N + col] = t;
   }
 }
-// layer blockIdx.y: its N columns' partial sums at `off` of part, the sums at boff of g
+
+// Weight gradients dW_l = d_l^T in_l and the bias gradients' chunk sums of up
+// to kGroup layers in one launch, after the chain of activation gradients: a
+// layer alone has 32 to 200 tiles for 256 CUs and each is a chain of rows / 64
+// steps, so layers one after another left most of the chip idle (1600 -> 3 x 512
+// -> 256 over 2048 rows: 87 us and four launches of column sums, 18, one after
+// another; 23 together).
+constexpr int kGroup = 8;
+struct WgradArgs {
+  int n, rows;
+  int tile0[kGroup + 1], col0[kGroup + 1];   // first product tile and first column-sum block of each layer
+  GemmArgs g[kGroup];
+  float* part[kGroup];
+};
+
+template <int BM>
+__global__ void __launch_bounds__(256) k_wgrad(WgradArgs w) {
+  __shared__ __attribute__((aligned(16))) unsigned short As[2][BM * BK];
+  __shared__ __attribute__((aligned(16))) unsigned short Bs[2][BN * BK];
+  int id = blockIdx.x, l = 0;
+  if (id < w.tile0[w.n]) {
+    while (id >= w.tile0[l + 1]) ++l;
+    gemm_tile<true, true, EPI_F32, BM>(w.g[l], id - w.tile0[l], As, Bs);
+  } else {
+    id -= w.tile0[w.n];
+    while (id >= w.col0[l + 1]) ++l;
+    id -= w.col0[l];
+    const int nb = w.g[l].M / 64;
+    colsum_part(w.rows, w.g[l].M, w.g[l].A, w.part[l], id % nb, id / nb, reinterpret_cast<float*>(As));
+  }
+}
+
+// layer blockIdx.y: its N columns' partial sums at `off` of part, the sums at
+// boff of g; the last row's first block sums the loss's partials into pinned memory
 struct ColLayer { int N; long long off, boff; };
-__global__ void k_colsum_fin(int chunks, const ColLayer* layers, const float* part, float* g) {
+__global__ void __launch_bounds__(256) k_grad_fin(int chunks, int n_layers, const ColLayer* layers, const float* part,
+                                                 float* g, int n_loss, const double* lpart, double* loss) {
+  if ((int)blockIdx.y == n_layers) {
+    if (blockIdx.x) return;
+    __shared__ double red[256];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < n_loss; i += 256) s += lpart[i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int st = 128; st > 0; st >>= 1) {
+      if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss = red[0];
+    return;
+  }
   const ColLayer L = layers[blockIdx.y];
   const int col = blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= L.N) return;
@@ -316,21 +391,27 @@ struct xg_mlp {
   hipStream_t stream = nullptr;
   Buf<float> w, g, m, v, Y, part, Zall;
   Buf<unsigned short> wb, Hall, dH, dY;
-  Buf<double> lpart, lsum;
+  Buf<double> lpart;
+  double* loss_sum = nullptr;             // pinned
   std::vector<ColLayer> col_layer;        // per layer: its partial column sums in `part`
   Buf<ColLayer> d_col;
   // Z_l / H_l at offset l * max_rows * width
   float* Z(int l) { return Zall.p + (size_t)l * max_rows * width; }
   unsigned short* H(int l) { return Hall.p + (size_t)l * max_rows * width; }
-  ~xg_mlp() { if (stream) (void)hipStreamDestroy(stream); }
+  // gradient with respect to layer l's output before its activation
+  unsigned short* D(int l) { return l + 1 == n_layers ? dY.p : dH.p + (size_t)l * max_rows * width; }
+  ~xg_mlp() {
+    if (stream) (void)hipStreamDestroy(stream);
+    if (loss_sum) (void)hipHostFree(loss_sum);
+  }
 
   template <bool TA, bool TB, int EPI>
   int gemm(const GemmArgs& a) {
     if (a.M % 64 || a.N % BN || a.K % BK || a.M <= 0 || a.N <= 0 || a.K <= 0) return XG_E_ARG;
     // 128-row tiles read B half as often, but their chain per step is longer: from
-    // two tiles per CU (256 of them) on (forward of 8192 rows 78 us against 80.5
-    // with 64-row tiles, of 4096 rows 61 against 53.6)
-    if (a.M % 128 == 0 && (long long)(a.N / BN) * (a.M / 128) >= 512)
+    // two tiles per CU (256 of them) on (forward of 4096 rows, one per CU: 58.6 us
+    // against 52 with 64-row tiles; of 8192 rows 78 against 80.5)
+    if (a.M % 128 == 0 && (long long)(a.N / BN) * (a.M / 128) >= kWideTiles)
       hipLaunchKernelGGL((k_gemm<TA, TB, EPI, 128>), dim3(a.N / BN * (a.M / 128)), dim3(256), 0, stream, a);
     else
       hipLaunchKernelGGL((k_gemm<TA, TB, EPI, 64>), dim3(a.N / BN * (a.M / 64)), dim3(256), 0, stream, a);
@@ -371,43 +452,49 @@ struct xg_mlp {
     return XG_OK;
   }
 
-  // partial column sums of layer l's gradient (k_colsum_fin adds the chunks)
-  int colsum(int rows, int l, const unsigned short* d) {
-    hipLaunchKernelGGL(k_colsum_part, dim3(dout[l] / 64, (rows + 255) / 256), dim3(256), 0, stream, rows, dout[l], d,
-                       part.p + col_layer[l].off);
-    HIPCHK(hipGetLastError());
-    return XG_OK;
-  }
-
-  // backward of the loss whose output gradient is in dY (bf16 [rows][out])
+  // backward of the loss whose output gradient is in dY (bf16 [rows][out]): the
+  // gradients with respect to each layer's output first, then all weights'
   int backward(int rows, const unsigned short* X) {
-    const unsigned short* dcur = dY.p;   // gradient w.r.t. this layer's output (pre-activation)
-    for (int l = n_layers - 1; l >= 0; --l) {
-      const unsigned short* in = l == 0 ? X : H(l - 1);
-      // dW_l = dcur^T in : C[dout][din] = sum_m dcur[m][o] in[m][i]
-      GemmArgs a{};
-      a.M = dout[l]; a.N = din[l]; a.K = rows;
-      a.A = dcur; a.lda = dout[l];
-      a.B = in; a.ldb = din[l];
-      a.C = g.p + woff[l]; a.ldc = din[l];
-      int st = gemm<true, true, EPI_F32>(a);
-      if (st != XG_OK) return st;
-      st = colsum(rows, l, dcur);
-      if (st != XG_OK) return st;
-      if (l == 0) break;
-      // d(pre-activation of layer l-1) = (dcur W_l) * gelu'(Z_{l-1})
+    for (int l = n_layers - 1; l > 0; --l) {
+      // d(pre-activation of layer l-1) = (d_l W_l) * gelu'(Z_{l-1})
       GemmArgs b{};
       b.M = rows; b.N = din[l]; b.K = dout[l];
-      b.A = dcur; b.lda = dout[l];
+      b.A = D(l); b.lda = dout[l];
       b.B = wb.p + woff[l]; b.ldb = din[l];
-      unsigned short* dst = dH.p + (size_t)((l - 1) & 1) * max_rows * width;
-      b.H = dst; b.ldc = width; b.Zin = Z(l - 1);
-      st = gemm<false, true, EPI_GELU_BWD>(b);
+      b.H = D(l - 1); b.ldc = width; b.Zin = Z(l - 1);
+      const int st = gemm<false, true, EPI_GELU_BWD>(b);
       if (st != XG_OK) return st;
-      dcur = dst;
     }
-    hipLaunchKernelGGL(k_colsum_fin, dim3(nblk(std::max(width, out_dim)), n_layers), dim3(256), 0, stream, (rows + 255) / 256,
-                       d_col.p, part.p, g.p);
+    const int chunks = (rows + 255) / 256;
+    for (int l0 = 0; l0 < n_layers; l0 += kGroup) {
+      WgradArgs w{};
+      w.n = std::min(kGroup, n_layers - l0);
+      w.rows = rows;
+      bool wide = true;
+      long long big = 0;
+      for (int j = 0; j < w.n; ++j) {
+        const int l = l0 + j;
+        // C[dout][din] = sum_m d[m][o] in[m][i]
+        GemmArgs& a = w.g[j];
+        a.M = dout[l]; a.N = din[l]; a.K = rows;
+        a.A = D(l); a.lda = dout[l];
+        a.B = l == 0 ? X : H(l - 1); a.ldb = din[l];
+        a.C = g.p + woff[l]; a.ldc = din[l];
+        w.part[j] = part.p + col_layer[l].off;
+        wide = wide && a.M % 128 == 0;
+        big += (long long)(a.N / BN) * (a.M / 128);
+      }
+      const int bm = wide && big >= kWideTiles ? 128 : 64;
+      for (int j = 0; j < w.n; ++j) {
+        w.tile0[j + 1] = w.tile0[j] + w.g[j].N / BN * (w.g[j].M / bm);
+        w.col0[j + 1] = w.col0[j] + w.g[j].M / 64 * chunks;
+      }
+      const dim3 grid(w.tile0[w.n] + w.col0[w.n]);
+      if (bm == 128) hipLaunchKernelGGL(k_wgrad<128>, grid, dim3(256), 0, stream, w);
+      else hipLaunchKernelGGL(k_wgrad<64>, grid, dim3(256), 0, stream, w);
+    }
+    hipLaunchKernelGGL(k_grad_fin, dim3(nblk(std::max(width, out_dim)), n_layers + 1), dim3(256), 0, stream, chunks,
+                       n_layers, d_col.p, part.p, g.p, (int)nblk((long long)rows * out_dim), lpart.p, loss_sum);
     HIPCHK(hipGetLastError());
     return XG_OK;
   }
@@ -459,7 +546,7 @@ int xg_mlp_create(int in_dim, int width, int hidden_layers, int out_dim, int max
   HIPCHK(net->wb.alloc(off));
   HIPCHK(net->Zall.alloc((size_t)hidden_layers * max_rows * width));
   HIPCHK(net->Hall.alloc((size_t)hidden_layers * max_rows * width));
-  HIPCHK(net->dH.alloc((size_t)2 * max_rows * width));
+  HIPCHK(net->dH.alloc((size_t)hidden_layers * max_rows * width));
   HIPCHK(net->dY.alloc((size_t)max_rows * out_dim));
   HIPCHK(net->Y.alloc((size_t)max_rows * out_dim));
   long long col_off = 0;
@@ -471,7 +558,7 @@ int xg_mlp_create(int in_dim, int width, int hidden_layers, int out_dim, int max
   HIPCHK(net->d_col.alloc(net->col_layer.size()));
   HIPCHK(hipMemcpy(net->d_col.p, net->col_layer.data(), sizeof(ColLayer) * net->col_layer.size(), hipMemcpyHostToDevice));
   HIPCHK(net->lpart.alloc(nblk((long long)max_rows * out_dim)));
-  HIPCHK(net->lsum.alloc(1));
+  HIPCHK(hipHostMalloc((void**)&net->loss_sum, sizeof(double), hipHostMallocDefault));
   HIPCHK(hipMemcpy(net->w.p, h.data(), off * sizeof(float), hipMemcpyHostToDevice));
   HIPCHK(hipMemset(net->m.p, 0, off * sizeof(float)));
   HIPCHK(hipMemset(net->v.p, 0, off * sizeof(float)));
@@ -523,15 +610,12 @@ int xg_mlp_loss_backward(xg_mlp* net, int rows, const unsigned short* x_dev, con
   const long long n = (long long)rows * net->out_dim;
   hipLaunchKernelGGL(k_mse, dim3(nblk(n)), dim3(256), 0, net->stream, (int)n, count, net->Y.p, t_dev, mask_dev,
                      net->dY.p, net->lpart.p);
-  hipLaunchKernelGGL(k_sum, dim3(1), dim3(256), 0, net->stream, (int)nblk(n), net->lpart.p, net->lsum.p);
   HIPCHK(hipGetLastError());
   st = net->backward(rows, x_dev);
   if (st != XG_OK) return st;
-  double l = 0.0;
-  HIPCHK(hipMemcpyAsync(&l, net->lsum.p, sizeof(double), hipMemcpyDeviceToHost, net->stream));
   if (grads) HIPCHK(hipMemcpyAsync(grads, net->g.p, net->n_params * sizeof(float), hipMemcpyDeviceToHost, net->stream));
   HIPCHK(hipStreamSynchronize(net->stream));
-  if (loss) *loss = l / count;
+  if (loss) *loss = *net->loss_sum / count;
   return XG_OK;
 }
 
