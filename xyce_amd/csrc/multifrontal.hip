@@ -828,12 +828,12 @@ __global__ void __launch_bounds__(64) k_mf_fwd_tiny(MfDev d, const int* list, co
 #pragma unroll
     for (int q = 0; q < 16; ++q) l[q] = row[min(k0 + q, np - 1)];
     __builtin_amdgcn_sched_barrier(0);
+    // (coefficients of no effect set to zero off the chain of steps)
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const T yk = mf_bcast(v, k0 + q);
-      const T w = v - l[q] * yk;
-      v = (k0 + q < np && t > k0 + q) ? w : v;
-    }
+    for (int q = 0; q < 16; ++q)
+      if (!(k0 + q < np && t > k0 + q)) l[q] = (T)0;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v -= l[q] * mf_bcast(v, k0 + q);
   }
   if (t < ms) V[f.vo + t] = v;
 }
@@ -849,24 +849,24 @@ __global__ void __launch_bounds__(64) k_mf_bwd_tiny(MfDev d, const int* list, co
   T v = t < np ? V[f.vo + t] : t < ms ? (T)x[g] : (T)0;
   const T* row = F + f.fo + (long long)min(t, np - 1) * ms;
   // each lane's pivot reciprocal first (in parallel): the sweep multiplies
-  const T rd = (T)1 / row[min(t, np - 1)];
+  const T rd = t < np ? (T)1 / row[t] : (T)1;
   for (int k1 = ms; k1 > 0; k1 -= 16) {
     T u[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) u[q] = row[max(k1 - 1 - q, 0)];
     __builtin_amdgcn_sched_barrier(0);
+    // (coefficients of no effect set to zero off the chain of steps; a branch in
+    // it would keep it from being unrolled)
+#pragma unroll
+    for (int q = 0; q < 16; ++q)
+      if (!(t < k1 - 1 - q && t < np)) u[q] = (T)0;
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
-      const int k = k1 - 1 - q;
-      if (k < 0) break;
-      T xk = mf_bcast(v, k);
-      if (k < np) {
-        xk *= mf_bcast(rd, k);
-        if (t == k) v = xk;
-      }
-      if (t < k && t < np) v -= u[q] * xk;
+      const int k = max(k1 - 1 - q, 0);
+      v -= u[q] * (mf_bcast(v, k) * mf_bcast(rd, k));
     }
   }
+  v *= rd;
   if (t < np) {
     x[g] = (double)v;
     if (!isfinite((double)v)) *nan_flag = 1;
@@ -903,14 +903,47 @@ __device__ __forceinline__ void mf_load_tri(const T* Fs, long long ld, int b0, i
   }
 }
 
-template <class T>
-__global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* list, const T* F, T* V, const double* b,
-                                                        int ldsv) {
+// A 64-row triangle by one wavefront, lane i holding row i's unknown: a row's
+// coefficients come from LDS sixteen at a time, the next ones under way, those of
+// no effect set to zero before, so that a step is a broadcast and a multiply-add
+// (a loop the compiler keeps rolled waits for LDS in each: 64 rows 5 us more)
+template <bool UPPER, class T>
+__device__ __forceinline__ T mf_triangle(const T* tri, int bw, int lane, T v) {
+  const T* row = tri + lane * 65;
+  const T rd = UPPER && lane < bw ? (T)1 / row[lane] : (T)1;
+  T l[2][16];
+  auto fetch = [&](int c, T (&to)[16]) MF_INLINE {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) to[q] = row[UPPER ? 63 - (16 * c + q) : 16 * c + q];
+  };
+  fetch(0, l[0]);
+  mf_for<4>([&](auto cc) MF_INLINE {
+    constexpr int c = cc;
+    if constexpr (c < 3) fetch(c + 1, l[(c + 1) & 1]);
+    // (opaque: else all 64 steps' masks are kept over the calls, in spilled registers)
+    int ln = lane < bw ? lane : UPPER ? 64 : -1, w = bw;
+    asm volatile("" : "+v"(ln), "+s"(w));
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      const int j = UPPER ? 63 - (16 * c + q) : 16 * c + q;
+      if (!(UPPER ? ln < j && j < w : ln > j)) l[c & 1][q] = (T)0;
+    }
+    mf_for<16>([&](auto qc) MF_INLINE {
+      constexpr int q = qc, j = UPPER ? 63 - (16 * c + q) : 16 * c + q;
+      v -= l[c & 1][q] * (UPPER ? mf_bcast(v, j) * mf_bcast(rd, j) : mf_bcast(v, j));
+    });
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  return UPPER ? v * rd : v;
+}
+
+template <class T, bool LDSV>
+__global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* list, const T* F, T* V, const double* b) {
   extern __shared__ unsigned char mf_sm[];
   T* tri = reinterpret_cast<T*>(mf_sm);
   const int2 en = list[blockIdx.x];             // front, rows below the pivots left to k_mf_fwd_rows
   const MfFront f = d.front[en.x];
-  T* x = ldsv ? tri + 2 * kMfTri : V + f.vo;    // the front's vector
+  T* x = LDSV ? tri + 2 * kMfTri : V + f.vo;    // the front's vector
   const int ms = f.m, np = f.np;
   const long long ld = ms;
   const T* Fs = F + f.fo;
@@ -923,7 +956,7 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* li
     for (int a = t; a < ch.nu; a += kMfSolve) x[d.emap[ch.em + a]] += V[ch.vsrc + a];
     __syncthreads();
   }
-  if (en.y && ldsv)
+  if (en.y && LDSV)
     for (int i = np + t; i < ms; i += kMfSolve) V[f.vo + i] = x[i];
   const int nb = (np + 63) / 64;
   for (int k = 0; k < nb; ++k) {
@@ -933,14 +966,7 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* li
     T acc[kMfNext], pre[kMfNext];
     if (wave == 0) {
       const int bw = min(64, np - b0);
-      const T* tr = tri + (k & 1) * kMfTri + lane * 65;
-      T v = lane < bw ? x[b0 + lane] : (T)0;
-#pragma unroll 16
-      for (int j = 0; j < bw; ++j) {
-        const T yj = mf_bcast(v, j);
-        const T l = tr[j];
-        if (lane > j) v -= l * yj;
-      }
+      const T v = mf_triangle<false>(tri + (k & 1) * kMfTri, bw, lane, lane < bw ? x[b0 + lane] : (T)0);
       if (lane < bw) x[b0 + lane] = v;
     } else {
       if (mine) {
@@ -974,7 +1000,7 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* li
         if (lane == 0 && k < nr) x[r + k] -= acc[k];
       }
     }
-  if (!ldsv) return;
+  if (!LDSV) return;
   __syncthreads();
   for (int i = t; i < (en.y ? np : ms); i += kMfSolve) V[f.vo + i] = x[i];
 }
@@ -1013,14 +1039,14 @@ __global__ void __launch_bounds__(256) k_mf_bwd_rows(MfDev d, const int2* ent, c
   }
 }
 
-template <class T>
+template <class T, bool LDSV>
 __global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* list, const T* F, T* V, double* xg,
-                                                        int ldsv, int* nan_flag) {
+                                                        int* nan_flag) {
   extern __shared__ unsigned char mf_sm[];
   T* tri = reinterpret_cast<T*>(mf_sm);
   const int2 en = list[blockIdx.x];             // front, U12 x_below already subtracted by k_mf_bwd_rows
   const MfFront f = d.front[en.x];
-  T* x = ldsv ? tri + 2 * kMfTri : V + f.vo;
+  T* x = LDSV ? tri + 2 * kMfTri : V + f.vo;
   const int ms = f.m, np = f.np;
   const long long ld = ms;
   const T* Fs = F + f.fo;
@@ -1030,7 +1056,7 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* li
   mf_load_tri(Fs, ld, 64 * (nb - 1), np - 64 * (nb - 1), t, kMfSolve, tri + ((nb - 1) & 1) * kMfTri);
   for (int i = t; i < (en.y ? np : ms); i += kMfSolve)
     if (i >= np) x[i] = (T)xg[ix[i]];
-    else if (ldsv) x[i] = V[f.vo + i];
+    else if (LDSV) x[i] = V[f.vo + i];
   __syncthreads();
   if (!en.y && ms > np) {
     for (int r = 4 * wave; r < np; r += 4 * (kMfSolve / 64)) {
@@ -1052,16 +1078,7 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* li
     const int nr = min(kMfNext, 64 - i0);
     T acc[kMfNext], pre[kMfNext];
     if (wave == 0) {
-      const T* tr = tri + (k & 1) * kMfTri + lane * 65;
-      T v = lane < bw ? x[b0 + lane] : (T)0;
-      const T rd = lane < bw ? (T)1 / tr[lane] : (T)0;
-#pragma unroll 16
-      for (int j = bw - 1; j >= 0; --j) {
-        const T xj = mf_bcast(v, j) * mf_bcast(rd, j);
-        const T u = tr[j];
-        if (lane == j) v = xj;
-        if (lane < j) v -= u * xj;
-      }
+      const T v = mf_triangle<true>(tri + (k & 1) * kMfTri, bw, lane, lane < bw ? x[b0 + lane] : (T)0);
       if (lane < bw) x[b0 + lane] = v;
     } else {
       if (mine) {
@@ -1399,9 +1416,12 @@ static int mf_solve_enqueue(MfLu::Impl& I, const T* F, T* V, const double* b_dev
     const int nt = I.tiny_off[l + 1] - I.tiny_off[l], nb = I.big_off[l + 1] - I.big_off[l];
     const int nr = I.frow_off[l + 1] - I.frow_off[l];
     if (nt) hipLaunchKernelGGL(k_mf_fwd_tiny<T>, dim3(nt), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l], F, V, b_dev);
-    if (nb)
-      hipLaunchKernelGGL(k_mf_fwd_big<T>, dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F, V, b_dev,
-                         (int)ldsv);
+    if (nb && ldsv)
+      hipLaunchKernelGGL((k_mf_fwd_big<T, true>), dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F, V,
+                         b_dev);
+    else if (nb)
+      hipLaunchKernelGGL((k_mf_fwd_big<T, false>), dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F,
+                         V, b_dev);
     if (nr) hipLaunchKernelGGL(k_mf_fwd_rows<T>, dim3(nr), dim3(256), 0, st, d, I.frow.p + I.frow_off[l], F, V);
   }
   for (int l = nl - 1; l >= 0; --l) {
@@ -1410,9 +1430,12 @@ static int mf_solve_enqueue(MfLu::Impl& I, const T* F, T* V, const double* b_dev
     if (nr)
       hipLaunchKernelGGL(k_mf_bwd_rows<T>, dim3(nr), dim3(256), 0, st, d, I.brow.p + I.brow_off[l], F, V,
                          (const double*)x_dev);
-    if (nb)
-      hipLaunchKernelGGL(k_mf_bwd_big<T>, dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F, V, x_dev,
-                         (int)ldsv, nan_flag);
+    if (nb && ldsv)
+      hipLaunchKernelGGL((k_mf_bwd_big<T, true>), dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F, V,
+                         x_dev, nan_flag);
+    else if (nb)
+      hipLaunchKernelGGL((k_mf_bwd_big<T, false>), dim3(nb), dim3(kMfSolve), lds, st, d, I.big_list.p + I.big_off[l], F,
+                         V, x_dev, nan_flag);
     if (nt)
       hipLaunchKernelGGL(k_mf_bwd_tiny<T>, dim3(nt), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l], F, (const T*)V,
                          x_dev, nan_flag);
