@@ -205,11 +205,66 @@ __device__ __forceinline__ float mf_bcast(float v, int src) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
 }
 
-template <class T>
-__device__ __forceinline__ T mf_wave_sum(T v) {
+// Sums over the wavefront, of four values at once: lanes of row k (16 k to 16 k +
+// 15) get the sum of the k-th.  Halves and rows are exchanged between two
+// registers (so that one addition serves two values), the rest within rows; the
+// order of each sum is the butterfly's (lane distances 32, 16, 8, 4, 2, 1).  In
+// registers, as a butterfly through LDS takes 48 accesses where this takes none
+// (solve of a 64-row block by 13 wavefronts: 6300 cycles of sums, 1300 now).
+__device__ __forceinline__ void mf_swap32(unsigned& a, unsigned& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+__device__ __forceinline__ void mf_swap16(unsigned& a, unsigned& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0]; b = r[1];
+}
+// upper half of a <-> lower half of b (odd rows of a <-> even rows of b), added
+template <int N, class T>
+__device__ __forceinline__ T mf_fold(T a, T b) {
+  constexpr int W = sizeof(T) / 4;
+  unsigned ua[W], ub[W];
+  __builtin_memcpy(ua, &a, sizeof(T));
+  __builtin_memcpy(ub, &b, sizeof(T));
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  for (int w = 0; w < W; ++w) {
+    if (N == 32) mf_swap32(ua[w], ub[w]);
+    else mf_swap16(ua[w], ub[w]);
+  }
+  __builtin_memcpy(&a, ua, sizeof(T));
+  __builtin_memcpy(&b, ub, sizeof(T));
+  return a + b;
+}
+template <int N, class T>
+__device__ __forceinline__ T mf_add_ror(T v) {
+  constexpr int W = sizeof(T) / 4;
+  int u[W];
+  __builtin_memcpy(u, &v, sizeof(T));
+#pragma unroll
+  for (int w = 0; w < W; ++w) u[w] = __builtin_amdgcn_update_dpp(0, u[w], 0x120 + N, 0xf, 0xf, true);
+  T o;
+  __builtin_memcpy(&o, u, sizeof(T));
+  return v + o;
+}
+template <class T>
+__device__ __forceinline__ T mf_sum4(T v0, T v1, T v2, T v3) {
+  T s = mf_fold<16>(mf_fold<32>(v0, v2), mf_fold<32>(v1, v3));
+  s = mf_add_ror<8>(s);
+  s = mf_add_ror<4>(s);
+  s = mf_add_ror<2>(s);
+  return mf_add_ror<1>(s);
+}
+// x[r + k] -= the sum of acc[k], k < min(nr, NR)
+template <int NR, class T>
+__device__ __forceinline__ void mf_sub_sums(T* x, int r, int nr, int lane, const T (&acc)[NR]) {
+  static_assert(NR == 4 || NR == 5, "");
+  const T s = mf_sum4(acc[0], acc[1], acc[2], acc[3]);
+  const int k = lane >> 4;
+  if ((lane & 15) == 0 && k < nr) x[r + k] -= s;
+  if (NR == 5) {
+    const T s4 = mf_sum4(acc[NR - 1], acc[NR - 1], acc[NR - 1], acc[NR - 1]);
+    if (lane == 0 && 4 < nr) x[r + 4] -= s4;
+  }
 }
 
 // Larger fronts: blocked by panels of kMfPanel columns, one launch per panel
@@ -781,16 +836,19 @@ __device__ __forceinline__ void mf_rows_part(const T* Fs, long long ld, int r, i
     T xv[4], f[NR][4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const int j = c + 64 * q + lane, jj = min(j, c1 - 1);
+      if (c + 64 * q >= c1) break;
+      const int jj = min(c + 64 * q + lane, c1 - 1);
 #pragma unroll
       for (int k = 0; k < NR; ++k) f[k][q] = row[k][jj];
-      xv[q] = j < c1 ? x(jj) : (T)0;
     }
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 4; ++q) {
+      const int j = c + 64 * q + lane;
+      if (c + 64 * q >= c1) break;
+      xv[q] = j < c1 ? x(j) : (T)0;
 #pragma unroll
-      for (int k = 0; k < NR; ++k)
-        if (c + 64 * q < c1) acc[k] += f[k][q] * xv[q];
+      for (int k = 0; k < NR; ++k) acc[k] += f[k][q] * xv[q];
+    }
   }
 }
 
@@ -881,27 +939,35 @@ __global__ void __launch_bounds__(64) k_mf_bwd_tiny(MfDev d, const int* list, co
 // stands one 64 x 64 product from registers.  The rows outside the pivot block
 // (L21 y, U12 x_below) are split over the GPU by the _rows kernels where they
 // have more than kMfSplit elements, which one workgroup would need longer for
-// than a launch takes (5 us).  512 x 512 grid, all levels, forward and
-// backward: 1.08 ms, 1.38 ms before the overlap and the split.
+// than a launch takes (5 us).  What bounds a block is one CU's reads (64 rows of
+// the solved columns at 27 bytes a cycle) above 128 solved columns, the triangle
+// below (64 steps of 55 cycles).  512 x 512 grid, all levels, forward and
+// backward: 0.59 ms; 0.78 with the sums as butterflies through LDS and whole
+// 256-column chunks read, 1.08 with the triangle's steps rolled, 1.38 before the
+// overlap and the split.
 constexpr int kMfSolve = 1024;
 constexpr int kMfSplit = 49152;
 constexpr int kMfTri = 64 * 65;
 constexpr int kMfNext = 5;                     // rows of the next block per wavefront
 
+// the triangle at b0 into `tri` by wavefronts w, w + nw, ..., straight to LDS (a
+// row is one or two loads of a dword per lane; no registers, so the products'
+// loads follow at once).  mf_tri_wait: before the barrier that publishes it.
 template <class T>
-__device__ __forceinline__ void mf_load_tri(const T* Fs, long long ld, int b0, int bw, int t, int nt, T* tri) {
-  T v[5];
+__device__ __forceinline__ void mf_load_tri(const T* Fs, long long ld, int b0, int bw, int w, int nw, int lane, T* tri) {
+  constexpr int D = sizeof(T) / 4;
+  for (int i = __builtin_amdgcn_readfirstlane(w); i < bw; i += nw) {
+    const char* src = reinterpret_cast<const char*>(Fs + (b0 + i) * ld + b0);
 #pragma unroll
-  for (int it = 0; it < 5; ++it) {
-    const int x = t + it * nt, i = min(x >> 6, bw - 1), j = min(x & 63, bw - 1);
-    v[it] = Fs[(b0 + i) * ld + b0 + j];
-  }
-#pragma unroll
-  for (int it = 0; it < 5; ++it) {
-    const int x = t + it * nt;
-    if (x < 4096) tri[(x >> 6) * 65 + (x & 63)] = v[it];
+    for (int h = 0; h < D; ++h) {
+      const int q = 64 * h + lane;
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(src + (min(q / D, bw - 1) * D + q % D) * 4),
+          (__attribute__((address_space(3))) void*)(reinterpret_cast<char*>(tri + i * 65) + 256 * h), 4, 0, 0);
+    }
   }
 }
+__device__ __forceinline__ void mf_tri_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // A 64-row triangle by one wavefront, lane i holding row i's unknown: a row's
 // coefficients come from LDS sixteen at a time, the next ones under way, those of
@@ -948,8 +1014,9 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* li
   const long long ld = ms;
   const T* Fs = F + f.fo;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  mf_load_tri(Fs, ld, 0, min(64, np), t, kMfSolve, tri);
+  mf_load_tri(Fs, ld, 0, min(64, np), wave, kMfSolve / 64, lane, tri);
   for (int i = t; i < ms; i += kMfSolve) x[i] = i < np ? (T)b[d.bidx[f.idx + i]] : (T)0;
+  mf_tri_wait();
   __syncthreads();
   for (int c = f.c0; c < f.c1; ++c) {
     const MfChild ch = d.child[c];
@@ -969,23 +1036,21 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* li
       const T v = mf_triangle<false>(tri + (k & 1) * kMfTri, bw, lane, lane < bw ? x[b0 + lane] : (T)0);
       if (lane < bw) x[b0 + lane] = v;
     } else {
+      if (k + 1 < nb)
+        mf_load_tri(Fs, ld, b0 + 64, min(64, np - b0 - 64), wave - 1, kMfSolve / 64 - 1, lane, tri + ((k + 1) & 1) * kMfTri);
       if (mine) {
 #pragma unroll
         for (int i = 0; i < kMfNext; ++i) pre[i] = Fs[(r + min(i, nr - 1)) * ld + b0 + lane];
         mf_rows_part<kMfNext>(Fs, ld, r, nr, 0, b0, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
       }
-      if (k + 1 < nb)
-        mf_load_tri(Fs, ld, b0 + 64, min(64, np - b0 - 64), t - 64, kMfSolve - 64, tri + ((k + 1) & 1) * kMfTri);
+      mf_tri_wait();
     }
     __syncthreads();
     if (mine) {
       const T y = x[b0 + lane];
 #pragma unroll
-      for (int i = 0; i < kMfNext; ++i) acc[i] = mf_wave_sum(acc[i] + pre[i] * y);
-      if (lane == 0)
-#pragma unroll
-        for (int i = 0; i < kMfNext; ++i)
-          if (i < nr) x[r + i] -= acc[i];
+      for (int i = 0; i < kMfNext; ++i) acc[i] += pre[i] * y;
+      mf_sub_sums<kMfNext>(x, r, nr, lane, acc);
     }
     __syncthreads();
   }
@@ -994,11 +1059,7 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_fwd_big(MfDev d, const int2* li
       const int nr = min(4, ms - r);
       T acc[4];
       mf_rows_part<4>(Fs, ld, r, nr, 0, np, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        acc[k] = mf_wave_sum(acc[k]);
-        if (lane == 0 && k < nr) x[r + k] -= acc[k];
-      }
+      mf_sub_sums<4>(x, r, nr, lane, acc);
     }
   if (!LDSV) return;
   __syncthreads();
@@ -1015,11 +1076,7 @@ __global__ void __launch_bounds__(256) k_mf_fwd_rows(MfDev d, const int2* ent, c
   T* v = V + f.vo;
   T acc[4];
   mf_rows_part<4>(F + f.fo, f.m, r, nr, 0, f.np, lane, [&](int j) MF_INLINE { return v[j]; }, acc);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    acc[k] = mf_wave_sum(acc[k]);
-    if (lane == 0 && k < nr) v[r + k] -= acc[k];
-  }
+  mf_sub_sums<4>(v, r, nr, lane, acc);
 }
 
 // pivot rows of a split front minus U12 x_below, 16 per workgroup
@@ -1032,11 +1089,7 @@ __global__ void __launch_bounds__(256) k_mf_bwd_rows(MfDev d, const int2* ent, c
   const int* ix = d.xidx + f.idx;
   T acc[4];
   mf_rows_part<4>(F + f.fo, f.m, r, nr, f.np, f.m, lane, [&](int j) MF_INLINE { return (T)x[ix[j]]; }, acc);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    acc[k] = mf_wave_sum(acc[k]);
-    if (lane == 0 && k < nr) V[f.vo + r + k] -= acc[k];
-  }
+  mf_sub_sums<4>(V + f.vo, r, nr, lane, acc);
 }
 
 template <class T, bool LDSV>
@@ -1053,21 +1106,18 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* li
   const int* ix = d.xidx + f.idx;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int nb = (np + 63) / 64;
-  mf_load_tri(Fs, ld, 64 * (nb - 1), np - 64 * (nb - 1), t, kMfSolve, tri + ((nb - 1) & 1) * kMfTri);
+  mf_load_tri(Fs, ld, 64 * (nb - 1), np - 64 * (nb - 1), wave, kMfSolve / 64, lane, tri + ((nb - 1) & 1) * kMfTri);
   for (int i = t; i < (en.y ? np : ms); i += kMfSolve)
     if (i >= np) x[i] = (T)xg[ix[i]];
     else if (LDSV) x[i] = V[f.vo + i];
+  mf_tri_wait();
   __syncthreads();
   if (!en.y && ms > np) {
     for (int r = 4 * wave; r < np; r += 4 * (kMfSolve / 64)) {
       const int nr = min(4, np - r);
       T acc[4];
       mf_rows_part<4>(Fs, ld, r, nr, np, ms, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        acc[k] = mf_wave_sum(acc[k]);
-        if (lane == 0 && k < nr) x[r + k] -= acc[k];
-      }
+      mf_sub_sums<4>(x, r, nr, lane, acc);
     }
     __syncthreads();
   }
@@ -1081,22 +1131,21 @@ __global__ void __launch_bounds__(kMfSolve) k_mf_bwd_big(MfDev d, const int2* li
       const T v = mf_triangle<true>(tri + (k & 1) * kMfTri, bw, lane, lane < bw ? x[b0 + lane] : (T)0);
       if (lane < bw) x[b0 + lane] = v;
     } else {
+      if (k > 0)
+        mf_load_tri(Fs, ld, b0 - 64, 64, wave - 1, kMfSolve / 64 - 1, lane, tri + ((k - 1) & 1) * kMfTri);
       if (mine) {
 #pragma unroll
         for (int i = 0; i < kMfNext; ++i) pre[i] = Fs[(r + min(i, nr - 1)) * ld + b0 + min(lane, bw - 1)];
         mf_rows_part<kMfNext>(Fs, ld, r, nr, b0 + bw, np, lane, [&](int j) MF_INLINE { return x[j]; }, acc);
       }
-      if (k > 0) mf_load_tri(Fs, ld, b0 - 64, 64, t - 64, kMfSolve - 64, tri + ((k - 1) & 1) * kMfTri);
+      mf_tri_wait();
     }
     __syncthreads();
     if (mine) {
       const T y = lane < bw ? x[b0 + lane] : (T)0;
 #pragma unroll
-      for (int i = 0; i < kMfNext; ++i) acc[i] = mf_wave_sum(acc[i] + pre[i] * y);
-      if (lane == 0)
-#pragma unroll
-        for (int i = 0; i < kMfNext; ++i)
-          if (i < nr) x[r + i] -= acc[i];
+      for (int i = 0; i < kMfNext; ++i) acc[i] += pre[i] * y;
+      mf_sub_sums<kMfNext>(x, r, nr, lane, acc);
     }
     __syncthreads();
   }
