@@ -346,27 +346,19 @@ __device__ __forceinline__ void mf_update_blocks(const T* Fs, long long ld, int 
   T l[NA][kMfPanel / 4], u[NB][kMfPanel / 4];
   const T* Lb = Fs + i0 * ld + q0;
   const T* Ub = Fs + q0 * ld + j0;
-  if (kw == kMfPanel) {
-    typedef T Pair __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+  // (in pairs, the last of an odd kw with the one before it: no branch, which
+  // would have the loads before it waited for; a front's last row may be read one
+  // value past its end, the buffer has it)
+  typedef T Pair __attribute__((ext_vector_type(2), aligned(sizeof(T))));
 #pragma unroll
-    for (int a = 0; a < NA; ++a) {
-      const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row + 8 * lk * (unsigned)sizeof(T);
+  for (int a = 0; a < NA; ++a) {
+    const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row;
 #pragma unroll
-      for (int k = 0; k < kMfPanel / 4; k += 2) {
-        const Pair p = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(Lb) + o + k * sizeof(T));
-        l[a][k] = -p.x;
-        l[a][k + 1] = -p.y;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < NA; ++a) {
-      const unsigned o = (unsigned)(min(i0 + 16 * a + lr, i1 - 1) - i0) * row;
-#pragma unroll
-      for (int k = 0; k < kMfPanel / 4; ++k) {
-        const T v = mf_at(Lb, o + (unsigned)min(8 * lk + k, kw - 1) * (unsigned)sizeof(T));
-        l[a][k] = 8 * lk + k < kw ? -v : (T)0;
-      }
+    for (int k = 0; k < kMfPanel / 4; k += 2) {
+      const unsigned c = (unsigned)max(min(8 * lk + k, kw - 2), 0);
+      const Pair p = *reinterpret_cast<const Pair*>(reinterpret_cast<const char*>(Lb) + o + c * (unsigned)sizeof(T));
+      l[a][k] = p.x;
+      l[a][k + 1] = p.y;
     }
   }
 #pragma unroll
@@ -375,12 +367,17 @@ __device__ __forceinline__ void mf_update_blocks(const T* Fs, long long ld, int 
 #pragma unroll
     for (int b = 0; b < NB; ++b) u[b][k] = mf_at(Ub, o + cj[b]);
   }
+  // (L's signs and its columns past kw only here, behind U's loads)
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int k = 0; k < kMfPanel / 4; ++k)
 #pragma unroll
-    for (int a = 0; a < NA; ++a)
+    for (int a = 0; a < NA; ++a) {
+      const int c = 8 * lk + k;
+      const T lv = c < kw ? -((k & 1) == 0 && c > 0 && c == kw - 1 ? l[a][k | 1] : l[a][k]) : (T)0;
 #pragma unroll
-      for (int b = 0; b < NB; ++b) acc[a][b] = MfAcc<T>::mma(l[a][k], u[b][k], acc[a][b]);
+      for (int b = 0; b < NB; ++b) acc[a][b] = MfAcc<T>::mma(lv, u[b][k], acc[a][b]);
+    }
 }
 
 // reciprocal of a pivot in four stages that run between the products of a row
@@ -628,34 +625,41 @@ __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list,
   if (__any(hard) && t == 0) atomicOr(bad + 1, 1);
 }
 
+#ifndef MF_K2
+#define MF_K2 8
+#endif
 constexpr int kMfStep = 192;              // threads of a step workgroup: three wavefronts
 constexpr int kMfTileRows = 96;           // rows of an update tile: 32 per wavefront
 constexpr int kMfDs = kMfPanel + 2;       // row stride of the diagonal factors in LDS (16-byte pairs)
 constexpr int kMfTile = 64 * (kMfPanel + 1) > kMfPanel * 65 ? 64 * (kMfPanel + 1) : kMfPanel * 65;
 
+// an entry and its front's numbers, so that the kernel's first loads are its tiles
+struct MfStep { int y, z, w, m, np, first; long long fo; };
+
 template <class T>
-__global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2))) k_mf_step(MfDev d, const int4* ent, int p0, T* F, T* dbuf, int half,
-                                                     int* bad, int* fail) {
+__global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2))) k_mf_step(const MfStep* ent, int p0, T* F, T* dbuf, int half, int* bad,
+                                                     int* fail) {
   constexpr int PW = kMfPanel;
   __shared__ __attribute__((aligned(16))) T Du[PW * kMfDs];   // U11 by rows
   __shared__ __attribute__((aligned(16))) T Dl[PW * kMfDs];   // L11 by columns; the updated block before it is factored
   __shared__ T Ts[2][kMfTile];
-  const int4 e = ent[blockIdx.x];
-  const int s = e.x, slot = e.w;
-  const int ms = d.m[s], np = d.sfirst[s + 1] - d.sfirst[s];
+  const MfStep e = ent[blockIdx.x];
+  const int slot = e.w, ms = e.m, np = e.np;
   const int base = min(np, p0 + PW), q0 = p0 - PW, kw = q0 >= 0 ? min(PW, np - q0) : 0;
-  T* Fs = F + d.fo[s];
+  T* Fs = F + e.fo;
   const long long ld = ms;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, lr = lane & 15, lk = lane >> 4;
   typedef typename MfAcc<T>::V V;
-  if (kw > 0 && e.y == 0 && e.z <= 0) {
-    // the front's first entry: panel j - 1's diagonal factors into the front
+  // the front's first entry: panel j - 1's diagonal factors into the front
+  auto copy_diagonal = [&](int t0, int nt) MF_INLINE {
+    if (kw <= 0 || e.y != 0 || e.z > 0) return;
     const T* db = dbuf + ((long long)slot * 2 + (half ^ 1)) * PW * PW;
-    for (int x = t; x < PW * PW; x += kMfStep) {
+    for (int x = t0; x < PW * PW; x += nt) {
       const int i = x / PW, j = x % PW;
       if (i < kw && j < kw) Fs[(q0 + i) * ld + q0 + j] = db[x];
     }
-  }
+  };
+  if (e.z != -1) copy_diagonal(t, kMfStep);
   if (e.z == -2) return;
   if (e.z >= 0) {
     const int i0 = base + e.y * kMfTileRows + 32 * wave, j0 = base + e.z * 64;
@@ -713,6 +717,7 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
 #pragma unroll
         for (int r = 0; r < 4; ++r) Tl[(16 * a + MfAcc<T>::row(lk, r)) * 65 + 16 * b + lr] = acc[a][b][r];
   }
+  if (wave > 0) copy_diagonal(t - 64, kMfStep - 64);      // (beside the diagonal's pivots)
   mf_wave_fence();          // each wavefront reads back its own tile: no wait for the others
   int failed = PW;          // first column whose pivot or multiplier fails
   bool hard = false;
@@ -748,41 +753,44 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
     for (int q = 0; q < PW; ++q) db[q] = v[q];
   }
   if (has) {
-    // the factors' rows come two values at a time from LDS; row k + 1 is read
-    // while row k is applied (its address is tied to v[k], so that no more than
-    // two rows are held in registers)
+    // the factors' rows come two values at a time from LDS, two rows ahead of the
+    // one applied (one ahead for the first, longest ones: registers); a row's
+    // address is tied to v[k], so that no more are held
     typedef T Pair __attribute__((ext_vector_type(2)));
     typedef const __attribute__((address_space(3))) T* Lds;
     typedef const __attribute__((address_space(3))) Pair* LdsPair;
+    constexpr int K2 = MF_K2;                     // from here on two rows ahead
     Lds pd = (Lds)(lower ? Du : Dl);
-    T u[PW], un[PW];
-    auto fetch = [&](auto kc, T (&to)[PW]) MF_INLINE {
+    T u[3][PW];
+    T rr[3] = {(T)1, (T)1, (T)1};
+    auto fetch = [&](auto kc) MF_INLINE {
       constexpr int k = kc;
+      if constexpr (k < PW) {
 #pragma unroll
-      for (int q = (k + 1) & ~1; q < PW; q += 2) {
-        const Pair p = *(LdsPair)(pd + k * kMfDs + q);
-        to[q] = p.x;
-        to[q + 1] = p.y;
+        for (int q = (k + 1) & ~1; q < PW; q += 2) {
+          const Pair p = *(LdsPair)(pd + k * kMfDs + q);
+          u[k % 3][q] = p.x;
+          u[k % 3][q + 1] = p.y;
+        }
+        if (lower) rr[k % 3] = pd[k * kMfDs + PW];
       }
     };
-    fetch(std::integral_constant<int, 0>{}, u);
+    auto ahead = [&](auto kc) MF_INLINE {
+      constexpr int k = kc;
+      asm volatile("" : "+v"(pd) : "v"(v[k]));
+      if constexpr (k <= K2) fetch(std::integral_constant<int, k + 1>{});
+      if constexpr (k >= K2) fetch(std::integral_constant<int, k + 2>{});
+    };
+    fetch(std::integral_constant<int, 0>{});
     if (lower) {
       const bool valid = o0 + lane < ms;
-      T r = pd[PW], rn = r;
       mf_for<PW>([&](auto kc) MF_INLINE {
         constexpr int k = kc;
-        asm volatile("" : "+v"(pd) : "v"(v[k]));
-        if constexpr (k + 1 < PW) {
-          fetch(std::integral_constant<int, k + 1>{}, un);
-          rn = pd[(k + 1) * kMfDs + PW];
-        }
-        v[k] *= r;
-        r = rn;
+        ahead(kc);
+        v[k] *= rr[k % 3];
         if (valid && !(fabs((double)v[k]) <= 1.0e3)) failed = min(failed, k);
 #pragma unroll
-        for (int q = k + 1; q < PW; ++q) v[q] -= v[k] * u[q];
-#pragma unroll
-        for (int q = k + 2; q < PW; ++q) u[q] = un[q];
+        for (int q = k + 1; q < PW; ++q) v[q] -= v[k] * u[k % 3][q];
         __builtin_amdgcn_sched_barrier(0);
       });
       // the lane's row of L21: 32 values next to each other
@@ -802,12 +810,9 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
       const int c = o0 + lane;
       mf_for<PW>([&](auto kc) MF_INLINE {
         constexpr int k = kc;
-        asm volatile("" : "+v"(pd) : "v"(v[k]));
-        if constexpr (k + 1 < PW) fetch(std::integral_constant<int, k + 1>{}, un);
+        ahead(kc);
 #pragma unroll
-        for (int q = k + 1; q < PW; ++q) v[q] -= u[q] * v[k];
-#pragma unroll
-        for (int q = k + 2; q < PW; ++q) u[q] = un[q];
+        for (int q = k + 1; q < PW; ++q) v[q] -= u[k % 3][q] * v[k];
         __builtin_amdgcn_sched_barrier(0);
       });
 #pragma unroll
@@ -815,7 +820,7 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
         if (c < ms && q < pw) Fs[(p0 + q) * ld + c] = v[q];
     }
   }
-  if (failed < pw) { atomicMin(bad, d.sfirst[s] + p0 + failed + 1); *fail = 1; }
+  if (failed < pw) { atomicMin(bad, e.first + p0 + failed + 1); *fail = 1; }
   if (__any(hard) && lane == 0) atomicOr(bad + 1, 1);
 }
 
@@ -1217,7 +1222,7 @@ struct MfLu::Impl {
   DevVec<int2> frow, brow;        // entries of those rows {front, first row}
   DevVec<int4> aent;              // assembly entries of the larger fronts, two each
   DevVec<int2> alo;               // per entry and child: the child's rows in the entry's range
-  DevVec<int4> sent;              // entries of the panel steps
+  DevVec<MfStep> sent;            // entries of the panel steps
   DevVec<double> dbuf;            // diagonal-block factors, two 32 x 32 slots per larger front of a level
   std::vector<int> tiny_off, tiny_half, big_off;   // fronts up to order 32 at [tiny_off, tiny_half), up to 64 from there
   int big_maxm = 0;
@@ -1276,8 +1281,8 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   MFCHK(I.bad.alloc(2));
   if (!I.fail) MFCHK(hipHostMalloc((void**)&I.fail, sizeof(int), hipHostMallocDefault));
   hipLaunchKernelGGL(k_mf_flag_init, dim3(1), dim3(1), 0, st, I.bad.p);
-  MFCHK(I.F64.alloc(P.fo[P.ns])); MFCHK(I.V64.alloc(P.vo[P.ns]));
-  if (want_fp32) { MFCHK(I.F32.alloc(P.fo[P.ns])); MFCHK(I.V32.alloc(P.vo[P.ns])); }
+  MFCHK(I.F64.alloc(P.fo[P.ns] + 1)); MFCHK(I.V64.alloc(P.vo[P.ns]));
+  if (want_fp32) { MFCHK(I.F32.alloc(P.fo[P.ns] + 1)); MFCHK(I.V32.alloc(P.vo[P.ns])); }
   // per level: tiny fronts (one launch), larger fronts (blocked panels, all
   // fronts of the level in each panel launch)
   const int nl = (int)P.lvl_ptr.size() - 1;
@@ -1285,7 +1290,7 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   std::vector<int2> bl2, fre, bre;
   I.frow_off.assign(nl + 1, 0);
   I.brow_off.assign(nl + 1, 0);
-  std::vector<int4> se;
+  std::vector<MfStep> se;
   int max_slots = 1;
   I.tiny_off.assign(nl + 1, 0);
   I.big_off.assign(nl + 1, 0);
@@ -1330,14 +1335,15 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
           if (S.p0 >= np + kMfPanel) continue;                 // finished at an earlier step
           const int rest = P.m[t] - std::min(np, S.p0 + kMfPanel);
           const int nrb = (rest + 63) / 64;
+          auto add = [&](int y, int z) { se.push_back(MfStep{y, z, slot, P.m[t], np, P.sfirst[t], P.fo[t]}); };
           if (pass == 0) {
             if (S.p0 < np)
-              for (int i = 0; i < std::max(1, nrb); ++i) se.push_back(make_int4(t, i, -1, slot));
-            else if (rest == 0) se.push_back(make_int4(t, 0, -2, slot));
+              for (int i = 0; i < std::max(1, nrb); ++i) add(i, -1);
+            else if (rest == 0) add(0, -2);
           } else if (j > 0) {
             // after the last panel tile (0, 0) copies the diagonal
             for (int ti = 0; ti * kMfTileRows < rest; ++ti)
-              for (int tj = 0; tj < nrb; ++tj) se.push_back(make_int4(t, ti, tj, slot));
+              for (int tj = 0; tj < nrb; ++tj) add(ti, tj);
           }
         }
       S.cnt = (int)se.size() - S.off;
@@ -1411,7 +1417,7 @@ static int mf_factor_enqueue(MfLu::Impl& I, const double* vals_dev, int nnz, T* 
       hipLaunchKernelGGL((k_mf_factor_tiny<T, kMfTiny>), dim3(n64), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_half[l],
                          vals_dev, F, I.bad.p, I.fail);
     for (const auto& S : I.steps[l])
-      hipLaunchKernelGGL(k_mf_step<T>, dim3(S.cnt), dim3(kMfStep), 0, st, d, I.sent.p + S.off, S.p0, F, dbuf,
+      hipLaunchKernelGGL(k_mf_step<T>, dim3(S.cnt), dim3(kMfStep), 0, st, I.sent.p + S.off, S.p0, F, dbuf,
                          (S.p0 / kMfPanel) & 1, I.bad.p, I.fail);
   }
   MFCHK(hipGetLastError());
