@@ -287,9 +287,10 @@ __device__ __forceinline__ void mf_sub_sums(T* x, int r, int nr, int lane, const
 // complement.  The chain of panels is what bounds a tree's top: one launch per
 // panel instead of a panel and an update launch, and no operand passes through
 // LDS on its way to the matrix cores, so that a step is one round of loads, the
-// diagonal's 32 dependent pivots and a substitution (12.5 us where the two
-// launches took 31.6, on the 865-order root of a 512 x 512 grid: loads and update
-// 3.8 us, pivots 4.5, substitution and stores 3.3; mean over all its steps 14.2).
+// diagonal's 32 dependent pivots and a substitution (12.2 us where the two
+// launches took 31.6, on the 865-order root of a 512 x 512 grid, of which the 32
+// pivots take 4.1; mean over all its steps 12.9, 14.2 with the loads of C and L
+// waited for before U's and the substitution's rows read one ahead).
 //
 // v_mfma_{f64,f32}_16x16x4: lane l holds A's row l % 16, column l / 16 of the
 // 16 x 4 block, B's row l / 16, column l % 16 of the 4 x 16 block; accumulator
@@ -487,49 +488,88 @@ __device__ __forceinline__ void mf_wave_fence() {
 // complements, one child after another in their fixed order, so that every
 // element receives the same sums in the same order on every refactor.  One
 // workgroup per range of rows and columns (entries {front, first row, rows,
-// offset into alo}, {first column, columns, 0, 0}; at most kMfAsm elements, held
+// offset into parts}, {first column, columns, parts, 0}; at most kMfAsm elements, held
 // in LDS until they are complete, so a front is written once and never cleared
 // or read back).  Wavefront w owns the rows with index % 4 = w: no wavefront
-// waits for another.  alo holds, per entry and child, the child's rows [x, y)
-// that land in the range; a child's rows map to increasing parent rows.  Per
-// child and 256 columns a wavefront issues the loads of up to four rows at
-// once (512 x 512 grid, all levels: 263 us with A's entries in, where clearing the
-// fronts, scattering A and adding the children in memory took 400).
+// waits for another.  The parts are the children with rows in the range (a front
+// with a supply row has many others), their positions loaded one part ahead; a
+// child's rows map to increasing parent rows.  Per part and 256 columns a wavefront
+// issues the loads of up to four rows at once; a part is a round trip, which bounds
+// fronts of many children (512 x 512 grid, all levels: 243 us with A's entries in,
+// where clearing the fronts, scattering A and adding the children in memory took
+// 400; roots of a 2000-gate array 42 us).
 constexpr int kMfAsmRows = 16;
+// a child in a range: its Schur complement, and its rows [a, b) that land there
+struct MfPart { long long src; int ld, nu, em, a, b, pad; };
 constexpr int kMfAsm = 4096;
 
 template <class T>
-__global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, const int2* alo, const double* vals,
+__global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, const MfPart* parts, const double* vals,
                                                      T* F) {
   __shared__ T R[kMfAsm];
   const int4 e = ent[2 * blockIdx.x], ec = ent[2 * blockIdx.x + 1];
   const MfFront f = d.front[e.x];
   const int r0 = e.y, rows = e.z, j0 = ec.x, w = ec.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int i = wave; i < rows; i += 4) {
-    for (int j = lane; j < w; j += 64) R[i * w + j] = (T)0;
-    mf_wave_fence();
-    const int* ar = d.arow + f.vo + r0 + i;
-    for (int q = ar[0] + lane; q < ar[1]; q += 64) {
-      const int j = d.acol[q] - j0;
-      // (an entry listed twice in a row adds up)
-      if (j >= 0 && j < w) atomicAdd(&R[i * w + j], (T)vals[d.aslot[q]]);
-    }
+  const MfPart* part = parts + e.w;
+  const int n_part = ec.z;
+  MfPart next{};
+  int next_er = -1, next_eb[4] = {-1, -1, -1, -1};
+  auto fetch = [&](int c) MF_INLINE {
+    if (c >= n_part) return;
+    next = part[c];
+    const int* em = d.emap + next.em;
+    next_er = next.a + lane < next.b ? em[next.a + lane] - r0 : -1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) next_eb[q] = lane + 64 * q < next.nu ? em[lane + 64 * q] - j0 : -1;
+  };
+  fetch(0);
+  // A's entries, the wavefront's rows side by side (each is three dependent loads)
+  constexpr int NR = kMfAsmRows / 4;
+  int q0[NR], q1[NR], col[NR], slot[NR];
+  T av[NR];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    const int i = min(4 * k + wave, rows - 1);
+    q0[k] = d.arow[f.vo + r0 + i];
+    q1[k] = 4 * k + wave < rows ? d.arow[f.vo + r0 + i + 1] : q0[k];
   }
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    const bool in = q0[k] + lane < q1[k];
+    col[k] = in ? d.acol[q0[k] + lane] - j0 : -1;
+    slot[k] = in ? d.aslot[q0[k] + lane] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < NR; ++k) av[k] = q0[k] + lane < q1[k] ? (T)vals[slot[k]] : (T)0;
+  for (int i = wave; i < rows; i += 4)
+    for (int j = lane; j < w; j += 64) R[i * w + j] = (T)0;
   mf_wave_fence();
-  const int2* lo = alo + e.w;
-  for (int c = f.c0; c < f.c1; ++c) {
-    const MfChild ch = d.child[c];
-    const int2 ab = lo[c - f.c0];
-    if (ab.x >= ab.y) continue;
+  // (an entry listed twice in a row adds up)
+#pragma unroll
+  for (int k = 0; k < NR; ++k)
+    if (col[k] >= 0 && col[k] < w) atomicAdd(&R[(4 * k + wave) * w + col[k]], av[k]);
+#pragma unroll
+  for (int k = 0; k < NR; ++k)
+    for (int q = q0[k] + 64 + lane; q < q1[k]; q += 64) {
+      const int j = d.acol[q] - j0;
+      if (j >= 0 && j < w) atomicAdd(&R[(4 * k + wave) * w + j], (T)vals[d.aslot[q]]);
+    }
+  mf_wave_fence();
+  // (the next child's positions are loaded beside this one's values)
+  for (int c = 0; c < n_part; ++c) {
+    const MfPart ch = next;
+    const int er = next_er;
+    int ebn[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ebn[q] = next_eb[q];
     const int* em = d.emap + ch.em;
     // slot k: the child's row that lands on this wavefront's row 4 k + wave
-    const int er = ab.x + lane < ab.y ? em[ab.x + lane] - r0 : -1;
     int a[kMfAsmRows / 4];
 #pragma unroll
     for (int k = 0; k < kMfAsmRows / 4; ++k) {
       const unsigned long long hit = __ballot(er == 4 * k + wave);
-      a[k] = hit ? ab.x + (int)__builtin_ctzll(hit) : -1;
+      a[k] = hit ? ch.a + (int)__builtin_ctzll(hit) : -1;
     }
     const T* Fc = F + ch.src;
     for (int c0 = lane; c0 - lane < ch.nu; c0 += 256) {
@@ -538,7 +578,7 @@ __global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, c
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int b = c0 + 64 * q;
-        const int j = b < ch.nu ? em[b] - j0 : -1;
+        const int j = c0 == lane ? ebn[q] : b < ch.nu ? em[b] - j0 : -1;
         eb[q] = j < w ? j : -1;
       }
 #pragma unroll
@@ -551,6 +591,7 @@ __global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, c
           cv[k][q] = b < ch.nu ? crow[b] : (T)0;
         }
       }
+      if (c0 == lane) fetch(c + 1);
 #pragma unroll
       for (int k = 0; k < kMfAsmRows / 4; ++k) {
         if (a[k] < 0) continue;
@@ -571,30 +612,54 @@ __global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, c
 // and the children's updates are added in LDS (row stride N + 1), one child
 // after another; then lane t holds row t in registers and the pivot rows are
 // broadcast from there: a pivot costs its reciprocal and the row updates, no
-// LDS traffic (512 x 512 grid, all levels: 300 us, 656 with the elimination in LDS).
+// LDS traffic (512 x 512 grid, all levels: 295 us, 656 with the elimination in LDS).
 template <class T, int N>
 __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list, const double* vals, T* F, int* bad, int* fail) {
   constexpr int ld = N + 1;
   __shared__ T A[N * ld];
   const MfFront f = d.front[list[blockIdx.x]];
   const int ms = f.m, np = f.np, t = threadIdx.x;
+  MfChild next{};
+  int next_e = 0;                                    // parent position of its row/column t
+  auto fetch = [&](int c) MF_INLINE {
+    if (c >= f.c1) return;
+    next = d.child[c];
+    next_e = t < next.nu ? d.emap[next.em + t] : 0;
+  };
+  fetch(f.c0);
   if (t < ms) {
     T* row = A + t * ld;
+    const int qa = d.arow[f.vo + t], qb = d.arow[f.vo + t + 1];
     for (int j = 0; j < ms; ++j) row[j] = (T)0;
-    const int q1 = d.arow[f.vo + t + 1];
-    for (int q = d.arow[f.vo + t]; q < q1; ++q) row[d.acol[q]] += (T)vals[d.aslot[q]];
+    // eight entries at a time: their positions, then their values
+    for (int q = qa; q < qb; q += 8) {
+      int col[8], slot[8];
+      T av[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int p = min(q + i, qb - 1);
+        col[i] = d.acol[p];
+        slot[i] = d.aslot[p];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) av[i] = (T)vals[slot[i]];
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (q + i < qb) row[col[i]] += av[i];
+    }
   }
   mf_wave_fence();
-  // a child's update has at most ms rows and columns: lane t adds column t
+  // a child's update has at most ms rows and columns: lane t adds column t; the
+  // next child's positions are loaded beside this one's values
   for (int c = f.c0; c < f.c1; ++c) {
-    const MfChild ch = d.child[c];
-    const int nu = ch.nu;
-    const int eb = t < nu ? d.emap[ch.em + t] : 0;   // parent position of the child's row/column t
+    const MfChild ch = next;
+    const int nu = ch.nu, eb = next_e;
     const T* cb = F + ch.src + t;
     for (int a = 0; a < nu; a += 16) {
       T v[16];
 #pragma unroll
       for (int q = 0; q < 16; ++q) v[q] = (t < nu && a + q < nu) ? cb[(long long)(a + q) * ch.ld] : (T)0;
+      if (a == 0) fetch(c + 1);
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
         if (a + q >= nu) break;
@@ -619,15 +684,13 @@ __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list,
   mf_wave_fence();
   const int first = mf_check_rows<N>(v, t, ms, np, [&](int k) MF_INLINE { return A[t * ld + k]; }, hard);
   T* Fs = F + f.fo;
+#pragma unroll 8
   for (int i = 0; i < ms; ++i)
     if (t < ms) Fs[(long long)i * ms + t] = A[i * ld + t];
   if (first < np) { atomicMin(bad, f.first + first + 1); *fail = 1; }
   if (__any(hard) && t == 0) atomicOr(bad + 1, 1);
 }
 
-#ifndef MF_K2
-#define MF_K2 8
-#endif
 constexpr int kMfStep = 192;              // threads of a step workgroup: three wavefronts
 constexpr int kMfTileRows = 96;           // rows of an update tile: 32 per wavefront
 constexpr int kMfDs = kMfPanel + 2;       // row stride of the diagonal factors in LDS (16-byte pairs)
@@ -759,7 +822,7 @@ __global__ void __launch_bounds__(kMfStep) __attribute__((amdgpu_waves_per_eu(2)
     typedef T Pair __attribute__((ext_vector_type(2)));
     typedef const __attribute__((address_space(3))) T* Lds;
     typedef const __attribute__((address_space(3))) Pair* LdsPair;
-    constexpr int K2 = MF_K2;                     // from here on two rows ahead
+    constexpr int K2 = 8;                         // from here on two rows ahead
     Lds pd = (Lds)(lower ? Du : Dl);
     T u[3][PW];
     T rr[3] = {(T)1, (T)1, (T)1};
@@ -1221,7 +1284,7 @@ struct MfLu::Impl {
   DevVec<int2> big_list;          // larger fronts {front, 1: rows outside the pivot block split over the GPU}
   DevVec<int2> frow, brow;        // entries of those rows {front, first row}
   DevVec<int4> aent;              // assembly entries of the larger fronts, two each
-  DevVec<int2> alo;               // per entry and child: the child's rows in the entry's range
+  DevVec<MfPart> parts;           // per entry: the children with rows in its range
   DevVec<MfStep> sent;            // entries of the panel steps
   DevVec<double> dbuf;            // diagonal-block factors, two 32 x 32 slots per larger front of a level
   std::vector<int> tiny_off, tiny_half, big_off;   // fronts up to order 32 at [tiny_off, tiny_half), up to 64 from there
@@ -1363,7 +1426,7 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   // assembly of the larger fronts, ranges of rows and columns (the tiny fronts
   // assemble themselves inside their factor kernel)
   std::vector<int4> ae;
-  std::vector<int2> lo;
+  std::vector<MfPart> parts;
   I.aoff.assign(nl + 1, 0);
   for (int l = 0; l < nl; ++l) {
     I.aoff[l] = (int)ae.size() / 2;
@@ -1371,23 +1434,24 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
       const int t = bl[b], m = P.m[t];
       const int w = std::min(m, kMfAsm / 4), rows = std::min(kMfAsmRows, kMfAsm / w);
       for (int r0 = 0; r0 < m; r0 += rows) {
-        const int off = (int)lo.size();
+        const int off = (int)parts.size();
         for (int c = P.cptr[t]; c < P.cptr[t + 1]; ++c) {
           const int ch = P.clist[c];
           const int* eb = P.emap.data() + P.eptr[ch];
           const int* ee = P.emap.data() + P.eptr[ch + 1];
-          lo.push_back(make_int2((int)(std::lower_bound(eb, ee, r0) - eb), (int)(std::lower_bound(eb, ee, r0 + rows) - eb)));
+          const int x = (int)(std::lower_bound(eb, ee, r0) - eb), y = (int)(std::lower_bound(eb, ee, r0 + rows) - eb);
+          if (x < y) parts.push_back(MfPart{chv[c].src, chv[c].ld, chv[c].nu, chv[c].em, x, y, 0});
         }
         for (int j0 = 0; j0 < m; j0 += w) {
           ae.push_back(make_int4(t, r0, std::min(rows, m - r0), off));
-          ae.push_back(make_int4(j0, std::min(w, m - j0), 0, 0));
+          ae.push_back(make_int4(j0, std::min(w, m - j0), (int)parts.size() - off, 0));
         }
       }
     }
   }
   I.aoff[nl] = (int)ae.size() / 2;
   MFCHK(I.aent.up(ae, st));
-  MFCHK(I.alo.up(lo, st));
+  MFCHK(I.parts.up(parts, st));
   MFCHK(hipStreamSynchronize(st));
   return XG_OK;
 }
@@ -1408,7 +1472,7 @@ static int mf_factor_enqueue(MfLu::Impl& I, const double* vals_dev, int nnz, T* 
   for (int l = 0; l < nl; ++l) {
     const int na = I.aoff[l + 1] - I.aoff[l];
     if (na)
-      hipLaunchKernelGGL(k_mf_assemble<T>, dim3(na), dim3(256), 0, st, d, I.aent.p + 2 * I.aoff[l], I.alo.p, vals_dev, F);
+      hipLaunchKernelGGL(k_mf_assemble<T>, dim3(na), dim3(256), 0, st, d, I.aent.p + 2 * I.aoff[l], I.parts.p, vals_dev, F);
     const int n32 = I.tiny_half[l] - I.tiny_off[l], n64 = I.tiny_off[l + 1] - I.tiny_half[l];
     if (n32)
       hipLaunchKernelGGL((k_mf_factor_tiny<T, kMfTiny / 2>), dim3(n32), dim3(64), 0, st, d, I.tiny_list.p + I.tiny_off[l],
