@@ -1,19 +1,18 @@
 // Multifrontal numeric LU for large systems (power-grid meshes, gate
 // arrays): the factorisation that AmesosSolver::doSolve
 // (src/LinearAlgebraServicesPKG/N_LAS_AmesosSolver.C:216-478) gets from KLU,
-// restructured for the GPU.  The symbolic analysis (maximum transversal,
-// approximate minimum degree, elimination tree) is the one the level-
-// scheduled path uses; here the columns of L are grouped into supernodes,
-// each with a dense frontal matrix, and the elimination tree of supernodes
-// is processed level by level (all fronts of a level in one launch):
+// restructured for the GPU.  The symbolic analysis (mf_analyse: maximum
+// transversal, the cheapest of minimum degree and nested dissection, a tree of
+// supernodes merged where that adds few zeros) gives each supernode a dense
+// frontal matrix; the tree is processed level by level (all fronts of a level in
+// the same launches):
 //
-//   assemble  F_s = A entries of s's columns + extend-add of the children's
-//             Schur complements (the j-th children of a level in launch j,
-//             rows split over workgroups: a fixed order)
+//   assemble  F_s = A entries of s's rows and columns + extend-add of the
+//             children's Schur complements, in LDS, in a fixed order
 //   factor    dense LU of the pivot block, L21, U12 and the Schur complement
-//             F22 -= L21 U12; small fronts one workgroup each, large fronts
-//             blocked by 32-column panels (diagonal block in LDS, row-parallel
-//             triangular solves for L21 and U12, tiled update over the GPU)
+//             F22 -= L21 U12; fronts of order <= 64 by one wavefront each (with
+//             their assembly), larger ones by 32-column panels, one launch per
+//             panel that updates by the panel before and factors its own
 //
 // Static pivots, as in the level-scheduled path, with KLU's threshold test
 // (|l_ij| <= 1/0.001, finite nonzero pivots) on every column.
