@@ -174,7 +174,6 @@ struct MfChild {
   int em, vsrc;                 // parent positions of its rows; their slots in the front vectors
 };
 struct MfDev {
-  const int* sfirst; const int* m; const long long* fo;
   const MfFront* front; const MfChild* child; const int* emap;
   const int* bidx; const int* xidx;      // of the fronts' rows: index into b, into x
   const int* arow; const int* acol; const int* aslot;
@@ -1273,8 +1272,7 @@ struct MfLu::Impl {
     for (auto& g : graphs)
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
   }
-  DevVec<int> sfirst, m, emap, bidx, xidx, bad, arow, acol, aslot;
-  DevVec<long long> fo;
+  DevVec<int> emap, bidx, xidx, bad, arow, acol, aslot;
   DevVec<MfFront> front;
   DevVec<MfChild> child;
   DevVec<double> F64, V64;
@@ -1294,7 +1292,7 @@ struct MfLu::Impl {
   std::vector<std::vector<Step>> steps;   // per level: its panel steps
   MfDev dev() const {
     MfDev d;
-    d.sfirst = sfirst.p; d.m = m.p; d.fo = fo.p; d.emap = emap.p; d.bidx = bidx.p; d.xidx = xidx.p;
+    d.emap = emap.p; d.bidx = bidx.p; d.xidx = xidx.p;
     d.front = front.p; d.child = child.p; d.arow = arow.p; d.acol = acol.p; d.aslot = aslot.p;
     return d;
   }
@@ -1336,7 +1334,7 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
   hipStream_t st = I.st;
   MFCHK(I.front.up(fr, st)); MFCHK(I.child.up(chv, st));
   MFCHK(I.arow.up(P.arow, st)); MFCHK(I.acol.up(P.acol, st)); MFCHK(I.aslot.up(P.aslot, st));
-  MFCHK(I.sfirst.up(P.sfirst, st)); MFCHK(I.m.up(P.m, st)); MFCHK(I.emap.up(P.emap, st)); MFCHK(I.fo.up(P.fo, st));
+  MFCHK(I.emap.up(P.emap, st));
   std::vector<int> bi(P.idx.size()), xi(P.idx.size());
   for (size_t q = 0; q < P.idx.size(); ++q) { bi[q] = s.perm_row[P.idx[q]]; xi[q] = s.perm_col[P.idx[q]]; }
   MFCHK(I.bidx.up(bi, st)); MFCHK(I.xidx.up(xi, st));
