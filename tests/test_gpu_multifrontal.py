@@ -275,3 +275,19 @@ def test_level_factors_in_lds_and_beyond(gpu, name, fp32):
     assert st != 0 and not x.any()
     st, x = s.solve(b)
     assert st == 0 and np.max(np.abs(A @ x - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("form", ["one", "diagonal", "path", "expander"])
+@pytest.mark.parametrize("k", [500, 700, 1000])
+def test_values_and_right_hand_side_far_from_one(gpu, form, k):
+    """A and b scaled by the same power of two: the solution's bits stay, although
+    the product of a pivot and an entry of b is beyond the largest double."""
+    A = _pattern(form)
+    A.sum_duplicates(); A.sort_indices()
+    n = A.shape[0]
+    b = np.random.default_rng(19).normal(size=n)
+    s = X.DirectSolver(n, A.indptr, A.indices, method=2)
+    st, x = s.doSolve(A.data, b)
+    assert st == 0
+    st, y = s.doSolve(np.ldexp(A.data, k), np.ldexp(b, k))
+    assert st == 0 and np.array_equal(x, y)

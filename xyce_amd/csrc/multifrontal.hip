@@ -952,10 +952,11 @@ __global__ void __launch_bounds__(64) k_mf_fwd_tiny(MfDev d, const int* list, co
 #pragma unroll
     for (int q = 0; q < 16; ++q) l[q] = row[min(k0 + q, np - 1)];
     __builtin_amdgcn_sched_barrier(0);
-    // (coefficients of no effect set to zero off the chain of steps)
+    // (coefficients of no effect set to zero off the chain of steps; those of the
+    // lanes past the front too, whose values every other lane gets times zero)
 #pragma unroll
     for (int q = 0; q < 16; ++q)
-      if (!(k0 + q < np && t > k0 + q)) l[q] = (T)0;
+      if (!(k0 + q < np && t > k0 + q && t < ms)) l[q] = (T)0;
 #pragma unroll
     for (int q = 0; q < 16; ++q) v -= l[q] * mf_bcast(v, k0 + q);
   }
