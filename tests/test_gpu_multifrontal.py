@@ -291,3 +291,35 @@ def test_values_and_right_hand_side_far_from_one(gpu, form, k):
     assert st == 0
     st, y = s.doSolve(np.ldexp(A.data, k), np.ldexp(b, k))
     assert st == 0 and np.array_equal(x, y)
+
+
+def _zero_diagonal_path(n):
+    """A chain whose every 7th diagonal entry is stored and zero: regular
+    (condition number 11 at 400), with pivots that are zero or not by the order."""
+    A = sp.csr_matrix(sp.diags([np.full(n, 4.0), np.full(n - 1, -1.0), np.full(n - 1, 1.0)], [0, 1, -1]))
+    A.sort_indices()
+    d = A.data.copy()
+    for i in range(3, n, 7):
+        r = slice(A.indptr[i], A.indptr[i + 1])
+        d[r][A.indices[r] == i] = 0.0
+    return A, d
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("n", [150, 300, 400, 1500])
+def test_zero_pivot_of_one_order_is_no_singular_matrix(gpu, n, fp32):
+    A, d = _zero_diagonal_path(n)
+    B = sp.csr_matrix((d, A.indices, A.indptr), shape=A.shape)
+    b = np.random.default_rng(20).normal(size=n)
+    s = X.DirectSolver(n, A.indptr, A.indices, method=2)
+    if fp32:
+        s.set_precision(1, ir_tol=1e-12, ir_max=10)
+    for v in (A.data, d, A.data, 2.0 * d):      # the order that was found is kept and serves others too
+        M = sp.csr_matrix((v, A.indices, A.indptr), shape=A.shape)
+        assert s.numeric(v) == 0
+        st, x = s.solve(b)
+        assert st == 0 and np.max(np.abs(M @ x - b)) <= 1e-12 * np.max(np.abs(b))
+    assert s.numeric(np.zeros_like(d)) > 0      # singular in every order
+    assert s.numeric(d) == 0
+    st, x = s.solve(b)
+    assert st == 0 and np.max(np.abs(B @ x - b)) <= 1e-12 * np.max(np.abs(b))

@@ -862,6 +862,7 @@ struct xg_lu {
   bool have64 = false;    // FP64 factors of the current values exist (refinement fallback)
   bool soft64 = false;    // those factors have multipliers beyond KLU's threshold: solves refine
   bool repivot_futile = false;  // a re-pivot left threshold failures: keep such factors at once
+  bool min_degree = false;      // multifrontal: a re-pivot in the order of its own choice met a zero pivot
   double stats[6] = {0, 0, 0, 0, 0, 0};  // last solve: refinements, rel. residual; totals: solves, refinements, fallbacks, FP32 pivot failures
   // method: 1 = level-scheduled entry LU (small systems), 2 = multifrontal
   int method = 1;
@@ -903,7 +904,7 @@ struct xg_lu {
     const int n = (int)a_rowptr.size() - 1;
     LuSymbolic t;
     int m = want_method ? want_method : n <= kLevelMaxN ? 1 : 2;
-    int st = m == 2 ? mf_analyse(n, a_rowptr.data(), a_colind.data(), values, t)
+    int st = m == 2 ? mf_analyse(n, a_rowptr.data(), a_colind.data(), values, t, min_degree)
                     : lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
     if (st != XG_OK) return st;
     // what the level-scheduled method can hold keeps its no-allocation solve
@@ -1816,21 +1817,27 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
     HIPCHK(hipStreamSynchronize(s));
   }
   const double* hvals = dev ? hv.data() : vals;
-  try {
-    if (lu->analyse(hvals, lu->method) != XG_OK) return bad;
-  } catch (...) {
-    return bad;
-  }
-  st = lu->upload();
-  if (st != XG_OK) return st;
-  HIPCHK(hipMemcpyAsync(lu->avals.p, hvals, sizeof(double) * lu->s.nnz_a, hipMemcpyHostToDevice, s));
-  if (lu->mode == 1) {
-    st = lu->factor_any(true, &bad, &hard);
+  for (;;) {
+    try {
+      if (lu->analyse(hvals, lu->method) != XG_OK) return bad;
+    } catch (...) {
+      return bad;
+    }
+    st = lu->upload();
     if (st != XG_OK) return st;
-    if (!bad) return XG_OK;
+    HIPCHK(hipMemcpyAsync(lu->avals.p, hvals, sizeof(double) * lu->s.nnz_a, hipMemcpyHostToDevice, s));
+    if (lu->mode == 1) {
+      st = lu->factor_any(true, &bad, &hard);
+      if (st != XG_OK) return st;
+      if (!bad) return XG_OK;
+    }
+    st = lu_factor64(lu, lu->mode == 1, &bad, &hard);
+    if (st != XG_OK) return st;
+    // a zero pivot in an order that is chosen for the GPU's sake: once more in
+    // minimum degree's, which the handle then keeps
+    if (!(bad && hard) || lu->method != 2 || lu->min_degree) break;
+    lu->min_degree = true;
   }
-  st = lu_factor64(lu, lu->mode == 1, &bad, &hard);
-  if (st != XG_OK) return st;
   if (bad && !hard) lu->repivot_futile = true;  // kept, refined from now on without a re-pivot
   return (bad && hard) ? bad : XG_OK;
 }

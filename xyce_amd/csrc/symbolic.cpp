@@ -121,6 +121,11 @@ std::vector<int> max_transversal(int n, const int* rowptr, const int* colind, co
 
 using Graph = std::vector<std::vector<int>>;
 
+// systems up to this size (the batched engine's classes) are ordered by multiple
+// minimum degree, whose independent sets keep the level schedule shallow; larger
+// ones by approximate minimum degree
+constexpr int kMmdMax = 256;
+
 // Multiple minimum degree on an explicit elimination graph: each round
 // eliminates an independent set of minimum-degree nodes, so a round is one
 // level of the elimination tree.
@@ -567,8 +572,10 @@ SuperTree build_tree(const Graph& g, const std::vector<int>& order0) {
 // and also less fill on large meshes (512 x 512 nodes: 2.6 GFLOP and 19 levels
 // against 5.8 and 34), so minimum degree is tried only on small systems or when a
 // separator is wide for its part (no locality: an expander fills in less
-// under minimum degree).
-int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s) {
+// under minimum degree).  min_degree: the order of the level-scheduled method
+// instead, whatever it costs (pivots that are zero in one order need not be in
+// another).
+int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s, bool min_degree) {
   s = LuSymbolic();
   s.n = n; s.nnz_a = rowptr[n];
   const std::vector<int> match = max_transversal(n, rowptr, colind, values);
@@ -589,24 +596,25 @@ int mf_analyse(int n, const int* rowptr, const int* colind, const double* values
     nd_order(g, sparse_nodes, order, leaf, tag, stamp, lvl, wide);
     return finish(order);
   };
-  auto min_degree = [&] {
+  const int m = (int)sparse_nodes.size();
+  auto least_degree = [&] {
     std::vector<int> order;
     order.reserve(n);
-    amd_order(g, sparse_nodes, order);
+    if (min_degree && m <= kMmdMax) mmd_order(g, sparse_nodes, order);
+    else amd_order(g, sparse_nodes, order);
     return finish(order);
   };
-  const int m = (int)sparse_nodes.size();
   SuperTree best;
   auto consider = [&](SuperTree t) {
     if (!t.order.empty() && (best.order.empty() || t.cost < best.cost)) best = std::move(t);
   };
-  if (m > 64) {
+  if (m > 64 && !min_degree) {
     std::future<SuperTree> coarse;
     if (m > 1024) coarse = std::async(std::launch::async, dissect, 1024, (double*)nullptr);
     consider(dissect(64, &widest));
     if (coarse.valid()) consider(coarse.get());
   }
-  if (best.order.empty() || m <= 8192 || widest > 3.0) consider(min_degree());
+  if (best.order.empty() || m <= 8192 || widest > 3.0) consider(least_degree());
   if (best.order.empty()) return XG_E_SETUP;
   s.dense_tail = (int)dense_nodes.size();
   s.perm_row.resize(n); s.perm_col.resize(n); s.rinv.resize(n); s.pinv.resize(n);
@@ -636,9 +644,7 @@ int lu_analyse(int n, const int* rowptr, const int* colind, const double* values
   split_dense(g, sparse_nodes, dense_nodes);
   std::vector<int> order;
   order.reserve(n);
-  // small systems (the batched engine's classes): multiple minimum degree,
-  // whose independent sets keep the level schedule shallow; larger: AMD
-  if ((int)sparse_nodes.size() <= 256) mmd_order(g, sparse_nodes, order);
+  if ((int)sparse_nodes.size() <= kMmdMax) mmd_order(g, sparse_nodes, order);
   else {
     amd_order(g, sparse_nodes, order);
     // a large system whose minimum-degree elimination tree is a long chain

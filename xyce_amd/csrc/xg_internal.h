@@ -116,8 +116,10 @@ int lu_analyse(int n, const int* rowptr, const int* colind, const double* values
                bool want_schedule = true);
 
 // Analysis for the multifrontal method: permutations and the supernode tree
-// (s.nlu and s.flops are those of the tree's fronts)
-int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s);
+// (s.nlu and s.flops are those of the tree's fronts).  min_degree: in the order
+// of lu_analyse.
+int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s,
+               bool min_degree = false);
 
 // Multifrontal plan of a symbolic analysis (multifrontal.hip)
 struct MfPlan {
