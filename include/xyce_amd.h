@@ -180,9 +180,10 @@ int xg_lu_numeric(xg_lu* lu, const double* vals);
 /* Solve A x = b with the last factors (:396); NaN -> XG_E_NAN, x zeroed.
  * transpose != 0 solves A^T x = b (doSolve(reuse_factors, transpose),
  * N_LAS_Solver.h:95-107; Amesos SetUseTranspose): FP64 factors of the
- * level-scheduled method, which a handle with an automatic method makes when
- * first asked, up to 65535 unknowns and 2e7 flops (XG_E_ARG otherwise; Xyce's
- * transient path does not use it). */
+ * level-scheduled method, up to 65535 unknowns and 2e7 flops (XG_E_ARG
+ * otherwise; Xyce's transient path does not use it).  An automatic handle above
+ * 128 unknowns makes that analysis with its first transpose solve, and those
+ * factors with the first after each refactor. */
 int xg_lu_solve(xg_lu* lu, const double* b, double* x, int transpose);
 /* xg_lu_numeric / xg_lu_solve on device arrays (HIP device memory); same
  * semantics; each call returns when its outputs are complete. */

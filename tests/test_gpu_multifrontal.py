@@ -323,3 +323,44 @@ def test_zero_pivot_of_one_order_is_no_singular_matrix(gpu, n, fp32):
     assert s.numeric(d) == 0
     st, x = s.solve(b)
     assert st == 0 and np.max(np.abs(B @ x - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+def test_transpose_solve_analyses_once(gpu):
+    """An automatic handle's first transpose solve makes the level-scheduled
+    analysis, one for a system it holds; what it can't hold is refused without
+    another analysis from the second call on (a tenth of the time of one)."""
+    def jac(nx, ny):
+        p = X.host_pattern(C.power_grid(nx, ny, seed=1, pad_pitch=16, n_sinks=16))
+        n, rp, ci = p["n"], p["rowptr"], p["colind"]
+        v = np.where(ci == np.repeat(np.arange(n), np.diff(rp)), 9.0, -1.0)
+        return n, rp, ci, v
+
+    def took(f):
+        t = time.perf_counter()
+        f()
+        return time.perf_counter() - t
+
+    n, rp, ci, v = jac(131, 97)                  # more flops than the level-scheduled method takes
+    s = X.DirectSolver(n, rp, ci)
+    assert s.numeric(v) == 0
+    b = np.ones(n)
+
+    def refused():
+        with pytest.raises(X.XgError, match="argument"):
+            s.solve(b, transpose=True)
+
+    first = took(refused)
+    again = min(took(refused) for _ in range(5))
+    print(f"refused after {1e3 * first:.2f} ms, then {1e3 * again:.3f} ms")
+    assert again < 0.1 * first
+    n, rp, ci, v = jac(48, 48)
+    s = X.DirectSolver(n, rp, ci)
+    assert s.numeric(v) == 0
+    b = np.random.default_rng(21).normal(size=n)
+    A = sp.csr_matrix((v, ci, rp), shape=(n, n))
+    for k in (1.0, -2.0):
+        assert s.numeric(k * v) == 0
+        st, x = s.solve(b, transpose=True)
+        assert st == 0 and np.max(np.abs(k * (A.T @ x) - b)) <= 1e-12 * np.max(np.abs(b))
+        st, x = s.solve(b)
+        assert st == 0 and np.max(np.abs(k * (A @ x) - b)) <= 1e-12 * np.max(np.abs(b))

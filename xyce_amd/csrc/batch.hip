@@ -1803,7 +1803,7 @@ int xg_batch_create(int n_inst, const xg_circuit_desc* descs, double tstop, doub
       std::vector<double> guide(hc.nnz, 1.0);
       for (int k = 0; k < hc.nnz; ++k) guide[k] = std::fabs(hc.linF[k]) + std::fabs(hc.linQ[k]) * 1e11 + 1e-3;
       try {
-        if (lu_analyse(hc.n, hc.rowptr.data(), hc.colind.data(), guide.data(), sym, true) != XG_OK) return XG_E_SETUP;
+        if (lu_analyse(hc.n, hc.rowptr.data(), hc.colind.data(), guide.data(), sym) != XG_OK) return XG_E_SETUP;
       } catch (...) {
         return XG_E_SETUP;
       }

@@ -30,7 +30,7 @@ int xg_host_lu_analyse(int n, const int* rowptr, const int* colind, const double
   if (n <= 0 || !rowptr || !colind || !info || !xg::valid_csr(n, rowptr, colind)) return XG_E_ARG;
   xg::LuSymbolic s;
   try {
-    const int st = xg::lu_analyse(n, rowptr, colind, values, s, true);
+    const int st = xg::lu_analyse(n, rowptr, colind, values, s);
     if (st != XG_OK) return st;
   } catch (...) {
     return XG_E_SETUP;

@@ -876,7 +876,7 @@ struct xg_lu {
   // made when a transpose solve first needs them
   int asked = 0;
   xg_lu* tlu = nullptr;
-  bool tlu_current = false;
+  bool tlu_current = false, tlu_refused = false;
 
   ~xg_lu() {
     if (tlu) (void)xg_lu_destroy(tlu);
@@ -884,12 +884,14 @@ struct xg_lu {
     if (hstage) (void)hipHostFree(hstage);
   }
 
-  bool level_fits(const double* values) const {
+  // what the level-scheduled method can hold for a handle with an automatic method
+  static constexpr int kLevelHoldN = 65535, kLevelHoldLu = 1 << 24;
+  static constexpr double kLevelHoldFlops = 2e7;
+  // its analysis, if the system is one of those
+  bool level_analysis(const double* values, LuSymbolic& t) const {
     const int n = (int)a_rowptr.size() - 1;
-    if (n > 65535) return false;
-    LuSymbolic t;
-    return lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, false) == XG_OK && t.flops <= 2e7 &&
-           t.nlu <= (1 << 24);
+    return n <= kLevelHoldN && lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, kLevelHoldFlops) == XG_OK &&
+           t.flops <= kLevelHoldFlops && t.nlu <= kLevelHoldLu;
   }
 
   // symbolic analysis for the chosen (or automatically picked) method.  The
@@ -905,13 +907,13 @@ struct xg_lu {
     LuSymbolic t;
     int m = want_method ? want_method : n <= kLevelMaxN ? 1 : 2;
     int st = m == 2 ? mf_analyse(n, a_rowptr.data(), a_colind.data(), values, t, min_degree)
-                    : lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
+                    : lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t);
     if (st != XG_OK) return st;
     // what the level-scheduled method can hold keeps its no-allocation solve
-    if (want_method == 0 && m == 2 && 4 * (size_t)n + t.srow.size() + 256 > kScratchDoubles && level_fits(values)) {
+    LuSymbolic lv;
+    if (want_method == 0 && m == 2 && 4 * (size_t)n + t.srow.size() + 256 > kScratchDoubles && level_analysis(values, lv)) {
       m = 1;
-      st = lu_analyse(n, a_rowptr.data(), a_colind.data(), values, t, true);
-      if (st != XG_OK) return st;
+      t = std::move(lv);
     }
     s = std::move(t);
     method = m;
@@ -1725,8 +1727,9 @@ int xg_combine_dev(xg_circuit* c, const double* q0, const double* q2, double* rh
 }
 
 // ---------------- LU ----------------
+// ready (may be null): the analysis, of the given method
 static int lu_create(int n, const int* rowptr, const int* colind, const double* values, int method, hipStream_t stream,
-                     xg_lu** out) {
+                     xg_lu** out, LuSymbolic* ready = nullptr) {
   if (n <= 0 || !rowptr || !colind || !out || method < 0 || method > 2) return XG_E_ARG;
   if (!xg::valid_csr(n, rowptr, colind)) return XG_E_ARG;
   int ndev = 0;
@@ -1736,11 +1739,16 @@ static int lu_create(int n, const int* rowptr, const int* colind, const double* 
   lu->a_colind.assign(colind, colind + rowptr[n]);
   lu->s.n = n;
   lu->asked = method;
-  try {
-    int st = lu->analyse(values, method);
-    if (st != XG_OK) return st;
-  } catch (...) {
-    return XG_E_SETUP;
+  if (ready) {
+    lu->s = std::move(*ready);
+    lu->method = method;
+  } else {
+    try {
+      int st = lu->analyse(values, method);
+      if (st != XG_OK) return st;
+    } catch (...) {
+      return XG_E_SETUP;
+    }
   }
   lu->stream = stream;
   if (!stream) {
@@ -1848,20 +1856,30 @@ int xg_lu_numeric_dev(xg_lu* lu, const double* vals) { return lu_numeric_impl(lu
 
 static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, bool dev);
 
-// A^T x = b on a handle that took the multifrontal method by itself: the
-// level-scheduled factors of the current values
-static int lu_solve_transpose_auto(xg_lu* lu, const double* b, double* x, bool dev) {
-  if (!lu->tlu) {
-    try {
-      if (!lu->level_fits(nullptr)) return XG_E_ARG;
-    } catch (...) {
-      return XG_E_SETUP;
+// The level-scheduled handle of a handle that took the multifrontal method by
+// itself, on the same stream: made once, and what it can't hold is refused at once
+// from then on.
+static int lu_level_twin(xg_lu* lu) {
+  if (lu->tlu) return XG_OK;
+  if (lu->tlu_refused) return XG_E_ARG;
+  LuSymbolic t;
+  try {
+    if (!lu->level_analysis(nullptr, t)) {
+      lu->tlu_refused = true;
+      return XG_E_ARG;
     }
-    const int st = xg_lu_symbolic_ex(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 1, &lu->tlu);
-    if (st != XG_OK) return st;
+  } catch (...) {
+    return XG_E_SETUP;
   }
+  return lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 1, lu->stream, &lu->tlu, &t);
+}
+
+// A^T x = b on such a handle: by the level-scheduled factors of the current values
+static int lu_solve_transpose_auto(xg_lu* lu, const double* b, double* x, bool dev) {
+  int st = lu_level_twin(lu);
+  if (st != XG_OK) return st;
   if (!lu->tlu_current) {
-    const int st = lu_numeric_impl(lu->tlu, lu->avals.p, true);
+    st = lu_numeric_impl(lu->tlu, lu->avals.p, true);
     if (st != XG_OK) return st < 0 ? st : XG_E_ARG;
     lu->tlu_current = true;
   }

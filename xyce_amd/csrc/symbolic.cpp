@@ -634,7 +634,7 @@ int mf_analyse(int n, const int* rowptr, const int* colind, const double* values
 }
 
 
-int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s, bool want_schedule) {
+int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s, double schedule_flops) {
   s = LuSymbolic();
   s.n = n; s.nnz_a = rowptr[n];
   std::vector<int> match = max_transversal(n, rowptr, colind, values);  // A'(c,:) = A(match[c],:)
@@ -738,7 +738,7 @@ int lu_analyse(int n, const int* rowptr, const int* colind, const double* values
     for (int k = 0; k < n; ++k) fl += 2.0 * (double)urow[k].size() * (double)urow[k].size() + (double)urow[k].size();
     s.flops = fl;
   }
-  if (!want_schedule) return XG_OK;
+  if (!(s.flops <= schedule_flops)) return XG_OK;
 
   // ---- entry-level factor schedule: target (i,j) += -L(i,k)*U(k,j), k ascending
   std::vector<int> level(s.nlu, 0);

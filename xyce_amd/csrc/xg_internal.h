@@ -1,5 +1,6 @@
 // Internal layout shared by the host setup code and the HIP kernels.
 #pragma once
+#include <cmath>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -100,7 +101,6 @@ struct LuSymbolic {
   std::vector<int> sfirst, sparent, srow_ptr, srow;
 };
 
-// want_schedule: build the entry-level factor / solve schedules
 // A square CSR pattern the symbolic analysis can read: rowptr[0] = 0,
 // non-decreasing, every column index in [0, n).
 inline bool valid_csr(int n, const int* rowptr, const int* colind) {
@@ -112,8 +112,10 @@ inline bool valid_csr(int n, const int* rowptr, const int* colind) {
   return true;
 }
 
+// schedule_flops: the entry-level factor and solve schedules are made up to this
+// many flops of a factorisation
 int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s,
-               bool want_schedule = true);
+               double schedule_flops = HUGE_VAL);
 
 // Analysis for the multifrontal method: permutations and the supernode tree
 // (s.nlu and s.flops are those of the tree's fronts).  min_degree: in the order
