@@ -170,8 +170,9 @@ int xg_lu_destroy(xg_lu* lu);
  * threshold (|l| > 1/0.001), makes it choose new pivots from these values and
  * refactor, as Xyce's KLU re-pivots at every factorisation (repivot_,
  * N_LAS_AmesosSolver.C:87,318); returns >0 (pivot+1) only if the new pivots
- * meet a zero pivot too (a singular matrix; the multifrontal method first
- * tries them in minimum degree's order, which the handle then keeps).  If the new pivots still leave
+ * meet a zero pivot too (a singular matrix).  New pivots that fail either test
+ * are tried in minimum degree's order too by the multifrontal method, and a
+ * handle keeps that order then.  If the new pivots still leave
  * multipliers beyond the threshold, those factors are kept and the solves
  * refine x against A in FP64 while the residual falls (at most ir_max
  * corrections, to ir_tol); from then on the handle keeps such factors

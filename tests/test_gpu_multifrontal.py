@@ -364,3 +364,41 @@ def test_transpose_solve_analyses_once(gpu):
         assert st == 0 and np.max(np.abs(k * (A.T @ x) - b)) <= 1e-12 * np.max(np.abs(b))
         st, x = s.solve(b)
         assert st == 0 and np.max(np.abs(k * (A @ x) - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+def _weak_diagonal(seed, n=160):
+    """Sparse systems (3 entries a row, diagonal 0.3 larger) that are regular
+    (condition number below 1e5), whose multipliers pass KLU's threshold in minimum
+    degree's order and not in the dissection's, also after a re-pivot."""
+    B = sp.random(n, n, density=3.0 / n, random_state=seed, data_rvs=np.random.default_rng(seed).standard_normal)
+    A = sp.csr_matrix(B + 0.3 * sp.eye(n))
+    A.sort_indices()
+    return A
+
+
+@pytest.mark.parametrize("method", [0, 2])
+@pytest.mark.parametrize("seed", [25, 72, 91, 209, 365])
+def test_threshold_failure_of_one_order_keeps_plain_factors(gpu, seed, method):
+    """Plain FP64 factors are found: solves refine nothing, the no-allocation
+    solve is accepted and an automatic handle solves the transpose.  Plain
+    factors' residual is growth * n * eps (growth up to the threshold 1e3)."""
+    import ctypes
+    import torch
+    A = _weak_diagonal(seed)
+    n = A.shape[0]
+    b = np.random.default_rng(22).normal(size=n)
+    s = X.DirectSolver(n, A.indptr, A.indices, method=method)
+    assert s.numeric(A.data) == 0
+    st, x = s.solve(b)
+    assert st == 0 and s.precision_stats()["corrections"] == 0
+    tol = 1e3 * n * 2.0 ** -52 * np.max(np.abs(A).sum(1)) * np.max(np.abs(x))
+    assert np.max(np.abs(A @ x - b)) <= tol
+    bd, xd = torch.from_numpy(b).cuda(), torch.zeros(n, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert X.lib().xg_lu_solve_noalloc(s.h, P(bd), P(xd)) == 0
+    assert np.array_equal(xd.cpu().numpy(), x)
+    if method == 0:
+        st, xt = s.solve(b, transpose=True)
+        assert st == 0
+        assert np.max(np.abs(A.T @ xt - b)) <= 1e3 * n * 2.0 ** -52 * np.max(np.abs(A).sum(0)) * np.max(np.abs(xt))

@@ -862,7 +862,7 @@ struct xg_lu {
   bool have64 = false;    // FP64 factors of the current values exist (refinement fallback)
   bool soft64 = false;    // those factors have multipliers beyond KLU's threshold: solves refine
   bool repivot_futile = false;  // a re-pivot left threshold failures: keep such factors at once
-  bool min_degree = false;      // multifrontal: a re-pivot in the order of its own choice met a zero pivot
+  bool min_degree = false;      // multifrontal: a re-pivot in the order of its own choice failed
   double stats[6] = {0, 0, 0, 0, 0, 0};  // last solve: refinements, rel. residual; totals: solves, refinements, fallbacks, FP32 pivot failures
   // method: 1 = level-scheduled entry LU (small systems), 2 = multifrontal
   int method = 1;
@@ -1841,9 +1841,9 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
     }
     st = lu_factor64(lu, lu->mode == 1, &bad, &hard);
     if (st != XG_OK) return st;
-    // a zero pivot in an order that is chosen for the GPU's sake: once more in
-    // minimum degree's, which the handle then keeps
-    if (!(bad && hard) || lu->method != 2 || lu->min_degree) break;
+    // a zero pivot or a multiplier beyond the threshold in an order that is chosen
+    // for the GPU's sake: once more in minimum degree's, which the handle then keeps
+    if (!bad || lu->method != 2 || lu->min_degree) break;
     lu->min_degree = true;
   }
   if (bad && !hard) lu->repivot_futile = true;  // kept, refined from now on without a re-pivot
