@@ -257,3 +257,36 @@ def test_batch_create_rejects_bad_arguments(tstop, tstep, hmax, rec):
     assert st != -1
     if st == 0:
         L.xg_batch_destroy(h)
+
+
+def test_multifrontal_analysis_without_threads():
+    """Where no thread can be started (a stack limit larger than the address
+    space) the plan is made by the calling thread, the same one."""
+    import resource
+    import subprocess
+    import sys
+    code = """
+import sys, threading
+sys.path.insert(0, %r)
+import xyce_amd as X
+from xyce_amd import circuits as C
+try:
+    threading.Thread(target=int).start()
+    print("threads")
+except RuntimeError:
+    pass
+h = X.host_pattern(C.power_grid(60, 60, seed=1, pad_pitch=16, n_sinks=16))
+print(X.host_mf_plan(h["n"], h["rowptr"], h["colind"]))
+""" % ROOT
+
+    def limit():
+        resource.setrlimit(resource.RLIMIT_STACK, (1 << 38, resource.RLIM_INFINITY))
+        resource.setrlimit(resource.RLIMIT_AS, (1 << 36, 1 << 36))
+
+    if resource.getrlimit(resource.RLIMIT_STACK)[1] not in (-1, resource.RLIM_INFINITY):
+        pytest.skip("stack limit can't be raised")
+    r = subprocess.run([sys.executable, "-c", code], preexec_fn=limit, capture_output=True, text=True,
+                       env=dict(os.environ, OPENBLAS_NUM_THREADS="1", OMP_NUM_THREADS="1"))
+    h = X.host_pattern(C.power_grid(60, 60, seed=1, pad_pitch=16, n_sinks=16))
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.strip() == str(X.host_mf_plan(h["n"], h["rowptr"], h["colind"]))

@@ -20,6 +20,7 @@
 #include <future>
 #include <numeric>
 #include <stdexcept>
+#include <system_error>
 
 #include "xg_internal.h"
 
@@ -610,7 +611,14 @@ int mf_analyse(int n, const int* rowptr, const int* colind, const double* values
   };
   if (m > 64 && !min_degree) {
     std::future<SuperTree> coarse;
-    if (m > 1024) coarse = std::async(std::launch::async, dissect, 1024, (double*)nullptr);
+    if (m > 1024) {
+      try {
+        coarse = std::async(std::launch::async, dissect, 1024, (double*)nullptr);
+      } catch (const std::system_error&) {
+        // no thread to be had: one after the other, in get()
+        coarse = std::async(std::launch::deferred, dissect, 1024, (double*)nullptr);
+      }
+    }
     consider(dissect(64, &widest));
     if (coarse.valid()) consider(coarse.get());
   }
