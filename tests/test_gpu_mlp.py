@@ -75,6 +75,56 @@ def test_grouped_weight_gradients(gpu, width, hidden, rows):
     test_forward_and_gradients_match_oracle(gpu, 128, width, hidden, 64, rows)
 
 
+def _seeded_net(in_dim, width, hidden, out_dim, rows):
+    net = X.MLP(in_dim, width, hidden, out_dim, max_rows=rows, seed=7)
+    rng = np.random.default_rng(11)
+    net.set_params(np.concatenate([v for di, do in net.dims() for v in
+                                   (rng.uniform(-1, 1, di * do) / np.sqrt(di), rng.normal(0, 0.1, do))]))
+    return net
+
+
+@pytest.mark.parametrize("rows", [8192, 8320])
+def test_128_row_tiles_give_the_64_row_tiles_bits(gpu, rows):
+    """512 and 520 tiles of 128 x 64 a layer (65 tile rows: no multiple of the
+    eight XCDs), so forward and activation gradients run on 128-row tiles; the
+    same rows in two calls run on 64-row ones.  Outputs are equal, weight gradients
+    (64-row tiles in both) are sums over the rows of equal terms, FP32: a sum of N
+    terms by steps of 16 is off by about sqrt(N / 16) eps, 1.4e-6 here."""
+    in_dim, width, hidden, out_dim = 128, 512, 2, 512
+    assert width // 64 * (rows // 128) >= 512 and width // 64 * (rows // 256 + 1) < 512
+    net = _seeded_net(in_dim, width, hidden, out_dim, rows)
+    x, t, mask = _data(rows, in_dim, out_dim, 3)
+    xd, td, md = _dev(x, torch.bfloat16), _dev(t), _dev(mask)
+    count = int(mask.sum())
+    y, y2 = (torch.zeros(rows, out_dim, dtype=torch.float32, device="cuda") for _ in range(2))
+    cut = rows // 128 * 64
+    net.forward(xd, y)
+    for r in (slice(0, cut), slice(cut, rows)):
+        net.forward(xd[r], y2[r])
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2)
+    loss, g = net.loss_backward(xd, td, md, count, want_grads=True)
+    parts = [net.loss_backward(xd[r].contiguous(), td[r].contiguous(), md[r].contiguous(), count, want_grads=True)
+             for r in (slice(0, cut), slice(cut, rows))]
+    assert abs(loss - sum(v[0] for v in parts)) <= 1e-12 * loss
+    ref = sum(v[1].astype(np.float64) for v in parts)
+    off = 0
+    for di, do in net.dims():
+        for n in (di * do, do):
+            a, b = g[off: off + n], ref[off: off + n]
+            assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
+            off += n
+
+
+@pytest.mark.parametrize("rows", [64, 320])
+def test_128_row_weight_gradient_tiles(gpu, rows):
+    """560 tiles of 128 x 64 in one launch of weight gradients; as the oracle's."""
+    in_dim, width, hidden, out_dim = 64, 2048, 2, 128
+    tiles = [(di // 64) * (do // 128) for di, do in ((in_dim, width), (width, width), (width, out_dim))]
+    assert sum(tiles) >= 512
+    test_forward_and_gradients_match_oracle(gpu, in_dim, width, hidden, out_dim, rows)
+
+
 def test_adam_step_matches_oracle(gpu):
     in_dim, width, hidden, out_dim, rows = 128, 128, 1, 64, 64
     net = X.MLP(in_dim, width, hidden, out_dim, max_rows=rows, seed=3)
