@@ -257,3 +257,13 @@ def test_host_and_device_loads_agree_on_both_sides_of_the_staging(gpu, stages):
     np.testing.assert_array_equal(j.cpu().numpy(), J)
     assert L.xg_combine_dev(d.h, P(q0d), None, P(r), None) == 0
     np.testing.assert_array_equal(r.cpu().numpy(), rhs0)
+
+
+@pytest.mark.parametrize("stages,copies", [(501, False), (7001, True)])
+def test_each_host_call_on_both_sides_of_the_staging(gpu, stages, copies):
+    """The same comparison with every one of the four host-array calls below, and
+    above, the 32768 doubles that go through the pinned staging."""
+    d = X.DeviceMgr(C.ring(stages, seed=stages, mc_seed=stages))
+    for doubles in (d.n + 2 * (d.nsta + d.nsto), 5 * d.n, 2 * d.nnz, 3 * d.n + d.nnz):
+        assert (doubles > 32768) == copies, doubles
+    test_host_and_device_loads_agree_on_both_sides_of_the_staging(gpu, stages)
