@@ -445,3 +445,28 @@ def test_fp32_elimination_error(gpu):
         e.append(np.linalg.norm(y - x) / np.linalg.norm(x))
     print("mean error", np.mean(e), e)
     assert np.mean(e) <= 9.7e-7
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_front_vector_beyond_lds(gpu, fp32):
+    """One front of order 10920: its vector does not fit LDS beside two triangles
+    in FP64 (10880 does), so the solves keep it in memory.  More than 10 sqrt(n)
+    entries a row make every node a dense one, and the fill is complete."""
+    n, deg = 10920, 1084
+    rng = np.random.default_rng(23)
+    i = np.repeat(np.arange(n), deg // 2)
+    A = sp.coo_matrix((rng.normal(size=i.size), (i, rng.integers(0, n, i.size))), shape=(n, n)).tocsr()
+    A = (A + sp.diags(np.full(n, 3.0 * deg))).tocsr()
+    A.sort_indices()
+    s = X.DirectSolver(n, A.indptr, A.indices, method=2)
+    assert s.info()["supernodes"] == 1
+    if fp32:
+        s.set_precision(1, ir_tol=1e-12, ir_max=10)
+    b = rng.normal(size=n)
+    for k in (1.0, -0.5):
+        assert s.numeric(k * A.data) == 0
+        st, x = s.solve(b)
+        assert st == 0 and np.max(np.abs(k * (A @ x) - b)) <= 1e-12 * np.max(np.abs(b))
+    b[n // 3] = np.inf
+    st, x = s.solve(b)
+    assert st != 0 and not x.any()
