@@ -39,6 +39,17 @@ int mf_plan(const LuSymbolic& s, const int* rowptr, const int* colind, MfPlan& p
   const int n = s.n;
   const int ns = (int)s.sfirst.size() - 1;
   if (ns < 1 || (int)s.sparent.size() != ns || (int)s.srow_ptr.size() != ns + 1 || s.sfirst[ns] != n) return XG_E_SETUP;
+  // every row and column is eliminated once, by one front; with the nesting of the
+  // rows and the place of every entry of A, checked below, the fronts hold all fill
+  if ((int)s.perm_row.size() != n || (int)s.perm_col.size() != n || (int)s.rinv.size() != n || (int)s.pinv.size() != n)
+    return XG_E_SETUP;
+  if (s.sfirst[0] != 0) return XG_E_SETUP;
+  for (int t = 0; t < ns; ++t)
+    if (s.sfirst[t + 1] <= s.sfirst[t]) return XG_E_SETUP;
+  for (int i = 0; i < n; ++i) {
+    const int r = s.perm_row[i], c = s.perm_col[i];
+    if (r < 0 || r >= n || c < 0 || c >= n || s.rinv[r] != i || s.pinv[c] != i) return XG_E_SETUP;
+  }
   p = MfPlan();
   p.n = n;
   p.ns = ns;
@@ -1337,7 +1348,7 @@ int MfLu::setup(const LuSymbolic& s, const int* rowptr, const int* colind, void*
     if (P.m[t] < P.sfirst[t + 1] - P.sfirst[t] || P.sfirst[t + 1] <= P.sfirst[t]) return XG_E_SETUP;
     for (int e = P.eptr[t]; e < P.eptr[t + 1]; ++e) {
       if (P.sparent[t] < 0 || P.emap[e] < 0 || P.emap[e] >= P.m[P.sparent[t]]) return XG_E_SETUP;
-      if (e > P.eptr[t] && P.emap[e] <= P.emap[e - 1]) return XG_E_SETUP;   // assembly bisects the map
+      if (e > P.eptr[t] && P.emap[e] <= P.emap[e - 1]) return XG_E_SETUP;   // the parts below are bisected from it
     }
   }
   std::vector<MfFront> fr(P.ns);
