@@ -172,7 +172,9 @@ int xg_lu_destroy(xg_lu* lu);
  * N_LAS_AmesosSolver.C:87,318); returns >0 (pivot+1) only if the new pivots
  * meet a zero pivot too (a singular matrix).  New pivots that fail either test
  * are tried in minimum degree's order too by the multifrontal method, and a
- * handle keeps that order then.  If the new pivots still leave
+ * handle keeps that order then.  (Pivots up to 2^-1024 count as zero to the
+ * multifrontal method; automatic handles factor values below 1e-290 level-
+ * scheduled if they have to, as far as that method holds the system.)  If the new pivots still leave
  * multipliers beyond the threshold, those factors are kept and the solves
  * refine x against A in FP64 while the residual falls (at most ir_max
  * corrections, to ir_tol); from then on the handle keeps such factors

@@ -470,3 +470,43 @@ def test_front_vector_beyond_lds(gpu, fp32):
     b[n // 3] = np.inf
     st, x = s.solve(b)
     assert st != 0 and not x.any()
+
+
+@pytest.mark.parametrize("form", ["diagonal", "path", "two_parts"])
+def test_values_below_the_normal_range(gpu, form):
+    """Pivots whose reciprocal overflows: an automatic handle solves with the
+    level-scheduled method's divisions (every way of solving, also after ordinary
+    values and back), a multifrontal one returns its pivot status (if they are all
+    below 2^-1024).  Sums carry
+    units of 2^-1074, 5e-15 of the right-hand side here, over a few hundred terms."""
+    import ctypes
+    import torch
+    A = _pattern(form)
+    A.sum_duplicates(); A.sort_indices()
+    n = A.shape[0]
+    b = np.random.default_rng(24).uniform(0.5, 1.0, size=n)
+    tiny, bt = A.data * 1e-309, b * 1e-309
+    s = X.DirectSolver(n, A.indptr, A.indices)
+    assert s.info()["method"] == 2
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+
+    def check(M, y, c):
+        assert np.max(np.abs(M @ (y * 1e9) - c * 1e9)) <= 1e-12 * np.max(np.abs(c * 1e9))
+
+    T = sp.csr_matrix((tiny, A.indices, A.indptr), shape=A.shape)
+    for v, M, c in ((A.data, A, b), (tiny, T, bt), (tiny, T, bt), (A.data, A, b)):
+        assert s.numeric(v) == 0
+        st, x = s.solve(c)
+        assert st == 0
+        check(M, x, c)
+        st, xt = s.solve(c, transpose=True)
+        assert st == 0
+        check(M.T, xt, c)
+        cd, xd = torch.from_numpy(c).cuda(), torch.zeros(n, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        assert X.lib().xg_lu_solve_noalloc(s.h, P(cd), P(xd)) == 0
+        assert np.array_equal(xd.cpu().numpy(), x)
+    m = X.DirectSolver(n, A.indptr, A.indices, method=2)
+    below = 1e-309 * A.diagonal().max() < 2.0 ** -1024      # (two_parts' pivots are about 9e-309)
+    assert (m.numeric(tiny) > 0) == below
+    assert m.numeric(A.data) == 0

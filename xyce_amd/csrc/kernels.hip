@@ -873,10 +873,11 @@ struct xg_lu {
 
   // a handle whose method was picked here (asked 0) also solves A^T x = b where
   // the level-scheduled method can hold the system: from factors of its own,
-  // made when a transpose solve first needs them
+  // made when first needed
   int asked = 0;
   xg_lu* tlu = nullptr;
   bool tlu_current = false, tlu_refused = false;
+  bool by_level = false;        // the current values have such factors only
 
   ~xg_lu() {
     if (tlu) (void)xg_lu_destroy(tlu);
@@ -1792,6 +1793,35 @@ static int lu_factor64(xg_lu* lu, bool fp32_failed, int* bad, int* hard) {
   return XG_OK;
 }
 
+static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev);
+
+// The level-scheduled handle of a handle that took the multifrontal method by
+// itself, on the same stream: made once, and what it can't hold is refused at once
+// from then on.
+static int lu_level_twin(xg_lu* lu) {
+  if (lu->tlu) return XG_OK;
+  if (lu->tlu_refused) return XG_E_ARG;
+  LuSymbolic t;
+  try {
+    if (!lu->level_analysis(nullptr, t)) {
+      lu->tlu_refused = true;
+      return XG_E_ARG;
+    }
+  } catch (...) {
+    return XG_E_SETUP;
+  }
+  return lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 1, lu->stream, &lu->tlu, &t);
+}
+
+// its factors of the current values
+static int lu_level_numeric(xg_lu* lu) {
+  int st = lu_level_twin(lu);
+  if (st != XG_OK || lu->tlu_current) return st;
+  st = lu_numeric_impl(lu->tlu, lu->avals.p, true);
+  lu->tlu_current = st == XG_OK;
+  return st;
+}
+
 static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
   if (!lu || !vals) return XG_E_ARG;
   hipStream_t s = lu->stream;
@@ -1806,7 +1836,7 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
   }
   lu->have64 = false;
   lu->soft64 = false;
-  lu->tlu_current = false;
+  lu->tlu_current = lu->by_level = false;
   int bad = 0, hard = 0, st;
   if (lu->mode == 1) {
     st = lu->factor_any(true, &bad, &hard);
@@ -1847,7 +1877,16 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
     lu->min_degree = true;
   }
   if (bad && !hard) lu->repivot_futile = true;  // kept, refined from now on without a re-pivot
-  return (bad && hard) ? bad : XG_OK;
+  if (!(bad && hard)) return XG_OK;
+  // pivots whose reciprocal overflows are zeros to the fronts and none to the
+  // level-scheduled method, which divides
+  if (lu->asked == 0 && lu->method == 2 &&
+      std::any_of(hvals, hvals + nnz, [](double v) { return v != 0.0 && std::fabs(v) < 1e-290; }) &&
+      lu_level_numeric(lu) == XG_OK) {
+    lu->by_level = true;
+    return XG_OK;
+  }
+  return bad;
 }
 
 int xg_lu_numeric(xg_lu* lu, const double* vals) { return lu_numeric_impl(lu, vals, false); }
@@ -1856,38 +1895,16 @@ int xg_lu_numeric_dev(xg_lu* lu, const double* vals) { return lu_numeric_impl(lu
 
 static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, bool dev);
 
-// The level-scheduled handle of a handle that took the multifrontal method by
-// itself, on the same stream: made once, and what it can't hold is refused at once
-// from then on.
-static int lu_level_twin(xg_lu* lu) {
-  if (lu->tlu) return XG_OK;
-  if (lu->tlu_refused) return XG_E_ARG;
-  LuSymbolic t;
-  try {
-    if (!lu->level_analysis(nullptr, t)) {
-      lu->tlu_refused = true;
-      return XG_E_ARG;
-    }
-  } catch (...) {
-    return XG_E_SETUP;
-  }
-  return lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 1, lu->stream, &lu->tlu, &t);
-}
-
-// A^T x = b on such a handle: by the level-scheduled factors of the current values
+// A^T x = b on a handle that took the multifrontal method by itself
 static int lu_solve_transpose_auto(xg_lu* lu, const double* b, double* x, bool dev) {
-  int st = lu_level_twin(lu);
-  if (st != XG_OK) return st;
-  if (!lu->tlu_current) {
-    st = lu_numeric_impl(lu->tlu, lu->avals.p, true);
-    if (st != XG_OK) return st < 0 ? st : XG_E_ARG;
-    lu->tlu_current = true;
-  }
+  const int st = lu_level_numeric(lu);
+  if (st != XG_OK) return st < 0 ? st : XG_E_ARG;
   return lu_solve_impl(lu->tlu, b, x, 1, dev);
 }
 
 static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, bool dev) {
   if (!lu || !b || !x) return XG_E_ARG;
+  if (lu->by_level && !(transpose && lu->mode == 1)) return lu_solve_impl(lu->tlu, b, x, transpose, dev);
   // transpose solves: the level-scheduled method with plain FP64 factors
   if (transpose && (lu->mode == 1 || !lu->have64 || lu->soft64)) return XG_E_ARG;
   if (transpose && lu->method != 1) return lu->asked == 0 ? lu_solve_transpose_auto(lu, b, x, dev) : XG_E_ARG;
@@ -1946,6 +1963,7 @@ int xg_lu_solve_dev(xg_lu* lu, const double* b, double* x, int transpose) {
 
 int xg_lu_solve_noalloc(xg_lu* lu, const double* b, double* x) {
   if (!lu || !b || !x) return XG_E_ARG;
+  if (lu->by_level) return xg_lu_solve_noalloc(lu->tlu, b, x);
   if (!lu->scratch_work) return XG_E_HIP;
   // FP32 factors, and FP64 factors with multipliers beyond the threshold,
   // are refined against A (and FP32 refinement may refactor in FP64): not a
@@ -2018,7 +2036,7 @@ LuDev lu_dev(xg_lu* lu) { return LuDev{lu->avals.p, lu->b.p, lu->x.p}; }
 int lu_step(xg_lu* lu, int* numeric) {
   *numeric = 0;
   if (lu->method == 2 && lu->mode == 0 && !lu->repivot_futile) {
-    lu->have64 = lu->soft64 = lu->tlu_current = false;
+    lu->have64 = lu->soft64 = lu->tlu_current = lu->by_level = false;
     *lu->nan_flag() = 0;
     int st = lu->mfp->factor_begin(lu->avals.p, lu->s.nnz_a, false);
     if (st != XG_OK) return st;

@@ -479,6 +479,10 @@ __device__ __forceinline__ unsigned mf_abs_high(double v) {
 }
 __device__ __forceinline__ unsigned mf_abs_high(float v) { return __float_as_uint(v) & 0x7fffffffu; }
 
+// pivots up to here have a reciprocal that overflows
+template <class T> constexpr T kMfNoPivot = (T)0x1p-1024;
+template <> constexpr float kMfNoPivot<float> = 0x1p-128f;
+
 // the lowest of the first np columns of factored rows (lane t: row t, t < rows;
 // also in memory, at(k)) with a bad pivot or a multiplier beyond KLU's
 // threshold, or N.  The high words of absolute values order like the values, NaN
@@ -496,13 +500,13 @@ __device__ __forceinline__ int mf_check_rows(const T (&v)[N], int lane, int rows
     top = max(top, lim > k ? h : 0);
     piv = own == k ? h : piv;
   }
-  const bool look = lane < rows && (top >= mf_abs_high((T)1.0e3) || piv == 0 || piv >= mf_abs_high((T)INFINITY));
+  const bool look = lane < rows && (top >= mf_abs_high((T)1.0e3) || piv <= mf_abs_high(kMfNoPivot<T>) || piv >= mf_abs_high((T)INFINITY));
   int first = N;
   if (__any(look) && lane < rows)
     for (int k = min(min(np, N) - 1, lane); k >= 0; --k) {
       const double a = fabs((double)at(k));
       const bool p = lane == k;
-      if (p ? !(a > 0.0) || !isfinite(a) : !(a <= 1.0e3)) { first = k; hard |= p; }
+      if (p ? !(a > (double)kMfNoPivot<T>) || !isfinite(a) : !(a <= 1.0e3)) { first = k; hard |= p; }
     }
   return first;
 }
