@@ -170,15 +170,15 @@ int xg_lu_destroy(xg_lu* lu);
  * threshold (|l| > 1/0.001), makes it choose new pivots from these values and
  * refactor, as Xyce's KLU re-pivots at every factorisation (repivot_,
  * N_LAS_AmesosSolver.C:87,318); returns >0 (pivot+1) only if the new pivots
- * meet a zero pivot too (a singular matrix).  New pivots that fail either test
- * are tried in minimum degree's order too by the multifrontal method, and a
- * handle keeps that order then.  (Pivots up to 2^-1024 count as zero to the
- * multifrontal method; automatic handles factor values below 1e-290 level-
- * scheduled if they have to, as far as that method holds the system.)  If the new pivots still leave
+ * meet a zero pivot too (a singular matrix).  If the new pivots still leave
  * multipliers beyond the threshold, those factors are kept and the solves
  * refine x against A in FP64 while the residual falls (at most ir_max
  * corrections, to ir_tol); from then on the handle keeps such factors
- * without choosing pivots again. */
+ * without choosing pivots again.  The multifrontal method tries new pivots that
+ * fail either test in minimum degree's order too, a second plan for such
+ * values.  Pivots up to 2^-1024 count as zero to it; an automatic handle factors
+ * values below 1e-290 level-scheduled if it has to, as far as that method holds
+ * the system. */
 int xg_lu_numeric(xg_lu* lu, const double* vals);
 /* Solve A x = b with the last factors (:396); NaN -> XG_E_NAN, x zeroed.
  * transpose != 0 solves A^T x = b (doSolve(reuse_factors, transpose),

@@ -510,3 +510,25 @@ def test_values_below_the_normal_range(gpu, form):
     below = 1e-309 * A.diagonal().max() < 2.0 ** -1024      # (two_parts' pivots are about 9e-309)
     assert (m.numeric(tiny) > 0) == below
     assert m.numeric(A.data) == 0
+
+
+def test_second_order_serves_only_its_values(gpu):
+    """Minimum degree's order (49 levels here, 7 in the handle's own) takes the
+    values whose pivots fail in the other; the handle's plan stays, and with FP32
+    factors the corrections are counted in one place."""
+    n = 1500
+    A, d = _zero_diagonal_path(n)
+    b = np.random.default_rng(25).normal(size=n)
+    s = X.DirectSolver(n, A.indptr, A.indices, method=2)
+    s.set_precision(1, ir_tol=1e-12, ir_max=10)
+    assert s.numeric(A.data) == 0
+    levels = s.info()["factor_levels"]
+    solves = 0
+    for v in (d, A.data, d, 3.0 * d, A.data):
+        M = sp.csr_matrix((v, A.indices, A.indptr), shape=A.shape)
+        assert s.numeric(v) == 0
+        st, x = s.solve(b)
+        assert st == 0 and np.max(np.abs(M @ x - b)) <= 1e-12 * np.max(np.abs(b))
+        solves += 1
+        assert s.precision_stats()["solves"] == solves
+        assert s.info()["factor_levels"] == levels

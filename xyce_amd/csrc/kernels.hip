@@ -862,8 +862,9 @@ struct xg_lu {
   bool have64 = false;    // FP64 factors of the current values exist (refinement fallback)
   bool soft64 = false;    // those factors have multipliers beyond KLU's threshold: solves refine
   bool repivot_futile = false;  // a re-pivot left threshold failures: keep such factors at once
-  bool min_degree = false;      // multifrontal: a re-pivot in the order of its own choice failed
-  double stats[6] = {0, 0, 0, 0, 0, 0};  // last solve: refinements, rel. residual; totals: solves, refinements, fallbacks, FP32 pivot failures
+  bool min_degree = false;      // multifrontal in minimum degree's order (another handle's second plan)
+  double own_stats[6] = {0, 0, 0, 0, 0, 0};
+  double* stats = own_stats;    // last solve: refinements, rel. residual; totals: solves, refinements, fallbacks, FP32 pivot failures
   // method: 1 = level-scheduled entry LU (small systems), 2 = multifrontal
   int method = 1;
   std::unique_ptr<MfLu> mfp;
@@ -871,16 +872,22 @@ struct xg_lu {
   // with the handle; null if the lookup failed)
   double* scratch_work = nullptr;
 
-  // a handle whose method was picked here (asked 0) also solves A^T x = b where
-  // the level-scheduled method can hold the system: from factors of its own,
-  // made when first needed
+  // Two more handles of the same system, made when first needed, on this one's
+  // stream:
+  //   md   (multifrontal handles) minimum degree's order, for values whose pivots
+  //        fail in the order that was chosen for the GPU's sake;
+  //   tlu  (handles whose method was picked here: asked 0) the level-scheduled
+  //        method, where it can hold the system: solves A^T x = b, and takes
+  //        pivots whose reciprocal overflows.
+  // by: the one that holds the factors of the current values, if this one doesn't
   int asked = 0;
-  xg_lu* tlu = nullptr;
+  xg_lu *md = nullptr, *tlu = nullptr, *by = nullptr;
+  bool md_last = false;         // md served the last values whose pivots failed here
   bool tlu_current = false, tlu_refused = false;
-  bool by_level = false;        // the current values have such factors only
 
   ~xg_lu() {
     if (tlu) (void)xg_lu_destroy(tlu);
+    if (md) (void)xg_lu_destroy(md);
     if (hflag) (void)hipHostFree(hflag);
     if (hstage) (void)hipHostFree(hstage);
   }
@@ -1793,7 +1800,7 @@ static int lu_factor64(xg_lu* lu, bool fp32_failed, int* bad, int* hard) {
   return XG_OK;
 }
 
-static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev);
+static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev, bool repivot = true);
 
 // The level-scheduled handle of a handle that took the multifrontal method by
 // itself, on the same stream: made once, and what it can't hold is refused at once
@@ -1822,7 +1829,31 @@ static int lu_level_numeric(xg_lu* lu) {
   return st;
 }
 
-static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
+// The factors of the current values in minimum degree's order; vals (may be null
+// once the handle is there): the values on the host, for its analysis.
+static int lu_md_numeric(xg_lu* lu, const double* vals) {
+  const bool first = !lu->md;
+  if (first) {
+    LuSymbolic t;
+    try {
+      const int st = mf_analyse(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), vals, t, true);
+      if (st != XG_OK) return st;
+    } catch (...) {
+      return XG_E_SETUP;
+    }
+    const int st = lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 2, lu->stream, &lu->md, &t);
+    if (st != XG_OK) return st;
+    lu->md->min_degree = true;
+    lu->md->stats = lu->stats;
+  }
+  lu->md->mode = lu->mode;
+  lu->md->ir_tol = lu->ir_tol;
+  lu->md->ir_max = lu->ir_max;
+  return lu_numeric_impl(lu->md, lu->avals.p, true, !first);
+}
+
+// repivot: new pivots if the present ones fail
+static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev, bool repivot) {
   if (!lu || !vals) return XG_E_ARG;
   hipStream_t s = lu->stream;
   const size_t nnz = lu->s.nnz_a;
@@ -1836,7 +1867,8 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
   }
   lu->have64 = false;
   lu->soft64 = false;
-  lu->tlu_current = lu->by_level = false;
+  lu->tlu_current = false;
+  lu->by = nullptr;
   int bad = 0, hard = 0, st;
   if (lu->mode == 1) {
     st = lu->factor_any(true, &bad, &hard);
@@ -1846,6 +1878,12 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
   st = lu_factor64(lu, lu->mode == 1, &bad, &hard);
   if (st != XG_OK) return st;
   if (!bad || (!hard && lu->repivot_futile)) return XG_OK;
+  if (!repivot) return hard ? bad : XG_OK;
+  const bool fronts = lu->method == 2 && !lu->min_degree;
+  if (fronts && lu->md_last && lu_md_numeric(lu, nullptr) == XG_OK && !lu->md->soft64) {
+    lu->by = lu->md;
+    return XG_OK;
+  }
   // a pivot that fails KLU's threshold or is zero (KLU would pivot elsewhere):
   // analyse again steering the transversal by the values, then refactor
   std::vector<double> hv;
@@ -1855,35 +1893,44 @@ static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev) {
     HIPCHK(hipStreamSynchronize(s));
   }
   const double* hvals = dev ? hv.data() : vals;
-  for (;;) {
-    try {
-      if (lu->analyse(hvals, lu->method) != XG_OK) return bad;
-    } catch (...) {
-      return bad;
-    }
-    st = lu->upload();
-    if (st != XG_OK) return st;
-    HIPCHK(hipMemcpyAsync(lu->avals.p, hvals, sizeof(double) * lu->s.nnz_a, hipMemcpyHostToDevice, s));
-    if (lu->mode == 1) {
-      st = lu->factor_any(true, &bad, &hard);
-      if (st != XG_OK) return st;
-      if (!bad) return XG_OK;
-    }
-    st = lu_factor64(lu, lu->mode == 1, &bad, &hard);
-    if (st != XG_OK) return st;
-    // a zero pivot or a multiplier beyond the threshold in an order that is chosen
-    // for the GPU's sake: once more in minimum degree's, which the handle then keeps
-    if (!bad || lu->method != 2 || lu->min_degree) break;
-    lu->min_degree = true;
+  try {
+    if (lu->analyse(hvals, lu->method) != XG_OK) return bad;
+  } catch (...) {
+    return bad;
   }
-  if (bad && !hard) lu->repivot_futile = true;  // kept, refined from now on without a re-pivot
-  if (!(bad && hard)) return XG_OK;
+  st = lu->upload();
+  if (st != XG_OK) return st;
+  HIPCHK(hipMemcpyAsync(lu->avals.p, hvals, sizeof(double) * lu->s.nnz_a, hipMemcpyHostToDevice, s));
+  if (lu->mode == 1) {
+    st = lu->factor_any(true, &bad, &hard);
+    if (st != XG_OK) return st;
+    if (!bad) return XG_OK;
+  }
+  st = lu_factor64(lu, lu->mode == 1, &bad, &hard);
+  if (st != XG_OK) return st;
+  if (!bad) return XG_OK;
+  // A zero pivot or multipliers beyond the threshold in an order that was chosen for
+  // the GPU's sake: minimum degree's, if that serves better, unless no order
+  // could.  For these values only: in that order a refactor and solve of 8000 gates'
+  // time step takes twice as long.
+  if (fronts) {
+    lu->md_last = (!hard || structurally_regular(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), hvals)) &&
+                  lu_md_numeric(lu, hvals) == XG_OK && (hard || !lu->md->soft64);
+    if (lu->md_last) {
+      lu->by = lu->md;
+      return XG_OK;
+    }
+  }
+  if (!hard) {
+    lu->repivot_futile = true;  // kept, refined from now on without a re-pivot
+    return XG_OK;
+  }
   // pivots whose reciprocal overflows are zeros to the fronts and none to the
   // level-scheduled method, which divides
   if (lu->asked == 0 && lu->method == 2 &&
       std::any_of(hvals, hvals + nnz, [](double v) { return v != 0.0 && std::fabs(v) < 1e-290; }) &&
       lu_level_numeric(lu) == XG_OK) {
-    lu->by_level = true;
+    lu->by = lu->tlu;
     return XG_OK;
   }
   return bad;
@@ -1904,9 +1951,10 @@ static int lu_solve_transpose_auto(xg_lu* lu, const double* b, double* x, bool d
 
 static int lu_solve_impl(xg_lu* lu, const double* b, double* x, int transpose, bool dev) {
   if (!lu || !b || !x) return XG_E_ARG;
-  if (lu->by_level && !(transpose && lu->mode == 1)) return lu_solve_impl(lu->tlu, b, x, transpose, dev);
+  const xg_lu* by = lu->by ? lu->by : lu;
   // transpose solves: the level-scheduled method with plain FP64 factors
-  if (transpose && (lu->mode == 1 || !lu->have64 || lu->soft64)) return XG_E_ARG;
+  if (transpose && (lu->mode == 1 || !by->have64 || by->soft64)) return XG_E_ARG;
+  if (!transpose && lu->by) return lu_solve_impl(lu->by, b, x, 0, dev);
   if (transpose && lu->method != 1) return lu->asked == 0 ? lu_solve_transpose_auto(lu, b, x, dev) : XG_E_ARG;
   hipStream_t s = lu->stream;
   const size_t n = lu->s.n;
@@ -1963,7 +2011,7 @@ int xg_lu_solve_dev(xg_lu* lu, const double* b, double* x, int transpose) {
 
 int xg_lu_solve_noalloc(xg_lu* lu, const double* b, double* x) {
   if (!lu || !b || !x) return XG_E_ARG;
-  if (lu->by_level) return xg_lu_solve_noalloc(lu->tlu, b, x);
+  if (lu->by) return xg_lu_solve_noalloc(lu->by, b, x);
   if (!lu->scratch_work) return XG_E_HIP;
   // FP32 factors, and FP64 factors with multipliers beyond the threshold,
   // are refined against A (and FP32 refinement may refactor in FP64): not a
@@ -2036,7 +2084,8 @@ LuDev lu_dev(xg_lu* lu) { return LuDev{lu->avals.p, lu->b.p, lu->x.p}; }
 int lu_step(xg_lu* lu, int* numeric) {
   *numeric = 0;
   if (lu->method == 2 && lu->mode == 0 && !lu->repivot_futile) {
-    lu->have64 = lu->soft64 = lu->tlu_current = lu->by_level = false;
+    lu->have64 = lu->soft64 = lu->tlu_current = false;
+    lu->by = nullptr;
     *lu->nan_flag() = 0;
     int st = lu->mfp->factor_begin(lu->avals.p, lu->s.nnz_a, false);
     if (st != XG_OK) return st;

@@ -642,6 +642,23 @@ int mf_analyse(int n, const int* rowptr, const int* colind, const double* values
 }
 
 
+bool structurally_regular(int n, const int* rowptr, const int* colind, const double* values) {
+  std::vector<int> rp(n + 1, 0), ci;
+  for (int r = 0; r < n; ++r) {
+    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) {
+      if (!std::isfinite(values[k])) return false;
+      if (values[k] != 0.0) ci.push_back(colind[k]);
+    }
+    rp[r + 1] = (int)ci.size();
+  }
+  try {
+    (void)max_transversal(n, rp.data(), ci.data(), nullptr);
+  } catch (const std::runtime_error&) {
+    return false;
+  }
+  return true;
+}
+
 int lu_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s, double schedule_flops) {
   s = LuSymbolic();
   s.n = n; s.nnz_a = rowptr[n];

@@ -123,6 +123,10 @@ int lu_analyse(int n, const int* rowptr, const int* colind, const double* values
 int mf_analyse(int n, const int* rowptr, const int* colind, const double* values, LuSymbolic& s,
                bool min_degree = false);
 
+// Whether the values are finite and those that are not zero hold a transversal:
+// else every pivot order fails.
+bool structurally_regular(int n, const int* rowptr, const int* colind, const double* values);
+
 // Multifrontal plan of a symbolic analysis (multifrontal.hip)
 struct MfPlan {
   int n = 0, ns = 0;
