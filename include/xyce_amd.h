@@ -395,7 +395,9 @@ int xg_batch_pred_counters(xg_batch* b, double* c);
  * kernels.  It proposes the Newton initial guess that
  * OneStep::obtainPredictor (N_TIA_OneStep.C:135) computes by polynomial
  * extrapolation; the polynomial predictor stays the fallback.  All
- * dimensions and row counts are multiples of 64.  Pointers named *_dev are
+ * dimensions and row counts are multiples of 64.  Device memory: 8 bytes per
+ * hidden layer, row and unit (pre-activations, activations, their gradients),
+ * 18 per parameter and 6 per row and output.  Pointers named *_dev are
  * device pointers; bf16 values are passed as their uint16 bit patterns. */
 int xg_mlp_create(int in_dim, int width, int hidden_layers, int out_dim, int max_rows, unsigned long long seed,
                   xg_mlp** out);

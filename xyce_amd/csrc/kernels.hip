@@ -502,12 +502,15 @@ __global__ void __launch_bounds__(1024) k_lu_solve_1wg(int n, const int* __restr
 // arrays: 197 us with the kernels above, which larger systems keep, 72 here, of
 // which 46 are the two calls' launches and waits (7 unknowns).
 constexpr int kLuSmall = 512;             // threads
+// (refactor and solve of a ring of 103 unknowns: 70 us with 8, 24 or 64 here, 96 if
+// no sum is shared; gate arrays of 66 and 124: 109 and 154 us with 24, 122 and 158
+// with 64, 111 and 166 if none is, 100 and 136 with 8)
 constexpr int kLuLong = 24;
 constexpr size_t kLuSmallLds = 65024;     // (beside 16 bytes of static LDS)
 
 struct LuSmall {
   int n, nlu, nnz_a;
-  const unsigned* prog;                   // packed program (LuProgram::pack)
+  const unsigned* prog;                   // packed program (xg_lu::pack_small)
   int words_f, words_s;                   // its factor and its solve part
   int nlev, nops, nfl, nbl;
 };
@@ -850,7 +853,9 @@ struct xg_lu {
   // systems), a non-finite solution, a failed pivot (other level systems)
   int* hflag = nullptr;
   int* nan_flag() const { return hflag + 2; }
-  // pinned staging of small host arrays, read and written by the kernels
+  // pinned staging of small host arrays, read and written by the kernels.  The line
+  // bounds the pinned memory of a handle (256 KiB), not the gain: a solve of 1604
+  // unknowns takes 110 us through it and 130 with copies, of 12716 220 and 235.
   double* hstage = nullptr;
   bool staged = false;          // the next factorisation reads its values there and keeps them
   static constexpr size_t kStage = 32768;
@@ -1289,7 +1294,10 @@ struct xg_circuit {
   }
   // vectors up to this many doubles in all go through the staging: the kernels
   // read and write it directly, which costs them a few microseconds where every
-  // copy costs about ten (ring of 101 stages, one load: 268 -> 106 us)
+  // copy costs about ten (ring of 101 stages, one load: 268 -> 106 us).  The line
+  // bounds the pinned memory of a circuit (256 KiB), not the gain: above it a state
+  // update of 59061 doubles takes 142 us with copies (49 through a staging that
+  // large), vectors of 35015 doubles 85 (44).
   static constexpr size_t kStageDirect = 32768;
   hipError_t stage(size_t cnt) {
     if (cnt <= hstage_n) return hipSuccess;

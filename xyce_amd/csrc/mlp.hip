@@ -546,6 +546,7 @@ int xg_mlp_create(int in_dim, int width, int hidden_layers, int out_dim, int max
   HIPCHK(net->wb.alloc(off));
   HIPCHK(net->Zall.alloc((size_t)hidden_layers * max_rows * width));
   HIPCHK(net->Hall.alloc((size_t)hidden_layers * max_rows * width));
+  // (a layer's each: the weight gradients of all layers are formed together)
   HIPCHK(net->dH.alloc((size_t)hidden_layers * max_rows * width));
   HIPCHK(net->dY.alloc((size_t)max_rows * out_dim));
   HIPCHK(net->Y.alloc((size_t)max_rows * out_dim));

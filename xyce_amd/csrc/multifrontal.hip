@@ -296,9 +296,9 @@ __device__ __forceinline__ void mf_sub_sums(T* x, int r, int nr, int lane, const
 // complement.  The chain of panels is what bounds a tree's top: one launch per
 // panel instead of a panel and an update launch, and no operand passes through
 // LDS on its way to the matrix cores, so that a step is one round of loads, the
-// diagonal's 32 dependent pivots and a substitution (12.2 us where the two
+// diagonal's 32 dependent pivots and a substitution (12.4 us where the two
 // launches took 31.6, on the 865-order root of a 512 x 512 grid, of which the 32
-// pivots take 4.1; mean over all its steps 12.9, 14.2 with the loads of C and L
+// pivots take 4.3; mean over all its steps 13.2, 14.4 with the loads of C and L
 // waited for before U's and the substitution's rows read one ahead).
 //
 // v_mfma_{f64,f32}_16x16x4: lane l holds A's row l % 16, column l / 16 of the
@@ -529,7 +529,7 @@ __device__ __forceinline__ void mf_wave_fence() {
 // with a supply row has many others), their positions loaded one part ahead; a
 // child's rows map to increasing parent rows.  Per part and 256 columns a wavefront
 // issues the loads of up to four rows at once; a part is a round trip, which bounds
-// fronts of many children (512 x 512 grid, all levels: 243 us with A's entries in,
+// fronts of many children (512 x 512 grid, all levels: 242 us with A's entries in,
 // where clearing the fronts, scattering A and adding the children in memory took
 // 400; roots of a 2000-gate array 42 us).
 constexpr int kMfAsmRows = 16;
@@ -646,7 +646,7 @@ __global__ void __launch_bounds__(256) k_mf_assemble(MfDev d, const int4* ent, c
 // and the children's updates are added in LDS (row stride N + 1), one child
 // after another; then lane t holds row t in registers and the pivot rows are
 // broadcast from there: a pivot costs its reciprocal and the row updates, no
-// LDS traffic (512 x 512 grid, all levels: 295 us, 656 with the elimination in LDS).
+// LDS traffic (512 x 512 grid, all levels: 297 us, 656 with the elimination in LDS).
 template <class T, int N>
 __global__ void __launch_bounds__(64) k_mf_factor_tiny(MfDev d, const int* list, const double* vals, T* F, int* bad, int* fail) {
   constexpr int ld = N + 1;

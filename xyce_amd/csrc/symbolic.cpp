@@ -412,8 +412,14 @@ struct SuperTree {
 // tree level a chain of launches, which a few padded entries do not.
 constexpr int kMergeOrder = 32;
 constexpr double kMergeFill = 0.1;
-// cost model (us): a tree level's launches in refactor and solve, a 32-column
-// panel step, a GFLOP, a million front elements
+// cost model (us) of a refactor and a solve: a tree level's launches, a 32-column
+// panel step, a GFLOP, a million front elements.  It only has to rank: with the
+// kernels as they are, its figure is 0.9 to 1.6 times the measured time (grid of
+// 131 x 97: 803 and 783, 60k gates: 1739 and 1712, ring of 501: 160 and 120), and
+// of 15 rings, meshes and gate arrays of 200 to 160k unknowns it takes the fastest
+// of the three candidates in 14 (a gate array of 187 unknowns: 155 us, minimum
+// degree 119); the next best are 1 to 70 % slower (131 x 97: 783, 895 and 1071 us; 10k
+// gates: 1033, 1526 and 2604).
 constexpr double kCostLevel = 40.0, kCostStep = 14.0, kCostGflop = 350.0, kCostMelem = 12.0;
 constexpr int kSmallFront = 64;      // orders up to this are factored by one wavefront
 
@@ -570,8 +576,8 @@ SuperTree build_tree(const Graph& g, const std::vector<int>& order0) {
 // The order is the one whose tree the GPU is expected to factor and solve
 // soonest: nested dissection down to 64 or to 1024 nodes, or minimum degree.
 // On meshes and locally wired gate arrays dissection has the shallower tree
-// and also less fill on large meshes (512 x 512 nodes: 2.6 GFLOP and 19 levels
-// against 5.8 and 34), so minimum degree is tried only on small systems or when a
+// and also less fill on large meshes (512 x 512 nodes: 3.1 GFLOP and 19 levels
+// against 6.9 and 31), so minimum degree is tried only on small systems or when a
 // separator is wide for its part (no locality: an expander fills in less
 // under minimum degree).  min_degree: the order of the level-scheduled method
 // instead, whatever it costs (pivots that are zero in one order need not be in
