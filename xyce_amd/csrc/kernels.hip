@@ -1810,6 +1810,14 @@ static int lu_factor64(xg_lu* lu, bool fp32_failed, int* bad, int* hard) {
 
 static int lu_numeric_impl(xg_lu* lu, const double* vals, bool dev, bool repivot = true);
 
+// a second handle of lu's system on its stream, from a finished analysis; one that
+// does not fit the device's memory leaves no error behind for later launches
+static int lu_create_beside(xg_lu* lu, int method, xg_lu** out, LuSymbolic* ready) {
+  const int st = lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, method, lu->stream, out, ready);
+  if (st != XG_OK) (void)hipGetLastError();
+  return st;
+}
+
 // The level-scheduled handle of a handle that took the multifrontal method by
 // itself, on the same stream: made once, and what it can't hold is refused at once
 // from then on.
@@ -1825,7 +1833,7 @@ static int lu_level_twin(xg_lu* lu) {
   } catch (...) {
     return XG_E_SETUP;
   }
-  return lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 1, lu->stream, &lu->tlu, &t);
+  return lu_create_beside(lu, 1, &lu->tlu, &t);
 }
 
 // its factors of the current values
@@ -1849,7 +1857,7 @@ static int lu_md_numeric(xg_lu* lu, const double* vals) {
     } catch (...) {
       return XG_E_SETUP;
     }
-    const int st = lu_create(lu->s.n, lu->a_rowptr.data(), lu->a_colind.data(), nullptr, 2, lu->stream, &lu->md, &t);
+    const int st = lu_create_beside(lu, 2, &lu->md, &t);
     if (st != XG_OK) return st;
     lu->md->min_degree = true;
     lu->md->stats = lu->stats;

@@ -649,18 +649,18 @@ int mf_analyse(int n, const int* rowptr, const int* colind, const double* values
 
 
 bool structurally_regular(int n, const int* rowptr, const int* colind, const double* values) {
-  std::vector<int> rp(n + 1, 0), ci;
-  for (int r = 0; r < n; ++r) {
-    for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) {
-      if (!std::isfinite(values[k])) return false;
-      if (values[k] != 0.0) ci.push_back(colind[k]);
-    }
-    rp[r + 1] = (int)ci.size();
-  }
   try {
+    std::vector<int> rp(n + 1, 0), ci;
+    for (int r = 0; r < n; ++r) {
+      for (int k = rowptr[r]; k < rowptr[r + 1]; ++k) {
+        if (!std::isfinite(values[k])) return false;
+        if (values[k] != 0.0) ci.push_back(colind[k]);
+      }
+      rp[r + 1] = (int)ci.size();
+    }
     (void)max_transversal(n, rp.data(), ci.data(), nullptr);
-  } catch (const std::runtime_error&) {
-    return false;
+  } catch (const std::exception&) {
+    return false;         // (none found, or no memory to look for one)
   }
   return true;
 }
